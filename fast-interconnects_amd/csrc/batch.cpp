@@ -68,7 +68,7 @@ struct ClassArena {
   std::vector<void*> allocs;
   PipelineDevice d{};
   HistParams* hist = nullptr;      // [2 * joins]
-  BatchScanJob* scan = nullptr;    // [2 * joins]
+  OffsetsScan* scan = nullptr;    // [2 * joins]
   ScatterParams* scat = nullptr;   // [2 * joins]
   BatchSide* sides = nullptr;      // [2 * joins]
   uint32_t* prefix = nullptr;      // [2 * joins + 1] first chunk of each join side
@@ -76,6 +76,7 @@ struct ClassArena {
   uint32_t* side_tiles = nullptr;  // [2 * joins] plan scratch: tiles of each join side
   uint32_t* counts = nullptr;      // per-chunk histograms of every join side
   uint64_t* local = nullptr;       // per-chunk write offsets of every join side
+  uint64_t* scan_state = nullptr;  // look-back state of every join side's offsets scan
   // capacities
   uint64_t joins = 0, rel1[2] = {0, 0}, rel2[2] = {0, 0}, tiles[2] = {0, 0}, chunk_words = 0, units = 0;
   // this submission: joins, chunks of all join sides, pass-2 tiles per side
@@ -142,15 +143,9 @@ hipError_t arena_alloc(ClassArena& a, T** out, uint64_t count) {
 }
 
 // Chunks of a batched join side: about 32768 tuples each, at most one per
-// compute unit, and never a chunk length that leaves the last chunk empty.
-uint32_t side_chunks(fij_type type, uint64_t n, uint32_t cus) {
-  uint32_t g = static_cast<uint32_t>(std::min<uint64_t>(cus, std::max<uint64_t>(1, (n + 32767) / 32768)));
-  auto fits = [&](uint32_t chunks) {
-    uint64_t c = 0;
-    return fij_input_chunk_size(type, n, chunks, &c) == FIJ_OK && c * (chunks - 1) <= n;
-  };
-  while (g > 1 && !fits(g)) --g;
-  return g;
+// compute unit.
+uint32_t side_chunks(KeyType kt, uint64_t n, uint32_t cus) {
+  return pass1_chunks(kt, n, static_cast<uint32_t>(std::min<uint64_t>(cus, std::max<uint64_t>(1, (n + 32767) / 32768))));
 }
 
 // Grows the class arena to hold `joins` joins with these totals; every
@@ -197,6 +192,7 @@ fij_status grow_arena(ClassArena& a, KeyType kt, uint32_t b1, uint32_t b2, uint6
   }
   if (e == hipSuccess) e = arena_alloc(n, &n.counts, n.chunk_words);
   if (e == hipSuccess) e = arena_alloc(n, &n.local, n.chunk_words);
+  if (e == hipSuccess) e = arena_alloc(n, &n.scan_state, 2 * n.joins * scan_state_words(F1));
   if (e == hipSuccess) e = arena_alloc(n, &d.work_counter, kJoinCounterWords);
   if (e == hipSuccess) e = arena_alloc(n, &d.overflow, parts * F2);
   if (e == hipSuccess) e = arena_alloc(n, &d.units, n.units);
@@ -227,7 +223,6 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
                          double* grow_ms) {
   const uint32_t b1 = ck.b1, b2 = ck.b2;
   const KeyType kt = b->kt;
-  const fij_type type = static_cast<fij_type>(b->cfg.type);
   const uint32_t F1 = 1u << b1, F2 = 1u << b2;
   const uint32_t pad = pad_tuples(kt);
   const uint32_t L = 128 / tuple_bytes(kt);
@@ -241,7 +236,7 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
     for (int s = 0; s < 2; ++s) {
       SideLayout& l = lay[2 * j + s];
       l.n = s ? jd.probe_len : jd.build_len;
-      l.chunks = side_chunks(type, l.n, b->cus);
+      l.chunks = side_chunks(kt, l.n, b->cus);
       l.counts_at = words;
       l.local_at = words;
       words += static_cast<uint64_t>(F1) * l.chunks;
@@ -264,12 +259,12 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
   *grow_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_grow).count();
   if (s != FIJ_OK) return s;
   // descriptors
-  const size_t n_hist = 2ull * J * sizeof(HistParams), n_scan = 2ull * J * sizeof(BatchScanJob),
+  const size_t n_hist = 2ull * J * sizeof(HistParams), n_scan = 2ull * J * sizeof(OffsetsScan),
                n_scat = 2ull * J * sizeof(ScatterParams), n_side = 2ull * J * sizeof(BatchSide),
                n_pre = (2ull * J + 1) * 4, n_slot = static_cast<size_t>(J) * 4;
   host.assign(n_hist + n_scan + n_scat + n_side + n_pre + n_slot, 0);
   HistParams* hh = reinterpret_cast<HistParams*>(host.data());
-  BatchScanJob* hs = reinterpret_cast<BatchScanJob*>(host.data() + n_hist);
+  OffsetsScan* hs = reinterpret_cast<OffsetsScan*>(host.data() + n_hist);
   ScatterParams* hc = reinterpret_cast<ScatterParams*>(host.data() + n_hist + n_scan);
   BatchSide* hb = reinterpret_cast<BatchSide*>(host.data() + n_hist + n_scan + n_scat);
   uint32_t* hp = reinterpret_cast<uint32_t*>(host.data() + n_hist + n_scan + n_scat + n_side);
@@ -285,9 +280,10 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
       PipelineSide& ps = side ? a.d.probe : a.d.build;
       const void* keys = side ? jd.probe_keys : jd.build_keys;
       const void* pays = side ? jd.probe_payloads : jd.build_payloads;
-      hh[js] = hist_params(kt, keys, l.n, l.chunks, b1, ck.block, a.counts + l.counts_at);
-      hs[js] = BatchScanJob{a.counts + l.counts_at, a.local + l.local_at, ps.off1 + static_cast<uint64_t>(j) * F1,
-                            l.rel1_at, F1, l.chunks, pad};
+      uint64_t* state = a.scan_state + js * scan_state_words(F1);
+      hh[js] = hist_params(kt, keys, l.n, l.chunks, b1, ck.block, a.counts + l.counts_at, state);
+      hs[js] = OffsetsScan{a.counts + l.counts_at, a.local + l.local_at, ps.off1 + static_cast<uint64_t>(j) * F1,
+                           state, l.rel1_at, F1, l.chunks, pad, 0};
       void* region = static_cast<uint8_t*>(ps.rel1) + l.rel1_at * tb;
       const hipError_t e = scatter_params_batched(kt, keys, pays, l.n, l.chunks, b1, a.local + l.local_at, region,
                                                   lds_total, ck.block, ck.ring, &hc[js]);
@@ -339,7 +335,7 @@ hipError_t launch_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, hi
   const uint32_t js = 2 * a.sub_joins;
   hipError_t e;
   if ((e = launch_hist_batched(kt, a.hist, a.prefix, js, a.sub_blocks, b1, ck.block, st)) != hipSuccess) return e;
-  if ((e = launch_offsets_batched(a.scan, js, st)) != hipSuccess) return e;
+  if ((e = launch_offsets_batched(a.scan, js, 1u << b1, st)) != hipSuccess) return e;
   if ((e = launch_partition_batched(kt, a.scat, a.prefix, js, a.sub_blocks, b1, lds_total, ck.block, ck.ring, st)) !=
       hipSuccess)
     return e;
@@ -713,7 +709,8 @@ fij_status fij_join_batch_device_bytes(const fij_join_batch* b, uint64_t* bytes)
     for (int s = 0; s < 2; ++s)
       total += (a.rel1[s] + a.rel2[s]) * tb + parts * (8 + 4 + 8 + 4) + (a.tiles[s] + 1) * F2 * 4;
     total += a.chunk_words * (4 + 8) + parts * F2 + a.units * 16 +
-             a.joins * 2 * (sizeof(HistParams) + sizeof(BatchScanJob) + sizeof(ScatterParams) + sizeof(BatchSide) + 4);
+             a.joins * 2 * (sizeof(HistParams) + sizeof(OffsetsScan) + sizeof(ScatterParams) + sizeof(BatchSide) + 4 +
+                            8 * scan_state_words(1ull << kv.first.b1));
   }
   *bytes = total;
   return FIJ_OK;

@@ -147,7 +147,7 @@ namespace {
 // stream first so that no in-flight kernel still uses the old buffers.
 fij_status ensure_scan_state(fij_partitioner* p, uint32_t fanout, hipStream_t stream) {
   const uint64_t n = static_cast<uint64_t>(fanout) * p->grid;
-  const uint64_t words = scan_state_words(n);
+  const uint64_t words = scan_state_words(fanout);
   if (n > p->counts_cap || words > p->scan_cap) FIJ_HIP(hipStreamSynchronize(stream));
   if (n > p->counts_cap) {
     if (p->counts) FIJ_HIP(hipFree(p->counts));
@@ -354,6 +354,13 @@ fij_status fij_partitioner_destroy(fij_partitioner* p) {
 
 namespace {
 
+// The contiguous prefix sum's scan of counts[grid][F] into the offsets.
+OffsetsScan offsets_scan(const uint32_t* counts, uint64_t* state, uint32_t fanout, uint32_t grid, fij_type type,
+                         const fij_partition_offsets* offsets) {
+  return OffsetsScan{counts, offsets->local_offsets, offsets->offsets, state, 0, fanout, grid,
+                     pad_tuples(key_type(type)), 0};
+}
+
 // Argument checks of prefix_sum (gpu_radix_partition.rs:561-696); sets *bits
 // to the pass's radix bits.
 fij_status prefix_sum_checks(const fij_partitioner* p, fij_radix_pass pass, fij_type type,
@@ -411,8 +418,7 @@ fij_status fij_prefix_sum(fij_partitioner* p, fij_radix_pass pass, fij_type type
     if (s != FIJ_OK) return s;
     FIJ_HIP(launch_hist_counts(key_type(type), partition_attr, nullptr, nullptr, nullptr, len, p->grid, bits, ignore,
                                p->counts, p->scan_state, p->scan_cap, p->block, st));
-    FIJ_HIP(launch_offsets_scan(p->counts, F, p->grid, pad_tuples(key_type(type)), offsets->local_offsets,
-                                offsets->offsets, p->scan_state, st));
+    FIJ_HIP(launch_offsets_scan(offsets_scan(p->counts, p->scan_state, F, p->grid, type, offsets), nullptr, st));
   }
   return FIJ_OK;
 }
@@ -446,9 +452,8 @@ fij_status fij_prefix_sum_noalloc(fij_partitioner* p, fij_radix_pass pass, fij_t
   FIJ_HIP(noalloc_scratch(&counts, &state));
   // the histogram kernel clears the scan state it needs before the scan
   FIJ_HIP(launch_hist_counts(key_type(type), partition_attr, nullptr, nullptr, nullptr, len, p->grid, bits, ignore,
-                             counts, state, scan_state_words(n), p->block, st));
-  FIJ_HIP(launch_offsets_scan(counts, F, p->grid, pad_tuples(key_type(type)), offsets->local_offsets,
-                              offsets->offsets, state, st));
+                             counts, state, scan_state_words(F), p->block, st));
+  FIJ_HIP(launch_offsets_scan(offsets_scan(counts, state, F, p->grid, type, offsets), nullptr, st));
   return FIJ_OK;
 }
 
@@ -488,8 +493,7 @@ fij_status fij_prefix_sum_and_copy_with_payload(fij_partitioner* p, fij_radix_pa
   FIJ_HIP(launch_hist_counts(key_type(type), src_partition_attr, src_payload_attr, dst_partition_attr,
                              dst_payload_attr, len, p->grid, bits, pass_ignore_bits(p->bits, pass), p->counts,
                              p->scan_state, p->scan_cap, p->block, st));
-  FIJ_HIP(launch_offsets_scan(p->counts, F, p->grid, pad_tuples(key_type(type)), offsets->local_offsets,
-                              offsets->offsets, p->scan_state, st));
+  FIJ_HIP(launch_offsets_scan(offsets_scan(p->counts, p->scan_state, F, p->grid, type, offsets), nullptr, st));
   return FIJ_OK;
 }
 
@@ -532,8 +536,7 @@ fij_status fij_prefix_sum_and_transform(fij_partitioner* p, fij_radix_pass pass,
                                   partition_id, dst_len, dst_partition_attr, dst_payload_attr, p->grid, bits,
                                   pass_ignore_bits(p->bits, pass), p->counts, p->scan_state, p->scan_cap, d->status,
                                   p->block, st));
-  FIJ_HIP(launch_offsets_scan(p->counts, F, p->grid, pad_tuples(key_type(type)), offsets->local_offsets,
-                              offsets->offsets, p->scan_state, st));
+  FIJ_HIP(launch_offsets_scan(offsets_scan(p->counts, p->scan_state, F, p->grid, type, offsets), nullptr, st));
   return FIJ_OK;
 }
 

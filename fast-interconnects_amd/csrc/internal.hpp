@@ -17,6 +17,16 @@ inline uint32_t key_bytes(KeyType t) { return t == KeyType::I32 ? 4u : 8u; }
 inline uint32_t tuple_bytes(KeyType t) { return 2u * key_bytes(t); }
 inline uint32_t pad_tuples(KeyType t) { return 128u / tuple_bytes(t); }
 
+// Chunk length of a pass 1 whose chunks are the library's own choice: ceil(n /
+// chunks) rounded up to 128 bytes of keys, so that no chunk is longer than
+// the others (the canonical length is rounded down and leaves up to 128
+// bytes of keys per chunk to the last one); the last chunks may be short or
+// empty.
+inline uint64_t balanced_chunk_len(KeyType t, uint64_t n, uint32_t chunks) {
+  const uint64_t align = 128u / key_bytes(t);
+  return ((n + chunks - 1) / chunks + align - 1) / align * align;
+}
+
 // Status bits a kernel may raise in the library's device status word.
 enum DeviceStatus : uint32_t {
   kStatusOk = 0,
@@ -25,18 +35,18 @@ enum DeviceStatus : uint32_t {
   kStatusPartitionOverflow = 1u << 2, // offsets inconsistent with the input
 };
 
-// Decoupled look-back scan state: one ticket word plus one word per tile.
+// Decoupled look-back scan state: one ticket word plus one word per tile of
+// kScanCols partitions.
 constexpr uint32_t kScanBlock = 1024;
-constexpr uint32_t kScanItems = 8;
-constexpr uint32_t kScanTile = kScanBlock * kScanItems;
-constexpr uint64_t scan_state_words(uint64_t n) { return 1 + (n + kScanTile - 1) / kScanTile; }
+constexpr uint32_t kScanCols = 16;
+constexpr uint64_t scan_state_words(uint64_t fanout) { return 1 + (fanout + kScanCols - 1) / kScanCols; }
 
 // ---- prefix sums (hist.hip) ----------------------------------------------
 // Chunked: one block per chunk; writes offsets[chunk][F] directly.
 hipError_t launch_hist_chunked(KeyType t, const void* keys, uint64_t n, uint32_t chunks,
                                uint32_t radix_bits, uint32_t ignore_bits, uint64_t* offsets,
                                uint32_t block, hipStream_t stream);
-// Contiguous, step 1: per-chunk counts in partition-major order counts[F][chunks];
+// Contiguous, step 1: per-chunk counts[chunks][F];
 // optionally copies keys/payloads (prefix_sum_and_copy_with_payload); clears
 // `scan_state` for the following scan.
 hipError_t launch_hist_counts(KeyType t, const void* keys, const void* pays, void* dst_keys,
@@ -52,11 +62,21 @@ hipError_t launch_transform_counts(KeyType t, const void* src_rel, const uint64_
                                    uint32_t radix_bits, uint32_t ignore_bits, uint32_t* counts,
                                    uint64_t* scan_state, uint64_t scan_state_len,
                                    uint32_t* status, uint32_t block, hipStream_t stream);
-// Contiguous, step 2: decoupled look-back exclusive scan of counts[F][chunks],
-// producing local_offsets[chunks][F] (+ (p+1)*pad) and offsets[F].
-hipError_t launch_offsets_scan(const uint32_t* counts, uint32_t fanout, uint32_t chunks,
-                               uint32_t pad, uint64_t* local_offsets, uint64_t* offsets,
-                               uint64_t* scan_state, hipStream_t stream);
+// Contiguous, step 2: decoupled look-back exclusive scan of counts[chunks][F]
+// in partition-major order, producing local[chunks][F] (+ (p+1)*pad) and
+// offsets[F] = region + local[0][F] (region: where the relation begins in a
+// larger array, 0 for one of its own).  `state`: scan_state_words(fanout)
+// words that the histogram cleared.
+struct OffsetsScan {
+  const uint32_t* counts;
+  uint64_t* local;
+  uint64_t* offsets;
+  uint64_t* state;
+  uint64_t region;
+  uint32_t fanout, chunks, pad, reserved;
+};
+// One launch for a, and for b (of the same fanout) unless it is null.
+hipError_t launch_offsets_scan(const OffsetsScan& a, const OffsetsScan* b, hipStream_t stream);
 
 // Allocation-free contiguous prefix sum: at most kNoAllocCounters per-chunk
 // counters (fanout x chunks).  noalloc_scratch returns the current device's
@@ -65,7 +85,7 @@ hipError_t launch_offsets_scan(const uint32_t* counts, uint32_t fanout, uint32_t
 constexpr uint64_t kNoAllocCounters = FIJ_NOALLOC_MAX_COUNTERS;
 hipError_t noalloc_scratch(uint32_t** counts, uint64_t** scan_state);
 
-// Histogram launch parameters (one relation, contiguous counts[F][chunks] or
+// Histogram launch parameters (one relation, contiguous counts[chunks][F] or
 // chunked offsets[chunks][F]).
 struct HistParams {
   const void* keys;
@@ -79,30 +99,25 @@ struct HistParams {
   uint32_t pad;
   uint32_t subhists;
   uint64_t* offsets;   // chunked: [G][F]
-  uint32_t* counts;    // contiguous: [F][G]
+  uint32_t* counts;    // contiguous: [G][F]
   uint64_t* scan_state;
   uint64_t scan_state_len;
 };
 
-// One relation of a batched offsets launch: counts[F][chunks] in, write
-// offsets local[chunks][F] (relative to the relation's region) and
-// partition starts off1[F] (in the plan's pass-1 array) out.
-struct BatchScanJob {
-  const uint32_t* counts;
-  uint64_t* local;
-  uint64_t* off1;
-  uint64_t region;
-  uint32_t fanout, chunks, pad;
-};
-// Contiguous histogram parameters of one relation of a batched launch.
+// Contiguous histogram parameters of one relation of a paired or batched
+// launch, in chunks of balanced_chunk_len; scan_state (scan_state_words(2^radix_bits) words) is cleared by it.
 HistParams hist_params(KeyType t, const void* keys, uint64_t n, uint32_t chunks, uint32_t radix_bits,
-                       uint32_t block, uint32_t* counts);
+                       uint32_t block, uint32_t* counts, uint64_t* scan_state);
+// Histograms of two relations of the same radix bits in one launch: ga chunks
+// of a, gb of b (gb = 0: a alone).
+hipError_t launch_hist_pair(KeyType t, const HistParams& a, const HistParams& b, uint32_t ga, uint32_t gb,
+                            uint32_t block, hipStream_t stream);
 // Histograms of njobs relations in one launch: block b counts chunk
 // b - prefix[j] of jobs[j] (prefix[njobs] = blocks, device memory).
 hipError_t launch_hist_batched(KeyType t, const HistParams* jobs, const uint32_t* prefix, uint32_t njobs,
                                uint32_t blocks, uint32_t radix_bits, uint32_t block, hipStream_t stream);
-// Offsets of njobs relations in one launch (one block each).
-hipError_t launch_offsets_batched(const BatchScanJob* jobs, uint32_t njobs, hipStream_t stream);
+// Offsets of njobs relations of one fanout in one launch.
+hipError_t launch_offsets_batched(const OffsetsScan* jobs, uint32_t njobs, uint32_t fanout, hipStream_t stream);
 
 // ---- partitioning (partition.hip) -----------------------------------------
 struct PartitionLaunch {
@@ -111,6 +126,7 @@ struct PartitionLaunch {
   const void* pays;
   uint64_t n;
   uint32_t chunks;            // == grid
+  uint64_t chunk_len;         // 0: the canonical length
   uint32_t radix_bits;
   uint32_t ignore_bits;
   const uint64_t* chunk_offsets;  // [chunks][F] absolute tuple offsets
@@ -127,6 +143,9 @@ struct PartitionLaunch {
   uint32_t spill_from = 0;
 };
 hipError_t launch_partition(const PartitionLaunch& a, hipStream_t stream);
+// Buffered scatters of two relations of one type, radix bits and block (no
+// spill): one launch where the line rings fit LDS, else one each.
+hipError_t launch_partition_pair(const PartitionLaunch& a, const PartitionLaunch& b, hipStream_t stream);
 // Buffered-scatter parameters of one relation of a batched launch.
 struct ScatterParams {
   const void* keys;

@@ -444,33 +444,29 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
     d.F1 = F1;
     d.bits1 = bits1;
     d.pad = static_cast<uint32_t>(pad);
-    PipelineSide side[2]{};
-    uint32_t G1 = cus;
-    auto fits = [&](uint64_t n, uint32_t chunks) {
-      uint64_t c = 0;
-      return fij_input_chunk_size(static_cast<fij_type>(cfg->type), n, chunks, &c) == FIJ_OK && c * (chunks - 1) <= n;
-    };
-    while (G1 > 1 && !(fits(build_len, G1) && fits(probe_len, G1))) G1 = G1 > 64 ? G1 - 32 : G1 - 1;
-    d.G1 = G1;
+    d.G1 = cus;
+    d.sides = 3;
+    PipelineSide* const side[2] = {&d.build, &d.probe};
     for (int r = 0; r < 2; ++r) {
-      PipelineSide& s = side[r];
+      PipelineSide& s = *side[r];
+      s.g1 = pass1_chunks(kt, lens[r], cus);
       s.keys = cols[r][0];
       s.pays = cols[r][1];
       s.n = lens[r];
       s.padded_len1 = s.n + F1 * pad;
-      s.scan1_len = scan_state_words(static_cast<uint64_t>(F1) * G1);
+      s.scan1_len = scan_state_words(F1);
       OOC_HIP(A.dalloc(&s.off1, F1));
-      OOC_HIP(A.dalloc(&s.local1, static_cast<uint64_t>(G1) * F1));
-      OOC_HIP(A.dalloc(&s.counts1, static_cast<uint64_t>(F1) * G1));
+      OOC_HIP(A.dalloc(&s.local1, static_cast<uint64_t>(s.g1) * F1));
+      OOC_HIP(A.dalloc(&s.counts1, static_cast<uint64_t>(F1) * s.g1));
       OOC_HIP(A.dalloc(&s.scan1, s.scan1_len));
     }
     OOC_HIP(hipEventRecord(ev[0], main_st));
-    for (int r = 0; r < 2; ++r) OOC_HIP(enqueue_side_prefix_sum(d, side[r], kt, 1024, main_st));
+    OOC_HIP(enqueue_pass1_prefix_sum(d, kt, 1024, main_st));
     OOC_HIP(hipEventRecord(ev[1], main_st));
     uint64_t* h_off = nullptr;
     OOC_HIP(A.halloc(&h_off, 2ull * F1));
     for (int r = 0; r < 2; ++r)
-      OOC_HIP(hipMemcpyAsync(h_off + r * F1, side[r].off1, F1 * 8ull, hipMemcpyDeviceToHost, main_st));
+      OOC_HIP(hipMemcpyAsync(h_off + r * F1, side[r]->off1, F1 * 8ull, hipMemcpyDeviceToHost, main_st));
     OOC_HIP(hipStreamSynchronize(main_st));
     float f = 0;
     OOC_HIP(hipEventElapsedTime(&f, ev[0], ev[1]));
@@ -504,13 +500,14 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
       a.keys = cols[r][0];
       a.pays = cols[r][1];
       a.n = lens[r];
-      a.chunks = G1;
+      a.chunks = side[r]->g1;
+      a.chunk_len = balanced_chunk_len(kt, lens[r], a.chunks);
       a.radix_bits = bits1;
       a.ignore_bits = 0;
-      a.chunk_offsets = side[r].local1;
+      a.chunk_offsets = side[r]->local1;
       // with everything spilled the relation pointer only anchors the
       // alignment: a 256-byte aligned device address
-      a.relation = rel[r].cache ? static_cast<void*>(rel[r].cache) : static_cast<void*>(side[r].off1);
+      a.relation = rel[r].cache ? static_cast<void*>(rel[r].cache) : static_cast<void*>(side[r]->off1);
       a.block = 1024;
       a.lds_bytes = lds_total;
       a.buffered = true;

@@ -20,9 +20,10 @@ struct PipelineSide {
   const void* keys;           // input columns
   const void* pays;
   uint64_t n;
+  uint32_t g1;                // pass-1 chunks of this side (at most PipelineDevice::G1)
   uint64_t* off1;             // [F1] partition starts in rel1
-  uint64_t* local1;           // [G1][F1] per-chunk write offsets
-  uint32_t* counts1;          // [F1][G1] per-chunk histograms
+  uint64_t* local1;           // [g1][F1] per-chunk write offsets
+  uint32_t* counts1;          // [g1][F1] per-chunk histograms
   uint64_t* scan1;            // look-back scan state of the offsets scan
   uint64_t scan1_len;
   void* rel1;                 // Tuple[padded_len1]
@@ -109,11 +110,22 @@ struct BatchSide {
 // tuples: the plan using it must set its pad to pad_tuples(t).
 hipError_t alloc_pipeline_side(PipelineSide& s, KeyType t, uint64_t n, uint32_t F1, uint32_t F2, uint32_t G1,
                                bool two_pass, uint32_t tiles, std::vector<void*>& allocs);
-// Pass 1 of one side: contiguous histogram + offsets scan, then the scatter.
-hipError_t enqueue_side_prefix_sum(const PipelineDevice& d, PipelineSide& s, KeyType t, uint32_t block,
-                                   hipStream_t stream);
-hipError_t enqueue_side_scatter(const PipelineDevice& d, PipelineSide& s, KeyType t, uint32_t block,
-                                uint32_t lds_total, hipStream_t stream);
+// Pass 1 of the sides in d.sides (each in its g1 chunks): contiguous
+// histograms + offsets scans, then the scatters, one launch each.
+hipError_t enqueue_pass1_prefix_sum(const PipelineDevice& d, KeyType t, uint32_t block, hipStream_t stream);
+hipError_t enqueue_pass1_scatter(const PipelineDevice& d, KeyType t, uint32_t block, uint32_t lds_total,
+                                 hipStream_t stream);
+// Chunks of n tuples: at most `most`, none shorter than a step of the
+// scatter (but for the last ones).
+uint32_t pass1_chunks(KeyType t, uint64_t n, uint32_t most);
+// Chunks of the two sides of one join when a launch covers both: `total`
+// blocks shared in proportion to the sides' lengths (at least one each), so
+// that every block has the same work and no launch waits for the tail of
+// another.  With one block per compute unit for each side in turn, the
+// histogram, scan and scatter of 2^20 + 2^24 int32 tuples at 9 bits took 26 +
+// 22 + 77 us, in one launch each 21 + 6 + 65 us; 2^27 + 2^27 int64 tuples 343 +
+// 22 + 1760 us and 330 + 6 + 1390 us (half as many pieces per partition).
+void split_chunks(KeyType t, uint64_t n_b, uint64_t n_p, uint32_t total, uint32_t* g_b, uint32_t* g_p);
 
 uint32_t pipeline_tile2(KeyType t);
 // Build tuples a deferred item may have to be joined from one block-shared

@@ -2,6 +2,7 @@
 // server (server.cpp): one side's buffers and its pass-1 launches.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "internal.hpp"
@@ -28,7 +29,8 @@ hipError_t alloc_pipeline_side(PipelineSide& s, KeyType t, uint64_t n, uint32_t 
   const uint32_t tb = tuple_bytes(t);
   s.n = n;
   s.padded_len1 = n + static_cast<uint64_t>(F1) * pad_tuples(t);
-  s.scan1_len = scan_state_words(static_cast<uint64_t>(F1) * G1);
+  s.g1 = G1;
+  s.scan1_len = scan_state_words(F1);
   hipError_t e;
   if ((e = alloc_n(&s.off1, F1, allocs)) != hipSuccess) return e;
   if ((e = alloc_n(&s.local1, static_cast<uint64_t>(G1) * F1, allocs)) != hipSuccess) return e;
@@ -54,22 +56,42 @@ hipError_t alloc_pipeline_side(PipelineSide& s, KeyType t, uint64_t n, uint32_t 
   return hipSuccess;
 }
 
-hipError_t enqueue_side_prefix_sum(const PipelineDevice& d, PipelineSide& s, KeyType t, uint32_t block,
-                                   hipStream_t stream) {
-  hipError_t e = launch_hist_counts(t, s.keys, nullptr, nullptr, nullptr, s.n, d.G1, d.bits1, 0, s.counts1, s.scan1,
-                                    s.scan1_len, block, stream);
-  if (e != hipSuccess) return e;
-  return launch_offsets_scan(s.counts1, d.F1, d.G1, d.pad, s.local1, s.off1, s.scan1, stream);
+uint32_t pass1_chunks(KeyType t, uint64_t n, uint32_t most) {
+  // at least one step of the scatter's loaders per chunk
+  const uint64_t step = t == KeyType::I32 ? 2048 : 1024;
+  return static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(most, (n + step - 1) / step)));
 }
 
-hipError_t enqueue_side_scatter(const PipelineDevice& d, PipelineSide& s, KeyType t, uint32_t block,
-                                uint32_t lds_total, hipStream_t stream) {
+void split_chunks(KeyType t, uint64_t n_b, uint64_t n_p, uint32_t total, uint32_t* g_b, uint32_t* g_p) {
+  uint32_t b = 1;
+  if (total > 2 && n_b + n_p) {
+    const double share = static_cast<double>(n_b) / static_cast<double>(n_b + n_p);
+    b = static_cast<uint32_t>(share * total + 0.5);
+    b = b < 1 ? 1 : (b > total - 1 ? total - 1 : b);
+  }
+  *g_b = pass1_chunks(t, n_b, b);
+  *g_p = pass1_chunks(t, n_p, total > b ? total - b : 1);
+}
+
+namespace {
+
+const PipelineSide* side_of(const PipelineDevice& d, uint32_t i) {
+  return (d.sides >> i) & 1u ? (i ? &d.probe : &d.build) : nullptr;
+}
+
+OffsetsScan scan_of(const PipelineDevice& d, const PipelineSide& s) {
+  return OffsetsScan{s.counts1, s.local1, s.off1, s.scan1, 0, d.F1, s.g1, d.pad, 0};
+}
+
+PartitionLaunch scatter_of(const PipelineDevice& d, const PipelineSide& s, KeyType t, uint32_t block,
+                           uint32_t lds_total) {
   PartitionLaunch a{};
   a.type = t;
   a.keys = s.keys;
   a.pays = s.pays;
   a.n = s.n;
-  a.chunks = d.G1;
+  a.chunks = s.g1;
+  a.chunk_len = balanced_chunk_len(t, s.n, s.g1);
   a.radix_bits = d.bits1;
   a.ignore_bits = 0;
   a.chunk_offsets = s.local1;
@@ -77,7 +99,28 @@ hipError_t enqueue_side_scatter(const PipelineDevice& d, PipelineSide& s, KeyTyp
   a.block = block;
   a.lds_bytes = lds_total;
   a.buffered = true;
-  return launch_partition(a, stream);
+  return a;
+}
+
+}  // namespace
+
+hipError_t enqueue_pass1_prefix_sum(const PipelineDevice& d, KeyType t, uint32_t block, hipStream_t stream) {
+  const PipelineSide* a = side_of(d, 0) ? side_of(d, 0) : side_of(d, 1);
+  const PipelineSide* b = d.sides == 3 ? &d.probe : nullptr;
+  const HistParams ha = hist_params(t, a->keys, a->n, a->g1, d.bits1, block, a->counts1, a->scan1);
+  const HistParams hb = b ? hist_params(t, b->keys, b->n, b->g1, d.bits1, block, b->counts1, b->scan1) : ha;
+  const hipError_t e = launch_hist_pair(t, ha, hb, a->g1, b ? b->g1 : 0, block, stream);
+  if (e != hipSuccess) return e;
+  const OffsetsScan sa = scan_of(d, *a), sb = b ? scan_of(d, *b) : sa;
+  return launch_offsets_scan(sa, b ? &sb : nullptr, stream);
+}
+
+hipError_t enqueue_pass1_scatter(const PipelineDevice& d, KeyType t, uint32_t block, uint32_t lds_total,
+                                 hipStream_t stream) {
+  if (d.sides == 3)
+    return launch_partition_pair(scatter_of(d, d.build, t, block, lds_total),
+                                 scatter_of(d, d.probe, t, block, lds_total), stream);
+  return launch_partition(scatter_of(d, d.sides & 1 ? d.build : d.probe, t, block, lds_total), stream);
 }
 
 }  // namespace fij

@@ -139,14 +139,6 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
   p->d.F1 = 1u << cfg->radix_bits_1;
   p->d.F2 = 1u << cfg->radix_bits_2;
   p->d.G1 = cfg->pass1_chunks ? cfg->pass1_chunks : cus;
-  if (!cfg->pass1_chunks) {
-    // automatic: one chunk per compute unit, fewer for short relations
-    auto fits = [&](uint64_t n, uint32_t chunks) {
-      uint64_t c = 0;
-      return fij_input_chunk_size(static_cast<fij_type>(cfg->type), n, chunks, &c) == FIJ_OK && c * (chunks - 1) <= n;
-    };
-    while (p->d.G1 > 1 && !(fits(cfg->build_len, p->d.G1) && fits(cfg->probe_len, p->d.G1))) --p->d.G1;
-  }
   p->g1_cap = p->d.G1;
   p->d.pad = pad_tuples(kt);
   p->d.tile2 = pipeline_tile2(kt);
@@ -159,8 +151,8 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
   const uint64_t lens[2] = {cfg->build_len, cfg->probe_len};
   for (int rel = 0; rel < 2 && st == FIJ_OK; ++rel) {
     uint64_t chunk = 0;
-    st = fij_input_chunk_size(static_cast<fij_type>(cfg->type), lens[rel], p->d.G1, &chunk);
-    if (st == FIJ_OK && chunk * (p->d.G1 - 1) > lens[rel])
+    if (cfg->pass1_chunks) st = fij_input_chunk_size(static_cast<fij_type>(cfg->type), lens[rel], p->d.G1, &chunk);
+    if (st == FIJ_OK && cfg->pass1_chunks && chunk * (p->d.G1 - 1) > lens[rel])
       st = plan_fail(FIJ_INVALID_ARGUMENT, "relation of %llu tuples is too short for %u chunks",
                      static_cast<unsigned long long>(lens[rel]), p->d.G1);
     // the scatter addresses a chunk's writes relative to its first partition
@@ -234,19 +226,6 @@ fij_status fij_join_plan_destroy(fij_join_plan* plan) {
 
 namespace {
 
-// Chunks of pass 1 for relations of n_b and n_p tuples: the plan's chunk
-// count, fewer when a relation is too short for it (every chunk but the last
-// has the canonical length, the last one the rest).
-uint32_t exec_chunks(const fij_join_plan* p, uint64_t n_b, uint64_t n_p) {
-  uint32_t g = p->g1_cap;
-  auto fits = [&](uint64_t n, uint32_t chunks) {
-    uint64_t c = 0;
-    return fij_input_chunk_size(static_cast<fij_type>(p->cfg.type), n, chunks, &c) == FIJ_OK && c * (chunks - 1) <= n;
-  };
-  while (g > 1 && !(fits(n_b, g) && fits(n_p, g))) g = g > 64 ? g - 32 : g - 1;
-  return g;
-}
-
 // Enqueues one join of the plan's shape over columns of n_b and n_p tuples
 // (at most the plan's lengths).  With events, the phases are timed and the
 // per-block aggregates are copied to the host; otherwise (capturable: no
@@ -274,13 +253,19 @@ fij_status enqueue_join(fij_join_plan* p, const void* build_keys, const void* bu
   d.probe.n = n_p;
   d.build.padded_len1 = n_b + static_cast<uint64_t>(d.F1) * d.pad;
   d.probe.padded_len1 = n_p + static_cast<uint64_t>(d.F1) * d.pad;
-  d.G1 = exec_chunks(p, n_b, n_p);
+  // pass-1 chunks: one block per compute unit, shared by the sides; a chunk
+  // count that the caller chose holds for each side
+  if (p->cfg.pass1_chunks) {
+    d.build.g1 = pass1_chunks(p->kt, n_b, p->g1_cap);
+    d.probe.g1 = pass1_chunks(p->kt, n_p, p->g1_cap);
+  } else {
+    split_chunks(p->kt, n_b, n_p, p->g1_cap, &d.build.g1, &d.probe.g1);
+  }
   d.big_block_tables = d.bits2 ? 0u : big_block_tables_for(p->kt, n_b, d.F1);
   if (events) PLAN_HIP(hipEventRecord(p->ev[0], st));
-  for (PipelineSide* s : {&d.build, &d.probe}) PLAN_HIP(enqueue_side_prefix_sum(d, *s, p->kt, p->block1, st));
+  PLAN_HIP(enqueue_pass1_prefix_sum(d, p->kt, p->block1, st));
   if (events) PLAN_HIP(hipEventRecord(p->ev[1], st));
-  for (PipelineSide* s : {&d.build, &d.probe})
-    PLAN_HIP(enqueue_side_scatter(d, *s, p->kt, p->block1, p->lds_total, st));
+  PLAN_HIP(enqueue_pass1_scatter(d, p->kt, p->block1, p->lds_total, st));
   if (events) PLAN_HIP(hipEventRecord(p->ev[2], st));
   PLAN_HIP(launch_pipeline_plan(d, st));
   if (d.bits2) PLAN_HIP(launch_pipeline_sort2(d, p->kt, p->sort2_grid, st));

@@ -163,17 +163,6 @@ PipelineDevice base_device(const fij_join_server* s, const ResidentBuild& b) {
   return d;
 }
 
-uint32_t chunks_for(KeyType kt, uint64_t n, uint32_t cap) {
-  uint32_t g = cap;
-  auto fits = [&](uint32_t chunks) {
-    uint64_t c = 0;
-    return fij_input_chunk_size(kt == KeyType::I32 ? FIJ_TYPE_I32 : FIJ_TYPE_I64, n, chunks, &c) == FIJ_OK &&
-           c * (chunks - 1) <= n;
-  };
-  while (g > 1 && !fits(g)) g = g > 64 ? g - 32 : g - 1;
-  return g;
-}
-
 // Launches request r on slot sl (scheduler thread, server lock held).
 fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
   const ResidentBuild& b = *s->builds[r.build];
@@ -193,8 +182,7 @@ fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
   d.probe.pays = r.pays;
   d.probe.n = r.len;
   d.probe.padded_len1 = r.len + static_cast<uint64_t>(d.F1) * d.pad;
-  d.probe.scan1_len = scan_state_words(static_cast<uint64_t>(d.F1) * s->cus);
-  d.G1 = chunks_for(s->kt, r.len, s->cus);
+  d.probe.g1 = pass1_chunks(s->kt, r.len, s->cus);
   d.big_block_tables = d.bits2 ? 0u : big_block_tables_for(s->kt, b.n, d.F1);
   d.sides = 2;
   d.work_counter = sl.work_counter;
@@ -203,8 +191,8 @@ fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
   d.unit_cap = sl.unit_cap;
   d.aggregates = sl.aggregates;
   hipStream_t st = sl.stream;
-  SRV_HIP(enqueue_side_prefix_sum(d, d.probe, s->kt, 1024, st));
-  SRV_HIP(enqueue_side_scatter(d, d.probe, s->kt, 1024, s->lds_total, st));
+  SRV_HIP(enqueue_pass1_prefix_sum(d, s->kt, 1024, st));
+  SRV_HIP(enqueue_pass1_scatter(d, s->kt, 1024, s->lds_total, st));
   SRV_HIP(launch_pipeline_plan(d, st));
   if (d.bits2) {
     const uint32_t tiles = static_cast<uint32_t>(r.len / d.tile2 + d.F1);
@@ -425,13 +413,13 @@ fij_status add_one_pass_build(fij_join_server* s, std::unique_ptr<ResidentBuild>
   d.build.keys = keys;
   d.build.pays = payloads;
   d.build.n = len;
-  d.G1 = chunks_for(s->kt, len, s->cus);
+  d.build.g1 = pass1_chunks(s->kt, len, s->cus);
   d.sides = 1;
   d.work_counter = s->scratch_counters;
   d.aggregates = s->scratch_agg;
   hipStream_t stm = s->setup;
-  if ((e = enqueue_side_prefix_sum(d, d.build, s->kt, 1024, stm)) != hipSuccess ||
-      (e = enqueue_side_scatter(d, d.build, s->kt, 1024, s->lds_total, stm)) != hipSuccess ||
+  if ((e = enqueue_pass1_prefix_sum(d, s->kt, 1024, stm)) != hipSuccess ||
+      (e = enqueue_pass1_scatter(d, s->kt, 1024, s->lds_total, stm)) != hipSuccess ||
       (e = launch_pipeline_plan(d, stm)) != hipSuccess || (e = hipStreamSynchronize(stm)) != hipSuccess) {
     free_all(b->allocs);
     return hip_status(e, "partitioning the build side");
@@ -526,13 +514,13 @@ fij_status fij_join_server_add_build(fij_join_server* s, const void* keys, const
   d.build.keys = keys;
   d.build.pays = payloads;
   d.build.n = len;
-  d.G1 = chunks_for(s->kt, len, s->cus);
+  d.build.g1 = pass1_chunks(s->kt, len, s->cus);
   d.sides = 1;
   d.work_counter = s->scratch_counters;
   d.aggregates = s->scratch_agg;
   hipStream_t stm = s->setup;
-  if ((e = enqueue_side_prefix_sum(d, d.build, s->kt, 1024, stm)) != hipSuccess ||
-      (e = enqueue_side_scatter(d, d.build, s->kt, 1024, s->lds_total, stm)) != hipSuccess ||
+  if ((e = enqueue_pass1_prefix_sum(d, s->kt, 1024, stm)) != hipSuccess ||
+      (e = enqueue_pass1_scatter(d, s->kt, 1024, s->lds_total, stm)) != hipSuccess ||
       (e = launch_pipeline_plan(d, stm)) != hipSuccess ||
       (e = launch_pipeline_sort2(d, s->kt, std::max(1u, std::min(s->cus, tiles)), stm)) != hipSuccess ||
       (e = hipStreamSynchronize(stm)) != hipSuccess) {
