@@ -194,8 +194,10 @@ fij_status grow_arena(ClassArena& a, KeyType kt, uint32_t b1, uint32_t b2, uint6
   if (e == hipSuccess) e = arena_alloc(n, &n.local, n.chunk_words);
   if (e == hipSuccess) e = arena_alloc(n, &n.scan_state, 2 * n.joins * scan_state_words(F1));
   if (e == hipSuccess) e = arena_alloc(n, &d.work_counter, kJoinCounterWords);
-  if (e == hipSuccess) e = arena_alloc(n, &d.overflow, parts * F2);
-  if (e == hipSuccess) e = arena_alloc(n, &d.units, n.units);
+  // work units: of deferred items (two passes) or of whole partitions (one)
+  if (e == hipSuccess && b2) e = arena_alloc(n, &d.overflow, parts * F2);
+  if (e == hipSuccess && b2) e = arena_alloc(n, &d.units, n.units);
+  if (e == hipSuccess && !b2) e = arena_alloc(n, &d.part_units, n.units);
   d.unit_cap = static_cast<uint32_t>(n.units);
   if (e == hipSuccess) e = arena_alloc(n, &d.aggregates, 1);
   if (e == hipSuccess) e = arena_alloc(n, &n.hist, 2 * n.joins);
@@ -206,7 +208,7 @@ fij_status grow_arena(ClassArena& a, KeyType kt, uint32_t b1, uint32_t b2, uint6
   if (e == hipSuccess) e = arena_alloc(n, &n.job_slot, n.joins);
   if (e == hipSuccess) e = arena_alloc(n, &n.side_tiles, 2 * n.joins);
   // the deferred-item flags start at zero; every join leaves them at zero
-  if (e == hipSuccess) e = hipMemset(d.overflow, 0, parts * F2);
+  if (e == hipSuccess && b2) e = hipMemset(d.overflow, 0, parts * F2);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   if (e != hipSuccess) {
     free_arena(n);
@@ -253,7 +255,8 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
   }
   if (static_cast<uint64_t>(J) * F1 * F2 >= 0xFFFFFFFFull || tiles[0] >= 0xFFFFFFFFull || tiles[1] >= 0xFFFFFFFFull)
     return batch_fail(FIJ_INTEGER_OVERFLOW, "size class %u+%u: too many joins for one submission", b1, b2);
-  const uint64_t units = static_cast<uint64_t>(J) * F1 * F2 + probe_total / 65536 + J + 1;
+  const uint64_t units = b2 ? static_cast<uint64_t>(J) * F1 * F2 + probe_total / 65536 + J + 1
+                            : part_unit_cap(static_cast<uint64_t>(J) * F1, probe_total);
   const auto t_grow = std::chrono::steady_clock::now();
   fij_status s = grow_arena(a, kt, b1, b2, J, rel1, rel2, tiles, words, units, st);
   *grow_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_grow).count();
@@ -339,22 +342,21 @@ hipError_t launch_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, hi
   if ((e = launch_partition_batched(kt, a.scat, a.prefix, js, a.sub_blocks, b1, lds_total, ck.block, ck.ring, st)) !=
       hipSuccess)
     return e;
+  if (ck.b2 == 0) {
+    if ((e = launch_one_pass_plan(a.d, kt, a.sides, a.sub_joins, st)) != hipSuccess) return e;
+    return launch_one_pass_join(a.d, kt, false, 2 * b->cus, st);
+  }
   if ((e = launch_pipeline_plan_batched(a.d, a.sides, a.sub_joins, a.side_tiles, a.d.build.n, a.d.probe.n, st)) !=
       hipSuccess)
     return e;
-  const bool one_pass = ck.b2 == 0;
-  if (!one_pass) {
-    const uint64_t tiles = static_cast<uint64_t>(a.sub_tiles[0]) + a.sub_tiles[1];
-    const uint32_t sort_grid = static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(b->cus, tiles)));
-    if ((e = launch_pipeline_sort2(a.d, kt, sort_grid, st)) != hipSuccess) return e;
-  }
+  const uint64_t tiles = static_cast<uint64_t>(a.sub_tiles[0]) + a.sub_tiles[1];
+  const uint32_t sort_grid = static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(b->cus, tiles)));
+  if ((e = launch_pipeline_sort2(a.d, kt, sort_grid, st)) != hipSuccess) return e;
   // the register join: four blocks per CU, as many as the lighter join shapes
   // of batched classes (fewer registers, smaller tables) keep resident; the
-  // others start as earlier blocks finish and find the items taken.  A
-  // single-pass class's items are whole pass-1 partitions (large tables);
-  // most go on to the block-table join.
-  if ((e = launch_pipeline_join(a.d, kt, one_pass, false, 4 * b->cus, st)) != hipSuccess) return e;
-  return launch_pipeline_join(a.d, kt, one_pass, true, 2 * b->cus, st);
+  // others start as earlier blocks finish and find the items taken
+  if ((e = launch_pipeline_join(a.d, kt, false, 4 * b->cus, st)) != hipSuccess) return e;
+  return launch_pipeline_join(a.d, kt, true, 2 * b->cus, st);
 }
 
 // The closed-form size-class rule (the built-in table's fallback).
@@ -708,7 +710,7 @@ fij_status fij_join_batch_device_bytes(const fij_join_batch* b, uint64_t* bytes)
     const uint64_t parts = a.joins << kv.first.b1, F2 = 1ull << kv.first.b2;
     for (int s = 0; s < 2; ++s)
       total += (a.rel1[s] + a.rel2[s]) * tb + parts * (8 + 4 + 8 + 4) + (a.tiles[s] + 1) * F2 * 4;
-    total += a.chunk_words * (4 + 8) + parts * F2 + a.units * 16 +
+    total += a.chunk_words * (4 + 8) + (kv.first.b2 ? parts * F2 + a.units * 16 : a.units * sizeof(PartUnit)) +
              a.joins * 2 * (sizeof(HistParams) + sizeof(OffsetsScan) + sizeof(ScatterParams) + sizeof(BatchSide) + 4 +
                             8 * scan_state_words(1ull << kv.first.b1));
   }

@@ -1,0 +1,528 @@
+// Single-pass joins: pass 1 leaves every partition of both relations as one
+// contiguous range, and a build partition that fits a block's LDS table is
+// joined by streaming its probe partition against it.
+//
+//   one_pass_plan_kernel  partition lengths, and work units {build range, probe
+//                         range} of every partition pair; a build partition
+//                         beyond the LDS table gets a hash table in the HBM
+//                         arena when the arena has room, else its units fill
+//                         the LDS table several times
+//   part_join_kernel      one block per unit: the build range goes into a
+//                         block-shared table, the probe range is streamed
+//                         against it; then the build sides of the HBM tables
+//   part_table_kernel     the probes of the HBM tables
+//
+// Semantics as in the other joins: every pair of equal keys counts, null keys
+// never join, count and sums wrap at 64 bits.
+#include "common.hpp"
+#include "hbm_table.hpp"
+#include "internal.hpp"
+#include "pipeline.hpp"
+
+namespace fij {
+namespace {
+
+template <typename U>
+__device__ __forceinline__ U uniform_load(const U* ptr) {
+  return *(const __attribute__((address_space(4))) U*)(ptr);
+}
+
+// Slots of the block-shared table: 64 KiB of keys and values, or 128 KiB
+// (big_block_tables).  A build range may fill 3/4 of them.
+template <typename K>
+constexpr uint32_t kSlots = 65536 / (2 * sizeof(K));
+
+constexpr uint32_t kTableUnitTuples = 65536;  // tuples of an HBM-table work unit
+
+// Probe tuples of a unit: 8 times its build tuples (a unit's build work is
+// paid once per unit), between kPartUnitMin and 65,536.
+__device__ __forceinline__ uint32_t unit_tuples(uint32_t build_n) {
+  return min(65536u, max(kPartUnitMin, 8 * min(build_n, 8192u)));
+}
+
+// One block per join.  `sides` == nullptr: one join, whose sides end at their
+// padded_len1; that block sets the counters.  In batches (which have no HBM
+// arena) the counters were reset by an earlier launch.
+__global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, const BatchSide* sides, uint32_t F1j,
+                                                             uint32_t rcap) {
+  extern __shared__ uint32_t lds[];
+  __shared__ uint32_t wave_tmp[1024 / kWave + 1];
+  __shared__ uint32_t s_base, s_slots, s_big, s_build_units, s_probe_units;
+  uint32_t* first = lds;           // [F1j] units of a partition, then their exclusive scan
+  uint32_t* probe_n = lds + F1j;   // [F1j]
+  uint32_t* per = lds + 2 * F1j;   // [F1j] probe tuples per unit
+  const uint32_t tid = threadIdx.x, j = blockIdx.x;
+  const uint64_t end_b = sides ? sides[2 * j].rel1_end : d.build.padded_len1;
+  const uint64_t end_p = sides ? sides[2 * j + 1].rel1_end : d.probe.padded_len1;
+  if (tid == 0) s_slots = s_big = s_build_units = s_probe_units = 0;
+  if (sides && tid == 0) d.job_results[d.job_slot[j]] = JoinAggregate{0, 0, 0};
+  __syncthreads();
+  auto range = [&](const PipelineSide& s, uint64_t end, uint32_t p, uint64_t& at) -> uint32_t {
+    const uint32_t vp = j * F1j + p;
+    at = s.off1[vp];
+    return static_cast<uint32_t>((p + 1 < F1j ? s.off1[vp + 1] - d.pad : end) - at);
+  };
+  for (uint32_t p = tid; p < F1j; p += blockDim.x) {
+    uint64_t at;
+    const uint32_t nb = range(d.build, end_b, p, at), np = range(d.probe, end_p, p, at);
+    uint32_t units = 0;
+    const uint32_t ut = unit_tuples(nb);
+    if (nb && np) {
+      units = (np + ut - 1) / ut;
+      if (nb > rcap && d.hbm_cap && nb <= (d.hbm_cap >> 1)) {
+        // an HBM table of at least twice the build tuples, if the arena (at
+        // most 2^26 slots) has room.  A partition that finds none takes no
+        // slots; the sum of the others' stays below 2^32.
+        const uint32_t lg = max(8u, 64u - static_cast<uint32_t>(__builtin_clzll(2ull * nb - 1)));
+        uint32_t slot = s_slots;
+        for (;;) {
+          const uint32_t seen = slot + (1u << lg) <= d.hbm_cap ? atomicCAS(&s_slots, slot, slot + (1u << lg)) : slot;
+          if (seen == slot) break;
+          slot = seen;
+        }
+        const uint32_t big = slot + (1u << lg) <= d.hbm_cap ? atomicAdd(&s_big, 1u) : d.big_cap;
+        if (big < d.big_cap) {
+          units = 0;
+          d.big[big] = make_uint4(j * F1j + p, slot, lg, 0u);
+          const uint32_t bu = (nb + kTableUnitTuples - 1) / kTableUnitTuples;
+          const uint32_t pu = (np + kTableUnitTuples - 1) / kTableUnitTuples;
+          const uint32_t b0 = atomicAdd(&s_build_units, bu), p0 = atomicAdd(&s_probe_units, pu);
+          for (uint32_t u = 0; u < bu; ++u)
+            d.hbm_units[b0 + u] = make_uint4(big, u * kTableUnitTuples, min(nb, (u + 1) * kTableUnitTuples), 0u);
+          for (uint32_t u = 0; u < pu; ++u)
+            d.hbm_units[d.hbm_unit_cap - 1 - (p0 + u)] =
+                make_uint4(big, u * kTableUnitTuples, min(np, (u + 1) * kTableUnitTuples), 0u);
+        }
+      }
+    }
+    first[p] = units;
+    probe_n[p] = np;
+    per[p] = ut;
+    if (d.sides & 1) d.build.plen[j * F1j + p] = nb;
+    if (d.sides & 2) d.probe.plen[j * F1j + p] = np;
+  }
+  __syncthreads();
+  const uint32_t total = block_exclusive_scan<uint32_t>(first, F1j, wave_tmp);
+  if (tid == 0) {
+    if (sides) {
+      s_base = total ? atomicAdd(d.work_counter + kUnitCount, total) : 0u;
+    } else {
+      s_base = 0;
+      d.work_counter[kUnitCount] = total;
+      d.work_counter[kBlockTicket] = 0;
+      d.work_counter[kHbmSlots] = s_slots;
+      d.work_counter[kHbmSlots + 1] = 0;
+      d.work_counter[kHbmBuildUnits] = s_build_units;
+      d.work_counter[kHbmProbeUnits] = s_probe_units;
+    }
+  }
+  __syncthreads();
+  for (uint32_t u = tid; u < total; u += blockDim.x) {
+    uint32_t lo = 0, hi = F1j;  // the last partition whose first unit is at or before u
+    while (hi - lo > 1) {
+      const uint32_t m = (lo + hi) / 2;
+      if (first[m] <= u) lo = m; else hi = m;
+    }
+    PartUnit w;
+    uint64_t build_at, probe_at;
+    w.build_n = range(d.build, end_b, lo, build_at);
+    range(d.probe, end_p, lo, probe_at);
+    const uint32_t from = (u - first[lo]) * per[lo];
+    w.build_at = build_at;
+    w.probe_at = probe_at + from;
+    w.probe_n = min(per[lo], probe_n[lo] - from);
+    w.part = j * F1j + lo;
+    w.reserved = 0;
+    d.part_units[s_base + u] = w;
+  }
+}
+
+__global__ void reset_counters_kernel(uint32_t* counters) {
+  for (uint32_t i = threadIdx.x; i < kJoinCounterWords; i += blockDim.x) counters[i] = 0;
+}
+
+// Block-shared table of buckets of four slots, filled in order and probed
+// linearly from the key's bucket: two LDS reads of a bucket's keys and values
+// (16 bytes each at i32) answer a probe unless the key's bucket was full.
+// Probing is bound by instructions (a wave of 64 takes 4 cycles for each), so
+// the common case is straight-line code: buckets are at most 1/4 full on
+// average where the table allows it, which leaves 0.4 % of the keys outside
+// their bucket, and a table without duplicate keys (the insert finds out: the
+// later of two equal keys passes the earlier one) stops at a match.
+//
+// The keys of a partition share their low digit, so a key of another digit
+// marks free slots: a null key (-1) needs no test of its own when it is
+// probed, and lanes past a range's end carry a second key of another digit.
+template <typename K>
+struct BucketTable {
+  typedef K Quad __attribute__((ext_vector_type(4)));
+  Quad* keys;      // [buckets]
+  Quad* vals;      // [buckets]
+  uint32_t shift;  // hash bits below the bucket index
+  uint32_t mask;   // buckets - 1
+  K free_key;
+
+  __device__ __forceinline__ uint32_t bucket(K key) const {
+    uint32_t h = static_cast<uint32_t>(key) * 2654435769u;
+    if constexpr (sizeof(K) == 8) h += static_cast<uint32_t>(static_cast<uint64_t>(key) >> 32) * 2246822519u;
+    return h >> shift;
+  }
+  // Returns whether an equal key was passed.
+  __device__ __forceinline__ bool insert(K key, K val) const {
+    bool dup = false;
+    uint32_t s = 4 * bucket(key);
+    K* const k = reinterpret_cast<K*>(keys);
+    for (;; s = (s + 1) & (4 * mask + 3)) {
+      K prev;
+      if constexpr (sizeof(K) == 8)
+        prev = static_cast<K>(atomicCAS(reinterpret_cast<unsigned long long*>(&k[s]),
+                                        static_cast<unsigned long long>(free_key),
+                                        static_cast<unsigned long long>(key)));
+      else
+        prev = static_cast<K>(atomicCAS(reinterpret_cast<unsigned int*>(&k[s]), static_cast<unsigned int>(free_key),
+                                        static_cast<unsigned int>(key)));
+      if (prev == free_key) {
+        reinterpret_cast<K*>(vals)[s] = val;
+        return dup;
+      }
+      dup |= prev == key;
+    }
+  }
+  static __device__ __forceinline__ void add(K v, K pay, uint64_t& sb, uint64_t& sp) {
+    sb += static_cast<uint64_t>(static_cast<int64_t>(v));
+    sp += static_cast<uint64_t>(static_cast<int64_t>(pay));
+  }
+  // Probes N tuples of a lane together in a table without duplicate keys; the
+  // matches in first buckets are counted by the scalar unit (wave_cnt).
+  template <uint32_t N>
+  __device__ __forceinline__ void probe_unique(const K (&key)[N], const K (&pay)[N], uint32_t& wave_cnt, uint64_t& cnt,
+                                               uint64_t& sb, uint64_t& sp) const {
+    uint32_t at[N];
+    Quad k[N], v[N];
+    bool more[N];
+#pragma unroll
+    for (uint32_t i = 0; i < N; ++i) {
+      at[i] = bucket(key[i]);
+      k[i] = keys[at[i]];
+      v[i] = vals[at[i]];
+    }
+    bool any = false;
+#pragma unroll
+    for (uint32_t i = 0; i < N; ++i) {
+      const bool m0 = k[i].x == key[i], m1 = k[i].y == key[i], m2 = k[i].z == key[i], m3 = k[i].w == key[i];
+      wave_cnt += static_cast<uint32_t>(__popcll(ballot(m0) | ballot(m1) | ballot(m2) | ballot(m3)));
+      const K val = m0 ? v[i].x : m1 ? v[i].y : m2 ? v[i].z : v[i].w;
+      if (m0 || m1 || m2 || m3) add(val, pay[i], sb, sp);
+      more[i] = !(m0 || m1 || m2 || m3) && k[i].w != free_key;
+      any |= more[i];
+    }
+    if (ballot(any)) {
+#pragma unroll
+      for (uint32_t i = 0; i < N; ++i)
+        if (more[i]) probe_from((at[i] + 1) & mask, key[i], pay[i], cnt, sb, sp);
+    }
+  }
+  // Probes from bucket b to the first bucket with a free slot: every match
+  // counts.
+  __device__ __forceinline__ void probe_from(uint32_t b, K key, K pay, uint64_t& cnt, uint64_t& sb,
+                                             uint64_t& sp) const {
+    for (;; b = (b + 1) & mask) {
+      const Quad k = keys[b];
+      const uint32_t m = (k.x == key ? 1u : 0u) | (k.y == key ? 2u : 0u) | (k.z == key ? 4u : 0u) |
+                         (k.w == key ? 8u : 0u);
+      if (m) {
+        const Quad v = vals[b];
+        cnt += __popc(m);
+        if (m & 1u) add(v.x, pay, sb, sp);
+        if (m & 2u) add(v.y, pay, sb, sp);
+        if (m & 4u) add(v.z, pay, sb, sp);
+        if (m & 8u) add(v.w, pay, sb, sp);
+      }
+      if (k.w == free_key) return;
+    }
+  }
+};
+
+// Sums over the block, in thread 0 (red: [3][waves]); ends with a barrier.
+template <uint32_t BLOCK>
+__device__ __forceinline__ void block_sums(uint64_t (*red)[BLOCK / kWave], uint64_t& cnt, uint64_t& sb, uint64_t& sp) {
+  const uint32_t w = threadIdx.x / kWave;
+  cnt = wave_broadcast_last(wave_inclusive_scan(cnt));
+  sb = wave_broadcast_last(wave_inclusive_scan(sb));
+  sp = wave_broadcast_last(wave_inclusive_scan(sp));
+  if (lane_id() == 0) {
+    red[0][w] = cnt;
+    red[1][w] = sb;
+    red[2][w] = sp;
+  }
+  __syncthreads();
+  cnt = sb = sp = 0;
+  if (threadIdx.x == 0)
+    for (uint32_t i = 0; i < BLOCK / kWave; ++i) {
+      cnt += red[0][i];
+      sb += red[1][i];
+      sp += red[2][i];
+    }
+  __syncthreads();
+}
+
+// Adds the block's sums to the result of join `job` (batches) or, for one join,
+// to the block's aggregate (FIRST: stores it, and zeros for blocks that this
+// grid does not have), and clears them.
+template <uint32_t BLOCK, bool FIRST>
+__device__ __forceinline__ void add_result(const PipelineDevice& d, uint64_t (*red)[BLOCK / kWave], uint32_t job,
+                                           uint64_t& cnt, uint64_t& sb, uint64_t& sp) {
+  block_sums<BLOCK>(red, cnt, sb, sp);
+  if (threadIdx.x == 0) {
+    if (d.job_results) {
+      if (cnt) {
+        JoinAggregate* r = d.job_results + d.job_slot[job];
+        atomicAdd(reinterpret_cast<unsigned long long*>(&r->count), static_cast<unsigned long long>(cnt));
+        atomicAdd(reinterpret_cast<unsigned long long*>(&r->sum_build), static_cast<unsigned long long>(sb));
+        atomicAdd(reinterpret_cast<unsigned long long*>(&r->sum_probe), static_cast<unsigned long long>(sp));
+      }
+    } else {
+      JoinAggregate* r = d.aggregates + blockIdx.x;
+      if constexpr (FIRST) {
+        *r = JoinAggregate{cnt, sb, sp};
+        for (uint32_t i = blockIdx.x + gridDim.x; i < d.agg_len; i += gridDim.x)
+          d.aggregates[i] = JoinAggregate{0, 0, 0};
+      } else {
+        r->count += cnt;
+        r->sum_build += sb;
+        r->sum_probe += sp;
+      }
+    }
+  }
+  cnt = sb = sp = 0;
+}
+
+// 16 bytes of tuples from 16-byte aligned memory.
+template <typename K>
+struct TupleVec {
+  static constexpr uint32_t N = 16 / sizeof(Tuple<K>);  // 2 of 8 bytes, 1 of 16
+  typedef K type __attribute__((ext_vector_type(16 / sizeof(K))));
+};
+
+// Joins the work units, one block per unit (the first by block index, the rest
+// by ticket, taken while the current unit runs).
+//
+// Bound by the read of the probe partitions and, for short units, by the chain
+// ticket -> unit -> tuples and the table's build.  2^20 + 2^24 int32 tuples in
+// 512 partitions: 44 us (3.2 TB/s) where the two-pass plans' register join
+// (23 us, every item only put off), unit counting (8 us) and block join (48
+// us, every tuple's run looked up although a partition is one run) ran before;
+// 20 batched joins of 2^18..2^20 int32 build tuples 1,053 -> 300 us.  Two and
+// four vectors per buffer, two or four probes together, blocks of 256 to 1,024
+// threads and 32 KiB tables all lie within 43-50 us; the smallest register
+// need was taken.
+template <typename K, uint32_t CAP, uint32_t BLOCK>
+__global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
+  using V = TupleVec<K>;
+  using VT = typename V::type;
+  constexpr uint32_t RCAP = CAP * 3 / 4;      // build tuples per table fill
+  constexpr uint32_t LG_CAP = 29u - __builtin_clz(CAP);  // of its buckets
+  constexpr uint32_t NV = 2;                  // vectors in flight per buffer
+  constexpr uint32_t NT = NV * V::N;          // their tuples
+  constexpr uint32_t PROBES = 2;              // probed together
+  extern __shared__ __attribute__((aligned(16))) uint64_t lds_u64[];
+  __shared__ uint32_t s_next, s_dup;
+  __shared__ uint64_t red[3][BLOCK / kWave];
+  const uint32_t tid = threadIdx.x;
+  uint64_t cnt = 0, sb = 0, sp = 0;
+  const uint32_t n_units = uniform_load(d.work_counter + kUnitCount);
+  uint32_t job = 0;
+  for (uint32_t u = blockIdx.x; u < n_units;) {
+    uint32_t ticket = 0;
+    if (tid == 0) ticket = atomicAdd(d.work_counter + kBlockTicket, 1u);
+    const PartUnit unit = scalar_load(d.part_units + u);
+    if (d.job_results && (unit.part >> d.job_shift) != job) {
+      add_result<BLOCK, true>(d, red, job, cnt, sb, sp);
+      job = unit.part >> d.job_shift;
+    }
+    const uint32_t nb = unit.build_n;
+    // a range as aligned 16-byte vectors: the first one may begin a tuple
+    // before the range (the padding in front of a partition, or the range
+    // before it) and the last end one after it (the next range, or the spare
+    // tuple behind the relation); those tuples are skipped
+    const uint32_t off_b = unit.build_at % V::N, off_p = unit.probe_at % V::N;
+    const auto vb = as_global(static_cast<const VT*>(d.build.rel1) + unit.build_at / V::N);
+    const auto vp = as_global(static_cast<const VT*>(d.probe.rel1) + unit.probe_at / V::N);
+    const uint32_t nvp = (unit.probe_n + off_p + V::N - 1) / V::N;
+    auto load = [&](VT (&x)[NV], uint32_t v0) {
+#pragma unroll
+      for (uint32_t k = 0; k < NV; ++k) x[k] = __builtin_nontemporal_load(vp + min(v0 + k * BLOCK + tid, nvp - 1));
+    };
+    const uint32_t digit = unit.part & ((1u << d.bits1) - 1u);
+    const K free_key = static_cast<K>(digit ^ 1u);
+    const K no_key = static_cast<K>((digit ^ 1u) | (1u << d.bits1));
+    uint32_t wave_cnt = 0;
+    VT xa[NV], xb[NV];
+    load(xa, 0);  // in flight while the table is built
+    for (uint32_t f0 = 0; f0 < nb; f0 += RCAP) {
+      const uint32_t nf = min(RCAP, nb - f0);
+      // at most 1/4 full where the table allows it, 3/4 at most
+      const uint32_t lg = min(LG_CAP, max(6u, 32u - static_cast<uint32_t>(__builtin_clz(nf))));
+      using Quad = typename BucketTable<K>::Quad;
+      const BucketTable<K> tab{reinterpret_cast<Quad*>(lds_u64), reinterpret_cast<Quad*>(lds_u64) + CAP / 4, 32u - lg,
+                               (1u << lg) - 1u, free_key};
+      for (uint32_t i = tid; i < (1u << lg); i += BLOCK) tab.keys[i] = Quad{free_key, free_key, free_key, free_key};
+      if (tid == 0) s_dup = 0;
+      __syncthreads();
+      {
+        const uint32_t lo = off_b + f0, hi = off_b + f0 + nf;  // tuples of the range, counted from vb
+        const uint32_t v_end = (hi + V::N - 1) / V::N;
+        bool dup = false;
+        for (uint32_t v0 = lo / V::N; v0 < v_end; v0 += 2 * BLOCK) {
+          VT x[2];
+#pragma unroll
+          for (uint32_t k = 0; k < 2; ++k) x[k] = vb[min(v0 + k * BLOCK + tid, v_end - 1)];
+#pragma unroll
+          for (uint32_t k = 0; k < 2; ++k) {
+            const uint32_t v = v0 + k * BLOCK + tid;
+#pragma unroll
+            for (uint32_t e = 0; e < V::N; ++e) {
+              const uint32_t at = v * V::N + e;
+              const K key = x[k][2 * e];
+              if (v < v_end && at >= lo && at < hi && key != null_key<K>()) dup |= tab.insert(key, x[k][2 * e + 1]);
+            }
+          }
+        }
+        if (dup) s_dup = 1;
+      }
+      __syncthreads();
+      const bool unique = __builtin_amdgcn_readfirstlane(s_dup) == 0;
+      auto probe = [&](const VT (&x)[NV], uint32_t v0) {
+        // batches inside the range need no test per tuple
+        const bool inside = v0 >= off_p && (v0 + NV * BLOCK) * V::N <= off_p + unit.probe_n;
+#pragma unroll
+        for (uint32_t g = 0; g < NT; g += PROBES) {
+          K key[PROBES], pay[PROBES];
+#pragma unroll
+          for (uint32_t i = 0; i < PROBES; ++i) {
+            key[i] = x[(g + i) / V::N][2 * ((g + i) % V::N)];
+            pay[i] = x[(g + i) / V::N][2 * ((g + i) % V::N) + 1];
+          }
+          if (!inside) {
+#pragma unroll
+            for (uint32_t i = 0; i < PROBES; ++i) {
+              // counted from the range's start (wraps below it)
+              const uint32_t at = (v0 + (g + i) / V::N * BLOCK + tid) * V::N + (g + i) % V::N - off_p;
+              if (at >= unit.probe_n) key[i] = no_key;
+            }
+          }
+          if (unique) {
+            tab.probe_unique(key, pay, wave_cnt, cnt, sb, sp);
+          } else {
+#pragma unroll
+            for (uint32_t i = 0; i < PROBES; ++i) tab.probe_from(tab.bucket(key[i]), key[i], pay[i], cnt, sb, sp);
+          }
+        }
+      };
+      if (f0) load(xa, 0);
+      constexpr uint32_t STEP = NV * BLOCK;
+      for (uint32_t v0 = 0;; v0 += 2 * STEP) {
+        load(xb, v0 + STEP);
+        probe(xa, v0);
+        if (v0 + STEP >= nvp) break;
+        load(xa, v0 + 2 * STEP);
+        probe(xb, v0 + STEP);
+        if (v0 + 2 * STEP >= nvp) break;
+      }
+      if (f0 + RCAP < nb) __syncthreads();  // probes done before the table is cleared
+    }
+    if (lane_id() == 0) cnt += wave_cnt;
+    if (tid == 0) s_next = gridDim.x + ticket;
+    __syncthreads();  // probes done; the table may be cleared
+    u = __builtin_amdgcn_readfirstlane(s_next);
+    __syncthreads();  // every thread has read s_next
+  }
+  // build sides of the HBM tables
+  const uint32_t n_big = d.hbm_cap ? uniform_load(d.work_counter + kHbmBuildUnits) : 0u;
+  for (uint32_t u = blockIdx.x; u < n_big; u += gridDim.x) {
+    const uint4 unit = scalar_load(d.hbm_units + u);
+    const uint4 big = scalar_load(d.big + unit.x);
+    Tuple<K>* const table = static_cast<Tuple<K>*>(d.hbm_table) + big.y;
+    const Tuple<K>* rel = static_cast<const Tuple<K>*>(d.build.rel1) + uniform_load(d.build.off1 + big.x);
+    for (uint32_t i = unit.y + tid; i < unit.z; i += BLOCK) {
+      const Tuple<K> t = load_tuple<K>(rel + i);
+      if (t.key != null_key<K>()) hbm_insert<K>(table, big.z, t.key, t.value);
+    }
+  }
+  add_result<BLOCK, true>(d, red, job, cnt, sb, sp);
+}
+
+// Probes of the HBM tables (plans of one join only: batches and served joins
+// have no arena).
+template <typename K, uint32_t BLOCK>
+__global__ __launch_bounds__(BLOCK) void part_table_kernel(PipelineDevice d) {
+  __shared__ uint64_t red[3][BLOCK / kWave];
+  const uint32_t n = uniform_load(d.work_counter + kHbmProbeUnits);
+  if (n == 0) return;
+  uint64_t cnt = 0, sb = 0, sp = 0;
+  for (uint32_t u = blockIdx.x; u < n; u += gridDim.x) {
+    const uint4 unit = scalar_load(d.hbm_units + (d.hbm_unit_cap - 1 - u));
+    const uint4 big = scalar_load(d.big + unit.x);
+    const Tuple<K>* const table = static_cast<const Tuple<K>*>(d.hbm_table) + big.y;
+    const Tuple<K>* rel = static_cast<const Tuple<K>*>(d.probe.rel1) + uniform_load(d.probe.off1 + big.x);
+    for (uint32_t i = unit.y + threadIdx.x; i < unit.z; i += BLOCK) {
+      const Tuple<K> t = load_tuple_nt<K>(rel + i);
+      if (t.key != null_key<K>()) hbm_probe<K>(table, big.z, t.key, t.value, cnt, sb, sp);
+    }
+  }
+  add_result<BLOCK, false>(d, red, 0, cnt, sb, sp);
+}
+
+template <typename K, uint32_t CAP, uint32_t BLOCK>
+hipError_t launch_part_join(const PipelineDevice& d, uint32_t grid, hipStream_t stream) {
+  auto kern = part_join_kernel<K, CAP, BLOCK>;
+  const size_t lds = CAP * 2 * sizeof(K);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            static_cast<int>(lds));
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, stream, d);
+  return hipGetLastError();
+}
+
+template <typename K>
+hipError_t launch_one_pass_join_t(const PipelineDevice& d, bool tables, uint32_t grid, hipStream_t stream) {
+  if (!tables) {
+    // 64 KiB tables: two blocks of 512 threads per CU; 128 KiB: one of 1024
+    if (d.big_block_tables) return launch_part_join<K, 2 * kSlots<K>, 1024>(d, (grid + 1) / 2, stream);
+    return launch_part_join<K, kSlots<K>, 512>(d, grid, stream);
+  }
+  // no build partition can exceed a table the whole build side fits
+  if (d.hbm_cap == 0 || d.build.n <= pipeline_block_table_tuples(sizeof(K) == 4 ? KeyType::I32 : KeyType::I64,
+                                                                 d.big_block_tables != 0))
+    return hipSuccess;
+  hipLaunchKernelGGL((part_table_kernel<K, 512>), dim3(grid), dim3(512), 0, stream, d);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return launch_hbm_clear(d, sizeof(Tuple<K>), grid, stream);
+}
+
+}  // namespace
+
+uint32_t pipeline_block_table_tuples(KeyType t, bool big) {
+  return (t == KeyType::I32 ? kSlots<int32_t> : kSlots<int64_t>) * (big ? 2 : 1) * 3 / 4;
+}
+
+hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchSide* sides, uint32_t joins,
+                                hipStream_t stream) {
+  if (joins == 0) return hipSuccess;
+  const uint32_t F1j = d.F1 / joins;
+  if (sides) {
+    hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(1024), 0, stream, d.work_counter);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(one_pass_plan_kernel, dim3(joins), dim3(1024), 3 * F1j * 4, stream, d, sides, F1j,
+                     pipeline_block_table_tuples(t, d.big_block_tables != 0));
+  return hipGetLastError();
+}
+
+hipError_t launch_one_pass_join(const PipelineDevice& d, KeyType t, bool tables, uint32_t grid, hipStream_t stream) {
+  if (t == KeyType::I32) return launch_one_pass_join_t<int32_t>(d, tables, grid, stream);
+  return launch_one_pass_join_t<int64_t>(d, tables, grid, stream);
+}
+
+}  // namespace fij

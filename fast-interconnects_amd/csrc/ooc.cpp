@@ -328,8 +328,8 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
       OOC_HIP(launch_pipeline_plan(d, st[s]));
       const uint32_t tiles = static_cast<uint32_t>((g.len[0] + g.len[1]) / tile2 + 2 * d.F1);
       OOC_HIP(launch_pipeline_sort2(d, kt, std::max(1u, std::min(cus, tiles)), st[s]));
-      OOC_HIP(launch_pipeline_join(d, kt, false, false, join_grid, st[s]));
-      OOC_HIP(launch_pipeline_join(d, kt, false, true, join_grid, st[s]));
+      OOC_HIP(launch_pipeline_join(d, kt, false, join_grid, st[s]));
+      OOC_HIP(launch_pipeline_join(d, kt, true, join_grid, st[s]));
       OOC_HIP(launch_sum_aggregates(d.aggregates, join_grid, results + gi, st[s]));
     }
     return FIJ_OK;

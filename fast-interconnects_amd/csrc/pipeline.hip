@@ -17,17 +17,22 @@
 //               probing) and probes the probe runs, aggregating match count,
 //               SUM(build.value) and SUM(probe.value)
 //
-// With bits2 == 0 (single pass) the join reads the pass-1 chunk pieces
-// directly.  Work items of the join are taken from an atomic counter so that
-// skewed partitions do not serialise a fixed wave; pairs too large for a
-// wave's registers are deferred, split into work units and joined from
-// block-shared (join_block_kernel) or wave LDS tables (join_general_kernel).
+// Work items of the join are taken from an atomic counter so that skewed
+// partitions do not serialise a fixed wave; pairs too large for a wave's
+// registers are deferred, split into work units and joined from block-shared
+// (join_block_kernel) or wave LDS tables (join_general_kernel).
+//
+// With bits2 == 0 (single pass) two launches follow pass 1:
+// one_pass_plan_kernel cuts every partition pair into work units, and
+// part_join_kernel streams each unit's probe tuples, contiguous in the pass-1
+// relation, against a block-shared LDS table of its build partition.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <vector>
 
 #include "common.hpp"
+#include "hbm_table.hpp"
 #include "internal.hpp"
 #include "pipeline.hpp"
 
@@ -55,7 +60,7 @@ __global__ __launch_bounds__(1024) void plan_kernel(PipelineDevice d) {
     const uint32_t n = static_cast<uint32_t>(e - b);
     s.plen[p] = n;
     starts[p] = n;
-    tiles[p] = d.bits2 ? (n + d.tile2 - 1) / d.tile2 : 0;
+    tiles[p] = (n + d.tile2 - 1) / d.tile2;
   }
   __syncthreads();
   const uint64_t total = block_exclusive_scan<uint64_t>(starts, F1, wave_tmp);
@@ -106,7 +111,7 @@ __global__ __launch_bounds__(1024) void plan_batched_kernel(PipelineDevice d, co
     const uint32_t n = static_cast<uint32_t>(e - b);
     s.plen[vp] = n;
     starts[p] = n;
-    tiles[p] = d.bits2 ? (n + d.tile2 - 1) / d.tile2 : 0;
+    tiles[p] = (n + d.tile2 - 1) / d.tile2;
   }
   __syncthreads();
   block_exclusive_scan<uint64_t>(starts, F1j, wave_tmp);
@@ -184,8 +189,7 @@ __device__ __forceinline__ U uniform_load(const U* ptr) {
 // ------------------------------------------------------------- sort2 ----
 
 // Slots of the block-shared LDS table of a deferred item (64 KiB of keys and
-// values; twice that in single-pass plans with big_block_tables); such an
-// item's build side may fill 3/4 of them.
+// values); such an item's build side may fill 3/4 of them.
 template <typename K>
 constexpr uint32_t kBlockTableSlots = 65536 / (2 * sizeof(K));
 
@@ -380,42 +384,30 @@ __global__ __launch_bounds__(BLOCK) void sort2_kernel(PipelineDevice d) {
 
 constexpr uint32_t kMaxRuns = 64;
 
-// Runs of one side of item (p, q): with two passes, one per pass-2 tile of
-// pass-1 partition p; with one pass, partition p cut into tile2-tuple pieces.
-__device__ __forceinline__ uint32_t run_count(const PipelineDevice& d, const PipelineSide& s, uint32_t p) {
-  if (d.bits2) return uniform_load(s.tile_start + p + 1) - uniform_load(s.tile_start + p);
-  return (uniform_load(s.plen + p) + d.tile2 - 1) / d.tile2;
+// Runs of one side of item (p, q): one per pass-2 tile of pass-1 partition p.
+__device__ __forceinline__ uint32_t run_count(const PipelineSide& s, uint32_t p) {
+  return uniform_load(s.tile_start + p + 1) - uniform_load(s.tile_start + p);
 }
 
-// Loaded, not yet combined, descriptor of run r0 + lane of item (p, q).  With
-// two passes run r is pass-2 digit q's range inside tile r of pass-1
-// partition p: a = first tuple of the tile, b0 = its meta word (start | end
-// << 16).  With one pass run r is piece r of partition p: a = its first
-// tuple, [b0, b1) = [0, its length).  Every lane loads from an in-bounds address
-// (lanes past the last run repeat it) and combining is left to the consumer:
-// no branch and no use follows the loads, so a prefetch does not make the
-// gathers issued before it wait.
+// Loaded, not yet combined, descriptor of run r0 + lane of item (p, q): run r
+// is pass-2 digit q's range inside tile r of pass-1 partition p; a = first
+// tuple of the tile, b = its meta word (start | end << 16).  Every lane loads
+// from an in-bounds address (lanes past the last run repeat it) and combining
+// is left to the consumer: no branch and no use follows the loads, so a
+// prefetch does not make the gathers issued before it wait.
 struct RawRun {
   uint64_t a;
-  uint32_t b0, b1;
+  uint32_t b;
 };
 
 // Descriptor of run r (in range) of item (p, q).
 __device__ __forceinline__ RawRun raw_run_at(const PipelineDevice& d, const PipelineSide& s, uint32_t p, uint32_t q,
                                              uint32_t r) {
   RawRun x;
-  if (d.bits2) {
-    // nruns == 0 reads row tile_start[p] <= tiles: the meta has a spare row
-    const uint32_t tile = uniform_load(s.tile_start + p) + r;
-    x.a = uniform_load(s.pstart + p) + static_cast<uint64_t>(r) * d.tile2;
-    x.b0 = s.meta[static_cast<uint64_t>(tile) * d.F2 + q];
-    x.b1 = 0;
-  } else {
-    const uint32_t plen = uniform_load(s.plen + p);
-    x.a = uniform_load(s.off1 + p) + static_cast<uint64_t>(r) * d.tile2;
-    x.b0 = 0;
-    x.b1 = min(d.tile2, plen - min(plen, r * d.tile2));
-  }
+  // nruns == 0 reads row tile_start[p] <= tiles: the meta has a spare row
+  const uint32_t tile = uniform_load(s.tile_start + p) + r;
+  x.a = uniform_load(s.pstart + p) + static_cast<uint64_t>(r) * d.tile2;
+  x.b = s.meta[static_cast<uint64_t>(tile) * d.F2 + q];
   return x;
 }
 
@@ -431,22 +423,18 @@ struct LaneRun {
   uint32_t len;
 };
 
-__device__ __forceinline__ LaneRun finish_run_at(const PipelineDevice& d, const RawRun& x, bool live) {
-  if (d.bits2) {
-    const uint32_t b = x.b0 & 0xffffu, e = x.b0 >> 16;
-    return LaneRun{x.a + b, live ? e - b : 0u};
-  }
-  return LaneRun{x.a, live ? x.b1 - x.b0 : 0u};
+__device__ __forceinline__ LaneRun finish_run_at(const RawRun& x, bool live) {
+  const uint32_t b = x.b & 0xffffu, e = x.b >> 16;
+  return LaneRun{x.a + b, live ? e - b : 0u};
 }
 
-__device__ __forceinline__ LaneRun finish_run(const PipelineDevice& d, const RawRun& x, uint32_t r0,
-                                              uint32_t nruns) {
-  return finish_run_at(d, x, r0 + lane_id() < nruns);
+__device__ __forceinline__ LaneRun finish_run(const RawRun& x, uint32_t r0, uint32_t nruns) {
+  return finish_run_at(x, r0 + lane_id() < nruns);
 }
 
 __device__ __forceinline__ LaneRun lane_run(const PipelineDevice& d, const PipelineSide& s, uint32_t p, uint32_t q,
                                             uint32_t r0, uint32_t nruns) {
-  return finish_run(d, raw_run(d, s, p, q, r0, nruns), r0, nruns);
+  return finish_run(raw_run(d, s, p, q, r0, nruns), r0, nruns);
 }
 
 // Per-wave LDS copy of one side's run batch: run starts and the exclusive
@@ -582,7 +570,7 @@ __device__ __forceinline__ void join_item_general(const PipelineDevice& d, uint3
   // every build tuple of the item joins the probe runs [pr0, pr1)
   const WaveTable<K, K, CAP> tab{table_keys, table_keys + CAP};
   const uint32_t lane = lane_id();
-  const uint32_t nb = run_count(d, d.build, p);
+  const uint32_t nb = run_count(d.build, p);
   for (uint32_t rb0 = 0; rb0 < nb; rb0 += kMaxRuns) {
     const uint32_t tb = publish_runs(lane_run(d, d.build, p, q, rb0, nb), rb);
     wave_lds_sync();
@@ -766,12 +754,6 @@ __device__ __forceinline__ void lane_item_side(const PipelineDevice& d, const Pi
                                                uint64_t& tuples) {
   runs = 0;
   tuples = 0;
-  if (!d.bits2) {
-    const uint32_t plen = live ? s.plen[p] : 0u;
-    runs = (plen + d.tile2 - 1) / d.tile2;
-    tuples = slice == 0 ? plen : 0u;
-    return;
-  }
   const uint32_t t0 = s.tile_start[p];
   runs = live ? s.tile_start[p + 1] - t0 : 0u;
   uint32_t most = runs;
@@ -796,7 +778,7 @@ __global__ __launch_bounds__(kUnitsWaves * 64) void join_units_kernel(PipelineDe
   __shared__ uint32_t s_ticket;
   __shared__ uint64_t part[2][kUnitsWaves][64];
   const uint32_t lane = lane_id(), w = threadIdx.x / 64;
-  const uint32_t F2 = d.bits2 ? d.F2 : 1;
+  const uint32_t F2 = d.F2;
   const uint32_t items = d.F1 * F2;
   for (;;) {
     if (threadIdx.x == 0) s_ticket = atomicAdd(d.work_counter + kOverflowTicket, 1u);
@@ -888,9 +870,9 @@ __global__ __launch_bounds__(WAVES * 64) void join_general_kernel(PipelineDevice
   extern __shared__ uint64_t lds_u64[];
   const WaveLds<K, CAP> l(lds_u64);
   const uint32_t lane = lane_id();
-  const uint32_t F2 = d.bits2 ? d.F2 : 1;
-  const T* rel_b = static_cast<const T*>(d.bits2 ? d.build.rel2 : d.build.rel1);
-  const T* rel_p = static_cast<const T*>(d.bits2 ? d.probe.rel2 : d.probe.rel1);
+  const uint32_t F2 = d.F2;
+  const T* rel_b = static_cast<const T*>(d.build.rel2);
+  const T* rel_p = static_cast<const T*>(d.probe.rel2);
   uint64_t cnt = 0, sb = 0, sp = 0;
   const uint32_t n = uniform_load(d.work_counter + kOverflowAny) ? uniform_load(d.work_counter + kWaveUnitCount) : 0;
   if (n) {
@@ -941,7 +923,7 @@ __device__ __forceinline__ uint32_t publish_block_runs(const PipelineDevice& d, 
                                                        uint32_t* wave_sums) {
   const uint32_t tid = threadIdx.x, w = tid / 64;
   const uint32_t r = r0 + tid;
-  const LaneRun x = finish_run_at(d, raw_run_at(d, s, p, q, min(r, nruns - 1)), r < nruns);
+  const LaneRun x = finish_run_at(raw_run_at(d, s, p, q, min(r, nruns - 1)), r < nruns);
   const uint32_t incl = wave_inclusive_scan(x.len);
   if (lane_id() == 63) wave_sums[w] = incl;
   __syncthreads();
@@ -1048,9 +1030,9 @@ __global__ __launch_bounds__(BLOCK) void join_block_kernel(PipelineDevice d) {
   uint32_t* const run_prefix = reinterpret_cast<uint32_t*>(run_start + BLOCK);
   const BlockRuns br{run_start, run_prefix, reinterpret_cast<uint16_t*>(run_prefix + BLOCK)};
   const uint32_t tid = threadIdx.x;
-  const uint32_t F2 = d.bits2 ? d.F2 : 1;
-  const T* rel_b = static_cast<const T*>(d.bits2 ? d.build.rel2 : d.build.rel1);
-  const T* rel_p = static_cast<const T*>(d.bits2 ? d.probe.rel2 : d.probe.rel1);
+  const uint32_t F2 = d.F2;
+  const T* rel_b = static_cast<const T*>(d.build.rel2);
+  const T* rel_p = static_cast<const T*>(d.probe.rel2);
   uint64_t cnt = 0, sb = 0, sp = 0;
   const uint32_t n = uniform_load(d.work_counter + kOverflowAny) ? uniform_load(d.work_counter + kUnitCount) : 0;
   auto clear = [&]() {
@@ -1069,7 +1051,7 @@ __global__ __launch_bounds__(BLOCK) void join_block_kernel(PipelineDevice d) {
       const uint32_t item = __builtin_amdgcn_readfirstlane(unit.x);
       const uint32_t p = item / F2, q = item % F2;
       const uint32_t pr0 = __builtin_amdgcn_readfirstlane(unit.y), pr1 = __builtin_amdgcn_readfirstlane(unit.z);
-      const uint32_t nb = run_count(d, d.build, p);
+      const uint32_t nb = run_count(d.build, p);
       for (uint32_t r0 = 0; r0 < nb; r0 += BLOCK) {
         const uint32_t tb = publish_block_runs<BLOCK>(d, d.build, p, q, r0, nb, br, wave_sums);
         const uint32_t s0 = publish_block_buckets<BLOCK>(br, min(nb - r0, BLOCK), tb);
@@ -1115,55 +1097,12 @@ __global__ __launch_bounds__(BLOCK) void join_block_kernel(PipelineDevice d) {
 
 // ----------------------------------------------------- HBM hash tables ----
 // A deferred item whose build side exceeds a block's LDS table gets a
-// linear-probing table of 2^lg slots (at least twice its build tuples) in
-// the plan's HBM arena: its build units insert the build side once, then its
-// probe units probe it, so the cost is linear in both sides (the LDS path
-// refills a wave table once per RCAP build tuples and streams the unit's
-// probe runs against every fill).  Hashing and probing follow the
-// no-partitioning join (no_partitioning_join.cu:39-249): multiply-shift from
-// the key, linear probing, every match counted; i32 entries are installed
-// by one 64-bit CAS of key and payload against an all-ones entry, i64 by a
-// CAS on the key and then the payload store.  The arena is all ones between
-// joins: the clear kernel restores the slots a join reserved.
-
-template <typename K>
-__device__ __forceinline__ void hbm_insert(Tuple<K>* tab, uint32_t lg, K key, K val) {
-  const uint64_t mask = (1ull << lg) - 1;
-  uint64_t h = mult_shift_hash<K>(key, lg);
-  for (uint64_t a = 0; a <= mask; ++a, h = (h + 1) & mask) {
-    if constexpr (sizeof(K) == 4) {
-      const unsigned long long want = static_cast<unsigned long long>(static_cast<uint32_t>(key)) |
-                                      (static_cast<unsigned long long>(static_cast<uint32_t>(val)) << 32);
-      if (atomicCAS(reinterpret_cast<unsigned long long*>(tab + h), ~0ull, want) == ~0ull) return;
-    } else {
-      if (atomicCAS(reinterpret_cast<unsigned long long*>(&tab[h].key), ~0ull, static_cast<unsigned long long>(key)) ==
-          ~0ull) {
-        tab[h].value = val;
-        return;
-      }
-    }
-  }
-}
-
-// Every build tuple with this key matches; probing ends at the first free
-// slot.  (The i64 payload of a slot whose key was just installed may still
-// be in flight only while the build kernel runs; probes run in a later
-// launch.)
-template <typename K>
-__device__ __forceinline__ void hbm_probe(const Tuple<K>* tab, uint32_t lg, K key, K pay, uint64_t& cnt, uint64_t& sb,
-                                          uint64_t& sp) {
-  const uint64_t mask = (1ull << lg) - 1;
-  uint64_t h = mult_shift_hash<K>(key, lg);
-  for (uint64_t a = 0; a <= mask; ++a, h = (h + 1) & mask) {
-    const Tuple<K> e = load_tuple<K>(tab + h);
-    if (e.key == null_key<K>()) return;
-    if (e.key == key) {
-      cnt += 1;
-      sb += static_cast<uint64_t>(static_cast<int64_t>(e.value));
-      sp += static_cast<uint64_t>(static_cast<int64_t>(pay));
-    }
-  }
-}
+// linear-probing table (hbm_table.hpp) in the plan's HBM arena: its build
+// units insert the build side once, then its probe units probe it, so the
+// cost is linear in both sides (the LDS path refills a wave table once per
+// RCAP build tuples and streams the unit's probe runs against every fill).
+// The arena is all ones between joins: the clear kernel restores the slots a
+// join reserved.
 
 // One block per HBM work unit (tickets over build units when BUILD, else over
 // probe units): the unit's runs of its item's build (probe) side, published
@@ -1178,9 +1117,9 @@ __global__ __launch_bounds__(BLOCK) void join_hbm_kernel(PipelineDevice d) {
   __shared__ uint16_t run_bucket[2 * BLOCK + 4];
   const BlockRuns br{run_start, run_prefix, run_bucket};
   const uint32_t tid = threadIdx.x;
-  const uint32_t F2 = d.bits2 ? d.F2 : 1;
+  const uint32_t F2 = d.F2;
   const PipelineSide& side = BUILD ? d.build : d.probe;
-  const T* rel = static_cast<const T*>(d.bits2 ? side.rel2 : side.rel1);
+  const T* rel = static_cast<const T*>(side.rel2);
   T* const arena = static_cast<T*>(d.hbm_table);
   uint64_t cnt = 0, sb = 0, sp = 0;
   const uint32_t n = uniform_load(d.work_counter + kOverflowAny)
@@ -1229,7 +1168,6 @@ __global__ __launch_bounds__(BLOCK) void join_hbm_kernel(PipelineDevice d) {
 
 // Restores the slots reserved in this join to all ones (16-byte stores).
 __global__ __launch_bounds__(256) void join_hbm_clear_kernel(PipelineDevice d, uint32_t tuple_bytes) {
-  if (uniform_load(d.work_counter + kOverflowAny) == 0) return;
   const uint64_t reserved = *reinterpret_cast<const volatile uint64_t*>(d.work_counter + kHbmSlots);
   const uint64_t slots = min<uint64_t>(reserved, d.hbm_cap);
   uint4* w = static_cast<uint4*>(d.hbm_table);
@@ -1264,10 +1202,10 @@ __global__ __launch_bounds__(WAVES * 64) void join_kernel(PipelineDevice d) {
   WaveTable<K, K, CAP>{table_keys, table_keys + CAP}.clear();
   for (uint32_t i = lane; i < 2 * kMarkBytes / 4; i += 64) reinterpret_cast<uint32_t*>(l.mb)[i] = 0;
   wave_lds_sync();
-  const T* rel_b = static_cast<const T*>(d.bits2 ? d.build.rel2 : d.build.rel1);
-  const T* rel_p = static_cast<const T*>(d.bits2 ? d.probe.rel2 : d.probe.rel1);
+  const T* rel_b = static_cast<const T*>(d.build.rel2);
+  const T* rel_p = static_cast<const T*>(d.probe.rel2);
   const uint32_t F1 = d.F1;
-  const uint32_t F2 = d.bits2 ? d.F2 : 1;
+  const uint32_t F2 = d.F2;
   const uint32_t shift = d.bits1 + d.bits2;
   const uint32_t items = F1 * F2;
   const T* const dummy = reinterpret_cast<const T*>(d.aggregates);  // 16 readable bytes, value unused
@@ -1313,8 +1251,8 @@ __global__ __launch_bounds__(WAVES * 64) void join_kernel(PipelineDevice d) {
   // current item's gathers without making them wait.
   auto fetch = [&](uint32_t i) {
     const uint32_t p = i / F2, q = i % F2;
-    nb = run_count(d, d.build, p);
-    np = run_count(d, d.probe, p);
+    nb = run_count(d.build, p);
+    np = run_count(d.probe, p);
     xb = raw_run(d, d.build, p, q, 0, nb);
     xp = raw_run(d, d.probe, p, q, 0, np);
   };
@@ -1347,7 +1285,7 @@ __global__ __launch_bounds__(WAVES * 64) void join_kernel(PipelineDevice d) {
 #pragma unroll
     for (uint32_t k = 0; k < SPL; ++k) ip[k] = 0;
     if (live) {
-      const LaneRun lb = finish_run(d, xb, 0, nb), lp = finish_run(d, xp, 0, np);
+      const LaneRun lb = finish_run(xb, 0, nb), lp = finish_run(xp, 0, np);
       tb = publish_runs(lb, rb);
       tp = publish_runs(lp, rp);
       wave_lds_sync();
@@ -1445,10 +1383,6 @@ hipError_t launch_sum_aggregates(const JoinAggregate* src, uint32_t n, JoinAggre
   return hipGetLastError();
 }
 
-uint32_t pipeline_block_table_tuples(KeyType t, bool big) {
-  return (t == KeyType::I32 ? kBlockTableSlots<int32_t> : kBlockTableSlots<int64_t>) * (big ? 2 : 1) * 3 / 4;
-}
-
 uint32_t pipeline_tile2(KeyType t) { return t == KeyType::I32 ? kTile2<int32_t> : kTile2<int64_t>; }
 
 hipError_t launch_pipeline_plan(const PipelineDevice& d, hipStream_t stream) {
@@ -1526,7 +1460,7 @@ static uint32_t register_join_lanes(uint64_t side_tuples, uint64_t items) {
 // more waves per CU.
 template <typename K, uint32_t CAP, uint32_t WAVES>
 hipError_t launch_register_join_sized(const PipelineDevice& d, uint32_t grid, hipStream_t stream) {
-  const uint64_t items = static_cast<uint64_t>(d.F1) * (d.bits2 ? d.F2 : 1u);
+  const uint64_t items = static_cast<uint64_t>(d.F1) * d.F2;
   const uint32_t bpl = register_join_lanes(d.build.n, items), spl = register_join_lanes(d.probe.n, items);
   if (bpl == 10 && spl == 10) return launch_register_join<K, CAP, WAVES, 10, 10>(d, grid, stream);
   if (spl == 10) {
@@ -1540,9 +1474,8 @@ hipError_t launch_register_join_sized(const PipelineDevice& d, uint32_t grid, hi
   return launch_register_join<K, CAP / 2, WAVES, 4, 4>(d, grid, stream);
 }
 
-// The deferred items' joins with block-shared tables of BCAP slots: 64 KiB
-// (two blocks of 512 threads per CU) or, for single-pass plans whose build
-// partitions need it, 128 KiB (one block per CU).
+// The deferred items' joins with block-shared tables of BCAP slots (64 KiB:
+// two blocks of 512 threads per CU).
 template <typename K, uint32_t BCAP, uint32_t GCAP, uint32_t GWAVES>
 hipError_t launch_deferred_t(const PipelineDevice& d, uint32_t grid, hipStream_t stream) {
   constexpr uint32_t BBLOCK = 512;
@@ -1571,34 +1504,23 @@ hipError_t launch_deferred_t(const PipelineDevice& d, uint32_t grid, hipStream_t
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL((join_hbm_kernel<K, 512, 8, false>), dim3(grid), dim3(512), 0, stream, d);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(join_hbm_clear_kernel, dim3(grid), dim3(256), 0, stream, d,
-                     static_cast<uint32_t>(sizeof(Tuple<K>)));
+  return launch_hbm_clear(d, sizeof(Tuple<K>), grid, stream);
+}
+
+hipError_t launch_hbm_clear(const PipelineDevice& d, uint32_t tuple_bytes, uint32_t grid, hipStream_t stream) {
+  hipLaunchKernelGGL(join_hbm_clear_kernel, dim3(grid), dim3(256), 0, stream, d, tuple_bytes);
   return hipGetLastError();
 }
 
-template <typename K, uint32_t CAP, uint32_t WAVES, uint32_t GCAP, uint32_t GWAVES>
+template <typename K, uint32_t GCAP>
 hipError_t launch_join_t(const PipelineDevice& d, bool deferred, uint32_t grid, hipStream_t stream) {
-  if (!deferred) {
-    // large tables (single-pass plans): one shape
-    if constexpr (CAP > 1024)
-      return launch_register_join<K, CAP, WAVES, 10, 10>(d, grid, stream);
-    else
-      return launch_register_join_sized<K, CAP, WAVES>(d, grid, stream);
-  }
-  if constexpr (CAP > 1024) {
-    if (d.big_block_tables) return launch_deferred_t<K, 2 * kBlockTableSlots<K>, GCAP, GWAVES>(d, grid, stream);
-  }
-  return launch_deferred_t<K, kBlockTableSlots<K>, GCAP, GWAVES>(d, grid, stream);
+  if (!deferred) return launch_register_join_sized<K, 1024, 4>(d, grid, stream);
+  return launch_deferred_t<K, kBlockTableSlots<K>, GCAP, 4>(d, grid, stream);
 }
 
-hipError_t launch_pipeline_join(const PipelineDevice& d, KeyType t, bool large_tables, bool deferred, uint32_t grid,
-                                hipStream_t stream) {
-  if (t == KeyType::I32) {
-    if (large_tables) return launch_join_t<int32_t, 8192, 2, 8192, 2>(d, deferred, grid, stream);
-    return launch_join_t<int32_t, 1024, 4, 4096, 4>(d, deferred, grid, stream);
-  }
-  if (large_tables) return launch_join_t<int64_t, 4096, 2, 4096, 2>(d, deferred, grid, stream);
-  return launch_join_t<int64_t, 1024, 4, 2048, 4>(d, deferred, grid, stream);
+hipError_t launch_pipeline_join(const PipelineDevice& d, KeyType t, bool deferred, uint32_t grid, hipStream_t stream) {
+  if (t == KeyType::I32) return launch_join_t<int32_t, 4096>(d, deferred, grid, stream);
+  return launch_join_t<int64_t, 2048>(d, deferred, grid, stream);
 }
 
 }  // namespace fij

@@ -60,6 +60,20 @@ constexpr uint32_t kHbmBuildTicket = (kJoinCounters + 10) * kJoinCounterStride;
 constexpr uint32_t kHbmProbeTicket = (kJoinCounters + 11) * kJoinCounterStride;
 constexpr uint32_t kJoinCounterWords = (kJoinCounters + 12) * kJoinCounterStride;
 
+// One work unit of a single-pass join: a whole pass-1 build partition against
+// a range of its probe partition (tuple indices in rel1).
+struct PartUnit {
+  uint64_t build_at, probe_at;
+  uint32_t build_n, probe_n;
+  uint32_t part, reserved;
+};
+// Probe tuples of a unit: at least kPartUnitMin (or the whole partition), so
+// that at most one unit per partition and one per kPartUnitMin tuples exist.
+constexpr uint32_t kPartUnitMin = 8192;
+inline uint64_t part_unit_cap(uint64_t partitions, uint64_t probe_len) {
+  return partitions + probe_len / kPartUnitMin + 1;
+}
+
 struct PipelineDevice {
   PipelineSide build;
   PipelineSide probe;
@@ -72,6 +86,7 @@ struct PipelineDevice {
   uint8_t* overflow;          // [F1 * F2] 1 = item deferred to the general join (zero between joins)
   uint4* units;               // [unit_cap] {item, first probe run, end probe run, 1 = wave table}
   uint32_t unit_cap;          // at least the items plus one per 65,536 probe tuples
+  PartUnit* part_units;       // single-pass plans: [part_unit_cap(F1, probe tuples)]
   JoinAggregate* aggregates;  // [agg_len]
   uint32_t agg_len;
   // Many joins in one plan (batched joins): pass-1 partition p belongs to
@@ -176,9 +191,19 @@ hipError_t launch_pipeline_plan_batched(const PipelineDevice& d, const BatchSide
 hipError_t launch_pipeline_sort2(const PipelineDevice& d, KeyType t, uint32_t grid, hipStream_t stream);
 // dst = the sum of the n per-block aggregates src (one block).
 hipError_t launch_sum_aggregates(const JoinAggregate* src, uint32_t n, JoinAggregate* dst, hipStream_t stream);
-// The register-resident join of every work item (deferred = false), then
-// the join of the items it deferred (deferred = true).
-hipError_t launch_pipeline_join(const PipelineDevice& d, KeyType t, bool large_tables, bool deferred, uint32_t grid,
+// Restores the HBM-arena slots that a join reserved to all ones.
+hipError_t launch_hbm_clear(const PipelineDevice& d, uint32_t tuple_bytes, uint32_t grid, hipStream_t stream);
+// Two passes: the register-resident join of every work item (deferred =
+// false), then the join of the items it deferred (deferred = true).
+hipError_t launch_pipeline_join(const PipelineDevice& d, KeyType t, bool deferred, uint32_t grid, hipStream_t stream);
+// Single pass, instead of the plan and join launches of two: partition
+// lengths and work units of the joins in d (sides of join j in sides[2 j],
+// sides[2 j + 1]; one join and sides == nullptr for a plan of its own), reset
+// of the join counters and aggregates (or of the joins' results).
+hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchSide* sides, uint32_t joins,
                                 hipStream_t stream);
+// ... the join of every unit and the builds of HBM hash tables, and (tables =
+// true, a launch of its own so that it can be timed) their probes.
+hipError_t launch_one_pass_join(const PipelineDevice& d, KeyType t, bool tables, uint32_t grid, hipStream_t stream);
 
 }  // namespace fij

@@ -32,7 +32,6 @@ struct fij_join_plan {
   uint32_t g1_cap;
   uint32_t block1;
   uint32_t lds_total;
-  bool large_tables;
   std::vector<void*> allocs;
   hipEvent_t ev[6];
   JoinAggregate* host_agg;
@@ -144,7 +143,6 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
   p->d.tile2 = pipeline_tile2(kt);
   p->d.sides = 3;
   p->block1 = cfg->pass1_block ? std::min<uint32_t>(cfg->pass1_block, 1024) : 1024;
-  p->large_tables = cfg->radix_bits_2 == 0;
   p->join_grid = cfg->join_blocks ? cfg->join_blocks : cus * 2;
   p->d.agg_len = p->join_grid;
   fij_status st = FIJ_OK;
@@ -170,14 +168,16 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
   if (st == FIJ_OK) st = alloc_side(p, p->d.probe, cfg->probe_len, p->max_tiles[1]);
   if (st == FIJ_OK) st = alloc(p, &p->d.work_counter, kJoinCounterWords);
   const uint64_t items = static_cast<uint64_t>(p->d.F1) * (p->d.bits2 ? p->d.F2 : 1);
-  if (st == FIJ_OK) st = alloc(p, &p->d.overflow, items);
   // work units of deferred items: at most one per item plus one per 65536
   // probe tuples
   p->d.unit_cap = static_cast<uint32_t>(items + cfg->probe_len / 65536 + 1);
-  if (st == FIJ_OK) st = alloc(p, &p->d.units, p->d.unit_cap);
+  if (st == FIJ_OK && p->d.bits2) st = alloc(p, &p->d.overflow, items);
+  if (st == FIJ_OK && p->d.bits2) st = alloc(p, &p->d.units, p->d.unit_cap);
+  if (st == FIJ_OK && !p->d.bits2) st = alloc(p, &p->d.part_units, part_unit_cap(items, cfg->probe_len));
   // the deferred-item flags start at zero (complete before any stream uses
   // them); every join leaves them at zero
-  if (st == FIJ_OK && (hipMemset(p->d.overflow, 0, items) != hipSuccess || hipDeviceSynchronize() != hipSuccess))
+  if (st == FIJ_OK && p->d.bits2 &&
+      (hipMemset(p->d.overflow, 0, items) != hipSuccess || hipDeviceSynchronize() != hipSuccess))
     st = plan_fail(FIJ_DEVICE_ERROR, "clearing the deferred-item flags failed");
   // HBM hash tables of deferred items with large build sides: an arena of
   // 2^k slots, twice the build relation (at most 2^26 slots), every word all
@@ -267,12 +267,20 @@ fij_status enqueue_join(fij_join_plan* p, const void* build_keys, const void* bu
   if (events) PLAN_HIP(hipEventRecord(p->ev[1], st));
   PLAN_HIP(enqueue_pass1_scatter(d, p->kt, p->block1, p->lds_total, st));
   if (events) PLAN_HIP(hipEventRecord(p->ev[2], st));
-  PLAN_HIP(launch_pipeline_plan(d, st));
-  if (d.bits2) PLAN_HIP(launch_pipeline_sort2(d, p->kt, p->sort2_grid, st));
-  if (events) PLAN_HIP(hipEventRecord(p->ev[3], st));
-  PLAN_HIP(launch_pipeline_join(d, p->kt, p->large_tables, false, p->join_grid, st));
-  if (events) PLAN_HIP(hipEventRecord(p->ev[4], st));
-  PLAN_HIP(launch_pipeline_join(d, p->kt, p->large_tables, true, p->join_grid, st));
+  if (d.bits2) {
+    PLAN_HIP(launch_pipeline_plan(d, st));
+    PLAN_HIP(launch_pipeline_sort2(d, p->kt, p->sort2_grid, st));
+    if (events) PLAN_HIP(hipEventRecord(p->ev[3], st));
+    PLAN_HIP(launch_pipeline_join(d, p->kt, false, p->join_grid, st));
+    if (events) PLAN_HIP(hipEventRecord(p->ev[4], st));
+    PLAN_HIP(launch_pipeline_join(d, p->kt, true, p->join_grid, st));
+  } else {
+    PLAN_HIP(launch_one_pass_plan(d, p->kt, nullptr, 1, st));
+    if (events) PLAN_HIP(hipEventRecord(p->ev[3], st));
+    PLAN_HIP(launch_one_pass_join(d, p->kt, false, p->join_grid, st));
+    if (events) PLAN_HIP(hipEventRecord(p->ev[4], st));
+    PLAN_HIP(launch_one_pass_join(d, p->kt, true, p->join_grid, st));
+  }
   if (events) {
     PLAN_HIP(hipEventRecord(p->ev[5], st));
     PLAN_HIP(hipMemcpyAsync(p->host_agg, d.aggregates, sizeof(JoinAggregate) * p->join_grid, hipMemcpyDeviceToHost,

@@ -101,6 +101,7 @@ struct Slot {
   uint8_t* overflow = nullptr;
   uint4* units = nullptr;
   uint32_t unit_cap = 0;
+  PartUnit* part_units = nullptr;
   JoinAggregate* aggregates = nullptr;
   JoinAggregate* d_result = nullptr;
   JoinAggregate* h_result = nullptr;
@@ -189,18 +190,21 @@ fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
   d.overflow = sl.overflow;
   d.units = sl.units;
   d.unit_cap = sl.unit_cap;
+  d.part_units = sl.part_units;
   d.aggregates = sl.aggregates;
   hipStream_t st = sl.stream;
   SRV_HIP(enqueue_pass1_prefix_sum(d, s->kt, 1024, st));
   SRV_HIP(enqueue_pass1_scatter(d, s->kt, 1024, s->lds_total, st));
-  SRV_HIP(launch_pipeline_plan(d, st));
   if (d.bits2) {
+    SRV_HIP(launch_pipeline_plan(d, st));
     const uint32_t tiles = static_cast<uint32_t>(r.len / d.tile2 + d.F1);
     SRV_HIP(launch_pipeline_sort2(d, s->kt, std::max(1u, std::min(s->cus, tiles)), st));
+    SRV_HIP(launch_pipeline_join(d, s->kt, false, s->join_grid, st));
+    SRV_HIP(launch_pipeline_join(d, s->kt, true, s->join_grid, st));
+  } else {
+    SRV_HIP(launch_one_pass_plan(d, s->kt, nullptr, 1, st));
+    SRV_HIP(launch_one_pass_join(d, s->kt, false, s->join_grid, st));
   }
-  const bool large = d.bits2 == 0;
-  SRV_HIP(launch_pipeline_join(d, s->kt, large, false, s->join_grid, st));
-  SRV_HIP(launch_pipeline_join(d, s->kt, large, true, s->join_grid, st));
   SRV_HIP(launch_sum_aggregates(sl.aggregates, s->join_grid, sl.d_result, st));
   SRV_HIP(hipMemcpyAsync(sl.h_result, sl.d_result, sizeof(JoinAggregate), hipMemcpyDeviceToHost, st));
   SRV_HIP(hipEventRecord(sl.done, st));
@@ -284,6 +288,7 @@ fij_status make_slot(fij_join_server* s, Slot& sl, uint64_t probe_cap) {
   SRV_HIP(hipMemset(sl.overflow, 0, items));
   sl.unit_cap = static_cast<uint32_t>(items + probe_cap / 65536 + 1);
   SRV_HIP(alloc(reinterpret_cast<void**>(&sl.units), sl.unit_cap * sizeof(uint4)));
+  SRV_HIP(alloc(reinterpret_cast<void**>(&sl.part_units), part_unit_cap(kMaxF1, probe_cap) * sizeof(PartUnit)));
   SRV_HIP(alloc(reinterpret_cast<void**>(&sl.aggregates), s->join_grid * sizeof(JoinAggregate)));
   SRV_HIP(alloc(reinterpret_cast<void**>(&sl.d_result), sizeof(JoinAggregate)));
   SRV_HIP(hipHostMalloc(reinterpret_cast<void**>(&sl.h_result), sizeof(JoinAggregate), hipHostMallocDefault));
