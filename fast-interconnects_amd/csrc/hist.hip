@@ -159,6 +159,7 @@ struct HistPair {
 template <typename K>
 __global__ __launch_bounds__(kHistBlockMax) void hist_pair_kernel(HistPair s, uint32_t ga) {
   const uint32_t i = blockIdx.x < ga ? 0u : 1u;
+  if (s.side[0].stamp && blockIdx.x == 0 && threadIdx.x == 0) *s.side[0].stamp = wall_clock64();
   const HistParams p = s.side[i];
   hist_body<K, false, false>(p, i ? blockIdx.x - ga : blockIdx.x, i ? gridDim.x - ga : ga);
 }

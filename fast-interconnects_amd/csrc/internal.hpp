@@ -102,6 +102,7 @@ struct HistParams {
   uint32_t* counts;    // contiguous: [G][F]
   uint64_t* scan_state;
   uint64_t scan_state_len;
+  uint64_t* stamp;     // time of the launch's start, or nullptr
 };
 
 // Contiguous histogram parameters of one relation of a paired or batched
@@ -141,6 +142,7 @@ struct PartitionLaunch {
   void* spill = nullptr;
   uint64_t spill_base = 0;
   uint32_t spill_from = 0;
+  uint64_t* stamp = nullptr;  // time of the launch's start, or nullptr
 };
 hipError_t launch_partition(const PartitionLaunch& a, hipStream_t stream);
 // Buffered scatters of two relations of one type, radix bits and block (no
@@ -160,6 +162,7 @@ struct ScatterParams {
   uint32_t queue_len;    // line queue entries per step buffer
   uintptr_t spill_addr;  // address tuple index 0 would have in the spill region
   uint32_t spill_from;   // first partition written to the spill region
+  uint64_t* stamp;       // time of the launch's start, or nullptr
 };
 
 // Scatter descriptor of one relation of a batched launch: the line ring is

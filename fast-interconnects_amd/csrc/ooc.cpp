@@ -330,7 +330,7 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
       OOC_HIP(launch_pipeline_sort2(d, kt, std::max(1u, std::min(cus, tiles)), st[s]));
       OOC_HIP(launch_pipeline_join(d, kt, false, join_grid, st[s]));
       OOC_HIP(launch_pipeline_join(d, kt, true, join_grid, st[s]));
-      OOC_HIP(launch_sum_aggregates(d.aggregates, join_grid, results + gi, st[s]));
+      OOC_HIP(launch_sum_aggregates(d.aggregates, join_grid, results + gi, nullptr, st[s]));
     }
     return FIJ_OK;
   };

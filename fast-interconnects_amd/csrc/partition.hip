@@ -53,10 +53,16 @@ __device__ __forceinline__ void chunk_range(const ScatterParams& p, uint32_t chu
   len = (chunk + 1 == G) ? p.n - begin : min(p.chunk_len, p.n - begin);
 }
 
+// Time of the launch's start (timed joins).
+__device__ __forceinline__ void stamp_start(uint64_t* stamp) {
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
+}
+
 // Direct scatter (reference NC): per-chunk LDS cursors, wave-aggregated ranks.
 template <typename K, bool SPILL>
 __global__ __launch_bounds__(1024) void scatter_direct_kernel(ScatterParams p) {
   extern __shared__ uint32_t cursors[];
+  stamp_start(p.stamp);
   const uint32_t F = 1u << p.radix_bits;
   const uint64_t mask = radix_mask(p.radix_bits, p.ignore_bits);
   const uint32_t tid = threadIdx.x, B = blockDim.x;
@@ -97,6 +103,7 @@ __global__ __launch_bounds__(BLOCK) void scatter_tile_kernel(ScatterParams p) {
   constexpr uint32_t TILE = ITEMS * BLOCK;
   extern __shared__ __attribute__((aligned(16))) uint64_t lds_u64[];
   __shared__ uint32_t wave_tmp[BLOCK / kWave + 1];
+  stamp_start(p.stamp);
   const uint32_t F = 1u << p.radix_bits;
   const uint64_t mask = radix_mask(p.radix_bits, p.ignore_bits);
   const uint32_t tid = threadIdx.x;
@@ -427,6 +434,7 @@ __device__ __forceinline__ void scatter_swwc_body(const ScatterParams& p, uint32
 
 template <typename K, int BLOCK, bool SPILL>
 __global__ __launch_bounds__(BLOCK) void scatter_swwc_kernel(ScatterParams p) {
+  stamp_start(p.stamp);
   scatter_swwc_body<K, BLOCK, SPILL>(p, blockIdx.x, gridDim.x);
 }
 
@@ -441,6 +449,7 @@ struct ScatterPair {
 template <typename K, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void scatter_swwc_pair_kernel(ScatterPair s, uint32_t ga) {
   const uint32_t i = blockIdx.x < ga ? 0u : 1u;
+  stamp_start(s.side[0].stamp);
   const ScatterParams p = s.side[i];
   scatter_swwc_body<K, BLOCK, false>(p, i ? blockIdx.x - ga : blockIdx.x, i ? gridDim.x - ga : ga);
 }
@@ -517,6 +526,7 @@ ScatterParams scatter_params(const PartitionLaunch& a) {
   p.ignore_bits = a.ignore_bits;
   p.chunk_offsets = a.chunk_offsets;
   p.relation = a.relation;
+  p.stamp = a.stamp;
   const uint32_t F = 1u << a.radix_bits;
   p.spill_from = a.spill != nullptr && a.spill_from < F ? a.spill_from : F;
   p.spill_addr = reinterpret_cast<uintptr_t>(a.spill) - static_cast<uintptr_t>(a.spill_base * sizeof(Tuple<K>));

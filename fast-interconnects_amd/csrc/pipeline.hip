@@ -49,6 +49,7 @@ namespace {
 __global__ __launch_bounds__(1024) void plan_kernel(PipelineDevice d) {
   extern __shared__ uint64_t buf[];
   __shared__ uint64_t wave_tmp[32];
+  stamp_phase(d.stamps, 2);
   const uint32_t rel = d.sides == 2 ? 1u : blockIdx.x;
   const PipelineSide& s = rel == 0 ? d.build : d.probe;
   const uint32_t F1 = d.F1;
@@ -774,6 +775,7 @@ __device__ __forceinline__ void lane_item_side(const PipelineDevice& d, const Pi
 }
 
 __global__ __launch_bounds__(kUnitsWaves * 64) void join_units_kernel(PipelineDevice d, uint32_t block_rcap) {
+  stamp_phase(d.stamps, 4);
   if (uniform_load(d.work_counter + kOverflowAny) == 0) return;
   __shared__ uint32_t s_ticket;
   __shared__ uint64_t part[2][kUnitsWaves][64];
@@ -1192,6 +1194,7 @@ __global__ __launch_bounds__(WAVES * 64) void join_kernel(PipelineDevice d) {
   constexpr uint32_t RCAP = CAP * 3 / 4;  // build tuples per table fill (load factor <= 3/4)
   constexpr uint32_t FAST_B = RCAP < BPL * 64 ? RCAP : BPL * 64;
   static_assert(WAVES <= 16, "aggregate scratch");
+  stamp_phase(d.stamps, 3);
   extern __shared__ uint64_t lds_u64[];
   const WaveLds<K, CAP> l(lds_u64);
   K* const table_keys = l.table_keys;
@@ -1349,7 +1352,7 @@ size_t sort2_lds_bytes(uint32_t F2) {
 
 // dst = the sum of src[0..n) (one block; wrapping 64-bit sums).
 __global__ __launch_bounds__(256) void sum_aggregates_kernel(const JoinAggregate* src, uint32_t n,
-                                                             JoinAggregate* dst) {
+                                                             JoinAggregate* dst, uint64_t* stamps) {
   __shared__ uint64_t red[3][4];
   uint64_t c = 0, b = 0, p = 0;
   for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
@@ -1371,6 +1374,7 @@ __global__ __launch_bounds__(256) void sum_aggregates_kernel(const JoinAggregate
     dst->count = red[0][0] + red[0][1] + red[0][2] + red[0][3];
     dst->sum_build = red[1][0] + red[1][1] + red[1][2] + red[1][3];
     dst->sum_probe = red[2][0] + red[2][1] + red[2][2] + red[2][3];
+    stamp_phase(stamps, 5);
   }
 }
 
@@ -1378,8 +1382,9 @@ __global__ __launch_bounds__(256) void sum_aggregates_kernel(const JoinAggregate
 
 // ------------------------------------------------------------- launches ----
 
-hipError_t launch_sum_aggregates(const JoinAggregate* src, uint32_t n, JoinAggregate* dst, hipStream_t stream) {
-  hipLaunchKernelGGL(sum_aggregates_kernel, dim3(1), dim3(256), 0, stream, src, n, dst);
+hipError_t launch_sum_aggregates(const JoinAggregate* src, uint32_t n, JoinAggregate* dst, uint64_t* stamps,
+                                 hipStream_t stream) {
+  hipLaunchKernelGGL(sum_aggregates_kernel, dim3(1), dim3(256), 0, stream, src, n, dst, stamps);
   return hipGetLastError();
 }
 

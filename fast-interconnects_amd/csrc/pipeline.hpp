@@ -60,6 +60,15 @@ constexpr uint32_t kHbmBuildTicket = (kJoinCounters + 10) * kJoinCounterStride;
 constexpr uint32_t kHbmProbeTicket = (kJoinCounters + 11) * kJoinCounterStride;
 constexpr uint32_t kJoinCounterWords = (kJoinCounters + 12) * kJoinCounterStride;
 
+// Phase stamps of a timed join (the device's constant-rate clock, written to
+// pinned host memory by the first block of a phase as it starts; the last
+// one as the result is written): histograms, scatter, pass 2, join, deferred
+// joins, end.  Events between the phases cost 5.5 us of device time each.
+constexpr uint32_t kStamps = 6;
+__device__ __forceinline__ void stamp_phase(uint64_t* stamps, uint32_t phase) {
+  if (stamps && blockIdx.x == 0 && threadIdx.x == 0) stamps[phase] = wall_clock64();
+}
+
 // One work unit of a single-pass join: a whole pass-1 build partition against
 // a range of its probe partition (tuple indices in rel1).
 struct PartUnit {
@@ -89,6 +98,7 @@ struct PipelineDevice {
   PartUnit* part_units;       // single-pass plans: [part_unit_cap(F1, probe tuples)]
   JoinAggregate* aggregates;  // [agg_len]
   uint32_t agg_len;
+  uint64_t* stamps;           // [kStamps] or nullptr: not timed
   // Many joins in one plan (batched joins): pass-1 partition p belongs to
   // join p >> job_shift, whose count and sums are added to
   // job_results[job_slot[join]] instead of the per-block aggregates.
@@ -189,8 +199,23 @@ hipError_t launch_pipeline_plan_batched(const PipelineDevice& d, const BatchSide
                                         hipStream_t stream);
 // Pass 2 of both relations in one persistent launch of `grid` blocks.
 hipError_t launch_pipeline_sort2(const PipelineDevice& d, KeyType t, uint32_t grid, hipStream_t stream);
-// dst = the sum of the n per-block aggregates src (one block).
-hipError_t launch_sum_aggregates(const JoinAggregate* src, uint32_t n, JoinAggregate* dst, hipStream_t stream);
+// dst = the sum of the n per-block aggregates src (one block); the end stamp of
+// a timed join.
+hipError_t launch_sum_aggregates(const JoinAggregate* src, uint32_t n, JoinAggregate* dst, uint64_t* stamps,
+                                 hipStream_t stream);
+// One join whose build side fits a block's LDS table (table_join_tuples): one
+// launch without partitioning.  partial: at least max_grid entries; done: a
+// word that is zero between joins.
+struct TableJoin {
+  const void *build_keys, *build_pays, *probe_keys, *probe_pays;
+  uint64_t n_b, n_p;
+  JoinAggregate* partial;
+  uint32_t* done;
+  JoinAggregate* result;
+  uint64_t* stamps;  // or nullptr
+};
+uint64_t table_join_tuples(KeyType t);
+hipError_t launch_table_join(KeyType t, const TableJoin& j, uint32_t cus, uint32_t max_grid, hipStream_t stream);
 // Restores the HBM-arena slots that a join reserved to all ones.
 hipError_t launch_hbm_clear(const PipelineDevice& d, uint32_t tuple_bytes, uint32_t grid, hipStream_t stream);
 // Two passes: the register-resident join of every work item (deferred =
@@ -204,6 +229,9 @@ hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchS
                                 hipStream_t stream);
 // ... the join of every unit and the builds of HBM hash tables, and (tables =
 // true, a launch of its own so that it can be timed) their probes.
+// Whether any build partition can need an HBM table (none can exceed an LDS
+// table that holds the whole build side): else the second launch does nothing.
+bool one_pass_tables(const PipelineDevice& d, KeyType t);
 hipError_t launch_one_pass_join(const PipelineDevice& d, KeyType t, bool tables, uint32_t grid, hipStream_t stream);
 
 }  // namespace fij

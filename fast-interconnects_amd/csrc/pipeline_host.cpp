@@ -107,7 +107,8 @@ PartitionLaunch scatter_of(const PipelineDevice& d, const PipelineSide& s, KeyTy
 hipError_t enqueue_pass1_prefix_sum(const PipelineDevice& d, KeyType t, uint32_t block, hipStream_t stream) {
   const PipelineSide* a = side_of(d, 0) ? side_of(d, 0) : side_of(d, 1);
   const PipelineSide* b = d.sides == 3 ? &d.probe : nullptr;
-  const HistParams ha = hist_params(t, a->keys, a->n, a->g1, d.bits1, block, a->counts1, a->scan1);
+  HistParams ha = hist_params(t, a->keys, a->n, a->g1, d.bits1, block, a->counts1, a->scan1);
+  ha.stamp = d.stamps;
   const HistParams hb = b ? hist_params(t, b->keys, b->n, b->g1, d.bits1, block, b->counts1, b->scan1) : ha;
   const hipError_t e = launch_hist_pair(t, ha, hb, a->g1, b ? b->g1 : 0, block, stream);
   if (e != hipSuccess) return e;
@@ -117,10 +118,10 @@ hipError_t enqueue_pass1_prefix_sum(const PipelineDevice& d, KeyType t, uint32_t
 
 hipError_t enqueue_pass1_scatter(const PipelineDevice& d, KeyType t, uint32_t block, uint32_t lds_total,
                                  hipStream_t stream) {
-  if (d.sides == 3)
-    return launch_partition_pair(scatter_of(d, d.build, t, block, lds_total),
-                                 scatter_of(d, d.probe, t, block, lds_total), stream);
-  return launch_partition(scatter_of(d, d.sides & 1 ? d.build : d.probe, t, block, lds_total), stream);
+  PartitionLaunch a = scatter_of(d, d.sides & 1 ? d.build : d.probe, t, block, lds_total);
+  a.stamp = d.stamps ? d.stamps + 1 : nullptr;
+  if (d.sides == 3) return launch_partition_pair(a, scatter_of(d, d.probe, t, block, lds_total), stream);
+  return launch_partition(a, stream);
 }
 
 }  // namespace fij

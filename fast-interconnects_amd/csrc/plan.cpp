@@ -33,8 +33,16 @@ struct fij_join_plan {
   uint32_t block1;
   uint32_t lds_total;
   std::vector<void*> allocs;
-  hipEvent_t ev[6];
-  JoinAggregate* host_agg;
+  uint32_t cus;
+  uint32_t clock_khz;  // rate of the device clock the phases are stamped with
+  uint32_t* done;      // finished blocks of a table join, zero between joins
+  // what the last enqueued join wrote or did not launch
+  struct Host {
+    JoinAggregate result;
+    uint64_t stamps[kStamps];
+  };
+  Host* host;
+  enum class Timed { None, Phases, NoDeferred, OneLaunch } timed;
 };
 
 namespace {
@@ -72,9 +80,7 @@ fij_status alloc(fij_join_plan* p, T** out, uint64_t count) {
 void release(fij_join_plan* p) {
   for (void* a : p->allocs) (void)hipFree(a);
   p->allocs.clear();
-  for (hipEvent_t& e : p->ev)
-    if (e) (void)hipEventDestroy(e);
-  if (p->host_agg) (void)hipHostFree(p->host_agg);
+  if (p->host) (void)hipHostFree(p->host);
 }
 
 fij_status alloc_side(fij_join_plan* p, PipelineSide& s, uint64_t n, uint32_t tiles) {
@@ -126,9 +132,14 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
     lds_total = std::max<uint32_t>(lds_total, static_cast<uint32_t>(optin));
   const uint32_t cus = static_cast<uint32_t>(prop.multiProcessorCount);
 
+  int clock_khz = 0;
+  PLAN_HIP(hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, dev));
+
   fij_join_plan* p = new fij_join_plan();
-  std::memset(p->ev, 0, sizeof(p->ev));
-  p->host_agg = nullptr;
+  p->clock_khz = static_cast<uint32_t>(std::max(clock_khz, 1));
+  p->host = nullptr;
+  p->timed = fij_join_plan::Timed::None;
+  p->cus = cus;
   p->cfg = *cfg;
   p->kt = kt;
   p->lds_total = lds_total;
@@ -189,6 +200,10 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
     p->d.big_cap = static_cast<uint32_t>(std::min<uint64_t>(items, slots / 256));
     p->d.hbm_unit_cap =
         static_cast<uint32_t>(2ull * p->d.big_cap + (cfg->build_len + cfg->probe_len) / 65536 + 2);
+    // (the block counter of table joins is cleared with the arena)
+    if (st == FIJ_OK) st = alloc(p, &p->done, 1);
+    if (st == FIJ_OK && hipMemset(p->done, 0, sizeof(uint32_t)) != hipSuccess)
+      st = plan_fail(FIJ_DEVICE_ERROR, "clearing the block counter failed");
     void* arena = nullptr;
     if (st == FIJ_OK && hipMalloc(&arena, slots * tuple_bytes(kt)) != hipSuccess)
       st = plan_fail(FIJ_OUT_OF_MEMORY, "cannot allocate the HBM hash-table arena");
@@ -201,11 +216,10 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
       st = plan_fail(FIJ_DEVICE_ERROR, "initialising the HBM hash-table arena failed");
   }
   if (st == FIJ_OK) st = alloc(p, &p->d.aggregates, p->join_grid);
-  for (int i = 0; i < 6 && st == FIJ_OK; ++i)
-    if (hipEventCreate(&p->ev[i]) != hipSuccess) st = plan_fail(FIJ_DEVICE_ERROR, "hipEventCreate failed");
-  if (st == FIJ_OK && hipHostMalloc(reinterpret_cast<void**>(&p->host_agg), sizeof(JoinAggregate) * p->join_grid,
+  if (st == FIJ_OK && hipHostMalloc(reinterpret_cast<void**>(&p->host), sizeof(fij_join_plan::Host),
                                     hipHostMallocDefault) != hipSuccess)
-    st = plan_fail(FIJ_OUT_OF_MEMORY, "cannot allocate pinned aggregates");
+    st = plan_fail(FIJ_OUT_OF_MEMORY, "cannot allocate the pinned result");
+  if (st == FIJ_OK) std::memset(p->host, 0, sizeof(fij_join_plan::Host));
   if (st != FIJ_OK) {
     release(p);
     delete p;
@@ -227,11 +241,11 @@ fij_status fij_join_plan_destroy(fij_join_plan* plan) {
 namespace {
 
 // Enqueues one join of the plan's shape over columns of n_b and n_p tuples
-// (at most the plan's lengths).  With events, the phases are timed and the
-// per-block aggregates are copied to the host; otherwise (capturable: no
-// events, no copies) they are summed into *device_result.
+// (at most the plan's lengths): launches only, so it can be captured.  The
+// result goes to *device_result or, timed, with the phases' stamps to the
+// plan's pinned memory (device_result == nullptr).
 fij_status enqueue_join(fij_join_plan* p, const void* build_keys, const void* build_pays, uint64_t n_b,
-                        const void* probe_keys, const void* probe_pays, uint64_t n_p, bool events,
+                        const void* probe_keys, const void* probe_pays, uint64_t n_p,
                         fij_join_aggregate* device_result, hipStream_t st) {
   if (n_b > p->cfg.build_len || n_p > p->cfg.probe_len)
     return plan_fail(FIJ_INVALID_ARGUMENT, "join of %llu x %llu tuples exceeds the plan's %llu x %llu",
@@ -244,7 +258,18 @@ fij_status enqueue_join(fij_join_plan* p, const void* build_keys, const void* bu
   for (const void* c : {build_keys, build_pays, probe_keys, probe_pays})
     if (c && reinterpret_cast<uintptr_t>(c) % kb)
       return plan_fail(FIJ_INVALID_ARGUMENT, "input columns must be aligned to their element size");
+  using Timed = fij_join_plan::Timed;
+  JoinAggregate* result = device_result ? reinterpret_cast<JoinAggregate*>(device_result) : &p->host->result;
+  uint64_t* stamps = device_result ? nullptr : p->host->stamps;
+  if (n_b <= table_join_tuples(p->kt)) {
+    // the whole build side fits a block's LDS table: no partitioning
+    const TableJoin j{build_keys, build_pays, probe_keys, probe_pays, n_b, n_p, p->d.aggregates, p->done, result, stamps};
+    PLAN_HIP(launch_table_join(p->kt, j, p->cus, p->join_grid, st));
+    if (!device_result) p->timed = Timed::OneLaunch;
+    return FIJ_OK;
+  }
   PipelineDevice& d = p->d;
+  d.stamps = stamps;
   d.build.keys = build_keys;
   d.build.pays = build_pays;
   d.probe.keys = probe_keys;
@@ -262,32 +287,22 @@ fij_status enqueue_join(fij_join_plan* p, const void* build_keys, const void* bu
     split_chunks(p->kt, n_b, n_p, p->g1_cap, &d.build.g1, &d.probe.g1);
   }
   d.big_block_tables = d.bits2 ? 0u : big_block_tables_for(p->kt, n_b, d.F1);
-  if (events) PLAN_HIP(hipEventRecord(p->ev[0], st));
   PLAN_HIP(enqueue_pass1_prefix_sum(d, p->kt, p->block1, st));
-  if (events) PLAN_HIP(hipEventRecord(p->ev[1], st));
   PLAN_HIP(enqueue_pass1_scatter(d, p->kt, p->block1, p->lds_total, st));
-  if (events) PLAN_HIP(hipEventRecord(p->ev[2], st));
+  Timed timed = Timed::Phases;
   if (d.bits2) {
     PLAN_HIP(launch_pipeline_plan(d, st));
     PLAN_HIP(launch_pipeline_sort2(d, p->kt, p->sort2_grid, st));
-    if (events) PLAN_HIP(hipEventRecord(p->ev[3], st));
     PLAN_HIP(launch_pipeline_join(d, p->kt, false, p->join_grid, st));
-    if (events) PLAN_HIP(hipEventRecord(p->ev[4], st));
     PLAN_HIP(launch_pipeline_join(d, p->kt, true, p->join_grid, st));
   } else {
     PLAN_HIP(launch_one_pass_plan(d, p->kt, nullptr, 1, st));
-    if (events) PLAN_HIP(hipEventRecord(p->ev[3], st));
     PLAN_HIP(launch_one_pass_join(d, p->kt, false, p->join_grid, st));
-    if (events) PLAN_HIP(hipEventRecord(p->ev[4], st));
     PLAN_HIP(launch_one_pass_join(d, p->kt, true, p->join_grid, st));
+    if (!one_pass_tables(d, p->kt)) timed = Timed::NoDeferred;
   }
-  if (events) {
-    PLAN_HIP(hipEventRecord(p->ev[5], st));
-    PLAN_HIP(hipMemcpyAsync(p->host_agg, d.aggregates, sizeof(JoinAggregate) * p->join_grid, hipMemcpyDeviceToHost,
-                            st));
-  }
-  if (device_result)
-    PLAN_HIP(launch_sum_aggregates(d.aggregates, p->join_grid, reinterpret_cast<JoinAggregate*>(device_result), st));
+  PLAN_HIP(launch_sum_aggregates(d.aggregates, p->join_grid, result, stamps, st));
+  if (!device_result) p->timed = timed;
   return FIJ_OK;
 }
 
@@ -298,7 +313,7 @@ extern "C" {
 fij_status fij_join_plan_enqueue(fij_join_plan* p, const void* build_keys, const void* build_pays,
                                  const void* probe_keys, const void* probe_pays, void* stream) {
   if (!p) return plan_fail(FIJ_INVALID_ARGUMENT, "plan is NULL");
-  return enqueue_join(p, build_keys, build_pays, p->cfg.build_len, probe_keys, probe_pays, p->cfg.probe_len, true,
+  return enqueue_join(p, build_keys, build_pays, p->cfg.build_len, probe_keys, probe_pays, p->cfg.probe_len,
                       nullptr, static_cast<hipStream_t>(stream));
 }
 
@@ -306,37 +321,34 @@ fij_status fij_join_plan_enqueue_sized(fij_join_plan* p, const void* build_keys,
                                        uint64_t build_len, const void* probe_keys, const void* probe_pays,
                                        uint64_t probe_len, fij_join_aggregate* device_result, void* stream) {
   if (!p || !device_result) return plan_fail(FIJ_INVALID_ARGUMENT, "plan or result is NULL");
-  return enqueue_join(p, build_keys, build_pays, build_len, probe_keys, probe_pays, probe_len, false, device_result,
+  return enqueue_join(p, build_keys, build_pays, build_len, probe_keys, probe_pays, probe_len, device_result,
                       static_cast<hipStream_t>(stream));
 }
 
 fij_status fij_join_plan_result(fij_join_plan* p, void* stream, fij_join_aggregate* result, fij_join_timing* timing) {
   if (!p) return plan_fail(FIJ_INVALID_ARGUMENT, "plan is NULL");
   PLAN_HIP(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
-  if (result) {
-    uint64_t c = 0, b = 0, s = 0;
-    for (uint32_t i = 0; i < p->join_grid; ++i) {
-      c += p->host_agg[i].count;
-      b += p->host_agg[i].sum_build;
-      s += p->host_agg[i].sum_probe;
-    }
-    result->count = c;
-    result->sum_build = b;
-    result->sum_probe = s;
-  }
+  const fij_join_plan::Host& h = *p->host;
+  if (result) *result = fij_join_aggregate{h.result.count, h.result.sum_build, h.result.sum_probe};
   if (timing) {
-    float ms[6] = {0, 0, 0, 0, 0, 0};
-    const int from[6] = {0, 1, 2, 0, 2, 3}, to[6] = {1, 2, 5, 5, 3, 4};
-    for (int i = 0; i < 6; ++i) PLAN_HIP(hipEventElapsedTime(&ms[i], p->ev[from[i]], p->ev[to[i]]));
-    float deferred = 0;
-    PLAN_HIP(hipEventElapsedTime(&deferred, p->ev[4], p->ev[5]));
-    timing->prefix_sum_ms = ms[0];
-    timing->partition_ms = ms[1];
-    timing->join_ms = ms[2];
-    timing->total_ms = ms[3];
-    timing->pass2_ms = ms[4];
-    timing->build_probe_ms = ms[5];
-    timing->deferred_ms = deferred;
+    using Timed = fij_join_plan::Timed;
+    if (p->timed == Timed::None) return plan_fail(FIJ_DEVICE_ERROR, "no join of this plan has been enqueued");
+    auto ms = [&](uint32_t from, uint32_t to) {
+      return static_cast<float>(static_cast<double>(h.stamps[to] - h.stamps[from]) / p->clock_khz);
+    };
+    *timing = fij_join_timing{};
+    timing->total_ms = ms(0, 5);
+    if (p->timed == Timed::OneLaunch) {
+      timing->join_ms = timing->build_probe_ms = timing->total_ms;
+    } else {
+      const bool deferred = p->timed == Timed::Phases;
+      timing->prefix_sum_ms = ms(0, 1);
+      timing->partition_ms = ms(1, 2);
+      timing->join_ms = ms(2, 5);
+      timing->pass2_ms = ms(2, 3);
+      timing->build_probe_ms = ms(3, deferred ? 4 : 5);
+      timing->deferred_ms = deferred ? ms(4, 5) : 0.0f;
+    }
   }
   return FIJ_OK;
 }

@@ -172,7 +172,7 @@ fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
     hipStream_t st = sl.stream;
     SRV_HIP(launch_np_probe_resident(s->kt, b.table, b.table_lg, r.keys, r.pays, r.len, sl.aggregates, s->join_grid,
                                      st));
-    SRV_HIP(launch_sum_aggregates(sl.aggregates, s->join_grid, sl.d_result, st));
+    SRV_HIP(launch_sum_aggregates(sl.aggregates, s->join_grid, sl.d_result, nullptr, st));
     SRV_HIP(hipMemcpyAsync(sl.h_result, sl.d_result, sizeof(JoinAggregate), hipMemcpyDeviceToHost, st));
     SRV_HIP(hipEventRecord(sl.done, st));
     return FIJ_OK;
@@ -205,7 +205,7 @@ fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
     SRV_HIP(launch_one_pass_plan(d, s->kt, nullptr, 1, st));
     SRV_HIP(launch_one_pass_join(d, s->kt, false, s->join_grid, st));
   }
-  SRV_HIP(launch_sum_aggregates(sl.aggregates, s->join_grid, sl.d_result, st));
+  SRV_HIP(launch_sum_aggregates(sl.aggregates, s->join_grid, sl.d_result, nullptr, st));
   SRV_HIP(hipMemcpyAsync(sl.h_result, sl.d_result, sizeof(JoinAggregate), hipMemcpyDeviceToHost, st));
   SRV_HIP(hipEventRecord(sl.done, st));
   return FIJ_OK;
