@@ -1019,9 +1019,11 @@ __device__ __forceinline__ void block_elements(const BlockRuns& br, const uint32
 // not runs: a batch of up to BLOCK runs is published block-wide and every
 // thread takes elements tid, tid + BLOCK, ... of it, SPL loads in flight, so
 // a unit of a few long runs (a heavy key, a small build side against a long
-// probe side) keeps every wave busy.
+// probe side) keeps every wave busy.  The loads in flight are as many as leave
+// two blocks per CU (128 VGPRs): 2^24.25 + 2^28 int64 tuples took 12.5 ms with
+// one block of 16 loads, 9.8 ms with two that spill, 8.8 ms with 12 loads.
 template <typename K, uint32_t CAP, uint32_t BLOCK, uint32_t SPL>
-__global__ __launch_bounds__(BLOCK) void join_block_kernel(PipelineDevice d) {
+__global__ __launch_bounds__(BLOCK, 4) void join_block_kernel(PipelineDevice d) {
   using T = Tuple<K>;
   extern __shared__ uint64_t lds_u64[];
   __shared__ uint32_t s_unit;
@@ -1488,7 +1490,7 @@ hipError_t launch_deferred_t(const PipelineDevice& d, uint32_t grid, hipStream_t
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   {
-    auto blk = join_block_kernel<K, BCAP, BBLOCK, 16>;
+    auto blk = join_block_kernel<K, BCAP, BBLOCK, sizeof(K) == 4 ? 16 : 12>;
     const size_t lds = BCAP * 2 * sizeof(K) + block_runs_bytes<BBLOCK>();
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(blk), hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(lds));
