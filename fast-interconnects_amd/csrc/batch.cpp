@@ -321,8 +321,18 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
   d.build.n = rel2[0];
   d.probe.n = rel2[1];
   d.big_block_tables = 0;
-  if (b2 == 0)
-    for (uint32_t j = 0; j < J; ++j) d.big_block_tables |= big_block_tables_for(kt, lay[2 * j].n, F1);
+  if (b2 == 0) {
+    // the build partitions' size, which chooses the block table: the mean over
+    // build tuples (large joins dominate the class's time)
+    double sum = 0, squares = 0;
+    for (uint32_t j = 0; j < J; ++j) {
+      const double n = static_cast<double>(lay[2 * j].n);
+      d.big_block_tables |= big_block_tables_for(kt, lay[2 * j].n, F1);
+      sum += n;
+      squares += n * n;
+    }
+    d.build.n = static_cast<uint64_t>(sum > 0 ? squares / sum * J : 0.0);
+  }
   a.sub_joins = J;
   a.sub_blocks = blocks;
   a.sub_tiles[0] = static_cast<uint32_t>(tiles[0]);

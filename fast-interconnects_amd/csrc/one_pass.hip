@@ -4,9 +4,9 @@
 //
 //   one_pass_plan_kernel  partition lengths, and work units {build range, probe
 //                         range} of every partition pair; a build partition
-//                         beyond the LDS table gets a hash table in the HBM
-//                         arena when the arena has room, else its units fill
-//                         the LDS table several times
+//                         beyond the LDS table fills it several times, beyond
+//                         kMaxFills fills it gets a hash table in the HBM arena
+//                         when the arena has room
 //   part_join_kernel      one block per unit: the build range goes into a
 //                         block-shared table, the probe range is streamed
 //                         against it; then the build sides of the HBM tables
@@ -20,6 +20,8 @@
 #include "internal.hpp"
 #include "pipeline.hpp"
 
+#include <algorithm>
+
 namespace fij {
 namespace {
 
@@ -28,17 +30,24 @@ __device__ __forceinline__ U uniform_load(const U* ptr) {
   return *(const __attribute__((address_space(4))) U*)(ptr);
 }
 
-// Slots of the block-shared table: 64 KiB of keys and values, or 128 KiB
-// (big_block_tables).  A build range may fill 3/4 of them.
+// Slots of the block-shared table: 64 KiB of keys and values, half of that
+// for small partitions, or 128 KiB (big_block_tables).  A build range may fill
+// 3/4 of them.
 template <typename K>
 constexpr uint32_t kSlots = 65536 / (2 * sizeof(K));
 
 constexpr uint32_t kTableUnitTuples = 65536;  // tuples of an HBM-table work unit
 
-// Probe tuples of a unit: 8 times its build tuples (a unit's build work is
-// paid once per unit), between kPartUnitMin and 65,536.
+// Table fills a build partition may take where the arena has room for a table:
+// every fill streams the probe tuples again (about 3 TB/s), an HBM table costs
+// a random access per probe tuple (about 45 G/s).
+constexpr uint32_t kMaxFills = 4;
+
+// Probe tuples of a unit, about: 16 times its build tuples (a unit's build work
+// is paid once per unit: 20 batched joins of 2^18..2^20 int32 build tuples took
+// 349 us with 8 times, 283 us with 16), between kPartUnitMin and 65,536.
 __device__ __forceinline__ uint32_t unit_tuples(uint32_t build_n) {
-  return min(65536u, max(kPartUnitMin, 8 * min(build_n, 8192u)));
+  return min(65536u, max(kPartUnitMin, 16 * min(build_n, 4096u)));
 }
 
 // One block per join.  `sides` == nullptr: one join, whose sides end at their
@@ -68,10 +77,11 @@ __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, c
     uint64_t at;
     const uint32_t nb = range(d.build, end_b, p, at), np = range(d.probe, end_p, p, at);
     uint32_t units = 0;
-    const uint32_t ut = unit_tuples(nb);
+    uint32_t ut = unit_tuples(nb);
     if (nb && np) {
       units = (np + ut - 1) / ut;
-      if (nb > rcap && d.hbm_cap && nb <= (d.hbm_cap >> 1)) {
+      ut = (np + units - 1) / units;  // even units
+      if (nb > kMaxFills * rcap && d.hbm_cap && nb <= (d.hbm_cap >> 1)) {
         // an HBM table of at least twice the build tuples, if the arena (at
         // most 2^26 slots) has room.  A partition that finds none takes no
         // slots; the sum of the others' stays below 2^32.
@@ -184,15 +194,16 @@ struct TupleVec {
 // Joins the work units, one block per unit (the first by block index, the rest
 // by ticket, taken while the current unit runs).
 //
-// Bound by the read of the probe partitions and, for short units, by the chain
-// ticket -> unit -> tuples and the table's build.  2^20 + 2^24 int32 tuples in
-// 512 partitions: 44 us (3.2 TB/s) where the two-pass plans' register join
-// (23 us, every item only put off), unit counting (8 us) and block join (48
-// us, every tuple's run looked up although a partition is one run) ran before;
-// 20 batched joins of 2^18..2^20 int32 build tuples 1,053 -> 300 us.  Two and
-// four vectors per buffer, two or four probes together, blocks of 256 to 1,024
-// threads and 32 KiB tables all lie within 43-50 us; the smallest register
-// need was taken.
+// Bound by the read of the probe partitions (with inserts and probes left out
+// of a copy: 36 of 46 us, 126 of 186 us, 230 of 240 us for the shapes below),
+// plus what the phases of a block do not overlap.  2^20 + 2^24 int32 tuples in
+// 512 partitions: 46 us, where the two-pass plans' register join (23 us, every
+// item only put off), unit counting (8 us) and block join (48 us, every
+// tuple's run looked up although a partition is one run) ran before; 20 batched
+// joins of 2^18..2^20 int32 build tuples 1,053 -> 240 us; 5,000,011 +
+// 20,000,003 int64 tuples (two fills) 186 us.  Two and four vectors per buffer,
+// two or four probes together and build tuples loaded a fill ahead all lay
+// within 3 % of each other; the smallest register need was taken.
 template <typename K, uint32_t CAP, uint32_t BLOCK>
 __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
   using V = TupleVec<K>;
@@ -237,8 +248,10 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
     uint32_t wave_cnt = 0;
     VT xa[NV], xb[NV];
     load(xa, 0);  // in flight while the table is built
-    for (uint32_t f0 = 0; f0 < nb; f0 += RCAP) {
-      const uint32_t nf = min(RCAP, nb - f0);
+    // equal fills: the emptier the table, the fewer probes leave their bucket
+    const uint32_t fill = nb <= RCAP ? nb : (nb + (nb + RCAP - 1) / RCAP - 1) / ((nb + RCAP - 1) / RCAP);
+    for (uint32_t f0 = 0; f0 < nb; f0 += fill) {
+      const uint32_t nf = min(fill, nb - f0);
       // at most 1/4 full where the table allows it, 3/4 at most
       const uint32_t lg = min(LG_CAP, max(6u, 32u - static_cast<uint32_t>(__builtin_clz(nf))));
       using Quad = typename BucketTable<K>::Quad;
@@ -307,7 +320,7 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
         probe(xb, v0 + STEP);
         if (v0 + 2 * STEP >= nvp) break;
       }
-      if (f0 + RCAP < nb) __syncthreads();  // probes done before the table is cleared
+      if (f0 + fill < nb) __syncthreads();  // probes done before the table is cleared
     }
     if (lane_id() == 0) cnt += wave_cnt;
     if (tid == 0) s_next = gridDim.x + ticket;
@@ -365,9 +378,14 @@ hipError_t launch_part_join(const PipelineDevice& d, uint32_t grid, hipStream_t 
 template <typename K>
 hipError_t launch_one_pass_join_t(const PipelineDevice& d, bool tables, uint32_t grid, hipStream_t stream) {
   if (!tables) {
-    // 64 KiB tables: two blocks of 512 threads per CU; 128 KiB: one of 1024
-    if (d.big_block_tables) return launch_part_join<K, 2 * kSlots<K>, 1024>(d, (grid + 1) / 2, stream);
-    return launch_part_join<K, kSlots<K>, 512>(d, grid, stream);
+    // One block of 1,024 threads per CU with a 128 KiB table, two of 512 with
+    // 64 KiB, three with 32 KiB: those take partitions that fill them half on
+    // average (the batched joins above: 283 us with 64 KiB tables, 240 us).
+    auto blocks = [&](uint32_t n) { return d.job_results ? n : std::min(n, d.agg_len); };
+    if (d.big_block_tables) return launch_part_join<K, 2 * kSlots<K>, 1024>(d, blocks((grid + 1) / 2), stream);
+    if (d.build.n <= static_cast<uint64_t>(d.F1) * (kSlots<K> / 4))
+      return launch_part_join<K, kSlots<K> / 2, 512>(d, blocks(grid + grid / 2), stream);
+    return launch_part_join<K, kSlots<K>, 512>(d, blocks(grid), stream);
   }
   if (!one_pass_tables(d, sizeof(K) == 4 ? KeyType::I32 : KeyType::I64)) return hipSuccess;
   hipLaunchKernelGGL((part_table_kernel<K, 512>), dim3(grid), dim3(512), 0, stream, d);
@@ -383,7 +401,7 @@ uint32_t pipeline_block_table_tuples(KeyType t, bool big) {
 }
 
 bool one_pass_tables(const PipelineDevice& d, KeyType t) {
-  return d.hbm_cap != 0 && d.build.n > pipeline_block_table_tuples(t, d.big_block_tables != 0);
+  return d.hbm_cap != 0 && d.build.n > kMaxFills * pipeline_block_table_tuples(t, d.big_block_tables != 0);
 }
 
 hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchSide* sides, uint32_t joins,

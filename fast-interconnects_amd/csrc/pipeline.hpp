@@ -172,6 +172,15 @@ inline bool block_tables_hold(KeyType t, uint64_t build_len, uint64_t partitions
 inline bool one_pass_fits(KeyType t, uint64_t build_len) {
   return block_tables_hold(t, build_len, 1ull << kOnePassBits, true);
 }
+// Build tuples up to which a two-pass plan runs in a single pass of
+// kOnePassBits instead: its partitions hold at most two fills of a 128 KiB
+// table on average (1/16 of headroom for uneven ones).  Per probe tuple of t
+// bytes a second fill reads t again, a second pass reads and writes t and
+// gathers short runs: pass 2 and join of 5,000,011 x 20,000,003 int64 tuples
+// take 385 us in 8 + 8 bits and 200 us in a single pass with two fills.
+inline uint64_t one_pass_limit(KeyType t) {
+  return (2ull * pipeline_block_table_tuples(t, true) << kOnePassBits) * 15 / 16;
+}
 // Pass-2 bits of a two-pass plan of 9 + b2 bits whose items hold about a
 // third of a 64 KiB block table's build tuples (1,024 int64, 2,048 int32):
 // for probe sides far longer than the build side, whose items go to the

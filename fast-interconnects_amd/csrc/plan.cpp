@@ -26,6 +26,8 @@ struct fij_join_plan {
   fij_join_plan_config cfg;
   KeyType kt;
   PipelineDevice d;
+  PipelineDevice one;  // two-pass plans: the same buffers as a single pass of kOnePassBits
+  bool two_pass;       // the plan has pass-2 buffers
   uint32_t max_tiles[2];
   uint32_t sort2_grid;
   uint32_t join_grid;
@@ -83,8 +85,15 @@ void release(fij_join_plan* p) {
   if (p->host) (void)hipHostFree(p->host);
 }
 
+// Partitions the pass-1 buffers are sized for: the plan's own, or those of
+// the single pass that a two-pass plan may take.
+uint32_t pass1_fanout(const fij_join_plan* p) {
+  return p->d.bits2 ? std::max(p->d.F1, 1u << kOnePassBits) : p->d.F1;
+}
+
 fij_status alloc_side(fij_join_plan* p, PipelineSide& s, uint64_t n, uint32_t tiles) {
-  const hipError_t e = alloc_pipeline_side(s, p->kt, n, p->d.F1, p->d.F2, p->d.G1, p->d.bits2 != 0, tiles, p->allocs);
+  const hipError_t e =
+      alloc_pipeline_side(s, p->kt, n, pass1_fanout(p), p->d.F2, p->d.G1, p->two_pass, tiles, p->allocs);
   return e == hipSuccess ? FIJ_OK : hip_fail(e, "hipMalloc");
 }
 
@@ -155,7 +164,9 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
   p->d.sides = 3;
   p->block1 = cfg->pass1_block ? std::min<uint32_t>(cfg->pass1_block, 1024) : 1024;
   p->join_grid = cfg->join_blocks ? cfg->join_blocks : cus * 2;
-  p->d.agg_len = p->join_grid;
+  // aggregates: the joins with small tables keep more than two blocks per CU
+  p->d.agg_len = cfg->join_blocks ? cfg->join_blocks : cus * 4;
+  p->two_pass = p->d.bits2 && cfg->build_len > one_pass_limit(kt);
   fij_status st = FIJ_OK;
   const uint64_t lens[2] = {cfg->build_len, cfg->probe_len};
   for (int rel = 0; rel < 2 && st == FIJ_OK; ++rel) {
@@ -182,12 +193,12 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
   // work units of deferred items: at most one per item plus one per 65536
   // probe tuples
   p->d.unit_cap = static_cast<uint32_t>(items + cfg->probe_len / 65536 + 1);
-  if (st == FIJ_OK && p->d.bits2) st = alloc(p, &p->d.overflow, items);
-  if (st == FIJ_OK && p->d.bits2) st = alloc(p, &p->d.units, p->d.unit_cap);
-  if (st == FIJ_OK && !p->d.bits2) st = alloc(p, &p->d.part_units, part_unit_cap(items, cfg->probe_len));
+  if (st == FIJ_OK && p->two_pass) st = alloc(p, &p->d.overflow, items);
+  if (st == FIJ_OK && p->two_pass) st = alloc(p, &p->d.units, p->d.unit_cap);
+  if (st == FIJ_OK) st = alloc(p, &p->d.part_units, part_unit_cap(pass1_fanout(p), cfg->probe_len));
   // the deferred-item flags start at zero (complete before any stream uses
   // them); every join leaves them at zero
-  if (st == FIJ_OK && p->d.bits2 &&
+  if (st == FIJ_OK && p->two_pass &&
       (hipMemset(p->d.overflow, 0, items) != hipSuccess || hipDeviceSynchronize() != hipSuccess))
     st = plan_fail(FIJ_DEVICE_ERROR, "clearing the deferred-item flags failed");
   // HBM hash tables of deferred items with large build sides: an arena of
@@ -215,7 +226,7 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
                          hipDeviceSynchronize() != hipSuccess))
       st = plan_fail(FIJ_DEVICE_ERROR, "initialising the HBM hash-table arena failed");
   }
-  if (st == FIJ_OK) st = alloc(p, &p->d.aggregates, p->join_grid);
+  if (st == FIJ_OK) st = alloc(p, &p->d.aggregates, p->d.agg_len);
   if (st == FIJ_OK && hipHostMalloc(reinterpret_cast<void**>(&p->host), sizeof(fij_join_plan::Host),
                                     hipHostMallocDefault) != hipSuccess)
     st = plan_fail(FIJ_OUT_OF_MEMORY, "cannot allocate the pinned result");
@@ -225,6 +236,11 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
     delete p;
     return st;
   }
+  p->one = p->d;
+  p->one.bits1 = kOnePassBits;
+  p->one.bits2 = 0;
+  p->one.F1 = 1u << kOnePassBits;
+  p->one.F2 = 1;
   *out = p;
   return FIJ_OK;
 }
@@ -264,11 +280,14 @@ fij_status enqueue_join(fij_join_plan* p, const void* build_keys, const void* bu
   if (n_b <= table_join_tuples(p->kt)) {
     // the whole build side fits a block's LDS table: no partitioning
     const TableJoin j{build_keys, build_pays, probe_keys, probe_pays, n_b, n_p, p->d.aggregates, p->done, result, stamps};
-    PLAN_HIP(launch_table_join(p->kt, j, p->cus, p->join_grid, st));
+    PLAN_HIP(launch_table_join(p->kt, j, p->cus, p->d.agg_len, st));
     if (!device_result) p->timed = Timed::OneLaunch;
     return FIJ_OK;
   }
-  PipelineDevice& d = p->d;
+  // A two-pass plan's join of a build side that a single pass leaves in
+  // partitions of at most two table fills is run in one: the probe tuples are
+  // read once more instead of partitioned once more.
+  PipelineDevice& d = p->d.bits2 && n_b <= one_pass_limit(p->kt) ? p->one : p->d;
   d.stamps = stamps;
   d.build.keys = build_keys;
   d.build.pays = build_pays;
@@ -301,7 +320,7 @@ fij_status enqueue_join(fij_join_plan* p, const void* build_keys, const void* bu
     PLAN_HIP(launch_one_pass_join(d, p->kt, true, p->join_grid, st));
     if (!one_pass_tables(d, p->kt)) timed = Timed::NoDeferred;
   }
-  PLAN_HIP(launch_sum_aggregates(d.aggregates, p->join_grid, result, stamps, st));
+  PLAN_HIP(launch_sum_aggregates(d.aggregates, d.agg_len, result, stamps, st));
   if (!device_result) p->timed = timed;
   return FIJ_OK;
 }
@@ -363,14 +382,16 @@ fij_status fij_join_plan_execute(fij_join_plan* p, const void* build_keys, const
 
 fij_status fij_join_plan_device_bytes(const fij_join_plan* p, uint64_t* bytes) {
   if (!p || !bytes) return plan_fail(FIJ_INVALID_ARGUMENT, "NULL argument");
-  const uint64_t tb = tuple_bytes(p->kt);
+  const uint64_t tb = tuple_bytes(p->kt), F1 = pass1_fanout(p);
+  const uint64_t lens[2] = {p->cfg.build_len, p->cfg.probe_len};
   uint64_t total = 0;
-  for (const PipelineSide* s : {&p->d.build, &p->d.probe}) {
-    total += s->padded_len1 * tb + static_cast<uint64_t>(p->d.F1) * (p->d.G1 + 1) * 8;
-    total += static_cast<uint64_t>(p->d.F1) * p->d.G1 * 4 + s->scan1_len * 8 + p->d.F1 * 4 + (p->d.F1 + 1) * 12;
-    if (p->d.bits2) total += s->n * tb;
+  for (uint64_t n : lens) {
+    total += (n + F1 * p->d.pad) * tb + F1 * (p->d.G1 + 1ull) * 8;
+    total += F1 * p->d.G1 * 4 + scan_state_words(F1) * 8 + F1 * 4 + (F1 + 1) * 12;
+    if (p->two_pass) total += n * tb;
   }
-  if (p->d.bits2) total += (static_cast<uint64_t>(p->max_tiles[0]) + p->max_tiles[1] + 2) * p->d.F2 * 4;
+  total += part_unit_cap(F1, p->cfg.probe_len) * sizeof(PartUnit);
+  if (p->two_pass) total += (static_cast<uint64_t>(p->max_tiles[0]) + p->max_tiles[1] + 2) * p->d.F2 * 4;
   total += static_cast<uint64_t>(p->d.hbm_cap) * tb + (static_cast<uint64_t>(p->d.big_cap) + p->d.hbm_unit_cap) * 16;
   *bytes = total;
   return FIJ_OK;

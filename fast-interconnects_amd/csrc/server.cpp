@@ -130,7 +130,7 @@ struct fij_join_server {
   fij_join_server_config cfg;
   KeyType kt;
   int device = 0;
-  uint32_t cus = 0, lds_total = 0, join_grid = 0;
+  uint32_t cus = 0, lds_total = 0, join_grid = 0, agg_len = 0;
   uint64_t budget_used = 0;
   std::vector<std::unique_ptr<ResidentBuild>> builds;
   std::vector<Slot> slots;
@@ -160,7 +160,7 @@ PipelineDevice base_device(const fij_join_server* s, const ResidentBuild& b) {
   d.G1 = s->cus;
   d.pad = pad_tuples(s->kt);
   d.tile2 = pipeline_tile2(s->kt);
-  d.agg_len = s->join_grid;
+  d.agg_len = s->agg_len;
   return d;
 }
 
@@ -205,7 +205,7 @@ fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
     SRV_HIP(launch_one_pass_plan(d, s->kt, nullptr, 1, st));
     SRV_HIP(launch_one_pass_join(d, s->kt, false, s->join_grid, st));
   }
-  SRV_HIP(launch_sum_aggregates(sl.aggregates, s->join_grid, sl.d_result, nullptr, st));
+  SRV_HIP(launch_sum_aggregates(sl.aggregates, s->agg_len, sl.d_result, nullptr, st));
   SRV_HIP(hipMemcpyAsync(sl.h_result, sl.d_result, sizeof(JoinAggregate), hipMemcpyDeviceToHost, st));
   SRV_HIP(hipEventRecord(sl.done, st));
   return FIJ_OK;
@@ -289,7 +289,7 @@ fij_status make_slot(fij_join_server* s, Slot& sl, uint64_t probe_cap) {
   sl.unit_cap = static_cast<uint32_t>(items + probe_cap / 65536 + 1);
   SRV_HIP(alloc(reinterpret_cast<void**>(&sl.units), sl.unit_cap * sizeof(uint4)));
   SRV_HIP(alloc(reinterpret_cast<void**>(&sl.part_units), part_unit_cap(kMaxF1, probe_cap) * sizeof(PartUnit)));
-  SRV_HIP(alloc(reinterpret_cast<void**>(&sl.aggregates), s->join_grid * sizeof(JoinAggregate)));
+  SRV_HIP(alloc(reinterpret_cast<void**>(&sl.aggregates), s->agg_len * sizeof(JoinAggregate)));
   SRV_HIP(alloc(reinterpret_cast<void**>(&sl.d_result), sizeof(JoinAggregate)));
   SRV_HIP(hipHostMalloc(reinterpret_cast<void**>(&sl.h_result), sizeof(JoinAggregate), hipHostMallocDefault));
   SRV_HIP(hipStreamCreateWithFlags(&sl.stream, hipStreamNonBlocking));
@@ -331,6 +331,7 @@ fij_status fij_join_server_create(const fij_join_server_config* cfg, fij_join_se
   s->device = dev;
   s->cus = static_cast<uint32_t>(prop.multiProcessorCount);
   s->join_grid = 2 * s->cus;
+  s->agg_len = 4 * s->cus;  // the joins with small tables keep more than two blocks per CU
   int optin = 0;
   s->lds_total = static_cast<uint32_t>(prop.sharedMemPerBlock);
   if (hipDeviceGetAttribute(&optin, hipDeviceAttributeSharedMemPerBlockOptin, dev) == hipSuccess && optin > 0)
@@ -344,7 +345,7 @@ fij_status fij_join_server_create(const fij_join_server_config* cfg, fij_join_se
       s->budget_used += s->slots[k++].bytes;
     }
   if (st == FIJ_OK && (hipMalloc(&s->scratch_counters, kJoinCounterWords * 4) != hipSuccess ||
-                       hipMalloc(&s->scratch_agg, s->join_grid * sizeof(JoinAggregate)) != hipSuccess ||
+                       hipMalloc(&s->scratch_agg, s->agg_len * sizeof(JoinAggregate)) != hipSuccess ||
                        hipStreamCreateWithFlags(&s->setup, hipStreamNonBlocking) != hipSuccess))
     st = server_fail(FIJ_OUT_OF_MEMORY, "cannot allocate the server's scratch");
   if (st == FIJ_OK && cfg->hbm_budget && s->budget_used > cfg->hbm_budget)

@@ -70,3 +70,29 @@ def test_probe_range_lengths(dtype, n_s):
     sk = orc.gen_uniform(n_s, 8, 2, 1, n_r, dtype)
     sp = orc.gen_iota(n_s, 1, dtype)
     assert plan_join(dtype, 1, (rk, rp, sk, sp)) == orc.sort_merge_join(rk, rp, sk, sp)
+
+
+@pytest.mark.parametrize("dtype,n_r", [(np.int32, 12_000_001), (np.int64, 6_000_001)])
+def test_two_pass_plan_beyond_two_fills(dtype, n_r):
+    """Build sides just beyond what a two-pass plan joins in a single pass,
+    and, sized, just within it: the same joins through both."""
+    n_s = 3_000_017
+    limit = {np.int32: 11_796_480, np.int64: 5_898_240}[dtype]
+    rk = orc.gen_perm(n_r, 11, dtype, 1)
+    rp = orc.gen_iota(n_r, 5, dtype)
+    sk = orc.gen_uniform(n_s, 11, 2, 1, n_r + n_r // 5, dtype)
+    sp = orc.gen_iota(n_s, 0, dtype)
+    plan = fij.JoinPlan(dtype, n_r, n_s, 9, 7)
+    d = [to_dev(c) for c in (rk, rp, sk, sp)]
+    res = fij.DeviceArray(3, np.uint64)
+    for n in (n_r, limit + 1, limit, n_r):
+        plan.enqueue_sized(d[0].view(0, n), d[1].view(0, n), d[2], d[3], res)
+        got = tuple(int(x) for x in res.to_host())
+        at = np.empty(n_r + 1, np.int64)
+        at.fill(-1)
+        at[rk[:n].astype(np.int64)] = np.arange(n)
+        hit = sk <= n_r
+        hit[hit] = at[sk[hit].astype(np.int64)] >= 0
+        rows = at[sk[hit].astype(np.int64)]
+        want = (int(hit.sum()), int(rp[rows].astype(np.int64).sum()), int(sp[hit].astype(np.int64).sum()))
+        assert got == want
