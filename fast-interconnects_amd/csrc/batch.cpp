@@ -87,11 +87,12 @@ struct ClassArena {
 constexpr uint32_t kMaxBatchLanes = 4;
 
 // A size class's configuration as batches run it: radix bits, pass-1 line
-// ring cap (0 = deepest) and pass-1 block shape.
+// ring cap (0 = deepest), pass-1 block shape, and build tuples of its joins at
+// most (single-pass classes; 0: two passes).
 struct ClassKey {
-  uint32_t b1, b2, ring, block;
+  uint32_t b1, b2, ring, block, build;
   bool operator<(const ClassKey& o) const {
-    return std::tie(b1, b2, ring, block) < std::tie(o.b1, o.b2, o.ring, o.block);
+    return std::tie(b1, b2, ring, block, build) < std::tie(o.b1, o.b2, o.ring, o.block, o.build);
   }
 };
 
@@ -320,18 +321,9 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
   d.job_shift = b1;
   d.build.n = rel2[0];
   d.probe.n = rel2[1];
-  d.big_block_tables = 0;
-  if (b2 == 0) {
-    // the build partitions' size, which chooses the block table: the mean over
-    // build tuples (large joins dominate the class's time)
-    double sum = 0, squares = 0;
-    for (uint32_t j = 0; j < J; ++j) {
-      const double n = static_cast<double>(lay[2 * j].n);
-      d.big_block_tables |= big_block_tables_for(kt, lay[2 * j].n, F1);
-      sum += n;
-      squares += n * n;
-    }
-    d.build.n = static_cast<uint64_t>(sum > 0 ? squares / sum * J : 0.0);
+  if (b2 == 0) {  // the class's largest build side chooses the block tables
+    d.build.n = static_cast<uint64_t>(J) * ck.build;
+    d.big_block_tables = big_block_tables_for(kt, ck.build, F1);
   }
   a.sub_joins = J;
   a.sub_blocks = blocks;
@@ -420,7 +412,7 @@ bool g_tuning_user[2] = {false, false};  // the table came from fij_join_tuning_
 // fij_join_tuning_set; else a single-pass plan where it applies; else the
 // built-in table's entry of its class (the small path only where the pair
 // qualifies for it); else the rule.
-fij_join_tuning tuned_class(KeyType kt, uint64_t build_len, uint64_t probe_len) {
+fij_join_tuning tuned_class(KeyType kt, uint64_t build_len, uint64_t probe_len, bool* user = nullptr) {
   const fij_join_tuning rule = class_rule(kt, build_len, probe_len);
   const int ti = kt == KeyType::I32 ? 0 : 1;
   std::lock_guard<std::mutex> lock(g_tuning_mutex);
@@ -435,6 +427,7 @@ fij_join_tuning tuned_class(KeyType kt, uint64_t build_len, uint64_t probe_len) 
       entry = &e;
       break;
     }
+  if (user) *user = entry && g_tuning_user[ti];
   // Build sides of 2^18 tuples up to what 64 KiB block tables hold after one
   // pass of 9 bits: a single-pass plan, measured faster than the two-pass
   // classes there (1.2-1.45x for single int32 joins at 2^19-2^21, up to 2.9x
@@ -459,6 +452,25 @@ fij_join_tuning tuned_class(KeyType kt, uint64_t build_len, uint64_t probe_len) 
     return t;
   }
   return rule;
+}
+
+// The class that a batch runs a partitioned join of these lengths in.  Build
+// sides of up to two table fills per partition (one_pass_limit) take a single
+// pass, in classes of a factor of four from 2^14 (int64: 2^13) tuples on: 5, 7
+// and 9 bits leave 512 to 2,048 (256 to 1,024) tuples in a partition, for 32
+// KiB tables; beyond, 9 bits with 64 KiB and then 128 KiB tables.
+ClassKey batch_class(KeyType kt, uint64_t build_len, uint64_t probe_len) {
+  bool user = false;
+  const fij_join_tuning tc = tuned_class(kt, build_len, probe_len, &user);
+  if (user || build_len > one_pass_limit(kt)) return {tc.radix_bits_1, tc.radix_bits_2, tc.ring_lines, tc.block, 0};
+  uint32_t b1 = 5;
+  uint64_t most = kt == KeyType::I32 ? 1u << 16 : 1u << 15;
+  for (; build_len > most && b1 < kOnePassBits; b1 += 2) most <<= 2;
+  if (build_len > most) {
+    most = static_cast<uint64_t>(pipeline_block_table_tuples(kt, false)) << kOnePassBits;
+    if (!block_tables_hold(kt, build_len, 1ull << kOnePassBits, false)) most = one_pass_limit(kt);
+  }
+  return {b1, 0, 0, 1024, static_cast<uint32_t>(most)};
 }
 
 }  // namespace
@@ -603,7 +615,7 @@ fij_status fij_join_batch_execute(fij_join_batch* b, uint32_t n, const fij_join_
       sj.probe_len = j.probe_len;
       sj.result = b->d_results + i;
     } else {
-      classes[ClassKey{tc.radix_bits_1, tc.radix_bits_2, tc.ring_lines, tc.block}].push_back(i);
+      classes[batch_class(b->kt, j.build_len, j.probe_len)].push_back(i);
       ++n_large;
     }
   }
@@ -626,15 +638,12 @@ fij_status fij_join_batch_execute(fij_join_batch* b, uint32_t n, const fij_join_
   if (use_graph) BATCH_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   fij_status s = FIJ_OK;
   if (!use_graph) BATCH_HIP(hipEventRecord(b->ev[0], st));
-  if (n_small) {
-    hipError_t e = launch_small_joins(b->kt, b->d_jobs, n_small, b->d_ticket, b->cus, st);
-    if (e != hipSuccess) s = batch_fail(FIJ_DEVICE_ERROR, "small joins: %s", hipGetErrorString(e));
-  }
   // Size classes are independent (each has its own buffers and result
   // slots), so they are spread over the lanes: largest class first, each to
-  // the lane with the fewest tuples so far.  Lane 0 is the submission stream
-  // (which also runs the small joins); the other lanes wait for it to reach
-  // this point and it waits for all of them at the end.
+  // the lane with the fewest tuples so far, and the small joins (one block
+  // each, so their launch leaves most of the GPU idle) behind the shortest
+  // lane.  Lane 0 is the submission stream; the other lanes wait for it to
+  // reach this point and it waits for all of them at the end.
   std::vector<std::pair<uint64_t, const ClassKey*>> order;
   for (auto& kv : classes) {
     uint64_t tuples = 0;
@@ -656,6 +665,11 @@ fij_status fij_join_batch_execute(fij_join_batch* b, uint32_t n, const fij_join_
     hipError_t e = launch_class(b, b->arenas[*key], *key, l ? b->lane[l] : st, b->lds_total);
     if (e != hipSuccess)
       s = batch_fail(FIJ_DEVICE_ERROR, "size class %u+%u: %s", key->b1, key->b2, hipGetErrorString(e));
+  }
+  if (n_small && s == FIJ_OK) {
+    const uint32_t l = static_cast<uint32_t>(std::min_element(lane_load, lane_load + lanes) - lane_load);
+    hipError_t e = launch_small_joins(b->kt, b->d_jobs, n_small, b->d_ticket, b->cus, l ? b->lane[l] : st);
+    if (e != hipSuccess) s = batch_fail(FIJ_DEVICE_ERROR, "small joins: %s", hipGetErrorString(e));
   }
   // every forked lane joins back, also after an error (a capture must end
   // with every stream it forked joined)
