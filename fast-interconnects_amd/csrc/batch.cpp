@@ -346,7 +346,7 @@ hipError_t launch_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, hi
     return e;
   if (ck.b2 == 0) {
     if ((e = launch_one_pass_plan(a.d, kt, a.sides, a.sub_joins, st)) != hipSuccess) return e;
-    return launch_one_pass_join(a.d, kt, false, 2 * b->cus, st);
+    return launch_one_pass_join(a.d, kt, 2 * b->cus, st);
   }
   if ((e = launch_pipeline_plan_batched(a.d, a.sides, a.sub_joins, a.side_tiles, a.d.build.n, a.d.probe.n, st)) !=
       hipSuccess)

@@ -1,6 +1,5 @@
 // Block-shared LDS hash table of the joins that stream a probe range against one
-// build range (single-pass partitions, build sides of one table), and the
-// block-wide sum of their results.
+// build range (single-pass partitions, build sides of one table).
 #pragma once
 
 #include "common.hpp"
@@ -112,28 +111,5 @@ struct BucketTable {
     }
   }
 };
-
-// Sums over the block, in thread 0 (red: [3][waves]); ends with a barrier.
-template <uint32_t BLOCK>
-__device__ __forceinline__ void block_sums(uint64_t (*red)[BLOCK / kWave], uint64_t& cnt, uint64_t& sb, uint64_t& sp) {
-  const uint32_t w = threadIdx.x / kWave;
-  cnt = wave_broadcast_last(wave_inclusive_scan(cnt));
-  sb = wave_broadcast_last(wave_inclusive_scan(sb));
-  sp = wave_broadcast_last(wave_inclusive_scan(sp));
-  if (lane_id() == 0) {
-    red[0][w] = cnt;
-    red[1][w] = sb;
-    red[2][w] = sp;
-  }
-  __syncthreads();
-  cnt = sb = sp = 0;
-  if (threadIdx.x == 0)
-    for (uint32_t i = 0; i < BLOCK / kWave; ++i) {
-      cnt += red[0][i];
-      sb += red[1][i];
-      sp += red[2][i];
-    }
-  __syncthreads();
-}
 
 }  // namespace fij

@@ -288,7 +288,9 @@ __global__ __launch_bounds__(kHistBlockMax) void transform_counts_kernel(Transfo
 // (whole 128-byte lines of the offsets), the sums over the chunks of a
 // partition are one wave scan.  Tiles take a dynamic ticket, so a tile only
 // ever waits on tiles that started before it.  Each state word packs
-// (value << 2) | flag with flag 1 = aggregate, 2 = inclusive prefix.
+// (value << 2) | flag with flag 1 = aggregate, 2 = inclusive prefix: all that
+// its reader needs, so the accesses are relaxed (a release writes back the
+// die's L2, an acquire drops it at every look).
 //
 // Bound by the latency of its chain (ticket, loads, look-back, stores), not
 // by its bytes.  512 partitions x 256 chunks: 11.1 us with 16 tiles of 8192
@@ -332,16 +334,16 @@ __device__ __forceinline__ void offsets_scan_body(const OffsetsScan& s) {
     uint64_t prefix = 0;
     if (tile == 0) {
       if (lane == 0)
-        __hip_atomic_store(&tile_state[0], (aggregate << 2) | kFlagIncl, __ATOMIC_RELEASE,
+        __hip_atomic_store(&tile_state[0], (aggregate << 2) | kFlagIncl, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     } else {
       if (lane == 0)
-        __hip_atomic_store(&tile_state[tile], (aggregate << 2) | kFlagAgg, __ATOMIC_RELEASE,
+        __hip_atomic_store(&tile_state[tile], (aggregate << 2) | kFlagAgg, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
       int64_t j = static_cast<int64_t>(tile) - 1;
       for (;;) {
         const int64_t idx = j - static_cast<int64_t>(lane);
-        uint64_t st = (idx >= 0) ? __hip_atomic_load(&tile_state[idx], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT)
+        uint64_t st = (idx >= 0) ? __hip_atomic_load(&tile_state[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                                  : kFlagIncl;  // virtual inclusive zero before tile 0
         const uint64_t flag = st & 3u;
         const uint64_t incl_mask = ballot(flag == kFlagIncl);
@@ -358,7 +360,7 @@ __device__ __forceinline__ void offsets_scan_body(const OffsetsScan& s) {
         j -= kWave;
       }
       if (lane == 0)
-        __hip_atomic_store(&tile_state[tile], ((prefix + aggregate) << 2) | kFlagIncl, __ATOMIC_RELEASE,
+        __hip_atomic_store(&tile_state[tile], ((prefix + aggregate) << 2) | kFlagIncl, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     }
     if (lane == 0) s_prefix = prefix;

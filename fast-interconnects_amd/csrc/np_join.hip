@@ -9,6 +9,7 @@
 // {count, SUM(build.value), SUM(probe.value)}.
 #include "common.hpp"
 #include "internal.hpp"
+#include "join_result.hpp"
 
 namespace fij {
 namespace {
@@ -141,11 +142,11 @@ __global__ __launch_bounds__(1024) void np_probe_kernel(const Tuple<K>* table, u
 // Probe of a resident linear-probing table of 2^lg entries (a served build
 // side that fits the GPU's cache): U probes in flight per thread, their first
 // slots loaded together; every match counts, probing ends at a free slot.
-// Block b writes (not adds) its {count, SUM(build.value), SUM(probe.value)}
-// to out[b].
+// *result = {count, SUM(build.value), SUM(probe.value)} (see finish_join).
 template <typename K, uint32_t U>
 __global__ __launch_bounds__(256) void np_probe_resident_kernel(const Tuple<K>* table, uint32_t lg, const K* keys,
-                                                                const K* pays, uint64_t n, JoinAggregate* out) {
+                                                                const K* pays, uint64_t n, JoinAggregate* partial,
+                                                                uint32_t* done, JoinAggregate* result) {
   const uint64_t mask = (1ull << lg) - 1;
   const uint64_t T = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   uint64_t cnt = 0, sb = 0, sp = 0;
@@ -183,27 +184,8 @@ __global__ __launch_bounds__(256) void np_probe_resident_kernel(const Tuple<K>* 
     }
   }
   __shared__ uint64_t red[3][256 / kWave];
-  const uint32_t w = threadIdx.x / kWave;
-  const uint64_t wc = wave_broadcast_last(wave_inclusive_scan(cnt));
-  const uint64_t wb = wave_broadcast_last(wave_inclusive_scan(sb));
-  const uint64_t wp = wave_broadcast_last(wave_inclusive_scan(sp));
-  if (lane_id() == 0) {
-    red[0][w] = wc;
-    red[1][w] = wb;
-    red[2][w] = wp;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint64_t a = 0, b = 0, d = 0;
-    for (uint32_t i = 0; i < blockDim.x / kWave; ++i) {
-      a += red[0][i];
-      b += red[1][i];
-      d += red[2][i];
-    }
-    out[blockIdx.x].count = a;
-    out[blockIdx.x].sum_build = b;
-    out[blockIdx.x].sum_probe = d;
-  }
+  __shared__ uint32_t s_last;
+  (void)finish_join<256>(partial, done, result, red, &s_last, cnt, sb, sp);
 }
 
 template <typename K>
@@ -260,16 +242,19 @@ hipError_t launch_np_build(KeyType t, JoinScheme s, bool selective, void* table,
 }
 
 hipError_t launch_np_probe_resident(KeyType t, const void* table, uint32_t lg, const void* keys, const void* pays,
-                                    uint64_t n, JoinAggregate* out, uint32_t grid, hipStream_t stream) {
+                                    uint64_t n, JoinAggregate* partial, uint32_t* done, JoinAggregate* result,
+                                    uint32_t grid, hipStream_t stream) {
   constexpr uint32_t U = 4;
+  // one step of every thread; a short request leaves the rest of the GPU to others
+  grid = static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(grid, (n + U * 256 - 1) / (U * 256))));
   if (t == KeyType::I32)
     hipLaunchKernelGGL((np_probe_resident_kernel<int32_t, U>), dim3(grid), dim3(256), 0, stream,
                        static_cast<const Tuple<int32_t>*>(table), lg, static_cast<const int32_t*>(keys),
-                       static_cast<const int32_t*>(pays), n, out);
+                       static_cast<const int32_t*>(pays), n, partial, done, result);
   else
     hipLaunchKernelGGL((np_probe_resident_kernel<int64_t, U>), dim3(grid), dim3(256), 0, stream,
                        static_cast<const Tuple<int64_t>*>(table), lg, static_cast<const int64_t*>(keys),
-                       static_cast<const int64_t*>(pays), n, out);
+                       static_cast<const int64_t*>(pays), n, partial, done, result);
   return hipGetLastError();
 }
 

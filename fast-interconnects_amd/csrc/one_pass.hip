@@ -9,8 +9,7 @@
 //                         when the arena has room
 //   part_join_kernel      one block per unit: the build range goes into a
 //                         block-shared table, the probe range is streamed
-//                         against it; then the build sides of the HBM tables
-//   part_table_kernel     the probes of the HBM tables
+//                         against it; then the HBM tables, and the sum
 //
 // Semantics as in the other joins: every pair of equal keys counts, null keys
 // never join, count and sums wrap at 64 bits.
@@ -18,6 +17,7 @@
 #include "common.hpp"
 #include "hbm_table.hpp"
 #include "internal.hpp"
+#include "join_result.hpp"
 #include "pipeline.hpp"
 
 #include <algorithm>
@@ -126,6 +126,7 @@ __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, c
       d.work_counter[kHbmSlots + 1] = 0;
       d.work_counter[kHbmBuildUnits] = s_build_units;
       d.work_counter[kHbmProbeUnits] = s_probe_units;
+      for (uint32_t c : {kHbmBuildTicket, kHbmBuildDone, kHbmProbeTicket, kHbmProbeDone}) d.work_counter[c] = 0;
     }
   }
   __syncthreads();
@@ -153,35 +154,83 @@ __global__ void reset_counters_kernel(uint32_t* counters) {
   for (uint32_t i = threadIdx.x; i < kJoinCounterWords; i += blockDim.x) counters[i] = 0;
 }
 
-// Adds the block's sums to the result of join `job` (batches) or, for one join,
-// to the block's aggregate (FIRST: stores it, and zeros for blocks that this
-// grid does not have), and clears them.
-template <uint32_t BLOCK, bool FIRST>
+// Adds the block's sums to the result of join `job` of a batch and clears them.
+template <uint32_t BLOCK>
 __device__ __forceinline__ void add_result(const PipelineDevice& d, uint64_t (*red)[BLOCK / kWave], uint32_t job,
                                            uint64_t& cnt, uint64_t& sb, uint64_t& sp) {
   block_sums<BLOCK>(red, cnt, sb, sp);
-  if (threadIdx.x == 0) {
-    if (d.job_results) {
-      if (cnt) {
-        JoinAggregate* r = d.job_results + d.job_slot[job];
-        atomicAdd(reinterpret_cast<unsigned long long*>(&r->count), static_cast<unsigned long long>(cnt));
-        atomicAdd(reinterpret_cast<unsigned long long*>(&r->sum_build), static_cast<unsigned long long>(sb));
-        atomicAdd(reinterpret_cast<unsigned long long*>(&r->sum_probe), static_cast<unsigned long long>(sp));
-      }
-    } else {
-      JoinAggregate* r = d.aggregates + blockIdx.x;
-      if constexpr (FIRST) {
-        *r = JoinAggregate{cnt, sb, sp};
-        for (uint32_t i = blockIdx.x + gridDim.x; i < d.agg_len; i += gridDim.x)
-          d.aggregates[i] = JoinAggregate{0, 0, 0};
-      } else {
-        r->count += cnt;
-        r->sum_build += sb;
-        r->sum_probe += sp;
-      }
-    }
+  if (threadIdx.x == 0 && cnt) {
+    JoinAggregate* r = d.job_results + d.job_slot[job];
+    atomicAdd(reinterpret_cast<unsigned long long*>(&r->count), static_cast<unsigned long long>(cnt));
+    atomicAdd(reinterpret_cast<unsigned long long*>(&r->sum_build), static_cast<unsigned long long>(sb));
+    atomicAdd(reinterpret_cast<unsigned long long*>(&r->sum_probe), static_cast<unsigned long long>(sp));
   }
   cnt = sb = sp = 0;
+}
+
+// The HBM tables of a join (plans of one join only: batches and served joins
+// have no arena): build, probe and clear, for blocks that have run out of work
+// units.  Units are taken by ticket and a block waits only once every unit of
+// the phase is taken, so it waits for blocks that are running and never for
+// one that has yet to start.  As launches of their own, which nearly every
+// join leaves without work, the probes and the clearing took 9 us of each.
+// No more blocks than units take part, so that few wait.
+template <typename K, uint32_t BLOCK>
+__device__ __forceinline__ void table_phases(const PipelineDevice& d, uint32_t n_build, uint32_t* s_next,
+                                             uint64_t& cnt, uint64_t& sb, uint64_t& sp) {
+  const uint32_t n_probe = uniform_load(d.work_counter + kHbmProbeUnits);
+  const uint32_t blocks = min(gridDim.x, max(n_build, n_probe));
+  if (blockIdx.x >= blocks) return;
+  const uint32_t tid = threadIdx.x;
+  auto take = [&](uint32_t ticket) {
+    if (tid == 0) *s_next = atomicAdd(d.work_counter + ticket, 1u);
+    __syncthreads();
+    const uint32_t u = __builtin_amdgcn_readfirstlane(*s_next);
+    __syncthreads();  // every thread has read it
+    return u;
+  };
+  // counts the block's finished units and waits for all n of the phase
+  auto finish = [&](uint32_t counter, uint32_t mine, uint32_t n) {
+    __threadfence();  // the thread's stores are visible before its units count
+    __syncthreads();
+    if (tid == 0) {
+      if (mine) atomicAdd(d.work_counter + counter, mine);
+      // relaxed: an acquire would drop the L2's lines at every look, while the
+      // chains of the blocks that work run through it
+      while (__hip_atomic_load(d.work_counter + counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < n)
+        __builtin_amdgcn_s_sleep(127);
+    }
+    __syncthreads();
+    __threadfence();  // what was read before is read again
+  };
+  uint32_t mine = 0;
+  for (uint32_t u; (u = take(kHbmBuildTicket)) < n_build; ++mine) {
+    const uint4 unit = scalar_load(d.hbm_units + u);
+    const uint4 big = scalar_load(d.big + unit.x);
+    Tuple<K>* const table = static_cast<Tuple<K>*>(d.hbm_table) + big.y;
+    const Tuple<K>* rel = static_cast<const Tuple<K>*>(d.build.rel1) + uniform_load(d.build.off1 + big.x);
+    for (uint32_t i = unit.y + tid; i < unit.z; i += BLOCK) {
+      const Tuple<K> t = load_tuple<K>(rel + i);
+      if (t.key != null_key<K>()) hbm_insert<K>(table, big.z, t.key, t.value);
+    }
+  }
+  finish(kHbmBuildDone, mine, n_build);
+  mine = 0;
+  for (uint32_t u; (u = take(kHbmProbeTicket)) < n_probe; ++mine) {
+    const uint4 unit = scalar_load(d.hbm_units + (d.hbm_unit_cap - 1 - u));
+    const uint4 big = scalar_load(d.big + unit.x);
+    const Tuple<K>* const table = static_cast<const Tuple<K>*>(d.hbm_table) + big.y;
+    const Tuple<K>* rel = static_cast<const Tuple<K>*>(d.probe.rel1) + uniform_load(d.probe.off1 + big.x);
+    for (uint32_t i = unit.y + tid; i < unit.z; i += BLOCK) {
+      const Tuple<K> t = load_tuple_nt<K>(rel + i);
+      if (t.key != null_key<K>()) hbm_probe<K>(table, big.z, t.key, t.value, cnt, sb, sp);
+    }
+  }
+  finish(kHbmProbeDone, mine, n_probe);
+  uint4* const words = static_cast<uint4*>(d.hbm_table);
+  const uint64_t n = static_cast<uint64_t>(uniform_load(d.work_counter + kHbmSlots)) * sizeof(Tuple<K>) / 16;
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * BLOCK + tid; i < n; i += static_cast<uint64_t>(blocks) * BLOCK)
+    words[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
 }
 
 // 16 bytes of tuples from 16-byte aligned memory.
@@ -226,7 +275,7 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
     if (tid == 0) ticket = atomicAdd(d.work_counter + kBlockTicket, 1u);
     const PartUnit unit = scalar_load(d.part_units + u);
     if (d.job_results && (unit.part >> d.job_shift) != job) {
-      add_result<BLOCK, true>(d, red, job, cnt, sb, sp);
+      add_result<BLOCK>(d, red, job, cnt, sb, sp);
       job = unit.part >> d.job_shift;
     }
     const uint32_t nb = unit.build_n;
@@ -328,41 +377,19 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
     u = __builtin_amdgcn_readfirstlane(s_next);
     __syncthreads();  // every thread has read s_next
   }
-  // build sides of the HBM tables
-  const uint32_t n_big = d.hbm_cap ? uniform_load(d.work_counter + kHbmBuildUnits) : 0u;
-  for (uint32_t u = blockIdx.x; u < n_big; u += gridDim.x) {
-    const uint4 unit = scalar_load(d.hbm_units + u);
-    const uint4 big = scalar_load(d.big + unit.x);
-    Tuple<K>* const table = static_cast<Tuple<K>*>(d.hbm_table) + big.y;
-    const Tuple<K>* rel = static_cast<const Tuple<K>*>(d.build.rel1) + uniform_load(d.build.off1 + big.x);
-    for (uint32_t i = unit.y + tid; i < unit.z; i += BLOCK) {
-      const Tuple<K> t = load_tuple<K>(rel + i);
-      if (t.key != null_key<K>()) hbm_insert<K>(table, big.z, t.key, t.value);
-    }
+  if (d.job_results) {
+    add_result<BLOCK>(d, red, job, cnt, sb, sp);
+    return;
   }
-  add_result<BLOCK, true>(d, red, job, cnt, sb, sp);
-}
-
-// Probes of the HBM tables (plans of one join only: batches and served joins
-// have no arena).
-template <typename K, uint32_t BLOCK>
-__global__ __launch_bounds__(BLOCK) void part_table_kernel(PipelineDevice d) {
-  __shared__ uint64_t red[3][BLOCK / kWave];
-  stamp_phase(d.stamps, 4);
-  const uint32_t n = uniform_load(d.work_counter + kHbmProbeUnits);
-  if (n == 0) return;
-  uint64_t cnt = 0, sb = 0, sp = 0;
-  for (uint32_t u = blockIdx.x; u < n; u += gridDim.x) {
-    const uint4 unit = scalar_load(d.hbm_units + (d.hbm_unit_cap - 1 - u));
-    const uint4 big = scalar_load(d.big + unit.x);
-    const Tuple<K>* const table = static_cast<const Tuple<K>*>(d.hbm_table) + big.y;
-    const Tuple<K>* rel = static_cast<const Tuple<K>*>(d.probe.rel1) + uniform_load(d.probe.off1 + big.x);
-    for (uint32_t i = unit.y + threadIdx.x; i < unit.z; i += BLOCK) {
-      const Tuple<K> t = load_tuple_nt<K>(rel + i);
-      if (t.key != null_key<K>()) hbm_probe<K>(table, big.z, t.key, t.value, cnt, sb, sp);
-    }
+  const uint32_t n_build = d.hbm_cap ? uniform_load(d.work_counter + kHbmBuildUnits) : 0u;
+  if (n_build) {
+    stamp_phase(d.stamps, 4);
+    table_phases<K, BLOCK>(d, n_build, &s_next, cnt, sb, sp);
   }
-  add_result<BLOCK, false>(d, red, 0, cnt, sb, sp);
+  if (finish_join<BLOCK>(d.aggregates, d.done, d.result, red, &s_next, cnt, sb, sp) && d.stamps && tid == 0) {
+    d.stamps[5] = wall_clock64();
+    if (!n_build) d.stamps[4] = d.stamps[5];
+  }
 }
 
 template <typename K, uint32_t CAP, uint32_t BLOCK>
@@ -376,32 +403,22 @@ hipError_t launch_part_join(const PipelineDevice& d, uint32_t grid, hipStream_t 
 }
 
 template <typename K>
-hipError_t launch_one_pass_join_t(const PipelineDevice& d, bool tables, uint32_t grid, hipStream_t stream) {
-  if (!tables) {
-    // One block of 1,024 threads per CU with a 128 KiB table, two of 512 with
-    // 64 KiB, three with 32 KiB: those take partitions that fill them half on
-    // average (the batched joins above: 283 us with 64 KiB tables, 240 us).
-    auto blocks = [&](uint32_t n) { return d.job_results ? n : std::min(n, d.agg_len); };
-    if (d.big_block_tables) return launch_part_join<K, 2 * kSlots<K>, 1024>(d, blocks((grid + 1) / 2), stream);
-    if (d.build.n <= static_cast<uint64_t>(d.F1) * (kSlots<K> / 4))
-      return launch_part_join<K, kSlots<K> / 2, 512>(d, blocks(grid + grid / 2), stream);
-    return launch_part_join<K, kSlots<K>, 512>(d, blocks(grid), stream);
-  }
-  if (!one_pass_tables(d, sizeof(K) == 4 ? KeyType::I32 : KeyType::I64)) return hipSuccess;
-  hipLaunchKernelGGL((part_table_kernel<K, 512>), dim3(grid), dim3(512), 0, stream, d);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return launch_hbm_clear(d, sizeof(Tuple<K>), grid, stream);
+hipError_t launch_one_pass_join_t(const PipelineDevice& d, uint32_t grid, hipStream_t stream) {
+  // One block of 1,024 threads per CU with a 128 KiB table, two of 512 with
+  // 64 KiB, three with 32 KiB: those take partitions that fill them half on
+  // average (20 batched joins of 2^18..2^20 int32 build tuples: 283 us with 64
+  // KiB tables, 240 us).
+  auto blocks = [&](uint32_t n) { return d.job_results ? n : std::min(n, d.agg_len); };
+  if (d.big_block_tables) return launch_part_join<K, 2 * kSlots<K>, 1024>(d, blocks((grid + 1) / 2), stream);
+  if (d.build.n <= static_cast<uint64_t>(d.F1) * (kSlots<K> / 4))
+    return launch_part_join<K, kSlots<K> / 2, 512>(d, blocks(grid + grid / 2), stream);
+  return launch_part_join<K, kSlots<K>, 512>(d, blocks(grid), stream);
 }
 
 }  // namespace
 
 uint32_t pipeline_block_table_tuples(KeyType t, bool big) {
   return (t == KeyType::I32 ? kSlots<int32_t> : kSlots<int64_t>) * (big ? 2 : 1) * 3 / 4;
-}
-
-bool one_pass_tables(const PipelineDevice& d, KeyType t) {
-  return d.hbm_cap != 0 && d.build.n > kMaxFills * pipeline_block_table_tuples(t, d.big_block_tables != 0);
 }
 
 hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchSide* sides, uint32_t joins,
@@ -418,9 +435,9 @@ hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchS
   return hipGetLastError();
 }
 
-hipError_t launch_one_pass_join(const PipelineDevice& d, KeyType t, bool tables, uint32_t grid, hipStream_t stream) {
-  if (t == KeyType::I32) return launch_one_pass_join_t<int32_t>(d, tables, grid, stream);
-  return launch_one_pass_join_t<int64_t>(d, tables, grid, stream);
+hipError_t launch_one_pass_join(const PipelineDevice& d, KeyType t, uint32_t grid, hipStream_t stream) {
+  if (t == KeyType::I32) return launch_one_pass_join_t<int32_t>(d, grid, stream);
+  return launch_one_pass_join_t<int64_t>(d, grid, stream);
 }
 
 }  // namespace fij

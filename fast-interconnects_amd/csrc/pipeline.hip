@@ -1511,11 +1511,7 @@ hipError_t launch_deferred_t(const PipelineDevice& d, uint32_t grid, hipStream_t
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL((join_hbm_kernel<K, 512, 8, false>), dim3(grid), dim3(512), 0, stream, d);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  return launch_hbm_clear(d, sizeof(Tuple<K>), grid, stream);
-}
-
-hipError_t launch_hbm_clear(const PipelineDevice& d, uint32_t tuple_bytes, uint32_t grid, hipStream_t stream) {
-  hipLaunchKernelGGL(join_hbm_clear_kernel, dim3(grid), dim3(256), 0, stream, d, tuple_bytes);
+  hipLaunchKernelGGL(join_hbm_clear_kernel, dim3(grid), dim3(256), 0, stream, d, static_cast<uint32_t>(sizeof(Tuple<K>)));
   return hipGetLastError();
 }
 

@@ -43,7 +43,8 @@ struct PipelineSide {
 // the block-table units, and the number of wave-table units (stored from the
 // back of `units`); then the HBM-table counters: slots reserved in the HBM
 // table arena (a 64-bit word), items given an HBM table, their build and
-// probe work units, and the tickets over those.
+// probe work units, the tickets over those, and their finished units (which
+// only the single-pass join counts).
 constexpr uint32_t kJoinCounters = 8;
 constexpr uint32_t kJoinCounterStride = 32;
 constexpr uint32_t kOverflowTicket = kJoinCounters * kJoinCounterStride;
@@ -58,7 +59,13 @@ constexpr uint32_t kHbmBuildUnits = (kJoinCounters + 8) * kJoinCounterStride;
 constexpr uint32_t kHbmProbeUnits = (kJoinCounters + 9) * kJoinCounterStride;
 constexpr uint32_t kHbmBuildTicket = (kJoinCounters + 10) * kJoinCounterStride;
 constexpr uint32_t kHbmProbeTicket = (kJoinCounters + 11) * kJoinCounterStride;
-constexpr uint32_t kJoinCounterWords = (kJoinCounters + 12) * kJoinCounterStride;
+constexpr uint32_t kHbmBuildDone = (kJoinCounters + 12) * kJoinCounterStride;
+constexpr uint32_t kHbmProbeDone = (kJoinCounters + 13) * kJoinCounterStride;
+constexpr uint32_t kJoinCounterWords = (kJoinCounters + 14) * kJoinCounterStride;
+
+// Counters of a join's finished blocks (finish_join), each on a line of its own.
+constexpr uint32_t kDoneGroups = 16, kDoneStride = 32;
+constexpr uint32_t kDoneWords = (kDoneGroups + 1) * kDoneStride;
 
 // Phase stamps of a timed join (the device's constant-rate clock, written to
 // pinned host memory by the first block of a phase as it starts; the last
@@ -98,6 +105,8 @@ struct PipelineDevice {
   PartUnit* part_units;       // single-pass plans: [part_unit_cap(F1, probe tuples)]
   JoinAggregate* aggregates;  // [agg_len]
   uint32_t agg_len;
+  JoinAggregate* result;      // single-pass joins of one plan or request: where the join's sums go, and
+  uint32_t* done;             // [kDoneWords] the finished blocks (zero between joins)
   uint64_t* stamps;           // [kStamps] or nullptr: not timed
   // Many joins in one plan (batched joins): pass-1 partition p belongs to
   // join p >> job_shift, whose count and sums are added to
@@ -213,8 +222,8 @@ hipError_t launch_pipeline_sort2(const PipelineDevice& d, KeyType t, uint32_t gr
 hipError_t launch_sum_aggregates(const JoinAggregate* src, uint32_t n, JoinAggregate* dst, uint64_t* stamps,
                                  hipStream_t stream);
 // One join whose build side fits a block's LDS table (table_join_tuples): one
-// launch without partitioning.  partial: at least max_grid entries; done: a
-// word that is zero between joins.
+// launch without partitioning.  partial: at least max_grid entries; done:
+// [kDoneWords], zero between joins.
 struct TableJoin {
   const void *build_keys, *build_pays, *probe_keys, *probe_pays;
   uint64_t n_b, n_p;
@@ -225,22 +234,17 @@ struct TableJoin {
 };
 uint64_t table_join_tuples(KeyType t);
 hipError_t launch_table_join(KeyType t, const TableJoin& j, uint32_t cus, uint32_t max_grid, hipStream_t stream);
-// Restores the HBM-arena slots that a join reserved to all ones.
-hipError_t launch_hbm_clear(const PipelineDevice& d, uint32_t tuple_bytes, uint32_t grid, hipStream_t stream);
 // Two passes: the register-resident join of every work item (deferred =
 // false), then the join of the items it deferred (deferred = true).
 hipError_t launch_pipeline_join(const PipelineDevice& d, KeyType t, bool deferred, uint32_t grid, hipStream_t stream);
 // Single pass, instead of the plan and join launches of two: partition
 // lengths and work units of the joins in d (sides of join j in sides[2 j],
 // sides[2 j + 1]; one join and sides == nullptr for a plan of its own), reset
-// of the join counters and aggregates (or of the joins' results).
+// of the join counters (and of the joins' results).
 hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchSide* sides, uint32_t joins,
                                 hipStream_t stream);
-// ... the join of every unit and the builds of HBM hash tables, and (tables =
-// true, a launch of its own so that it can be timed) their probes.
-// Whether any build partition can need an HBM table (none can exceed an LDS
-// table that holds the whole build side): else the second launch does nothing.
-bool one_pass_tables(const PipelineDevice& d, KeyType t);
-hipError_t launch_one_pass_join(const PipelineDevice& d, KeyType t, bool tables, uint32_t grid, hipStream_t stream);
+// ... the join of every unit and of the partitions with HBM hash tables, and
+// the sum in *d.result (d.job_results: in the joins' results).
+hipError_t launch_one_pass_join(const PipelineDevice& d, KeyType t, uint32_t grid, hipStream_t stream);
 
 }  // namespace fij

@@ -37,14 +37,14 @@ struct fij_join_plan {
   std::vector<void*> allocs;
   uint32_t cus;
   uint32_t clock_khz;  // rate of the device clock the phases are stamped with
-  uint32_t* done;      // finished blocks of a table join, zero between joins
+  uint32_t* done;      // [kDoneWords] finished blocks, zero between joins
   // what the last enqueued join wrote or did not launch
   struct Host {
     JoinAggregate result;
     uint64_t stamps[kStamps];
   };
   Host* host;
-  enum class Timed { None, Phases, NoDeferred, OneLaunch } timed;
+  enum class Timed { None, Phases, OneLaunch } timed;
 };
 
 namespace {
@@ -211,10 +211,10 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
     p->d.big_cap = static_cast<uint32_t>(std::min<uint64_t>(items, slots / 256));
     p->d.hbm_unit_cap =
         static_cast<uint32_t>(2ull * p->d.big_cap + (cfg->build_len + cfg->probe_len) / 65536 + 2);
-    // (the block counter of table joins is cleared with the arena)
-    if (st == FIJ_OK) st = alloc(p, &p->done, 1);
-    if (st == FIJ_OK && hipMemset(p->done, 0, sizeof(uint32_t)) != hipSuccess)
-      st = plan_fail(FIJ_DEVICE_ERROR, "clearing the block counter failed");
+    // (the block counters are cleared with the arena)
+    if (st == FIJ_OK) st = alloc(p, &p->done, kDoneWords);
+    if (st == FIJ_OK && hipMemset(p->done, 0, kDoneWords * sizeof(uint32_t)) != hipSuccess)
+      st = plan_fail(FIJ_DEVICE_ERROR, "clearing the block counters failed");
     void* arena = nullptr;
     if (st == FIJ_OK && hipMalloc(&arena, slots * tuple_bytes(kt)) != hipSuccess)
       st = plan_fail(FIJ_OUT_OF_MEMORY, "cannot allocate the HBM hash-table arena");
@@ -308,20 +308,19 @@ fij_status enqueue_join(fij_join_plan* p, const void* build_keys, const void* bu
   d.big_block_tables = d.bits2 ? 0u : big_block_tables_for(p->kt, n_b, d.F1);
   PLAN_HIP(enqueue_pass1_prefix_sum(d, p->kt, p->block1, st));
   PLAN_HIP(enqueue_pass1_scatter(d, p->kt, p->block1, p->lds_total, st));
-  Timed timed = Timed::Phases;
   if (d.bits2) {
     PLAN_HIP(launch_pipeline_plan(d, st));
     PLAN_HIP(launch_pipeline_sort2(d, p->kt, p->sort2_grid, st));
     PLAN_HIP(launch_pipeline_join(d, p->kt, false, p->join_grid, st));
     PLAN_HIP(launch_pipeline_join(d, p->kt, true, p->join_grid, st));
+    PLAN_HIP(launch_sum_aggregates(d.aggregates, d.agg_len, result, stamps, st));
   } else {
+    d.result = result;
+    d.done = p->done;
     PLAN_HIP(launch_one_pass_plan(d, p->kt, nullptr, 1, st));
-    PLAN_HIP(launch_one_pass_join(d, p->kt, false, p->join_grid, st));
-    PLAN_HIP(launch_one_pass_join(d, p->kt, true, p->join_grid, st));
-    if (!one_pass_tables(d, p->kt)) timed = Timed::NoDeferred;
+    PLAN_HIP(launch_one_pass_join(d, p->kt, p->join_grid, st));
   }
-  PLAN_HIP(launch_sum_aggregates(d.aggregates, d.agg_len, result, stamps, st));
-  if (!device_result) p->timed = timed;
+  if (!device_result) p->timed = Timed::Phases;
   return FIJ_OK;
 }
 
@@ -360,13 +359,12 @@ fij_status fij_join_plan_result(fij_join_plan* p, void* stream, fij_join_aggrega
     if (p->timed == Timed::OneLaunch) {
       timing->join_ms = timing->build_probe_ms = timing->total_ms;
     } else {
-      const bool deferred = p->timed == Timed::Phases;
       timing->prefix_sum_ms = ms(0, 1);
       timing->partition_ms = ms(1, 2);
       timing->join_ms = ms(2, 5);
       timing->pass2_ms = ms(2, 3);
-      timing->build_probe_ms = ms(3, deferred ? 4 : 5);
-      timing->deferred_ms = deferred ? ms(4, 5) : 0.0f;
+      timing->build_probe_ms = ms(3, 4);
+      timing->deferred_ms = ms(4, 5);
     }
   }
   return FIJ_OK;

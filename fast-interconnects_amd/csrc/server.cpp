@@ -103,8 +103,8 @@ struct Slot {
   uint32_t unit_cap = 0;
   PartUnit* part_units = nullptr;
   JoinAggregate* aggregates = nullptr;
-  JoinAggregate* d_result = nullptr;
-  JoinAggregate* h_result = nullptr;
+  uint32_t* blocks_done = nullptr;    // [kDoneWords] zero between requests
+  JoinAggregate* h_result = nullptr;  // pinned, written by the request's last kernel
   hipStream_t stream = nullptr;
   hipEvent_t done = nullptr;
   std::vector<void*> allocs;
@@ -170,10 +170,8 @@ fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
   if (b.table) {
     // a resident table: one probe launch, no partitioning of the probe side
     hipStream_t st = sl.stream;
-    SRV_HIP(launch_np_probe_resident(s->kt, b.table, b.table_lg, r.keys, r.pays, r.len, sl.aggregates, s->join_grid,
-                                     st));
-    SRV_HIP(launch_sum_aggregates(sl.aggregates, s->join_grid, sl.d_result, nullptr, st));
-    SRV_HIP(hipMemcpyAsync(sl.h_result, sl.d_result, sizeof(JoinAggregate), hipMemcpyDeviceToHost, st));
+    SRV_HIP(launch_np_probe_resident(s->kt, b.table, b.table_lg, r.keys, r.pays, r.len, sl.aggregates, sl.blocks_done,
+                                     sl.h_result, s->join_grid, st));
     SRV_HIP(hipEventRecord(sl.done, st));
     return FIJ_OK;
   }
@@ -192,6 +190,8 @@ fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
   d.unit_cap = sl.unit_cap;
   d.part_units = sl.part_units;
   d.aggregates = sl.aggregates;
+  d.result = sl.h_result;
+  d.done = sl.blocks_done;
   hipStream_t st = sl.stream;
   SRV_HIP(enqueue_pass1_prefix_sum(d, s->kt, 1024, st));
   SRV_HIP(enqueue_pass1_scatter(d, s->kt, 1024, s->lds_total, st));
@@ -201,12 +201,11 @@ fij_status launch_request(fij_join_server* s, Slot& sl, const Request& r) {
     SRV_HIP(launch_pipeline_sort2(d, s->kt, std::max(1u, std::min(s->cus, tiles)), st));
     SRV_HIP(launch_pipeline_join(d, s->kt, false, s->join_grid, st));
     SRV_HIP(launch_pipeline_join(d, s->kt, true, s->join_grid, st));
+    SRV_HIP(launch_sum_aggregates(sl.aggregates, s->agg_len, sl.h_result, nullptr, st));
   } else {
     SRV_HIP(launch_one_pass_plan(d, s->kt, nullptr, 1, st));
-    SRV_HIP(launch_one_pass_join(d, s->kt, false, s->join_grid, st));
+    SRV_HIP(launch_one_pass_join(d, s->kt, s->join_grid, st));
   }
-  SRV_HIP(launch_sum_aggregates(sl.aggregates, s->agg_len, sl.d_result, nullptr, st));
-  SRV_HIP(hipMemcpyAsync(sl.h_result, sl.d_result, sizeof(JoinAggregate), hipMemcpyDeviceToHost, st));
   SRV_HIP(hipEventRecord(sl.done, st));
   return FIJ_OK;
 }
@@ -290,7 +289,8 @@ fij_status make_slot(fij_join_server* s, Slot& sl, uint64_t probe_cap) {
   SRV_HIP(alloc(reinterpret_cast<void**>(&sl.units), sl.unit_cap * sizeof(uint4)));
   SRV_HIP(alloc(reinterpret_cast<void**>(&sl.part_units), part_unit_cap(kMaxF1, probe_cap) * sizeof(PartUnit)));
   SRV_HIP(alloc(reinterpret_cast<void**>(&sl.aggregates), s->agg_len * sizeof(JoinAggregate)));
-  SRV_HIP(alloc(reinterpret_cast<void**>(&sl.d_result), sizeof(JoinAggregate)));
+  SRV_HIP(alloc(reinterpret_cast<void**>(&sl.blocks_done), kDoneWords * sizeof(uint32_t)));
+  SRV_HIP(hipMemset(sl.blocks_done, 0, kDoneWords * sizeof(uint32_t)));
   SRV_HIP(hipHostMalloc(reinterpret_cast<void**>(&sl.h_result), sizeof(JoinAggregate), hipHostMallocDefault));
   SRV_HIP(hipStreamCreateWithFlags(&sl.stream, hipStreamNonBlocking));
   SRV_HIP(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));

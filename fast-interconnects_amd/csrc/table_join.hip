@@ -5,6 +5,7 @@
 #include "bucket_table.hpp"
 #include "common.hpp"
 #include "internal.hpp"
+#include "join_result.hpp"
 #include "pipeline.hpp"
 
 namespace fij {
@@ -122,8 +123,7 @@ struct ColumnStream {
   }
 };
 
-// One join.  done counts finished blocks (zero between joins); the last one
-// writes the sums of all to *result.
+// One join; the last block writes the sums of all to *result (finish_join).
 //
 // Bound by the chain launch -> build -> probe for short probe sides and by the
 // read of the probe columns for long ones.  1,500 x 6,007 int32 tuples: one
@@ -147,30 +147,8 @@ __global__ __launch_bounds__(BLOCK) void table_join_kernel(TableJoin j) {
                                                 &s_dup, unique);
     s.run(tab, unique, cnt, sb, sp);
   }
-  block_sums<BLOCK>(red, cnt, sb, sp);
-  if (gridDim.x > 1) {
-    if (threadIdx.x == 0) {
-      j.partial[blockIdx.x] = JoinAggregate{cnt, sb, sp};
-      __threadfence();  // the partial sums are visible before the block is counted
-      s_last = atomicAdd(j.done, 1u) == gridDim.x - 1 ? 1u : 0u;
-    }
-    __syncthreads();
-    if (!s_last) return;  // uniform
-    __threadfence();
-    cnt = sb = sp = 0;
-    for (uint32_t i = threadIdx.x; i < gridDim.x; i += BLOCK) {
-      const uint64_t* r = reinterpret_cast<const uint64_t*>(j.partial + i);
-      cnt += __hip_atomic_load(r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      sb += __hip_atomic_load(r + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      sp += __hip_atomic_load(r + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    block_sums<BLOCK>(red, cnt, sb, sp);
-    if (threadIdx.x == 0) *j.done = 0;
-  }
-  if (threadIdx.x == 0) {
-    *j.result = JoinAggregate{cnt, sb, sp};
-    if (j.stamps) j.stamps[5] = wall_clock64();
-  }
+  if (finish_join<BLOCK>(j.partial, j.done, j.result, red, &s_last, cnt, sb, sp) && j.stamps && threadIdx.x == 0)
+    j.stamps[5] = wall_clock64();
 }
 
 template <typename K, uint32_t CAP, uint32_t BLOCK>

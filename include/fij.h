@@ -341,7 +341,7 @@ typedef struct fij_join_plan_config {
   uint32_t radix_bits_2; /* pass-2 bits; 0 = single pass */
   uint32_t pass1_chunks; /* pass-1 chunks (= blocks); 0 = one per compute unit (fewer for short relations) */
   uint32_t pass1_block;  /* threads per pass-1 block; 0 = 1024 */
-  uint32_t join_blocks;  /* resident blocks of the join; 0 = two per compute unit */
+  uint32_t join_blocks;  /* resident blocks of the join at most; 0 = one to four per compute unit */
   uint64_t build_len;    /* |R| */
   uint64_t probe_len;    /* |S| */
 } fij_join_plan_config;
@@ -350,8 +350,9 @@ typedef struct fij_join_plan_config {
  * (radix-join/src/measurement/data_point.rs:29-74): prefix sum (pass-1
  * histograms), partition (pass-1 scatter), join (pass 2 + build/probe);
  * join_ms splits into pass2_ms (plan + pass-2 sort), build_probe_ms (the
- * register-resident build/probe launch) and deferred_ms (the launch that
- * joins the partitions too large for it). */
+ * register-resident or block-table build/probe) and deferred_ms (the join of
+ * the partitions too large for it).  A join whose build side fits one LDS
+ * table is not partitioned: all of its time is build_probe_ms. */
 typedef struct fij_join_timing {
   float prefix_sum_ms;
   float partition_ms;
