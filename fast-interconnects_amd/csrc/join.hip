@@ -7,6 +7,7 @@
 // per-thread partials; this library writes those partials unchanged (when
 // asked) and additionally a per-block {match count, SUM(build.value),
 // SUM(probe.value)} as wrapping 64-bit integers.
+#include "bucket_table.hpp"
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -30,6 +31,7 @@ struct JoinParams {
   JoinAggregate* aggregates;
   const uint32_t* task_assignments;
   uint32_t* status;
+  uint32_t table_slots;  // of the largest bucket table (a power of two)
 };
 
 // Largest fanout whose task assignment runs by pointer doubling (its LDS:
@@ -120,8 +122,75 @@ __global__ __launch_bounds__(1024) void assign_tasks_kernel(const uint64_t* prob
   }
 }
 
-// Probe tuples in flight per thread in the LDS joins.
-constexpr uint32_t kJoinLoads = 8;
+// The partitions part .. end - 1 of a block, whose results are task `owner`'s.
+struct TaskPart {
+  uint32_t part, end, owner;
+};
+
+// A task takes partitions up to the average number of probe tuples, so tasks
+// of about two partitions alternate with tasks of one and as many blocks are
+// left without any.  With at least as many blocks as partitions those blocks
+// take the second and later partitions of the others' tasks, and a launch
+// lasts one partition instead of two: with N tasks the i-th block behind them
+// takes the i-th such partition, partition i + k + 1 of the task k with
+// ta[k] - k <= i < ta[k + 1] - (k + 1).
+__device__ __forceinline__ TaskPart block_task(const JoinParams& p) {
+  const uint32_t* const ta = p.task_assignments;
+  const uint32_t F = 1u << p.radix_bits, b = blockIdx.x;
+  if (F > gridDim.x) return {ta[b], ta[b + 1], b};
+  __shared__ uint32_t s_tasks, s_owner;
+  if (threadIdx.x == 0) s_tasks = s_owner = 0;
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < gridDim.x; k += blockDim.x)
+    if (ta[k] < F) atomicMax(&s_tasks, k + 1);
+  __syncthreads();
+  const uint32_t n = s_tasks, i = b - n;
+  if (b < n) return {ta[b], ta[b] + 1, b};
+  if (i >= F - n) return {F, F, b};  // uniform
+  for (uint32_t k = threadIdx.x; k < n; k += blockDim.x)
+    if (ta[k] - k <= i && i < ta[k + 1] - (k + 1)) s_owner = k;
+  __syncthreads();
+  const uint32_t k = s_owner;
+  return {i + k + 1, i + k + 2, k};
+}
+
+// Probe tuples q0 .. q1 - 1 (at least one) of a block, streamed through two
+// buffers of N tuples per thread: thread i takes tuples q0 + i, q0 + i +
+// blockDim, ... (lanes past the end repeat the last tuple).
+template <typename K>
+struct ProbeStream {
+  static constexpr uint32_t N = 4;
+  const Tuple<K>* probe;
+  uint64_t q0, q1;
+  Tuple<K> a[N], b[N];
+
+  __device__ __forceinline__ void load(Tuple<K> (&t)[N], uint64_t i0) {
+#pragma unroll
+    for (uint32_t k = 0; k < N; ++k)
+      t[k] = load_tuple<K>(probe + min<uint64_t>(i0 + k * blockDim.x + threadIdx.x, q1 - 1));
+  }
+  __device__ __forceinline__ void start() {
+    if (q0 < q1) load(a, q0);
+  }
+  // f(tuples, live): bit k of live = tuple k is in the range.
+  template <typename Fn>
+  __device__ __forceinline__ void run(Fn f) {
+    const uint64_t step = static_cast<uint64_t>(N) * blockDim.x;
+    auto live = [&](uint64_t i0) {
+      uint32_t m = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < N; ++k) m |= i0 + k * blockDim.x + threadIdx.x < q1 ? 1u << k : 0u;
+      return m;
+    };
+    for (uint64_t i0 = q0; i0 < q1; i0 += 2 * step) {
+      load(b, i0 + step);
+      f(a, live(i0));
+      if (i0 + step >= q1) break;
+      load(a, i0 + 2 * step);
+      f(b, live(i0 + step));
+    }
+  }
+};
 
 __device__ __forceinline__ void partition_range(const uint64_t* offsets, uint64_t padded_len, uint32_t F,
                                                 uint32_t p, uint32_t pad, uint64_t& begin, uint64_t& end) {
@@ -143,7 +212,14 @@ __device__ __forceinline__ uint32_t chain_bucket(K key, uint32_t ignore_bits, ui
   return mult_shift_hash<K>(static_cast<K>(perfect_index<K>(key, ignore_bits)), log2_buckets);
 }
 
-// Block-wide sum of three u64 values into aggregates[blockIdx.x] (+=).
+template <typename U>
+__device__ __forceinline__ void add_u64(U* at, uint64_t v) {
+  static_assert(sizeof(U) == 8, "64-bit words");
+  atomicAdd(reinterpret_cast<unsigned long long*>(at), static_cast<unsigned long long>(v));
+}
+
+// Block-wide sum of three u64 values into *out (+=), which other blocks of its
+// task may add to.
 __device__ void block_aggregate(JoinAggregate* out, uint64_t c, uint64_t sb, uint64_t sp) {
   __shared__ uint64_t red[3][16];
   const uint32_t w = threadIdx.x / kWave;
@@ -163,9 +239,9 @@ __device__ void block_aggregate(JoinAggregate* out, uint64_t c, uint64_t sb, uin
       b += red[1][i];
       d += red[2][i];
     }
-    out[blockIdx.x].count += a;
-    out[blockIdx.x].sum_build += b;
-    out[blockIdx.x].sum_probe += d;
+    add_u64(&out->count, a);
+    add_u64(&out->sum_build, b);
+    add_u64(&out->sum_probe, d);
   }
 }
 
@@ -181,10 +257,15 @@ __global__ __launch_bounds__(1024) void join_perfect_kernel(JoinParams p) {
   uint64_t cnt = 0, sb = 0, sp = 0;
   int64_t ref_sum = 0;
   bool overflow = false;
-  for (uint32_t part = p.task_assignments[blockIdx.x]; part < p.task_assignments[blockIdx.x + 1]; ++part) {
-    uint64_t b0, b1, q0, q1;
+  const TaskPart task = block_task(p);
+  if (task.part == task.end) return;  // uniform: adds nothing
+  for (uint32_t part = task.part; part < task.end; ++part) {
+    ProbeStream<K> stream;
+    stream.probe = probe;
+    uint64_t b0, b1;
     partition_range(p.build_offsets, p.build_len, F, part, pad, b0, b1);
-    partition_range(p.probe_offsets, p.probe_len, F, part, pad, q0, q1);
+    partition_range(p.probe_offsets, p.probe_len, F, part, pad, stream.q0, stream.q1);
+    stream.start();  // in flight while the table is built
     for (uint32_t i = threadIdx.x; i < E; i += blockDim.x) {
       ht[i].key = null_key<K>();
       ht[i].value = 0;
@@ -198,35 +279,85 @@ __global__ __launch_bounds__(1024) void join_perfect_kernel(JoinParams p) {
       else overflow = true;
     }
     __syncthreads();
-    // thread i takes tuples q0 + i, q0 + i + blockDim, ... (kJoinLoads loads
-    // in flight; lanes past the end re-read the last tuple and skip it)
-    for (uint64_t i0 = q0; i0 < q1; i0 += kJoinLoads * blockDim.x) {
-      Tuple<K> t[kJoinLoads];
+    stream.run([&](const Tuple<K>(&t)[ProbeStream<K>::N], uint32_t live) {
 #pragma unroll
-      for (uint32_t k = 0; k < kJoinLoads; ++k)
-        t[k] = load_tuple<K>(probe + min<uint64_t>(i0 + k * blockDim.x + threadIdx.x, q1 - 1));
-#pragma unroll
-      for (uint32_t k = 0; k < kJoinLoads; ++k) {
+      for (uint32_t k = 0; k < ProbeStream<K>::N; ++k) {
         const uint32_t idx = perfect_index<K>(t[k].key, p.ignore_bits);
-        if (i0 + k * blockDim.x + threadIdx.x < q1 && t[k].key != null_key<K>() && idx < E &&
-            ht[idx].key == t[k].key) {
+        if (((live >> k) & 1u) && t[k].key != null_key<K>() && idx < E && ht[idx].key == t[k].key) {
           cnt += 1;
           sb += static_cast<uint64_t>(static_cast<int64_t>(ht[idx].value));
           sp += static_cast<uint64_t>(static_cast<int64_t>(t[k].value));
           ref_sum += static_cast<int64_t>(t[k].value);
         }
       }
-    }
+    });
     __syncthreads();
   }
   if (overflow && p.status) atomicOr(p.status, kStatusHashTableFull);
-  if (p.result_set) p.result_set[static_cast<uint64_t>(blockDim.x) * blockIdx.x + threadIdx.x] += ref_sum;
-  if (p.aggregates) block_aggregate(p.aggregates, cnt, sb, sp);
+  if (p.result_set)
+    add_u64(p.result_set + static_cast<uint64_t>(blockDim.x) * task.owner + threadIdx.x, static_cast<uint64_t>(ref_sum));
+  if (p.aggregates) block_aggregate(p.aggregates + task.owner, cnt, sb, sp);
 }
 
+// One partition's build tuples (at most 3/4 of p.table_slots) in a bucket table
+// and its probe tuples against it.
+template <typename K>
+__device__ __forceinline__ void bucket_join(const JoinParams& p, uint64_t* lds, uint32_t* s_dup,
+                                            const Tuple<K>* build, uint32_t nbuild, ProbeStream<K>& stream,
+                                            uint64_t& cnt, uint64_t& sb, uint64_t& sp) {
+  using Table = BucketTable<K, true>;
+  using Quad = typename Table::Quad;
+  // at most 1/4 full where the table allows it, 3/4 at most
+  const uint32_t lg = min(29u - static_cast<uint32_t>(__builtin_clz(p.table_slots)),
+                          max(6u, 32u - static_cast<uint32_t>(__builtin_clz(nbuild | 1u))));
+  const Table tab{reinterpret_cast<Quad*>(lds), reinterpret_cast<Quad*>(lds) + p.table_slots / 4, 32u - lg,
+                  (1u << lg) - 1u, null_key<K>()};
+  for (uint32_t i = threadIdx.x; i < (1u << lg); i += blockDim.x)
+    tab.keys[i] = Quad{null_key<K>(), null_key<K>(), null_key<K>(), null_key<K>()};
+  if (threadIdx.x == 0) *s_dup = 0;
+  __syncthreads();
+  bool dup = false;
+  for (uint32_t i = threadIdx.x; i < nbuild; i += blockDim.x) {
+    const Tuple<K> t = load_tuple<K>(build + i);
+    if (t.key != null_key<K>()) dup |= tab.insert(t.key, t.value);  // null keys never join
+  }
+  if (dup) *s_dup = 1;
+  __syncthreads();
+  const bool unique = __builtin_amdgcn_readfirstlane(*s_dup) == 0;
+  uint32_t wave_cnt = 0;
+  stream.run([&](const Tuple<K>(&t)[ProbeStream<K>::N], uint32_t live) {
+#pragma unroll
+    for (uint32_t g = 0; g < ProbeStream<K>::N; g += 2) {
+      K key[2], pay[2];
+#pragma unroll
+      for (uint32_t i = 0; i < 2; ++i) {
+        key[i] = (live >> (g + i)) & 1u ? t[g + i].key : null_key<K>();
+        pay[i] = t[g + i].value;
+      }
+      if (unique) {
+        tab.probe_unique(key, pay, wave_cnt, cnt, sb, sp);
+      } else {
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i)
+          if (key[i] != null_key<K>()) tab.probe_from(tab.bucket(key[i]), key[i], pay[i], cnt, sb, sp);
+      }
+    }
+  });
+  if (lane_id() == 0) cnt += wave_cnt;
+}
+
+// Small build sides go into chains (radix_join.cu:208-392's layout): as long
+// as chains are short, their three reads per entry cost less than clearing and
+// filling a table (586 build and 7,800 probe tuples per block at int64: 10.2 us,
+// 12.1 us with tables).  Beyond half an entry per bucket a bucket table answers
+// a probe with two reads, where the longest chain among a wave's lanes is four
+// and more entries deep (4,096 and 65,536 tuples at int32: 41 us, 57 us with
+// chains).  Build sides that no bucket table holds, up to ht_entries, fit
+// chains only.
 template <typename K>
 __global__ __launch_bounds__(1024) void join_chaining_kernel(JoinParams p) {
-  extern __shared__ uint64_t lds_u64[];
+  extern __shared__ __attribute__((aligned(16))) uint64_t lds_u64[];
+  __shared__ uint32_t s_dup;
   const uint32_t E = p.ht_entries;  // entries (<= 0xFFFF)
   K* keys = reinterpret_cast<K*>(lds_u64);
   K* vals = keys + E;
@@ -238,15 +369,24 @@ __global__ __launch_bounds__(1024) void join_chaining_kernel(JoinParams p) {
   const Tuple<K>* build = static_cast<const Tuple<K>*>(p.build_rel);
   const Tuple<K>* probe = static_cast<const Tuple<K>*>(p.probe_rel);
   uint64_t cnt = 0, sb = 0, sp = 0;
-  int64_t ref_sum = 0;
   bool overflow = false;
-  for (uint32_t part = p.task_assignments[blockIdx.x]; part < p.task_assignments[blockIdx.x + 1]; ++part) {
-    uint64_t b0, b1, q0, q1;
+  const TaskPart task = block_task(p);
+  if (task.part == task.end) return;  // uniform: adds nothing
+  for (uint32_t part = task.part; part < task.end; ++part) {
+    ProbeStream<K> stream;
+    stream.probe = probe;
+    uint64_t b0, b1;
     partition_range(p.build_offsets, p.build_len, F, part, pad, b0, b1);
-    partition_range(p.probe_offsets, p.probe_len, F, part, pad, q0, q1);
+    partition_range(p.probe_offsets, p.probe_len, F, part, pad, stream.q0, stream.q1);
+    stream.start();  // in flight while the table is built
     const uint64_t nb = b1 - b0;
     if (nb > E) overflow = true;
     const uint32_t nbuild = nb > E ? E : static_cast<uint32_t>(nb);
+    if (nbuild > kChainBuckets / 2 && nbuild <= p.table_slots / 4 * 3) {
+      bucket_join<K>(p, lds_u64, &s_dup, build + b0, nbuild, stream, cnt, sb, sp);
+      __syncthreads();
+      continue;
+    }
     for (uint32_t i = threadIdx.x; i < kChainBuckets; i += blockDim.x) heads[i] = kChainTail;
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < nbuild; i += blockDim.x) {
@@ -258,30 +398,47 @@ __global__ __launch_bounds__(1024) void join_chaining_kernel(JoinParams p) {
       links[i] = static_cast<uint16_t>(atomicExch(&heads[bucket], i));
     }
     __syncthreads();
-    for (uint64_t i0 = q0; i0 < q1; i0 += kJoinLoads * blockDim.x) {
-      Tuple<K> t[kJoinLoads];
+    // the chains of a buffer's tuples are walked together: a step's LDS reads
+    // are in flight at once (entry 0 is read where a chain has ended)
+    stream.run([&](const Tuple<K>(&t)[ProbeStream<K>::N], uint32_t live) {
+      constexpr uint32_t N = ProbeStream<K>::N;
+      uint32_t e[N];
 #pragma unroll
-      for (uint32_t k = 0; k < kJoinLoads; ++k)
-        t[k] = load_tuple<K>(probe + min<uint64_t>(i0 + k * blockDim.x + threadIdx.x, q1 - 1));
+      for (uint32_t k = 0; k < N; ++k) {
+        const uint32_t head = heads[chain_bucket<K>(t[k].key, p.ignore_bits, log2_buckets)];
+        e[k] = ((live >> k) & 1u) && t[k].key != null_key<K>() ? head : kChainTail;
+      }
+      for (;;) {
+        bool any = false;
 #pragma unroll
-      for (uint32_t k = 0; k < kJoinLoads; ++k) {
-        if (i0 + k * blockDim.x + threadIdx.x >= q1 || t[k].key == null_key<K>()) continue;
-        const uint32_t bucket = chain_bucket<K>(t[k].key, p.ignore_bits, log2_buckets);
-        for (uint32_t e = heads[bucket]; e != kChainTail; e = links[e]) {
-          if (keys[e] == t[k].key) {
+        for (uint32_t k = 0; k < N; ++k) any |= e[k] != kChainTail;
+        if (!ballot(any)) break;
+        K key[N], val[N];
+        uint32_t next[N];
+#pragma unroll
+        for (uint32_t k = 0; k < N; ++k) {
+          const uint32_t at = e[k] != kChainTail ? e[k] : 0u;
+          key[k] = keys[at];
+          val[k] = vals[at];
+          next[k] = links[at];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < N; ++k) {
+          if (e[k] == kChainTail) continue;
+          if (key[k] == t[k].key) {
             cnt += 1;
-            sb += static_cast<uint64_t>(static_cast<int64_t>(vals[e]));
+            sb += static_cast<uint64_t>(static_cast<int64_t>(val[k]));
             sp += static_cast<uint64_t>(static_cast<int64_t>(t[k].value));
-            ref_sum += static_cast<int64_t>(t[k].value);
           }
+          e[k] = next[k];
         }
       }
-    }
+    });
     __syncthreads();
   }
   if (overflow && p.status) atomicOr(p.status, kStatusHashTableFull);
-  if (p.result_set) p.result_set[static_cast<uint64_t>(blockDim.x) * blockIdx.x + threadIdx.x] += ref_sum;
-  if (p.aggregates) block_aggregate(p.aggregates, cnt, sb, sp);
+  if (p.result_set) add_u64(p.result_set + static_cast<uint64_t>(blockDim.x) * task.owner + threadIdx.x, sp);
+  if (p.aggregates) block_aggregate(p.aggregates + task.owner, cnt, sb, sp);
 }
 
 template <typename K>
@@ -316,6 +473,9 @@ hipError_t launch_join_t(const JoinLaunch& a, hipStream_t stream) {
     uint32_t entries = (lds - kChainBuckets * 4) / (2 + 2 * sizeof(K));
     if (entries > kChainTail) entries = kChainTail;
     p.ht_entries = entries;
+    uint32_t slots = 4;
+    while (4 * sizeof(K) * slots <= lds) slots *= 2;  // two columns of twice as many
+    p.table_slots = slots;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(lds));
     hipLaunchKernelGGL(kern, dim3(a.grid), dim3(a.block), lds, stream, p);
