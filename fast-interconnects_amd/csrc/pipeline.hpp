@@ -138,10 +138,42 @@ struct BatchSide {
   uint32_t reserved;
 };
 
-// Allocates one side's buffers (capacity n tuples, F1 x F2 partitions, G1
-// chunks; rel2 and meta only for two passes, meta with `tiles` + 1 rows) and
-// records every allocation in `allocs`.  rel1 holds n + F1 * pad_tuples(t)
+// Arrays placed in one allocation, 256-byte aligned (a first round without base
+// adds up their sizes, a second one sets the pointers), or each allocated by
+// itself and recorded in `allocs`.
+struct Placer {
+  uint8_t* base = nullptr;
+  uint64_t used = 0;
+  std::vector<void*>* allocs = nullptr;
+  hipError_t error = hipSuccess;  // of the allocations
+  template <typename T>
+  void take(T** p, uint64_t count) {
+    const uint64_t bytes = (count ? count : 1) * sizeof(T);
+    void* v = base ? base + used : nullptr;
+    if (allocs && error == hipSuccess && (error = hipMalloc(&v, bytes)) == hipSuccess) allocs->push_back(v);
+    used += (bytes + 255) / 256 * 256;
+    *p = static_cast<T*>(v);
+  }
+};
+// Places arrays with place(Placer&) in one new device allocation, recorded in
+// `allocs`.
+template <typename Place>
+hipError_t place_on_device(std::vector<void*>& allocs, Place place) {
+  Placer sizes, at;
+  place(sizes);
+  const hipError_t e = hipMalloc(reinterpret_cast<void**>(&at.base), sizes.used);
+  if (e != hipSuccess) return e;
+  allocs.push_back(at.base);
+  place(at);
+  return hipSuccess;
+}
+
+// One side's buffers (capacity n tuples, F1 x F2 partitions, G1 chunks; rel2
+// and meta only for two passes, meta with `tiles` + 1 rows), placed by `a` or
+// allocated and recorded in `allocs`.  rel1 holds n + F1 * pad_tuples(t)
 // tuples: the plan using it must set its pad to pad_tuples(t).
+void place_pipeline_side(PipelineSide& s, KeyType t, uint64_t n, uint32_t F1, uint32_t F2, uint32_t G1, bool two_pass,
+                         uint32_t tiles, Placer& a);
 hipError_t alloc_pipeline_side(PipelineSide& s, KeyType t, uint64_t n, uint32_t F1, uint32_t F2, uint32_t G1,
                                bool two_pass, uint32_t tiles, std::vector<void*>& allocs);
 // Pass 1 of the sides in d.sides (each in its g1 chunks): contiguous

@@ -10,50 +10,39 @@
 
 namespace fij {
 
-namespace {
-
-template <typename T>
-hipError_t alloc_n(T** out, uint64_t count, std::vector<void*>& allocs) {
-  void* p = nullptr;
-  const hipError_t e = hipMalloc(&p, (count ? count : 1) * sizeof(T));
-  if (e != hipSuccess) return e;
-  allocs.push_back(p);
-  *out = static_cast<T*>(p);
-  return hipSuccess;
-}
-
-}  // namespace
-
-hipError_t alloc_pipeline_side(PipelineSide& s, KeyType t, uint64_t n, uint32_t F1, uint32_t F2, uint32_t G1,
-                               bool two_pass, uint32_t tiles, std::vector<void*>& allocs) {
+void place_pipeline_side(PipelineSide& s, KeyType t, uint64_t n, uint32_t F1, uint32_t F2, uint32_t G1, bool two_pass,
+                         uint32_t tiles, Placer& a) {
   const uint32_t tb = tuple_bytes(t);
   s.n = n;
   s.padded_len1 = n + static_cast<uint64_t>(F1) * pad_tuples(t);
   s.g1 = G1;
   s.scan1_len = scan_state_words(F1);
-  hipError_t e;
-  if ((e = alloc_n(&s.off1, F1, allocs)) != hipSuccess) return e;
-  if ((e = alloc_n(&s.local1, static_cast<uint64_t>(G1) * F1, allocs)) != hipSuccess) return e;
-  if ((e = alloc_n(&s.counts1, static_cast<uint64_t>(F1) * G1, allocs)) != hipSuccess) return e;
-  if ((e = alloc_n(&s.scan1, s.scan1_len, allocs)) != hipSuccess) return e;
-  uint8_t* rel1 = nullptr;
+  a.take(&s.off1, F1);
+  a.take(&s.local1, static_cast<uint64_t>(G1) * F1);
+  a.take(&s.counts1, static_cast<uint64_t>(F1) * G1);
+  a.take(&s.scan1, s.scan1_len);
+  uint8_t *rel1 = nullptr, *rel2 = nullptr;
   // one spare tuple after the end: pass 2 reads 8-byte tuples in aligned
   // pairs, and the last pair may end one tuple past the relation
-  if ((e = alloc_n(&rel1, (s.padded_len1 + 1) * tb, allocs)) != hipSuccess) return e;
-  s.rel1 = rel1;
-  if ((e = alloc_n(&s.plen, F1, allocs)) != hipSuccess) return e;
-  if ((e = alloc_n(&s.pstart, F1 + 1, allocs)) != hipSuccess) return e;
-  if ((e = alloc_n(&s.tile_start, F1 + 1, allocs)) != hipSuccess) return e;
+  a.take(&rel1, (s.padded_len1 + 1) * tb);
+  a.take(&s.plen, F1);
+  a.take(&s.pstart, F1 + 1);
+  a.take(&s.tile_start, F1 + 1);
+  s.meta = nullptr;
   if (two_pass) {
-    uint8_t* rel2 = nullptr;
-    if ((e = alloc_n(&rel2, n * tb, allocs)) != hipSuccess) return e;
-    s.rel2 = rel2;
-    if ((e = alloc_n(&s.meta, (static_cast<uint64_t>(tiles) + 1) * F2, allocs)) != hipSuccess) return e;
-  } else {
-    s.rel2 = nullptr;
-    s.meta = nullptr;
+    a.take(&rel2, n * tb);
+    a.take(&s.meta, (static_cast<uint64_t>(tiles) + 1) * F2);
   }
-  return hipSuccess;
+  s.rel1 = rel1;
+  s.rel2 = rel2;
+}
+
+hipError_t alloc_pipeline_side(PipelineSide& s, KeyType t, uint64_t n, uint32_t F1, uint32_t F2, uint32_t G1,
+                               bool two_pass, uint32_t tiles, std::vector<void*>& allocs) {
+  Placer a;
+  a.allocs = &allocs;
+  place_pipeline_side(s, t, n, F1, F2, G1, two_pass, tiles, a);
+  return a.error;
 }
 
 uint32_t pass1_chunks(KeyType t, uint64_t n, uint32_t most) {
