@@ -244,13 +244,13 @@ struct TupleVec {
 // by ticket, taken while the current unit runs).
 //
 // Bound by the read of the probe partitions (with inserts and probes left out
-// of a copy: 36 of 46 us, 126 of 186 us, 230 of 240 us for the shapes below),
+// of a copy: 36 of 46 us, 126 of 174 us, 230 of 240 us for the shapes below),
 // plus what the phases of a block do not overlap.  2^20 + 2^24 int32 tuples in
 // 512 partitions: 46 us, where the two-pass plans' register join (23 us, every
 // item only put off), unit counting (8 us) and block join (48 us, every
 // tuple's run looked up although a partition is one run) ran before; 20 batched
 // joins of 2^18..2^20 int32 build tuples 1,053 -> 240 us; 5,000,011 +
-// 20,000,003 int64 tuples (two fills) 186 us.  Two and four vectors per buffer,
+// 20,000,003 int64 tuples (two fills) 174 us.  Two and four vectors per buffer,
 // two or four probes together and build tuples loaded a fill ahead all lay
 // within 3 % of each other; the smallest register need was taken.
 template <typename K, uint32_t CAP, uint32_t BLOCK>
