@@ -455,20 +455,20 @@ fij_join_tuning tuned_class(KeyType kt, uint64_t build_len, uint64_t probe_len, 
 }
 
 // The class that a batch runs a partitioned join of these lengths in.  Build
-// sides of up to two table fills per partition (one_pass_limit) take a single
+// sides of up to two table fills per partition (one_pass_join) take a single
 // pass, in classes of a factor of four from 2^14 (int64: 2^13) tuples on: 5, 7
 // and 9 bits leave 512 to 2,048 (256 to 1,024) tuples in a partition, for 32
 // KiB tables; beyond, 9 bits with 64 KiB and then 128 KiB tables.
 ClassKey batch_class(KeyType kt, uint64_t build_len, uint64_t probe_len) {
   bool user = false;
   const fij_join_tuning tc = tuned_class(kt, build_len, probe_len, &user);
-  if (user || build_len > one_pass_limit(kt)) return {tc.radix_bits_1, tc.radix_bits_2, tc.ring_lines, tc.block, 0};
+  if (user || !one_pass_join(kt, build_len, probe_len)) return {tc.radix_bits_1, tc.radix_bits_2, tc.ring_lines, tc.block, 0};
   uint32_t b1 = 5;
   uint64_t most = kt == KeyType::I32 ? 1u << 16 : 1u << 15;
   for (; build_len > most && b1 < kOnePassBits; b1 += 2) most <<= 2;
   if (build_len > most) {
     most = static_cast<uint64_t>(pipeline_block_table_tuples(kt, false)) << kOnePassBits;
-    if (!block_tables_hold(kt, build_len, 1ull << kOnePassBits, false)) most = one_pass_limit(kt);
+    if (!block_tables_hold(kt, build_len, 1ull << kOnePassBits, false)) most = 2 * one_pass_fill(kt) << kOnePassBits;
   }
   return {b1, 0, 0, 1024, static_cast<uint32_t>(most)};
 }

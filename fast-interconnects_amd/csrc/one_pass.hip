@@ -31,8 +31,8 @@ __device__ __forceinline__ U uniform_load(const U* ptr) {
 }
 
 // Slots of the block-shared table: 64 KiB of keys and values, half of that
-// for small partitions, or 128 KiB (big_block_tables).  A build range may fill
-// 3/4 of them.
+// for small partitions, or 128 KiB (big_block_tables).  A fill takes at most
+// 9/16 (int32) or 5/8 (int64) of them.
 template <typename K>
 constexpr uint32_t kSlots = 65536 / (2 * sizeof(K));
 
@@ -257,7 +257,7 @@ template <typename K, uint32_t CAP, uint32_t BLOCK>
 __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
   using V = TupleVec<K>;
   using VT = typename V::type;
-  constexpr uint32_t RCAP = CAP * 3 / 4;      // build tuples per table fill
+  constexpr uint32_t FILL = CAP / 16 * (sizeof(K) == 4 ? 9 : 10);  // build tuples per table fill (one_pass_fill)
   constexpr uint32_t LG_CAP = 29u - __builtin_clz(CAP);  // of its buckets
   constexpr uint32_t NV = 2;                  // vectors in flight per buffer
   constexpr uint32_t NT = NV * V::N;          // their tuples
@@ -297,11 +297,11 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
     uint32_t wave_cnt = 0;
     VT xa[NV], xb[NV];
     load(xa, 0);  // in flight while the table is built
-    // equal fills: the emptier the table, the fewer probes leave their bucket
-    const uint32_t fill = nb <= RCAP ? nb : (nb + (nb + RCAP - 1) / RCAP - 1) / ((nb + RCAP - 1) / RCAP);
+    // equal fills
+    const uint32_t fills = (nb + FILL - 1) / FILL, fill = (nb + fills - 1) / fills;
     for (uint32_t f0 = 0; f0 < nb; f0 += fill) {
       const uint32_t nf = min(fill, nb - f0);
-      // at most 1/4 full where the table allows it, 3/4 at most
+      // at most 1/4 full where the table allows it
       const uint32_t lg = min(LG_CAP, max(6u, 32u - static_cast<uint32_t>(__builtin_clz(nf))));
       using Quad = typename BucketTable<K>::Quad;
       const BucketTable<K> tab{reinterpret_cast<Quad*>(lds_u64), reinterpret_cast<Quad*>(lds_u64) + CAP / 4, 32u - lg,

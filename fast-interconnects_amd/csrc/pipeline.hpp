@@ -213,14 +213,37 @@ inline bool block_tables_hold(KeyType t, uint64_t build_len, uint64_t partitions
 inline bool one_pass_fits(KeyType t, uint64_t build_len) {
   return block_tables_hold(t, build_len, 1ull << kOnePassBits, true);
 }
+// Build tuples of one fill of a 128 KiB table in each of 2^kOnePassBits
+// partitions.  A fill takes 5/8 of the slots at int64, 9/16 at int32: fuller
+// buckets overflow, and probes that leave theirs (in a table with duplicate
+// keys every one whose bucket is full) made fills of 70 % 0.7 to 0.9 times as
+// fast as two passes, at int32 fills of 60 % 0.94 to 1.5 times.
+inline uint64_t one_pass_fill(KeyType t) {
+  return static_cast<uint64_t>(pipeline_block_table_tuples(t, true)) * (t == KeyType::I32 ? 9 : 10) / 12;
+}
 // Build tuples up to which a two-pass plan runs in a single pass of
-// kOnePassBits instead: its partitions hold at most two fills of a 128 KiB
-// table on average (1/16 of headroom for uneven ones).  Per probe tuple of t
-// bytes a second fill reads t again, a second pass reads and writes t and
-// gathers short runs: pass 2 and join of 5,000,011 x 20,000,003 int64 tuples
-// take 385 us in 8 + 8 bits and 200 us in a single pass with two fills.
+// kOnePassBits instead, whatever the probe side: two fills of 9/16 of the slots
+// on average at int64, one at int32 (1/32 of headroom for uneven partitions).
+// Per probe tuple of t bytes a second fill reads t again, a second pass reads
+// and writes t and gathers short runs: 3 M x 2^28 int64 tuples take 3.4 ms in a
+// single pass and 4.5 ms in two, 4.56 M x 2^29 int32 tuples 3.0 and 5.0 ms
+// (with three copies of every build key 6.0 and 6.5 ms).
 inline uint64_t one_pass_limit(KeyType t) {
-  return (2ull * pipeline_block_table_tuples(t, true) << kOnePassBits) * 15 / 16;
+  return (static_cast<uint64_t>(pipeline_block_table_tuples(t, true)) * (t == KeyType::I32 ? 3 : 6) / 4 << kOnePassBits) *
+         31 / 32;
+}
+// Whether it does for these lengths: beyond, two fills pay for probe sides that
+// are not too long: int32 tuples are moved in half the time and probed in the
+// same (7,300,000 x 10 M tuples: 167 against 323 us; 7 M x 220 M 1.7 to 2.8
+// against 2.1 to 2.8 ms, by keys; x 2^29 4.0 to 6.9 against 4.7 to 6.4 ms); at
+// int64 the tables fill up (5,000,011 x 20,000,003 tuples: 390 against 590 us,
+// with copies 560 against 660; 5,070,000 x 150 M 2.2 to 3.6 against 2.6 to 3.3
+// ms).
+inline bool one_pass_join(KeyType t, uint64_t build_len, uint64_t probe_len) {
+  if (build_len <= one_pass_limit(t)) return true;
+  const uint64_t fill = one_pass_fill(t) << kOnePassBits;
+  return t == KeyType::I32 ? build_len <= fill * 3 / 2 && probe_len / 32 <= build_len
+                           : build_len <= 2 * fill * 31 / 32 && probe_len / 16 <= build_len;
 }
 // Pass-2 bits of a two-pass plan of 9 + b2 bits whose items hold about a
 // third of a 64 KiB block table's build tuples (1,024 int64, 2,048 int32):

@@ -287,7 +287,7 @@ fij_status enqueue_join(fij_join_plan* p, const void* build_keys, const void* bu
   // A two-pass plan's join of a build side that a single pass leaves in
   // partitions of at most two table fills is run in one: the probe tuples are
   // read once more instead of partitioned once more.
-  PipelineDevice& d = p->d.bits2 && n_b <= one_pass_limit(p->kt) ? p->one : p->d;
+  PipelineDevice& d = p->d.bits2 && one_pass_join(p->kt, n_b, n_p) ? p->one : p->d;
   d.stamps = stamps;
   d.build.keys = build_keys;
   d.build.pays = build_pays;

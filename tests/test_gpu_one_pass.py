@@ -96,3 +96,21 @@ def test_two_pass_plan_beyond_two_fills(dtype, n_r):
         rows = at[sk[hit].astype(np.int64)]
         want = (int(hit.sum()), int(rp[rows].astype(np.int64).sum()), int(sp[hit].astype(np.int64).sum()))
         assert got == want
+
+
+@pytest.mark.parametrize("dtype,limits", [(np.int32, (4_571_136, 7_077_888)), (np.int64, (4_571_136, 5_079_040))])
+def test_two_pass_plan_at_the_single_pass_limits(dtype, limits):
+    """Sized joins of a two-pass plan around the build sides up to which it
+    takes a single pass, for every probe side and for short ones."""
+    n_r, n_s = limits[1] + 1, 2_000_003
+    rk = orc.gen_perm(n_r, 12, dtype, 1)
+    rk[: n_r // 3] = rk[n_r // 3 : 2 * (n_r // 3)]  # a third of the keys twice
+    rp = orc.gen_iota(n_r, 5, dtype)
+    sk = orc.gen_uniform(n_s, 12, 2, 1, n_r + n_r // 5, dtype)
+    sp = orc.gen_iota(n_s, 0, dtype)
+    plan = fij.JoinPlan(dtype, n_r, n_s, 9, 7)
+    d = [to_dev(c) for c in (rk, rp, sk, sp)]
+    res = fij.DeviceArray(3, np.uint64)
+    for n in (limits[0], limits[0] + 1, limits[1], limits[1] + 1):
+        plan.enqueue_sized(d[0].view(0, n), d[1].view(0, n), d[2], d[3], res)
+        assert tuple(int(x) for x in res.to_host()) == orc.sort_merge_join(rk[:n], rp[:n], sk, sp)
