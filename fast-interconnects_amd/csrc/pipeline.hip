@@ -742,8 +742,14 @@ constexpr uint64_t kUnitTuples = 65536;
 // by join_general_kernel's wave tables with refills (path 1).  Blocks take
 // tickets of 64 items, one item per lane; the waves of a block split the
 // items' run rows between them, so the partition of a heavy key (thousands
-// of pass-2 tiles, one run row each) is summed by the whole block.  Flags
-// found are cleared, so they are all zero again for the next join.
+// of pass-2 tiles, one run row each) is summed by the whole block, and the
+// units of such an item are written by a whole wave (one lane and two 64-bit
+// divisions for each of 800 units took 167 us of a Zipf join of 2^27 + 2^30
+// int32 tuples).  Flags found are cleared, so they are all zero again for the
+// next join.
+//
+// all: the register join did not run, every item is deferred (items without a
+// match on either side need no unit).
 constexpr uint32_t kUnitsWaves = 8;
 constexpr uint32_t kUnitsRows = 32;  // rows in flight per lane
 
@@ -774,9 +780,14 @@ __device__ __forceinline__ void lane_item_side(const PipelineDevice& d, const Pi
   }
 }
 
-__global__ __launch_bounds__(kUnitsWaves * 64) void join_units_kernel(PipelineDevice d, uint32_t block_rcap) {
+__global__ __launch_bounds__(kUnitsWaves * 64) void join_units_kernel(PipelineDevice d, uint32_t block_rcap, uint32_t all) {
   stamp_phase(d.stamps, 4);
-  if (uniform_load(d.work_counter + kOverflowAny) == 0) return;
+  if (all) {
+    stamp_phase(d.stamps, 3);
+    if (blockIdx.x == 0 && threadIdx.x == 0) d.work_counter[kOverflowAny] = 1;
+  } else if (uniform_load(d.work_counter + kOverflowAny) == 0) {
+    return;
+  }
   __shared__ uint32_t s_ticket;
   __shared__ uint64_t part[2][kUnitsWaves][64];
   const uint32_t lane = lane_id(), w = threadIdx.x / 64;
@@ -790,7 +801,7 @@ __global__ __launch_bounds__(kUnitsWaves * 64) void join_units_kernel(PipelineDe
     if (static_cast<uint64_t>(t) * 64 >= items) break;
     // one item per lane, the same in every wave
     const uint32_t item = min(t * 64 + lane, items - 1);
-    const bool flagged = t * 64 + lane < items && d.overflow[item] != 0;
+    bool flagged = t * 64 + lane < items && (all || d.overflow[item] != 0);
     if (__builtin_amdgcn_ballot_w64(flagged) == 0) continue;
     const uint32_t p = item / F2, q = item % F2;
     uint32_t np, nb;
@@ -805,7 +816,8 @@ __global__ __launch_bounds__(kUnitsWaves * 64) void join_units_kernel(PipelineDe
       tuples += part[0][i][lane];
       btuples += part[1][i][lane];
     }
-    if (flagged) d.overflow[item] = 0;
+    if (flagged && !all) d.overflow[item] = 0;
+    flagged = flagged && tuples != 0 && btuples != 0;
     uint32_t path = btuples <= block_rcap ? 0u : 1u;
     // A larger build side gets a hash table in the HBM arena when the arena
     // has room for it (at least twice its tuples, a power of two): path 2.
@@ -846,18 +858,34 @@ __global__ __launch_bounds__(kUnitsWaves * 64) void join_units_kernel(PipelineDe
     base_w = __builtin_amdgcn_readlane(base_w, 63) + incl_w - uw;
     base_hb = __builtin_amdgcn_readlane(base_hb, 63) + incl_hb - hb;
     base_hp = __builtin_amdgcn_readlane(base_hp, 63) + incl_hp - hp;
-    for (uint32_t u = 0; u < units; ++u) {
-      const uint32_t r0 = static_cast<uint32_t>(static_cast<uint64_t>(u) * np / units);
-      const uint32_t r1 = static_cast<uint32_t>(static_cast<uint64_t>(u + 1) * np / units);
-      if (path == 2)
-        d.hbm_units[d.hbm_unit_cap - 1 - (base_hp + u)] = make_uint4(big_idx, r0, r1, 0u);
-      else
-        d.units[path == 0 ? base_b + u : d.unit_cap - 1 - (base_w + u)] = make_uint4(t * 64 + lane, r0, r1, path);
-    }
-    for (uint32_t u = 0; u < bunits; ++u) {
-      const uint32_t r0 = static_cast<uint32_t>(static_cast<uint64_t>(u) * nb / bunits);
-      const uint32_t r1 = static_cast<uint32_t>(static_cast<uint64_t>(u + 1) * nb / bunits);
-      d.hbm_units[base_hb + u] = make_uint4(big_idx, r0, r1, 0u);
+    struct ItemUnits {
+      uint32_t units, np, path, base, big_idx, bunits, nb, base_hb;
+    };
+    const ItemUnits mine{units, np, path, path == 0 ? base_b : path == 1 ? base_w : base_hp, big_idx, bunits, nb, base_hb};
+    // units first, first + step, ... of item t * 64 + l
+    auto write = [&](const ItemUnits& x, uint32_t l, uint32_t first, uint32_t step) {
+      for (uint32_t u = first; u < x.units; u += step) {
+        const uint32_t r0 = static_cast<uint32_t>(static_cast<uint64_t>(u) * x.np / x.units);
+        const uint32_t r1 = static_cast<uint32_t>(static_cast<uint64_t>(u + 1) * x.np / x.units);
+        if (x.path == 2)
+          d.hbm_units[d.hbm_unit_cap - 1 - (x.base + u)] = make_uint4(x.big_idx, r0, r1, 0u);
+        else
+          d.units[x.path == 0 ? x.base + u : d.unit_cap - 1 - (x.base + u)] = make_uint4(t * 64 + l, r0, r1, x.path);
+      }
+      for (uint32_t u = first; u < x.bunits; u += step) {
+        const uint32_t r0 = static_cast<uint32_t>(static_cast<uint64_t>(u) * x.nb / x.bunits);
+        const uint32_t r1 = static_cast<uint32_t>(static_cast<uint64_t>(u + 1) * x.nb / x.bunits);
+        d.hbm_units[x.base_hb + u] = make_uint4(x.big_idx, r0, r1, 0u);
+      }
+    };
+    const bool many = units > 4 || bunits > 4;
+    if (!many) write(mine, lane, 0, 1);
+    for (uint64_t m = __builtin_amdgcn_ballot_w64(many); m; m &= m - 1) {
+      const uint32_t l = static_cast<uint32_t>(__builtin_ctzll(m));
+      auto of = [&](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(v, l)); };
+      write(ItemUnits{of(mine.units), of(mine.np), of(mine.path), of(mine.base), of(mine.big_idx), of(mine.bunits),
+                      of(mine.nb), of(mine.base_hb)},
+            l, lane, 64);
     }
   }
 }
@@ -1481,12 +1509,22 @@ hipError_t launch_register_join_sized(const PipelineDevice& d, uint32_t grid, hi
   return launch_register_join<K, CAP / 2, WAVES, 4, 4>(d, grid, stream);
 }
 
+// Whether the register join would only put off nearly every item of a join: one
+// of its sides exceeds the registers (640 tuples) four times on average.  It is
+// not launched then (it took 97 us to look at 65,536 items of 2,048 + 16,384
+// int32 tuples).
+static bool all_deferred(const PipelineDevice& d) {
+  const uint64_t items = static_cast<uint64_t>(d.F1) * d.F2;
+  return !d.job_results && std::max(d.build.n, d.probe.n) / items >= 4 * 640;
+}
+
 // The deferred items' joins with block-shared tables of BCAP slots (64 KiB:
 // two blocks of 512 threads per CU).
 template <typename K, uint32_t BCAP, uint32_t GCAP, uint32_t GWAVES>
 hipError_t launch_deferred_t(const PipelineDevice& d, uint32_t grid, hipStream_t stream) {
   constexpr uint32_t BBLOCK = 512;
-  hipLaunchKernelGGL(join_units_kernel, dim3(grid), dim3(kUnitsWaves * 64), 0, stream, d, BCAP * 3 / 4);
+  hipLaunchKernelGGL(join_units_kernel, dim3(grid), dim3(kUnitsWaves * 64), 0, stream, d, BCAP * 3 / 4,
+                     all_deferred(d) ? 1u : 0u);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   {
@@ -1517,7 +1555,7 @@ hipError_t launch_deferred_t(const PipelineDevice& d, uint32_t grid, hipStream_t
 
 template <typename K, uint32_t GCAP>
 hipError_t launch_join_t(const PipelineDevice& d, bool deferred, uint32_t grid, hipStream_t stream) {
-  if (!deferred) return launch_register_join_sized<K, 1024, 4>(d, grid, stream);
+  if (!deferred) return all_deferred(d) ? hipSuccess : launch_register_join_sized<K, 1024, 4>(d, grid, stream);
   return launch_deferred_t<K, kBlockTableSlots<K>, GCAP, 4>(d, grid, stream);
 }
 
