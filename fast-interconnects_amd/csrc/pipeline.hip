@@ -781,9 +781,9 @@ __device__ __forceinline__ void lane_item_side(const PipelineDevice& d, const Pi
 }
 
 __global__ __launch_bounds__(kUnitsWaves * 64) void join_units_kernel(PipelineDevice d, uint32_t block_rcap, uint32_t all) {
+  if (all) stamp_phase(d.stamps, 3);
   stamp_phase(d.stamps, 4);
   if (all) {
-    stamp_phase(d.stamps, 3);
     if (blockIdx.x == 0 && threadIdx.x == 0) d.work_counter[kOverflowAny] = 1;
   } else if (uniform_load(d.work_counter + kOverflowAny) == 0) {
     return;

@@ -28,4 +28,6 @@ def test_deferred_units(dtype, n_r, bits, spread):
     plan = fij.JoinPlan(dtype, n_r, n_s, *bits)
     dev = [to_dev(c) for c in (rk, rp, sk, sp)]
     for _ in range(2):
-        assert plan.execute(*dev)[0] == want
+        got, times = plan.execute(*dev)
+        assert got == want
+        assert all(0 <= t <= times["total_ms"] for t in times.values()), times
