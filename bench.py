@@ -295,7 +295,8 @@ def batched_main(a):
     # each tuple's key and payload once (t); a partitioned join with P passes
     # moves k + (2P + 1) t per tuple (key histogram, P scatters, join read)
     classes = [fij.autotune(np.int32, int(r), int(s_)) for r, s_ in zip(n_r, n_s)]
-    b_alg = sum((int(r) + int(s_)) * (8 if small else 4 + (2 * (2 if b2 else 1) + 1) * 8)
+    # (batches take one pass up to 4,571,136 int32 build tuples)
+    b_alg = sum((int(r) + int(s_)) * (8 if small else 4 + (2 * (2 if b2 and r > 4_571_136 else 1) + 1) * 8)
                 for (small, _, b2), r, s_ in zip(classes, n_r, n_s))
     # the plain per-join launch: each join through a plan of the bits a
     # join run alone takes (fij_join_plan_bits: one pass where the build
@@ -887,9 +888,9 @@ def main():
     t_bytes = 16
     b_alg = 2 * n * (8 + (2 * 2 + 1) * t_bytes)  # (|R|+|S|) * (k + (2P+1) t), P = 2
     med = {k: float(np.median(v)) for k, v in phases.items()}
-    # Per-kernel launch times from the HIP events around each phase, and the
-    # algorithmic HBM bytes of one launch (each tuple's bytes read and written
-    # once; relation-sized kernels run once per relation).
+    # Per-kernel times from the stamps around each phase, and the algorithmic
+    # HBM bytes (each tuple's bytes read and written once); the histogram and
+    # the scatter of both relations are one launch, given here per relation.
     # (hist includes the small offsets scan; sort2 the small plan kernel; the
     # deferred-item join moves no bytes of its own at this shape)
     kernels = {

@@ -431,11 +431,7 @@ fij_join_tuning tuned_class(KeyType kt, uint64_t build_len, uint64_t probe_len, 
   // Build sides of 2^18 tuples up to what 64 KiB block tables hold after one
   // pass of 9 bits: a single-pass plan, measured faster than the two-pass
   // classes there (1.2-1.45x for single int32 joins at 2^19-2^21, up to 2.9x
-  // for long probe sides at int64; batched int32 joins of log-uniform sizes
-  // 6 % faster); below 2^18 the two are level.  Going on to the 128 KiB
-  // tables that single joins take up to twice that size (fij_join_plan_bits)
-  // left the batched mix as fast (0.238 s either way on one box), so batched
-  // classes stop here.
+  // for long probe sides at int64).  Batches go further (batch_class).
   if (!(entry && g_tuning_user[ti]) && !rule.small && build_len >= (1u << 18) &&
       block_tables_hold(kt, build_len, 1ull << kOnePassBits, false)) {
     fij_join_tuning t = rule;

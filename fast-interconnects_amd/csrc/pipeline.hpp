@@ -124,8 +124,7 @@ struct PipelineDevice {
   uint4* hbm_units;           // [hbm_unit_cap] {big index, first run, end run, 0}: build units from the front,
                               // probe units from the back
   uint32_t hbm_unit_cap;
-  // single-pass plans: deferred items joined from 128 KiB block tables (one
-  // block per CU) instead of 64 KiB ones (build partitions beyond the latter)
+  // single pass: 128 KiB block tables (one block per CU) instead of 64 KiB ones
   uint32_t big_block_tables;
 };
 

@@ -328,10 +328,15 @@ fij_status fij_np_probe_sum(fij_type type, fij_hashing_scheme scheme, const void
  * (radix-join/src/execution_methods/gpu_radix_join.rs:90-565), which the
  * reference builds from the operators above with a host loop of six launches
  * per pass-1 partition.  A plan allocates every intermediate buffer of one
- * join shape once; executing it runs pass 1 (chunked histogram + buffered
- * scatter), pass 2 (per-partition LDS counting sort of tiles) and the LDS
- * hash join for all partitions with a fixed, small number of launches, and
- * returns {count, SUM(build.value), SUM(probe.value)}. */
+ * join shape once; executing it runs pass 1 (histogram + buffered scatter of
+ * both relations), pass 2 (per-partition LDS counting sort of tiles) and the
+ * LDS hash join for all partitions with a fixed, small number of launches, and
+ * returns {count, SUM(build.value), SUM(probe.value)}.  radix_bits are what a
+ * plan has buffers for; a join whose build side is small for them takes fewer
+ * passes: none where one block's LDS table holds it (12,288 int32 or 6,144
+ * int64 tuples), one of 9 bits instead of two where its partitions then make at
+ * most two table fills (up to 4.57 M tuples; 7.08 M int32 or 5.08 M int64 for
+ * probe sides of at most 32 or 16 times the build side). */
 
 typedef struct fij_join_plan fij_join_plan;
 
@@ -401,10 +406,11 @@ fij_status fij_join_plan_execute(fij_join_plan *plan, const void *build_keys, co
 /* Many independent joins with one submission (no counterpart in the
  * reference, which joins one pair per run of the radix-join binary).  Joins
  * whose build side fits one block's LDS table are joined together by one
- * persistent launch without partitioning; every other join is partitioned
- * in one or two passes with the radix bits of its size class
- * (fij_join_autotune: one pass of 9 bits for build sides from 2^18 tuples up
- * to what 64 KiB block tables hold after it: 2^20 int64, 2^21 int32),
+ * persistent launch without partitioning.  Every other join is partitioned, in
+ * one pass of 5, 7 or 9 bits by its build side up to two table fills per
+ * partition (as a plan's join), else in two passes with the radix bits of its
+ * size class (fij_join_autotune; also where fij_join_tuning_set has given the
+ * class an entry),
  * all joins of a class together: one launch per pass (histograms, offsets,
  * scatter, pass 2, join) covers every join of the class.  The submission is
  * recorded into one HIP graph when use_graph is set.  The size classes are
@@ -469,7 +475,8 @@ typedef struct fij_join_tuning {
   uint32_t from_table;   /* lookup output: 1 = a table entry, 0 = the closed-form rule */
 } fij_join_tuning;
 
-/* The configuration batched joins of these lengths run with. */
+/* The configuration of these lengths' class, from the table or the rule:
+ * batched joins that run in two passes take its bits, ring and block. */
 fij_status fij_join_tuning_lookup(fij_type type, uint64_t build_len, uint64_t probe_len, fij_join_tuning *out);
 /* Replaces the active table of `type` with entries[0..n) (n = 0: the rule
  * only); a later call with use_builtin = 1 restores the built-in table.
