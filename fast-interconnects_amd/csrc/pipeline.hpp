@@ -177,7 +177,9 @@ hipError_t alloc_pipeline_side(PipelineSide& s, KeyType t, uint64_t n, uint32_t 
                                bool two_pass, uint32_t tiles, std::vector<void*>& allocs);
 // Pass 1 of the sides in d.sides (each in its g1 chunks): contiguous
 // histograms + offsets scans, then the scatters, one launch each.
-hipError_t enqueue_pass1_prefix_sum(const PipelineDevice& d, KeyType t, uint32_t block, hipStream_t stream);
+// The histograms copy the keys to key_copies[side] (device columns) if given.
+hipError_t enqueue_pass1_prefix_sum(const PipelineDevice& d, KeyType t, uint32_t block, hipStream_t stream,
+                                    void* const* key_copies = nullptr);
 hipError_t enqueue_pass1_scatter(const PipelineDevice& d, KeyType t, uint32_t block, uint32_t lds_total,
                                  hipStream_t stream);
 // Chunks of n tuples: at most `most`, none shorter than a step of the

@@ -93,12 +93,17 @@ PartitionLaunch scatter_of(const PipelineDevice& d, const PipelineSide& s, KeyTy
 
 }  // namespace
 
-hipError_t enqueue_pass1_prefix_sum(const PipelineDevice& d, KeyType t, uint32_t block, hipStream_t stream) {
+hipError_t enqueue_pass1_prefix_sum(const PipelineDevice& d, KeyType t, uint32_t block, hipStream_t stream,
+                                    void* const* key_copies) {
   const PipelineSide* a = side_of(d, 0) ? side_of(d, 0) : side_of(d, 1);
   const PipelineSide* b = d.sides == 3 ? &d.probe : nullptr;
   HistParams ha = hist_params(t, a->keys, a->n, a->g1, d.bits1, block, a->counts1, a->scan1);
   ha.stamp = d.stamps;
-  const HistParams hb = b ? hist_params(t, b->keys, b->n, b->g1, d.bits1, block, b->counts1, b->scan1) : ha;
+  HistParams hb = b ? hist_params(t, b->keys, b->n, b->g1, d.bits1, block, b->counts1, b->scan1) : ha;
+  if (key_copies) {
+    ha.dst_keys = key_copies[a == &d.build ? 0 : 1];
+    hb.dst_keys = key_copies[1];
+  }
   const hipError_t e = launch_hist_pair(t, ha, hb, a->g1, b ? b->g1 : 0, block, stream);
   if (e != hipSuccess) return e;
   const OffsetsScan sa = scan_of(d, *a), sb = b ? scan_of(d, *b) : sa;
