@@ -143,10 +143,21 @@ hipError_t arena_alloc(ClassArena& a, T** out, uint64_t count) {
   return hipSuccess;
 }
 
-// Chunks of a batched join side: about 32768 tuples each, at most one per
-// compute unit.
-uint32_t side_chunks(KeyType kt, uint64_t n, uint32_t cus) {
-  return pass1_chunks(kt, n, static_cast<uint32_t>(std::min<uint64_t>(cus, std::max<uint64_t>(1, (n + 32767) / 32768))));
+// Tuples of a chunk in pass 1 of b1 bits of a class of `total` tuples: every
+// chunk ends within a line in each partition and adds a row to the offsets scan,
+// so single-pass classes that leave four chunks per CU take longer ones, up to
+// 512 tuples per partition (GPU time of 54 joins of 2^14 to 2^20 int32 build
+// tuples 1.01 ms with 32,768 tuples per chunk, 0.92 ms).
+uint64_t class_chunk_len(uint64_t total, uint32_t b1, uint32_t b2, uint32_t cus) {
+  constexpr uint64_t kLeast = 32768;
+  if (b2) return kLeast;
+  return std::max(kLeast, std::min<uint64_t>(512ull << b1, total / (4ull * cus)));
+}
+
+// Chunks of a batched join side: at most one per compute unit.
+uint32_t side_chunks(KeyType kt, uint64_t n, uint64_t chunk_len, uint32_t cus) {
+  return pass1_chunks(
+      kt, n, static_cast<uint32_t>(std::min<uint64_t>(cus, std::max<uint64_t>(1, (n + chunk_len - 1) / chunk_len))));
 }
 
 // Grows the class arena to hold `joins` joins with these totals; every
@@ -234,12 +245,15 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
   std::vector<SideLayout> lay(2 * J);
   uint64_t rel1[2] = {0, 0}, rel2[2] = {0, 0}, tiles[2] = {0, 0}, words = 0, probe_total = 0;
   uint32_t blocks = 0;
+  uint64_t total = 0;
+  for (uint32_t id : ids) total += joins[id].build_len + joins[id].probe_len;
+  const uint64_t chunk_len = class_chunk_len(total, b1, b2, b->cus);
   for (uint32_t j = 0; j < J; ++j) {
     const fij_join_desc& jd = joins[ids[j]];
     for (int s = 0; s < 2; ++s) {
       SideLayout& l = lay[2 * j + s];
       l.n = s ? jd.probe_len : jd.build_len;
-      l.chunks = side_chunks(kt, l.n, b->cus);
+      l.chunks = side_chunks(kt, l.n, chunk_len, b->cus);
       l.counts_at = words;
       l.local_at = words;
       words += static_cast<uint64_t>(F1) * l.chunks;

@@ -32,3 +32,15 @@ def test_class_edges(dtype, lanes, graph):
     want = [orc.sort_merge_join(*[c[h[k] != -1] for k, c in ((0, h[0]), (0, h[1]), (2, h[2]), (2, h[3]))]) for h in host]
     for _ in range(2):
         assert batch.execute(dev)[0] == want
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_long_chunks(dtype):
+    """A class of more tuples than four chunks of 32,768 per compute unit: longer
+    chunks, of which a short probe side beside the long ones is less than one."""
+    sizes = [(600_011, 12_000_007), (530_000, 12_000_001), (524_289, 12_500_000), (700_001, 50_021), (640_000, 7)]
+    host = [relations(dtype, r, s, 60 + i) for i, (r, s) in enumerate(sizes)]
+    batch = fij.JoinBatch(dtype, len(sizes))
+    dev = [tuple(to_dev(c) for c in h) for h in host]
+    want = [orc.sort_merge_join(*[c[h[k] != -1] for k, c in ((0, h[0]), (0, h[1]), (2, h[2]), (2, h[3]))]) for h in host]
+    assert batch.execute(dev)[0] == want
