@@ -18,6 +18,7 @@
 #include "hbm_table.hpp"
 #include "internal.hpp"
 #include "join_result.hpp"
+#include "one_pass_rules.hpp"
 #include "pipeline.hpp"
 
 #include <algorithm>
@@ -42,13 +43,6 @@ constexpr uint32_t kTableUnitTuples = 65536;  // tuples of an HBM-table work uni
 // every fill streams the probe tuples again (about 3 TB/s), an HBM table costs
 // a random access per probe tuple (about 45 G/s).
 constexpr uint32_t kMaxFills = 4;
-
-// Probe tuples of a unit, about: 16 times its build tuples (a unit's build work
-// is paid once per unit: 20 batched joins of 2^18..2^20 int32 build tuples took
-// 349 us with 8 times, 283 us with 16), between kPartUnitMin and 65,536.
-__device__ __forceinline__ uint32_t unit_tuples(uint32_t build_n) {
-  return min(65536u, max(kPartUnitMin, 16 * min(build_n, 4096u)));
-}
 
 // One block per join.  `sides` == nullptr: one join, whose sides end at their
 // padded_len1; that block sets the counters.  In batches (which have no HBM
@@ -76,11 +70,8 @@ __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, c
   for (uint32_t p = tid; p < F1j; p += blockDim.x) {
     uint64_t at;
     const uint32_t nb = range(d.build, end_b, p, at), np = range(d.probe, end_p, p, at);
-    uint32_t units = 0;
-    uint32_t ut = unit_tuples(nb);
-    if (nb && np) {
-      units = (np + ut - 1) / ut;
-      ut = (np + units - 1) / units;  // even units
+    PartUnits cut = part_units_of(nb, np);
+    if (cut.units) {
       if (nb > kMaxFills * rcap && d.hbm_cap && nb <= (d.hbm_cap >> 1)) {
         // an HBM table of at least twice the build tuples, if the arena (at
         // most 2^26 slots) has room.  A partition that finds none takes no
@@ -94,22 +85,21 @@ __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, c
         }
         const uint32_t big = slot + (1u << lg) <= d.hbm_cap ? atomicAdd(&s_big, 1u) : d.big_cap;
         if (big < d.big_cap) {
-          units = 0;
+          cut.units = 0;
           d.big[big] = make_uint4(j * F1j + p, slot, lg, 0u);
-          const uint32_t bu = (nb + kTableUnitTuples - 1) / kTableUnitTuples;
-          const uint32_t pu = (np + kTableUnitTuples - 1) / kTableUnitTuples;
+          const uint32_t bu = range_count(nb, kTableUnitTuples), pu = range_count(np, kTableUnitTuples);
           const uint32_t b0 = atomicAdd(&s_build_units, bu), p0 = atomicAdd(&s_probe_units, pu);
           for (uint32_t u = 0; u < bu; ++u)
-            d.hbm_units[b0 + u] = make_uint4(big, u * kTableUnitTuples, min(nb, (u + 1) * kTableUnitTuples), 0u);
+            d.hbm_units[b0 + u] = make_uint4(big, u * kTableUnitTuples, range_end(nb, kTableUnitTuples, u), 0u);
           for (uint32_t u = 0; u < pu; ++u)
             d.hbm_units[d.hbm_unit_cap - 1 - (p0 + u)] =
-                make_uint4(big, u * kTableUnitTuples, min(np, (u + 1) * kTableUnitTuples), 0u);
+                make_uint4(big, u * kTableUnitTuples, range_end(np, kTableUnitTuples, u), 0u);
         }
       }
     }
-    first[p] = units;
+    first[p] = cut.units;
     probe_n[p] = np;
-    per[p] = ut;
+    per[p] = cut.per;
     if (d.sides & 1) d.build.plen[j * F1j + p] = nb;
     if (d.sides & 2) d.probe.plen[j * F1j + p] = np;
   }
@@ -298,9 +288,9 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
     VT xa[NV], xb[NV];
     load(xa, 0);  // in flight while the table is built
     // equal fills
-    const uint32_t fills = (nb + FILL - 1) / FILL, fill = (nb + fills - 1) / fills;
-    for (uint32_t f0 = 0; f0 < nb; f0 += fill) {
-      const uint32_t nf = min(fill, nb - f0);
+    const uint32_t fills = range_count(nb, FILL), fill = range_count(nb, fills);
+    for (uint32_t f = 0; f < fills; ++f) {
+      const uint32_t f0 = f * fill, nf = range_end(nb, fill, f) - f0;
       // at most 1/4 full where the table allows it
       const uint32_t lg = min(LG_CAP, max(6u, 32u - static_cast<uint32_t>(__builtin_clz(nf))));
       using Quad = typename BucketTable<K>::Quad;
@@ -369,7 +359,7 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
         probe(xb, v0 + STEP);
         if (v0 + 2 * STEP >= nvp) break;
       }
-      if (f0 + fill < nb) __syncthreads();  // probes done before the table is cleared
+      if (f + 1 < fills) __syncthreads();  // probes done before the table is cleared
     }
     if (lane_id() == 0) cnt += wave_cnt;
     if (tid == 0) s_next = gridDim.x + ticket;

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "internal.hpp"
+#include "one_pass_rules.hpp"
 
 namespace fij {
 
@@ -83,13 +84,6 @@ struct PartUnit {
   uint32_t build_n, probe_n;
   uint32_t part, reserved;
 };
-// Probe tuples of a unit: at least kPartUnitMin (or the whole partition), so
-// that at most one unit per partition and one per kPartUnitMin tuples exist.
-constexpr uint32_t kPartUnitMin = 8192;
-inline uint64_t part_unit_cap(uint64_t partitions, uint64_t probe_len) {
-  return partitions + probe_len / kPartUnitMin + 1;
-}
-
 struct PipelineDevice {
   PipelineSide build;
   PipelineSide probe;

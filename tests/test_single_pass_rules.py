@@ -1,0 +1,51 @@
+"""The rules that cut single-pass joins into work units, compiled for the host:
+up to the longest partitions that a plan accepts (nearly 2^32 tuples)."""
+import os
+import subprocess
+
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = """
+#include <cstdio>
+#include <cstdlib>
+#include "one_pass_rules.hpp"
+using namespace fij;
+int main(int argc, char** argv) {
+  for (int i = 1; i + 1 < argc; i += 2) {
+    const uint32_t nb = strtoul(argv[i], nullptr, 10), np = strtoul(argv[i + 1], nullptr, 10);
+    const PartUnits u = part_units_of(nb, np);
+    const uint32_t r = range_count(np, 65536);
+    printf("%u %u %u %u\\n", u.units, u.per, r, r ? range_end(np, 65536, r - 1) : 0u);
+  }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.cpp").write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I", os.path.join(REPO, "include"),
+                    "-I", os.path.join(REPO, "fast-interconnects_amd", "csrc"), "rules.cpp", "-o", "rules"], cwd=d, check=True)
+
+    def ask(pairs):
+        out = subprocess.run([str(d / "rules")] + [str(x) for p in pairs for x in p], check=True, capture_output=True, text=True)
+        return [tuple(int(x) for x in line.split()) for line in out.stdout.splitlines()]
+    return ask
+
+
+def test_units_cover_partitions_of_every_length(rules):
+    builds = [0, 1, 511, 512, 513, 2048, 4095, 4096, 5000, (1 << 32) - 20_000]
+    probes = [0, 1, 8191, 8192, 8193, 65_536, 65_537, 1 << 24, (1 << 32) - 65_536, (1 << 32) - 65_535, (1 << 32) - 20_000,
+              (1 << 32) - 514, (1 << 32) - 1]
+    pairs = [(b, p) for b in builds for p in probes]
+    for (nb, np_), (units, per, ranges, end) in zip(pairs, rules(pairs)):
+        assert ranges == -(-np_ // 65_536) and end == np_
+        if nb == 0 or np_ == 0:
+            assert units == 0
+            continue
+        assert 1 <= per <= max(8192, min(16 * nb, 65_536))
+        assert (units - 1) * per < np_ <= units * per  # no tuple left out, no empty unit
+        assert units <= np_ // 8192 + 1
