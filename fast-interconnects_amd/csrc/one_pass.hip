@@ -407,10 +407,6 @@ hipError_t launch_one_pass_join_t(const PipelineDevice& d, uint32_t grid, hipStr
 
 }  // namespace
 
-uint32_t pipeline_block_table_tuples(KeyType t, bool big) {
-  return (t == KeyType::I32 ? kSlots<int32_t> : kSlots<int64_t>) * (big ? 2 : 1) * 3 / 4;
-}
-
 hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchSide* sides, uint32_t joins,
                                 hipStream_t stream) {
   if (joins == 0) return hipSuccess;

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "internal.hpp"
+
 namespace fij {
 
 // n tuples cut into ranges of `per` tuples: how many, and where range r ends.
@@ -34,6 +36,87 @@ __host__ __device__ constexpr PartUnits part_units_of(uint32_t build_n, uint32_t
   const uint32_t want = build_n < kPartUnitMax / 16 ? 16 * build_n : kPartUnitMax;
   const uint32_t units = range_count(probe_n, want < kPartUnitMin ? kPartUnitMin : want);
   return {units, range_count(probe_n, units)};
+}
+
+// Build tuples a deferred item may have to be joined from one block-shared
+// LDS table (3/4 of its slots): the 64 KiB table, or the 128 KiB one of
+// single-pass plans with big_block_tables.
+constexpr uint32_t pipeline_block_table_tuples(KeyType t, bool big = false) {
+  return (big ? 131072u : 65536u) / (t == KeyType::I32 ? 8u : 16u) * 3 / 4;
+}
+
+
+// Single-pass plans (fij_join_plan_bits, single-pass batched classes): 9
+// bits, the widest pass-1 fanout whose line rings fit LDS.
+constexpr uint32_t kOnePassBits = 9;
+// Whether a build side's single-pass partitions hold on average at most 2/3
+// of a (big) block table (half again of headroom for uneven ones).
+inline bool block_tables_hold(KeyType t, uint64_t build_len, uint64_t partitions, bool big) {
+  return build_len * 3 <= static_cast<uint64_t>(pipeline_block_table_tuples(t, big)) * partitions * 2;
+}
+// Single pass of kOnePassBits: with 128 KiB tables where 64 KiB ones do not
+// hold the partitions (the big ones run one block per CU and are slower for
+// build sides the small ones hold).
+inline bool one_pass_fits(KeyType t, uint64_t build_len) {
+  return block_tables_hold(t, build_len, 1ull << kOnePassBits, true);
+}
+// Build tuples of one fill of a 128 KiB table in each of 2^kOnePassBits
+// partitions.  A fill takes 5/8 of the slots at int64, 9/16 at int32: fuller
+// buckets overflow, and probes that leave theirs (in a table with duplicate
+// keys every one whose bucket is full) made fills of 70 % 0.7 to 0.9 times as
+// fast as two passes, at int32 fills of 60 % 0.94 to 1.5 times.
+inline uint64_t one_pass_fill(KeyType t) {
+  return static_cast<uint64_t>(pipeline_block_table_tuples(t, true)) * (t == KeyType::I32 ? 9 : 10) / 12;
+}
+// Whether the scatter's 32-bit offsets reach the end of a relation of `len`
+// tuples in this many partitions, each behind its padding.
+inline bool pass1_offsets_fit(KeyType t, uint64_t len, uint64_t partitions) {
+  return len + partitions * pad_tuples(t) * 2 < 0xFFFFFFFFull;
+}
+// Build tuples up to which a two-pass plan runs in a single pass of
+// kOnePassBits instead, whatever the probe side: two fills of 9/16 of the slots
+// on average at int64, one at int32 (1/32 of headroom for uneven partitions).
+// Per probe tuple of t bytes a second fill reads t again, a second pass reads
+// and writes t and gathers short runs: 3 M x 2^28 int64 tuples take 3.4 ms in a
+// single pass and 4.5 ms in two, 4.56 M x 2^29 int32 tuples 3.0 and 5.0 ms
+// (with three copies of every build key 6.0 and 6.5 ms).
+inline uint64_t one_pass_limit(KeyType t) {
+  return (static_cast<uint64_t>(pipeline_block_table_tuples(t, true)) * (t == KeyType::I32 ? 3 : 6) / 4 << kOnePassBits) *
+         31 / 32;
+}
+// Whether it does for these lengths: beyond, two fills pay for probe sides that
+// are not too long: int32 tuples are moved in half the time and probed in the
+// same (7,300,000 x 10 M tuples: 167 against 323 us; 7 M x 220 M 1.7 to 2.8
+// against 2.1 to 2.8 ms, by keys; x 2^29 4.0 to 6.9 against 4.7 to 6.4 ms); at
+// int64 the tables fill up (5,000,011 x 20,000,003 tuples: 390 against 590 us,
+// with copies 560 against 660; 5,070,000 x 150 M 2.2 to 3.6 against 2.6 to 3.3
+// ms).
+inline bool one_pass_join(KeyType t, uint64_t build_len, uint64_t probe_len) {
+  if (!pass1_offsets_fit(t, probe_len, 1u << kOnePassBits)) return false;
+  if (build_len <= one_pass_limit(t)) return true;
+  const uint64_t fill = one_pass_fill(t) << kOnePassBits;
+  return t == KeyType::I32 ? build_len <= fill * 3 / 2 && probe_len / 32 <= build_len
+                           : build_len <= 2 * fill * 31 / 32 && probe_len / 16 <= build_len;
+}
+// Whether every join of at most these lengths runs in a single pass: a plan for
+// them needs no pass-2 buffers.
+inline bool one_pass_always(KeyType t, uint64_t build_len, uint64_t probe_len) {
+  return build_len <= one_pass_limit(t) && pass1_offsets_fit(t, probe_len, 1u << kOnePassBits);
+}
+// Pass-2 bits of a two-pass plan of 9 + b2 bits whose items hold about a
+// third of a 64 KiB block table's build tuples (1,024 int64, 2,048 int32):
+// for probe sides far longer than the build side, whose items go to the
+// block join anyway, fewer pass-2 digits give longer runs.
+inline uint32_t probe_heavy_bits2(KeyType t, uint64_t build_len) {
+  const uint64_t per_item = pipeline_block_table_tuples(t, false) / 3;
+  const uint64_t items = (build_len >> kOnePassBits) / per_item;
+  uint32_t b2 = 1;
+  while (b2 < 12 && (1ull << b2) < items) ++b2;
+  return b2;
+}
+// big_block_tables of a single-pass plan of `partitions` partitions.
+inline uint32_t big_block_tables_for(KeyType t, uint64_t build_len, uint64_t partitions) {
+  return block_tables_hold(t, build_len, partitions, false) ? 0u : 1u;
 }
 
 }  // namespace fij

@@ -166,7 +166,7 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
   p->join_grid = cfg->join_blocks ? cfg->join_blocks : cus * 2;
   // aggregates: the joins with small tables keep more than two blocks per CU
   p->d.agg_len = cfg->join_blocks ? cfg->join_blocks : cus * 4;
-  p->two_pass = p->d.bits2 && cfg->build_len > one_pass_limit(kt);
+  p->two_pass = p->d.bits2 && !one_pass_always(kt, cfg->build_len, cfg->probe_len);
   fij_status st = FIJ_OK;
   const uint64_t lens[2] = {cfg->build_len, cfg->probe_len};
   for (int rel = 0; rel < 2 && st == FIJ_OK; ++rel) {
@@ -177,7 +177,7 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
                      static_cast<unsigned long long>(lens[rel]), p->d.G1);
     // the scatter addresses a chunk's writes relative to its first partition
     // with 32-bit offsets; in the contiguous layout they span the relation
-    if (st == FIJ_OK && lens[rel] + static_cast<uint64_t>(p->d.F1) * p->d.pad * 2 >= 0xFFFFFFFFull)
+    if (st == FIJ_OK && !pass1_offsets_fit(kt, lens[rel], p->d.F1))
       st = plan_fail(FIJ_INTEGER_OVERFLOW, "relation of %llu tuples exceeds the 32-bit pass-1 offsets",
                      static_cast<unsigned long long>(lens[rel]));
     p->max_tiles[rel] = p->d.bits2 ? static_cast<uint32_t>((lens[rel] + p->d.tile2 - 1) / p->d.tile2 + p->d.F1) : 0;

@@ -457,7 +457,7 @@ fij_status fij_join_server_add_build(fij_join_server* s, const void* keys, const
   const size_t kb = key_bytes(s->kt);
   if (reinterpret_cast<uintptr_t>(keys) % kb || reinterpret_cast<uintptr_t>(payloads) % kb)
     return server_fail(FIJ_INVALID_ARGUMENT, "columns must be aligned to their element size");
-  if (len + static_cast<uint64_t>(kMaxF1) * pad_tuples(s->kt) * 2 >= 0xFFFFFFFFull)
+  if (!pass1_offsets_fit(s->kt, len, kMaxF1))
     return server_fail(FIJ_INTEGER_OVERFLOW, "build side exceeds the 32-bit pass-1 offsets");
   auto b = std::make_unique<ResidentBuild>();
   if (len == 0) {  // joins nothing: requests against it complete at submission

@@ -13,6 +13,12 @@ PROGRAM = """
 #include "one_pass_rules.hpp"
 using namespace fij;
 int main(int argc, char** argv) {
+  if (argc == 4) {  // type, build and probe tuples: one pass, always one pass
+    const KeyType t = argv[1][0] == '0' ? KeyType::I32 : KeyType::I64;
+    const uint64_t b = strtoull(argv[2], nullptr, 10), p = strtoull(argv[3], nullptr, 10);
+    printf("%d %d\\n", one_pass_join(t, b, p), one_pass_always(t, b, p));
+    return 0;
+  }
   for (int i = 1; i + 1 < argc; i += 2) {
     const uint32_t nb = strtoul(argv[i], nullptr, 10), np = strtoul(argv[i + 1], nullptr, 10);
     const PartUnits u = part_units_of(nb, np);
@@ -31,7 +37,8 @@ def rules(tmp_path_factory):
                     "-I", os.path.join(REPO, "fast-interconnects_amd", "csrc"), "rules.cpp", "-o", "rules"], cwd=d, check=True)
 
     def ask(pairs):
-        out = subprocess.run([str(d / "rules")] + [str(x) for p in pairs for x in p], check=True, capture_output=True, text=True)
+        args = [str(x) for p in pairs for x in p]
+        out = subprocess.run([str(d / "rules")] + args, check=True, capture_output=True, text=True)
         return [tuple(int(x) for x in line.split()) for line in out.stdout.splitlines()]
     return ask
 
@@ -49,3 +56,15 @@ def test_units_cover_partitions_of_every_length(rules):
         assert 1 <= per <= max(8192, min(16 * nb, 65_536))
         assert (units - 1) * per < np_ <= units * per  # no tuple left out, no empty unit
         assert units <= np_ // 8192 + 1
+
+
+@pytest.mark.parametrize("type,pad", [(0, 16), (1, 8)])
+def test_single_pass_offsets_stay_below_2_32(rules, type, pad):
+    """A plan of few pass-1 bits accepts relations that 512 padded partitions
+    would carry past 2^32: those take two passes."""
+    last = (1 << 32) - 2 - 512 * pad * 2
+    for build in (20_000, 4_571_136):
+        assert rules([(type, build, last)]) == [(1, 1)]
+        assert rules([(type, build, last + 1)]) == [(0, 0)]
+        assert rules([(type, build, (1 << 32) - 600)]) == [(0, 0)]
+    assert rules([(type, 4_571_137, 5_000_000)]) == [(1, 0)]  # by its lengths, not always
