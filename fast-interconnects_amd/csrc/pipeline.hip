@@ -61,7 +61,7 @@ __global__ __launch_bounds__(1024) void plan_kernel(PipelineDevice d) {
     const uint32_t n = static_cast<uint32_t>(e - b);
     s.plen[p] = n;
     starts[p] = n;
-    tiles[p] = (n + d.tile2 - 1) / d.tile2;
+    tiles[p] = range_count(n, d.tile2);
   }
   __syncthreads();
   const uint64_t total = block_exclusive_scan<uint64_t>(starts, F1, wave_tmp);
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(1024) void plan_batched_kernel(PipelineDevice d, co
     const uint32_t n = static_cast<uint32_t>(e - b);
     s.plen[vp] = n;
     starts[p] = n;
-    tiles[p] = (n + d.tile2 - 1) / d.tile2;
+    tiles[p] = range_count(n, d.tile2);
   }
   __syncthreads();
   block_exclusive_scan<uint64_t>(starts, F1j, wave_tmp);

@@ -32,12 +32,14 @@ def test_one_probe_partition(n_r, stride):
     assert got == (n_s, int(rp[77]) * n_s, n_s)
 
 
-def test_few_pass_1_bits():
+@pytest.mark.parametrize("keys", [20_000, 1])
+def test_few_pass_1_bits(keys):
     """16 partitions fit the 32-bit offsets of pass 1, the 512 of a single pass
-    would not."""
+    would not; with one key, one partition has nearly 2^32 tuples to cut into
+    tiles."""
     n_r, n_s = 20_000, (1 << 32) - 1000
     rk, rp = orc.gen_perm(n_r, 6, np.int32, 1), np.full(n_r, 7, np.int32)
-    sk, sp = columns(n_s, 1, n_r)  # every probe key matches
+    sk, sp = columns(n_s, 1, keys)  # every probe key matches
     plan = fij.JoinPlan(np.int32, n_r, n_s, 4, 4)
     got = plan.execute(to_dev(rk), to_dev(rp), sk, sp)[0]
     assert got == (n_s, 7 * n_s, n_s)
