@@ -306,14 +306,8 @@ __device__ __forceinline__ void bucket_join(const JoinParams& p, uint64_t* lds, 
                                             const Tuple<K>* build, uint32_t nbuild, ProbeStream<K>& stream,
                                             uint64_t& cnt, uint64_t& sb, uint64_t& sp) {
   using Table = BucketTable<K, true>;
-  using Quad = typename Table::Quad;
-  // at most 1/4 full where the table allows it, 3/4 at most
-  const uint32_t lg = min(29u - static_cast<uint32_t>(__builtin_clz(p.table_slots)),
-                          max(6u, 32u - static_cast<uint32_t>(__builtin_clz(nbuild | 1u))));
-  const Table tab{reinterpret_cast<Quad*>(lds), reinterpret_cast<Quad*>(lds) + p.table_slots / 4, 32u - lg,
-                  (1u << lg) - 1u, null_key<K>()};
-  for (uint32_t i = threadIdx.x; i < (1u << lg); i += blockDim.x)
-    tab.keys[i] = Quad{null_key<K>(), null_key<K>(), null_key<K>(), null_key<K>()};
+  const Table tab(lds, p.table_slots, Table::lg_buckets(p.table_slots, nbuild), null_key<K>());
+  tab.clear();
   if (threadIdx.x == 0) *s_dup = 0;
   __syncthreads();
   bool dup = false;
@@ -334,13 +328,7 @@ __device__ __forceinline__ void bucket_join(const JoinParams& p, uint64_t* lds, 
         key[i] = (live >> (g + i)) & 1u ? t[g + i].key : null_key<K>();
         pay[i] = t[g + i].value;
       }
-      if (unique) {
-        tab.probe_unique(key, pay, wave_cnt, cnt, sb, sp);
-      } else {
-#pragma unroll
-        for (uint32_t i = 0; i < 2; ++i)
-          if (key[i] != null_key<K>()) tab.probe_from(tab.bucket(key[i]), key[i], pay[i], cnt, sb, sp);
-      }
+      tab.probe(unique, key, pay, wave_cnt, cnt, sb, sp);
     }
   });
   if (lane_id() == 0) cnt += wave_cnt;
@@ -473,9 +461,8 @@ hipError_t launch_join_t(const JoinLaunch& a, hipStream_t stream) {
     uint32_t entries = (lds - kChainBuckets * 4) / (2 + 2 * sizeof(K));
     if (entries > kChainTail) entries = kChainTail;
     p.ht_entries = entries;
-    uint32_t slots = 4;
-    while (4 * sizeof(K) * slots <= lds) slots *= 2;  // two columns of twice as many
-    p.table_slots = slots;
+    p.table_slots = 256;
+    while (bucket_table_bytes<K>(2 * p.table_slots) <= lds) p.table_slots *= 2;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(lds));
     hipLaunchKernelGGL(kern, dim3(a.grid), dim3(a.block), lds, stream, p);

@@ -244,11 +244,10 @@ struct TupleVec {
 // two or four probes together and build tuples loaded a fill ahead all lay
 // within 3 % of each other; the smallest register need was taken.
 template <typename K, uint32_t CAP, uint32_t BLOCK>
-__global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
+__global__ __launch_bounds__(BLOCK, CAP * 2 * sizeof(K) <= 32768 ? 6 : 4) void part_join_kernel(PipelineDevice d) {
   using V = TupleVec<K>;
   using VT = typename V::type;
   constexpr uint32_t FILL = CAP / 16 * (sizeof(K) == 4 ? 9 : 10);  // build tuples per table fill (one_pass_fill)
-  constexpr uint32_t LG_CAP = 29u - __builtin_clz(CAP);  // of its buckets
   constexpr uint32_t NV = 2;                  // vectors in flight per buffer
   constexpr uint32_t NT = NV * V::N;          // their tuples
   constexpr uint32_t PROBES = 2;              // probed together
@@ -291,12 +290,8 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
     const uint32_t fills = range_count(nb, FILL), fill = range_count(nb, fills);
     for (uint32_t f = 0; f < fills; ++f) {
       const uint32_t f0 = f * fill, nf = range_end(nb, fill, f) - f0;
-      // at most 1/4 full where the table allows it
-      const uint32_t lg = min(LG_CAP, max(6u, 32u - static_cast<uint32_t>(__builtin_clz(nf))));
-      using Quad = typename BucketTable<K>::Quad;
-      const BucketTable<K> tab{reinterpret_cast<Quad*>(lds_u64), reinterpret_cast<Quad*>(lds_u64) + CAP / 4, 32u - lg,
-                               (1u << lg) - 1u, free_key};
-      for (uint32_t i = tid; i < (1u << lg); i += BLOCK) tab.keys[i] = Quad{free_key, free_key, free_key, free_key};
+      const BucketTable<K> tab(lds_u64, CAP, BucketTable<K>::lg_buckets(CAP, nf), free_key);
+      tab.clear();
       if (tid == 0) s_dup = 0;
       __syncthreads();
       {
@@ -341,12 +336,7 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
               if (at >= unit.probe_n) key[i] = no_key;
             }
           }
-          if (unique) {
-            tab.probe_unique(key, pay, wave_cnt, cnt, sb, sp);
-          } else {
-#pragma unroll
-            for (uint32_t i = 0; i < PROBES; ++i) tab.probe_from(tab.bucket(key[i]), key[i], pay[i], cnt, sb, sp);
-          }
+          tab.probe(unique, key, pay, wave_cnt, cnt, sb, sp);
         }
       };
       if (f0) load(xa, 0);
@@ -385,7 +375,7 @@ __global__ __launch_bounds__(BLOCK) void part_join_kernel(PipelineDevice d) {
 template <typename K, uint32_t CAP, uint32_t BLOCK>
 hipError_t launch_part_join(const PipelineDevice& d, uint32_t grid, hipStream_t stream) {
   auto kern = part_join_kernel<K, CAP, BLOCK>;
-  const size_t lds = CAP * 2 * sizeof(K);
+  const size_t lds = bucket_table_bytes<K>(CAP);
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                             static_cast<int>(lds));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, stream, d);

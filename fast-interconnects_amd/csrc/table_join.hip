@@ -18,23 +18,17 @@ struct ColumnVec {
   typedef K type __attribute__((ext_vector_type(16 / sizeof(K)), aligned(sizeof(K))));
 };
 
-// The build side (n tuples, at most 3/4 of CAP) into the block's table, at
-// most 1/4 full where CAP allows it.  Returns the table; `dup`: whether two
-// build keys are equal.  Begins and ends with a barrier.
+// The build side (n tuples, at most 3/4 of CAP) into the block's table.
+// Returns the table; `unique`: no build key occurs twice.  Begins and ends with a barrier.
 template <typename K, uint32_t CAP, uint32_t BLOCK>
 __device__ __forceinline__ BucketTable<K, true> build_table(uint64_t* lds, const K* keys, const K* pays, uint32_t n,
                                                             uint32_t* s_dup, bool& unique) {
   using Table = BucketTable<K, true>;
-  using Quad = typename Table::Quad;
-  constexpr uint32_t LG_CAP = 29u - __builtin_clz(CAP);  // of its buckets
-  constexpr uint32_t U = 4;                              // build tuples in flight per thread
+  constexpr uint32_t U = 4;  // build tuples in flight per thread
   const uint32_t tid = threadIdx.x;
-  const uint32_t lg = min(LG_CAP, max(6u, 32u - static_cast<uint32_t>(__builtin_clz(n | 1u))));
-  const Table tab{reinterpret_cast<Quad*>(lds), reinterpret_cast<Quad*>(lds) + CAP / 4, 32u - lg, (1u << lg) - 1u,
-                  null_key<K>()};
+  const Table tab(lds, CAP, Table::lg_buckets(CAP, n), null_key<K>());
   __syncthreads();  // the table may still be probed
-  for (uint32_t i = tid; i < (1u << lg); i += BLOCK)
-    tab.keys[i] = Quad{tab.free_key, tab.free_key, tab.free_key, tab.free_key};
+  tab.clear();
   if (tid == 0) *s_dup = 0;
   __syncthreads();
   bool dup = false;
@@ -93,13 +87,7 @@ struct ColumnStream {
       for (uint32_t g = 0; g < V; g += 2) {
         const K key[2] = {live ? k[u][g] : null_key<K>(), live ? k[u][g + 1] : null_key<K>()};
         const K pay[2] = {p[u][g], p[u][g + 1]};
-        if (unique) {
-          tab.probe_unique(key, pay, wave_cnt, cnt, sb, sp);
-        } else {
-#pragma unroll
-          for (uint32_t i = 0; i < 2; ++i)
-            if (key[i] != null_key<K>()) tab.probe_from(tab.bucket(key[i]), key[i], pay[i], cnt, sb, sp);
-        }
+        tab.probe(unique, key, pay, wave_cnt, cnt, sb, sp);
       }
     }
   }
@@ -118,7 +106,7 @@ struct ColumnStream {
     const uint64_t i = nv * V + threadIdx.x;
     if (first == 0 && i < n && keys[i] != null_key<K>()) {
       const K key = keys[i];
-      tab.probe_from(tab.bucket(key), key, pays[i], cnt, sb, sp);
+      tab.template probe_from<false>(tab.bucket(key), key, pays[i], cnt, sb, sp);
     }
   }
 };
@@ -131,7 +119,7 @@ struct ColumnStream {
 // the whole call 140 -> 19 us.  Every block pays the build, so a block gets at
 // least 4 steps of probe tuples.
 template <typename K, uint32_t CAP, uint32_t BLOCK>
-__global__ __launch_bounds__(BLOCK) void table_join_kernel(TableJoin j) {
+__global__ __launch_bounds__(BLOCK, CAP * 2 * sizeof(K) <= 32768 ? 6 : 4) void table_join_kernel(TableJoin j) {
   extern __shared__ __attribute__((aligned(16))) uint64_t lds_u64[];
   __shared__ uint32_t s_dup, s_last;
   __shared__ uint64_t red[3][BLOCK / kWave];
@@ -154,7 +142,7 @@ __global__ __launch_bounds__(BLOCK) void table_join_kernel(TableJoin j) {
 template <typename K, uint32_t CAP, uint32_t BLOCK>
 hipError_t launch_table_join_t(const TableJoin& j, uint32_t grid, hipStream_t stream) {
   auto kern = table_join_kernel<K, CAP, BLOCK>;
-  const size_t lds = static_cast<size_t>(CAP) * 2 * sizeof(K);
+  const size_t lds = bucket_table_bytes<K>(CAP);
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                             static_cast<int>(lds));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), lds, stream, j);
