@@ -133,11 +133,16 @@ struct TaskPart {
 // take the second and later partitions of the others' tasks, and a launch
 // lasts one partition instead of two: with N tasks the i-th block behind them
 // takes the i-th such partition, partition i + k + 1 of the task k with
-// ta[k] - k <= i < ta[k + 1] - (k + 1).
+// ta[k] - k <= i < ta[k + 1] - (k + 1).  Blocks with a task start on it and
+// those that no partition is left for end without a look at the others (each
+// block has a compute unit's LDS: 13.4 us for the launches of 64 partitions of
+// 1,000 + 4,000 tuples became 15 with that look).
 __device__ __forceinline__ TaskPart block_task(const JoinParams& p) {
   const uint32_t* const ta = p.task_assignments;
   const uint32_t F = 1u << p.radix_bits, b = blockIdx.x;
   if (F > gridDim.x) return {ta[b], ta[b + 1], b};
+  if (ta[b] < F) return {ta[b], ta[b] + 1, b};
+  if (ta[F - 1] < F) return {F, F, b};  // a task per partition
   __shared__ uint32_t s_tasks, s_owner;
   if (threadIdx.x == 0) s_tasks = s_owner = 0;
   __syncthreads();
@@ -145,7 +150,6 @@ __device__ __forceinline__ TaskPart block_task(const JoinParams& p) {
     if (ta[k] < F) atomicMax(&s_tasks, k + 1);
   __syncthreads();
   const uint32_t n = s_tasks, i = b - n;
-  if (b < n) return {ta[b], ta[b] + 1, b};
   if (i >= F - n) return {F, F, b};  // uniform
   for (uint32_t k = threadIdx.x; k < n; k += blockDim.x)
     if (ta[k] - k <= i && i < ta[k + 1] - (k + 1)) s_owner = k;
@@ -299,10 +303,25 @@ __global__ __launch_bounds__(1024) void join_perfect_kernel(JoinParams p) {
   if (p.aggregates) block_aggregate(p.aggregates + task.owner, cnt, sb, sp);
 }
 
-// One partition's build tuples (at most 3/4 of p.table_slots) in a bucket table
-// and its probe tuples against it.
+// Whether a bucket table answers a partition's probes faster than chains, whose
+// build costs half as much and for which copies of a key are cheaper.  64
+// partitions of n build tuples and r * n probe tuples, chains and tables, us:
+// int32, different keys: n = 1,500 r = 8 16.5 16.5, r = 32 31 28; 4,096 r = 4 21
+// 20, r = 8 31 25; 12,000 r = 4 68 67, r = 16 225 174; int64: 2,048 r = 16 27 27;
+// 4,096 r = 8 31 29, r = 16 49 41; 5,000 r = 16 65 67.  Keys of two copies: int32
+// 4,096 r = 8 35 36, 12,000 r = 16 250 308; int64 4,096 r = 16 57 69.
 template <typename K>
-__device__ __forceinline__ void bucket_join(const JoinParams& p, uint64_t* lds, uint32_t* s_dup,
+__device__ __forceinline__ bool table_pays(uint32_t slots, uint32_t nbuild, uint64_t nprobe) {
+  const bool few = sizeof(K) == 4 && nbuild <= slots / 8 * 3;  // level also where keys repeat
+  return nbuild > kChainBuckets / 2 && nbuild <= slots / 16 * (sizeof(K) == 4 ? 12 : 9) && nprobe >= 32768 &&
+         nprobe >= static_cast<uint64_t>(few ? 8 : 16) * nbuild;
+}
+
+// One partition's build tuples (at most 3/4 of p.table_slots) in a bucket table
+// and its probe tuples against it; false, with nothing joined, if keys repeat
+// and chains are better then.
+template <typename K>
+__device__ __forceinline__ bool bucket_join(const JoinParams& p, uint64_t* lds, uint32_t* s_dup,
                                             const Tuple<K>* build, uint32_t nbuild, ProbeStream<K>& stream,
                                             uint64_t& cnt, uint64_t& sb, uint64_t& sp) {
   using Table = BucketTable<K, true>;
@@ -318,6 +337,7 @@ __device__ __forceinline__ void bucket_join(const JoinParams& p, uint64_t* lds, 
   if (dup) *s_dup = 1;
   __syncthreads();
   const bool unique = __builtin_amdgcn_readfirstlane(*s_dup) == 0;
+  if (!unique && (sizeof(K) == 8 || nbuild > p.table_slots / 8 * 3)) return false;
   uint32_t wave_cnt = 0;
   stream.run([&](const Tuple<K>(&t)[ProbeStream<K>::N], uint32_t live) {
 #pragma unroll
@@ -332,16 +352,14 @@ __device__ __forceinline__ void bucket_join(const JoinParams& p, uint64_t* lds, 
     }
   });
   if (lane_id() == 0) cnt += wave_cnt;
+  return true;
 }
 
-// Small build sides go into chains (radix_join.cu:208-392's layout): as long
-// as chains are short, their three reads per entry cost less than clearing and
-// filling a table (586 build and 7,800 probe tuples per block at int64: 10.2 us,
-// 12.1 us with tables).  Beyond half an entry per bucket a bucket table answers
-// a probe with two reads, where the longest chain among a wave's lanes is four
-// and more entries deep (4,096 and 65,536 tuples at int32: 41 us, 57 us with
-// chains).  Build sides that no bucket table holds, up to ht_entries, fit
-// chains only.
+// Build partitions go into chains (radix_join.cu:208-392's layout), or, where
+// table_pays, into a bucket table.  Chains cost two reads per entry, and the
+// value of a match (reading it with each key: 85 instead of 82 us for the probes
+// of 64 partitions of 6,000 + 96,000 int64 tuples); as long as they are short,
+// that is less than clearing and filling a table.
 template <typename K>
 __global__ __launch_bounds__(1024) void join_chaining_kernel(JoinParams p) {
   extern __shared__ __attribute__((aligned(16))) uint64_t lds_u64[];
@@ -370,8 +388,8 @@ __global__ __launch_bounds__(1024) void join_chaining_kernel(JoinParams p) {
     const uint64_t nb = b1 - b0;
     if (nb > E) overflow = true;
     const uint32_t nbuild = nb > E ? E : static_cast<uint32_t>(nb);
-    if (nbuild > kChainBuckets / 2 && nbuild <= p.table_slots / 4 * 3) {
-      bucket_join<K>(p, lds_u64, &s_dup, build + b0, nbuild, stream, cnt, sb, sp);
+    if (table_pays<K>(p.table_slots, nbuild, stream.q1 - stream.q0) &&
+        bucket_join<K>(p, lds_u64, &s_dup, build + b0, nbuild, stream, cnt, sb, sp)) {
       __syncthreads();
       continue;
     }
@@ -401,13 +419,12 @@ __global__ __launch_bounds__(1024) void join_chaining_kernel(JoinParams p) {
 #pragma unroll
         for (uint32_t k = 0; k < N; ++k) any |= e[k] != kChainTail;
         if (!ballot(any)) break;
-        K key[N], val[N];
+        K key[N];
         uint32_t next[N];
 #pragma unroll
         for (uint32_t k = 0; k < N; ++k) {
           const uint32_t at = e[k] != kChainTail ? e[k] : 0u;
           key[k] = keys[at];
-          val[k] = vals[at];
           next[k] = links[at];
         }
 #pragma unroll
@@ -415,7 +432,7 @@ __global__ __launch_bounds__(1024) void join_chaining_kernel(JoinParams p) {
           if (e[k] == kChainTail) continue;
           if (key[k] == t[k].key) {
             cnt += 1;
-            sb += static_cast<uint64_t>(static_cast<int64_t>(val[k]));
+            sb += static_cast<uint64_t>(static_cast<int64_t>(vals[e[k]]));
             sp += static_cast<uint64_t>(static_cast<int64_t>(t[k].value));
           }
           e[k] = next[k];

@@ -2,12 +2,15 @@
 others, more heavy keys than a block table's side entries take, values at the
 ends of their type; in every join that builds block tables.  And what a heavy
 key may cost."""
+import time
+
 import numpy as np
 import pytest
 
 import fij
 import oracle_lib as orc
 from gpu_helpers import to_dev
+from test_gpu_join import partition_one_pass
 from test_gpu_operator_join import join_case
 
 pytestmark = pytest.mark.gpu
@@ -64,6 +67,19 @@ def test_operators(dtype, copies):
         join_case(dtype, *columns(dtype, n, 9001, copies), 0, 1, 256)
 
 
+# build partitions around the lengths that go into bucket tables (chains below,
+# beyond, and, for some, where a key repeats) against probe partitions around
+# the length from which they do
+@pytest.mark.parametrize("dtype,n", [(np.int32, n) for n in (1024, 1025, 4097, 6144, 6145, 12_288, 12_289)] +
+                         [(np.int64, n) for n in (1024, 1025, 4608, 4609)])
+@pytest.mark.parametrize("copies", [1, 3, "heavy"])
+def test_operator_tables_and_chains(dtype, n, copies):
+    few = dtype == np.int32 and n <= 6144
+    least = max(32_768, n * (8 if few else 16))
+    for n_s in (least - 1, least):
+        join_case(dtype, *columns(dtype, n, n_s, copies), 0, 1, 1024)
+
+
 @pytest.mark.parametrize("dtype", [np.int32, np.int64])
 def test_batches_and_served_joins(dtype):
     cols = [columns(dtype, 20_000 + 9000 * i, 40_001, c, 30 + i) for i, c in enumerate(COPIES[:-1])]
@@ -74,6 +90,30 @@ def test_batches_and_served_joins(dtype):
     for d, w in zip(dev, want):
         assert srv.wait(srv.submit(srv.add_build(d[0], d[1]), d[2], d[3]))[0] == w
     srv.close()
+
+
+def test_a_heavy_key_costs_an_operator_little():
+    """... where the partition goes into a bucket table."""
+    dtype, n, n_s = np.int32, 6000, 100_000
+    pays = orc.gen_iota(n, 1, dtype), orc.gen_iota(n_s, 1, dtype)
+    rk = orc.gen_perm(n, 9, np.int64, 1).astype(dtype)
+    sk = orc.gen_uniform(n_s, 9, 3, 8, n, dtype)
+    heavy = rk.copy()
+    heavy[:2000] = 7
+
+    def best(keys):
+        build, probe = (partition_one_pass(k, p, 0, fij.KeyType.I32) for k, p in ((keys, pays[0]), (sk, pays[1])))
+        tasks, agg = fij.DeviceArray.zeros(2, np.uint32), fij.aggregates_array(1)
+        join = fij.HipRadixJoin(fij.RadixPass.First, fij.RadixBits(0), fij.HashingScheme.BucketChaining, 1, 1024)
+        times = []
+        for _ in range(6):
+            fij.synchronize()
+            t = time.perf_counter()
+            join.join(build, probe, None, tasks, agg)
+            fij.synchronize()
+            times.append(time.perf_counter() - t)
+        return min(times)
+    assert best(heavy) < 4 * best(rk)
 
 
 @pytest.mark.parametrize("dtype", [np.int32, np.int64])
