@@ -73,6 +73,7 @@ struct ClassArena {
   BatchSide* sides = nullptr;      // [2 * joins]
   uint32_t* prefix = nullptr;      // [2 * joins + 1] first chunk of each join side
   uint32_t* job_slot = nullptr;    // [joins]
+  uint32_t* hashed = nullptr;      // [joins] single-pass classes: whether the join's digits are hashed
   uint32_t* side_tiles = nullptr;  // [2 * joins] plan scratch: tiles of each join side
   uint32_t* counts = nullptr;      // per-chunk histograms of every join side
   uint64_t* local = nullptr;       // per-chunk write offsets of every join side
@@ -218,6 +219,7 @@ fij_status grow_arena(ClassArena& a, KeyType kt, uint32_t b1, uint32_t b2, uint6
   if (e == hipSuccess) e = arena_alloc(n, &n.sides, 2 * n.joins);
   if (e == hipSuccess) e = arena_alloc(n, &n.prefix, 2 * n.joins + 1);
   if (e == hipSuccess) e = arena_alloc(n, &n.job_slot, n.joins);
+  if (e == hipSuccess && !b2) e = arena_alloc(n, &n.hashed, n.joins);
   if (e == hipSuccess) e = arena_alloc(n, &n.side_tiles, 2 * n.joins);
   // the deferred-item flags start at zero; every join leaves them at zero
   if (e == hipSuccess && b2) e = hipMemset(d.overflow, 0, parts * F2);
@@ -302,10 +304,12 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
       hh[js] = hist_params(kt, keys, l.n, l.chunks, b1, ck.block, a.counts + l.counts_at, state);
       hs[js] = OffsetsScan{a.counts + l.counts_at, a.local + l.local_at, ps.off1 + static_cast<uint64_t>(j) * F1,
                            state, l.rel1_at, F1, l.chunks, pad, 0};
+      if (b2 == 0) sample_build_keys(hh[js], jd.build_keys, jd.build_len, a.hashed + j);
       void* region = static_cast<uint8_t*>(ps.rel1) + l.rel1_at * tb;
       const hipError_t e = scatter_params_batched(kt, keys, pays, l.n, l.chunks, b1, a.local + l.local_at, region,
                                                   lds_total, ck.block, ck.ring, &hc[js]);
       if (e != hipSuccess) return batch_fail(FIJ_UNSUPPORTED, "size class %u+%u: pass-1 buffers do not fit LDS", b1, b2);
+      hc[js].hashed = b2 == 0 ? a.hashed + j : nullptr;
       hb[js] = BatchSide{l.rel1_at + l.n + static_cast<uint64_t>(F1) * pad, l.rel2_at, j * F1, 0};
       hp[js] = at;
       at += l.chunks;
@@ -335,6 +339,7 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
   d.job_shift = b1;
   d.build.n = rel2[0];
   d.probe.n = rel2[1];
+  d.hashed = a.hashed;
   if (b2 == 0) {  // the class's largest build side chooses the block tables
     d.build.n = static_cast<uint64_t>(J) * ck.build;
     d.big_block_tables = big_block_tables_for(kt, ck.build, F1);
@@ -353,10 +358,10 @@ hipError_t launch_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, hi
   const uint32_t b1 = ck.b1;
   const uint32_t js = 2 * a.sub_joins;
   hipError_t e;
-  if ((e = launch_hist_batched(kt, a.hist, a.prefix, js, a.sub_blocks, b1, ck.block, st)) != hipSuccess) return e;
+  if ((e = launch_hist_batched(kt, a.hist, a.prefix, js, a.sub_blocks, b1, ck.b2 == 0, ck.block, st)) != hipSuccess) return e;
   if ((e = launch_offsets_batched(a.scan, js, 1u << b1, st)) != hipSuccess) return e;
-  if ((e = launch_partition_batched(kt, a.scat, a.prefix, js, a.sub_blocks, b1, lds_total, ck.block, ck.ring, st)) !=
-      hipSuccess)
+  if ((e = launch_partition_batched(kt, a.scat, a.prefix, js, a.sub_blocks, b1, ck.b2 == 0, lds_total, ck.block, ck.ring,
+                                    st)) != hipSuccess)
     return e;
   if (ck.b2 == 0) {
     if ((e = launch_one_pass_plan(a.d, kt, a.sides, a.sub_joins, st)) != hipSuccess) return e;

@@ -38,17 +38,18 @@ constexpr uint32_t bucket_table_bytes(uint32_t slots) {
 // later of two equal keys passes the earlier one) stops at a match.
 //
 // free_key marks free slots; no build tuple may have it.  The keys of a
-// partition share their low digit, so the single-pass joins take a key of
-// another digit: a null key (-1) then needs no test of its own when it is
-// probed, and lanes past a range's end carry a second key of another digit.
+// partition share their digit, so the single-pass joins take a key of another
+// digit: a null key (-1) then needs no test of its own when it is probed, and
+// lanes past a range's end carry a second key of another digit.
 // NULLS: free_key is the null key itself, and null keys are kept from probing.
 template <typename K, bool NULLS = false>
 struct BucketTable {
   typedef K Quad __attribute__((ext_vector_type(4)));
   Quad* keys;      // [buckets]
   Quad* vals;      // [buckets]
-  uint32_t shift;  // hash bits below the bucket index
+  uint32_t shift;  // bits of the key's word below the bucket index
   uint32_t mask;   // buckets - 1
+  KeyMul mul;      // of the word (kBucketMul when NULLS)
   K free_key;
   // the side table, [buckets / 2]: sums of values (int32: at most 2^14 values of
   // 32 bits below bit 46 and their count above it), keys, counts (int64)
@@ -57,9 +58,13 @@ struct BucketTable {
   uint32_t* copy_counts;
 
   // A table of at most `slots` slots (a power of two, at least 256) in `lds`,
-  // of 2^lg buckets.
-  __device__ __forceinline__ BucketTable(uint64_t* lds, uint32_t slots, uint32_t lg, K free)
-      : keys(reinterpret_cast<Quad*>(lds)), vals(keys + slots / 4), shift(32u - lg), mask((1u << lg) - 1u), free_key(free),
+  // of 2^lg buckets; hashed: for keys that share the top `bits` bits of their
+  // word as digit (not when NULLS).
+  __device__ __forceinline__ BucketTable(uint64_t* lds, uint32_t slots, uint32_t lg, K free, bool hashed = false,
+                                         uint32_t bits = 0)
+      : keys(reinterpret_cast<Quad*>(lds)), vals(keys + slots / 4), shift(32u - lg),
+        mask((1u << lg) - 1u), mul(hashed ? KeyMul{kDigitMul.lo << bits, kDigitMul.hi << bits} : kBucketMul),
+        free_key(free),
         copy_sums(reinterpret_cast<uint64_t*>(vals + slots / 4)), copy_keys(reinterpret_cast<K*>(copy_sums + slots / 8)),
         copy_counts(reinterpret_cast<uint32_t*>(copy_keys + slots / 8)) {}
   // log2 of the buckets for n tuples: at most 1/4 full where `slots` allow it.
@@ -77,9 +82,7 @@ struct BucketTable {
     }
   }
   __device__ __forceinline__ uint32_t bucket(K key) const {
-    uint32_t h = static_cast<uint32_t>(key) * 2654435769u;
-    if constexpr (sizeof(K) == 8) h += static_cast<uint32_t>(static_cast<uint64_t>(key) >> 32) * 2246822519u;
-    return h >> shift;
+    return key_word<K>(key, NULLS ? kBucketMul : mul) >> shift;
   }
   // Puts the key into a slot if it is free; returns what the slot held.
   __device__ __forceinline__ K take(K* slot, K key) const {

@@ -45,6 +45,52 @@ __host__ __device__ inline uint64_t radix_mask(uint32_t radix_bits, uint32_t ign
   return static_cast<uint64_t>((1u << radix_bits) - 1u) << ignore_bits;
 }
 
+// 32 bits of a key by multiplication: multiples of any stride spread over the
+// top bits as evenly as consecutive keys.
+struct KeyMul {
+  uint32_t lo, hi;  // of the key's halves
+};
+template <typename K>
+__device__ __forceinline__ uint32_t key_word(K key, KeyMul m) {
+  uint32_t h = static_cast<uint32_t>(key) * m.lo;
+  if constexpr (sizeof(K) == 8) h += static_cast<uint32_t>(static_cast<uint64_t>(key) >> 32) * m.hi;
+  return h;
+}
+// Of bucket tables (the golden ratio's; the first one is mult_shift_hash's).
+constexpr KeyMul kBucketMul{2654435769u, 2246822519u};
+// Of hashed pass-1 digits (the fractional parts of the square roots of 2 and 3):
+// not the same, since keys that share the top bits of one hash would share few
+// slots of a table that takes its slots by these bits.
+constexpr KeyMul kDigitMul{0x6A09E667u, 0xBB67AE85u};
+constexpr uint32_t kDigitMulInverse = 0x0B39D557u;
+static_assert(kDigitMul.lo * kDigitMulInverse == 1u, "inverse modulo 2^32");
+
+// The pass-1 digit of a key.  ADAPTIVE: of joins in one pass that were not asked
+// for it, the radix digit or (hashed) the top bits of the key's word, as the
+// histogram decides from the build keys.  Multiples of 2^k leave all but one of
+// 2^k radix partitions empty (1,048,576 x 2^24 int32 tuples, multiples of 64:
+// 1.63 ms with radix digits, 0.40 ms in two passes of 8 bits, 0.19 ms hashed),
+// while for consecutive keys with copies the buckets of radix partitions fill
+// more evenly (2,300,003 x 2^24 int32 tuples: 188 us, 226 us hashed).  The
+// multiplication costs the histogram and the scatter nothing.
+template <typename K, bool ADAPTIVE>
+struct DigitOf {
+  uint64_t mask;
+  uint32_t shift;
+  KeyMul mul;
+  __device__ __forceinline__ DigitOf(uint32_t bits, uint32_t ignore_bits, bool hashed)
+      : mask(radix_mask(bits, ignore_bits)), shift(ignore_bits), mul{1u, 0u} {
+    if (ADAPTIVE && hashed) {
+      shift = 32u - bits;
+      mul = kDigitMul;
+    }
+  }
+  __device__ __forceinline__ uint32_t operator()(K key) const {
+    if constexpr (ADAPTIVE) return (key_word<K>(key, mul) >> shift) & static_cast<uint32_t>(mask);
+    return key_to_partition<K>(key, mask, shift);
+  }
+};
+
 // Canonical input chunk length: ceil(n / chunks) rounded down to a multiple of
 // 128 bytes of keys; the last chunk takes the remainder
 // (sql-ops/src/partition/partition_input_chunk.rs:24-35).

@@ -103,20 +103,30 @@ struct HistParams {
   uint64_t* scan_state;
   uint64_t scan_state_len;
   uint64_t* stamp;     // time of the launch's start, or nullptr
+  // adaptive digits: the build keys to decide by, sample_n of them (0: decided),
+  // one of every sample_part; the least number of different digits among them;
+  // the decision
+  const void* sample;
+  uint32_t sample_n, sample_part, sample_digits, reserved;
+  uint32_t* hashed;
 };
+constexpr uint32_t kSampleKeys = 256;
 
 // Contiguous histogram parameters of one relation of a paired or batched
 // launch, in chunks of balanced_chunk_len; scan_state (scan_state_words(2^radix_bits) words) is cleared by it.
 HistParams hist_params(KeyType t, const void* keys, uint64_t n, uint32_t chunks, uint32_t radix_bits,
                        uint32_t block, uint32_t* counts, uint64_t* scan_state);
+// Adaptive digits by the n build keys; the decision goes to *hashed.
+void sample_build_keys(HistParams& p, const void* keys, uint64_t n, uint32_t* hashed);
 // Histograms of two relations of the same radix bits in one launch: ga chunks
-// of a, gb of b (gb = 0: a alone).
+// of a, gb of b (gb = 0: a alone).  adaptive, here and below: digits as the
+// build keys want them (DigitOf).
 hipError_t launch_hist_pair(KeyType t, const HistParams& a, const HistParams& b, uint32_t ga, uint32_t gb,
-                            uint32_t block, hipStream_t stream);
+                            bool adaptive, uint32_t block, hipStream_t stream);
 // Histograms of njobs relations in one launch: block b counts chunk
 // b - prefix[j] of jobs[j] (prefix[njobs] = blocks, device memory).
 hipError_t launch_hist_batched(KeyType t, const HistParams* jobs, const uint32_t* prefix, uint32_t njobs,
-                               uint32_t blocks, uint32_t radix_bits, uint32_t block, hipStream_t stream);
+                               uint32_t blocks, uint32_t radix_bits, bool adaptive, uint32_t block, hipStream_t stream);
 // Offsets of njobs relations of one fanout in one launch.
 hipError_t launch_offsets_batched(const OffsetsScan* jobs, uint32_t njobs, uint32_t fanout, hipStream_t stream);
 
@@ -135,6 +145,7 @@ struct PartitionLaunch {
   uint32_t block;             // requested threads per block
   uint32_t lds_bytes;         // LDS the scatter may use per block
   bool buffered;              // software write-combining vs. direct scatter
+  const uint32_t* hashed = nullptr;  // adaptive digits: the histogram's decision (buffered, up to 9 bits, no spill)
   // Optional spill region: partitions spill_from.. are written to
   // `spill` instead of `relation`, spill[0] standing for tuple index
   // spill_base of the relation (so the relation's first spill_base tuples
@@ -163,6 +174,7 @@ struct ScatterParams {
   uintptr_t spill_addr;  // address tuple index 0 would have in the spill region
   uint32_t spill_from;   // first partition written to the spill region
   uint64_t* stamp;       // time of the launch's start, or nullptr
+  const uint32_t* hashed;  // adaptive digits: the histogram's decision
 };
 
 // Scatter descriptor of one relation of a batched launch: the line ring is
@@ -175,7 +187,7 @@ hipError_t scatter_params_batched(KeyType t, const void* keys, const void* pays,
 // chunk b - prefix[j] of jobs[j] (prefix[njobs] = blocks, device memory);
 // block and ring_cap as given to scatter_params_batched for every job.
 hipError_t launch_partition_batched(KeyType t, const ScatterParams* jobs, const uint32_t* prefix, uint32_t njobs,
-                                    uint32_t blocks, uint32_t radix_bits, uint32_t lds_total, uint32_t block,
+                                    uint32_t blocks, uint32_t radix_bits, bool adaptive, uint32_t lds_total, uint32_t block,
                                     uint32_t ring_cap, hipStream_t stream);
 // Pass 1 on the CPU (host memory in and out): the contiguous layout of the
 // GPU's pass 1; offsets[F] receives the partition starts.

@@ -281,8 +281,10 @@ __global__ __launch_bounds__(BLOCK, CAP * 2 * sizeof(K) <= 32768 ? 6 : 4) void p
       for (uint32_t k = 0; k < NV; ++k) x[k] = __builtin_nontemporal_load(vp + min(v0 + k * BLOCK + tid, nvp - 1));
     };
     const uint32_t digit = unit.part & ((1u << d.bits1) - 1u);
-    const K free_key = static_cast<K>(digit ^ 1u);
-    const K no_key = static_cast<K>((digit ^ 1u) | (1u << d.bits1));
+    const bool hashed = d.hashed && uniform_load(d.hashed + (d.job_results ? unit.part >> d.job_shift : 0u)) != 0;
+    const uint32_t other = hashed ? (digit ^ 1u) << (32u - d.bits1) : digit ^ 1u;
+    const K free_key = static_cast<K>(hashed ? other * kDigitMulInverse : other);
+    const K no_key = static_cast<K>(hashed ? (other + 1u) * kDigitMulInverse : other | (1u << d.bits1));
     uint32_t wave_cnt = 0;
     VT xa[NV], xb[NV];
     load(xa, 0);  // in flight while the table is built
@@ -290,7 +292,7 @@ __global__ __launch_bounds__(BLOCK, CAP * 2 * sizeof(K) <= 32768 ? 6 : 4) void p
     const uint32_t fills = range_count(nb, FILL), fill = range_count(nb, fills);
     for (uint32_t f = 0; f < fills; ++f) {
       const uint32_t f0 = f * fill, nf = range_end(nb, fill, f) - f0;
-      const BucketTable<K> tab(lds_u64, CAP, BucketTable<K>::lg_buckets(CAP, nf), free_key);
+      const BucketTable<K> tab(lds_u64, CAP, BucketTable<K>::lg_buckets(CAP, nf), free_key, hashed, d.bits1);
       tab.clear();
       if (tid == 0) s_dup = 0;
       __syncthreads();

@@ -198,7 +198,7 @@ struct Vec16 {
 };
 
 // Buffered scatter of chunk `chunk` of G (one block).
-template <typename K, int BLOCK, bool SPILL>
+template <typename K, int BLOCK, bool SPILL, bool ADAPTIVE>
 __device__ __forceinline__ void scatter_swwc_body(const ScatterParams& p, uint32_t chunk, uint32_t G) {
   using T = Tuple<K>;
   using VK = typename Vec16<K>::type;
@@ -218,7 +218,7 @@ __device__ __forceinline__ void scatter_swwc_body(const ScatterParams& p, uint32
   const uint32_t R = p.ring_lines;
   const uint32_t RL = R * L;
   const uint32_t QL = p.queue_len;
-  const uint64_t mask = radix_mask(p.radix_bits, p.ignore_bits);
+  const DigitOf<K, ADAPTIVE> digit(p.radix_bits, p.ignore_bits, ADAPTIVE && scalar_load(p.hashed) != 0);
   const uint32_t tid = threadIdx.x;
   const uint32_t w = __builtin_amdgcn_readfirstlane(tid / kWave);
   const uint32_t lane = lane_id();
@@ -267,7 +267,7 @@ __device__ __forceinline__ void scatter_swwc_body(const ScatterParams& p, uint32
     uint32_t d[V], pos[V], lm[V];
 #pragma unroll
     for (uint32_t k = 0; k < V; ++k) {
-      d[k] = key_to_partition<K>(key[k], mask, p.ignore_bits);
+      d[k] = digit(key[k]);
       pos[k] = 0;
       lm[k] = 0;
       if ((act >> k) & 1u) {
@@ -435,7 +435,7 @@ __device__ __forceinline__ void scatter_swwc_body(const ScatterParams& p, uint32
 template <typename K, int BLOCK, bool SPILL>
 __global__ __launch_bounds__(BLOCK) void scatter_swwc_kernel(ScatterParams p) {
   stamp_start(p.stamp);
-  scatter_swwc_body<K, BLOCK, SPILL>(p, blockIdx.x, gridDim.x);
+  scatter_swwc_body<K, BLOCK, SPILL, false>(p, blockIdx.x, gridDim.x);
 }
 
 // Two relations in one launch (the sides of one join, of the same fanout): the
@@ -446,17 +446,17 @@ __global__ __launch_bounds__(BLOCK) void scatter_swwc_kernel(ScatterParams p) {
 struct ScatterPair {
   ScatterParams side[2];
 };
-template <typename K, int BLOCK>
+template <typename K, int BLOCK, bool ADAPTIVE>
 __global__ __launch_bounds__(BLOCK) void scatter_swwc_pair_kernel(ScatterPair s, uint32_t ga) {
   const uint32_t i = blockIdx.x < ga ? 0u : 1u;
   stamp_start(s.side[0].stamp);
   const ScatterParams p = s.side[i];
-  scatter_swwc_body<K, BLOCK, false>(p, i ? blockIdx.x - ga : blockIdx.x, i ? gridDim.x - ga : ga);
+  scatter_swwc_body<K, BLOCK, false, ADAPTIVE>(p, i ? blockIdx.x - ga : blockIdx.x, i ? gridDim.x - ga : ga);
 }
 
 // Many relations in one launch: block b scatters chunk b - prefix[j] of
 // relation j (batched joins; every relation has the same fanout).
-template <typename K, int BLOCK>
+template <typename K, int BLOCK, bool ADAPTIVE>
 __global__ __launch_bounds__(BLOCK) void scatter_swwc_batched_kernel(const ScatterParams* __restrict__ jobs,
                                                                      const uint32_t* __restrict__ prefix,
                                                                      uint32_t njobs) {
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(BLOCK) void scatter_swwc_batched_kernel(const Scatt
   // loaded from them as global)
   const ScatterParams p = jobs[lo];
   const uint32_t c0 = scalar_load(prefix + lo);
-  scatter_swwc_body<K, BLOCK, false>(p, blockIdx.x - c0, scalar_load(prefix + lo + 1) - c0);
+  scatter_swwc_body<K, BLOCK, false, ADAPTIVE>(p, blockIdx.x - c0, scalar_load(prefix + lo + 1) - c0);
 }
 
 // Queue entries per step buffer: a step completes at most one line per
@@ -527,6 +527,7 @@ ScatterParams scatter_params(const PartitionLaunch& a) {
   p.chunk_offsets = a.chunk_offsets;
   p.relation = a.relation;
   p.stamp = a.stamp;
+  p.hashed = a.hashed;
   const uint32_t F = 1u << a.radix_bits;
   p.spill_from = a.spill != nullptr && a.spill_from < F ? a.spill_from : F;
   p.spill_addr = reinterpret_cast<uintptr_t>(a.spill) - static_cast<uintptr_t>(a.spill_base * sizeof(Tuple<K>));
@@ -566,10 +567,10 @@ hipError_t launch_swwc_t(ScatterParams p, uint32_t fanout, uint32_t chunks, uint
   return hipGetLastError();
 }
 
-template <typename K, int BLOCK>
+template <typename K, int BLOCK, bool ADAPTIVE>
 hipError_t launch_swwc_pair(ScatterParams a, ScatterParams b, uint32_t fanout, uint32_t ga, uint32_t gb,
                             uint32_t lds_total, hipStream_t stream) {
-  auto kern = scatter_swwc_pair_kernel<K, BLOCK>;
+  auto kern = scatter_swwc_pair_kernel<K, BLOCK, ADAPTIVE>;
   const uint32_t lds = size_ring<K>(reinterpret_cast<const void*>(kern), fanout, BLOCK, lds_total, a);
   if (lds == 0) return hipErrorNotSupported;
   b.ring_lines = a.ring_lines;
@@ -580,13 +581,13 @@ hipError_t launch_swwc_pair(ScatterParams a, ScatterParams b, uint32_t fanout, u
   return hipGetLastError();
 }
 
-template <typename K>
+template <typename K, bool ADAPTIVE>
 hipError_t launch_partition_pair_t(const PartitionLaunch& a, const PartitionLaunch& b, hipStream_t stream) {
   const ScatterParams pa = scatter_params<K>(a), pb = scatter_params<K>(b);
   const uint32_t F = 1u << a.radix_bits;
-  if (a.block >= 1024) return launch_swwc_pair<K, 1024>(pa, pb, F, a.chunks, b.chunks, a.lds_bytes, stream);
-  if (a.block >= 512) return launch_swwc_pair<K, 512>(pa, pb, F, a.chunks, b.chunks, a.lds_bytes, stream);
-  return launch_swwc_pair<K, 256>(pa, pb, F, a.chunks, b.chunks, a.lds_bytes, stream);
+  if (a.block >= 1024) return launch_swwc_pair<K, 1024, ADAPTIVE>(pa, pb, F, a.chunks, b.chunks, a.lds_bytes, stream);
+  if (a.block >= 512) return launch_swwc_pair<K, 512, ADAPTIVE>(pa, pb, F, a.chunks, b.chunks, a.lds_bytes, stream);
+  return launch_swwc_pair<K, 256, ADAPTIVE>(pa, pb, F, a.chunks, b.chunks, a.lds_bytes, stream);
 }
 
 template <typename K>
@@ -627,13 +628,22 @@ uint32_t swwc_lds_bytes(uint32_t fanout, uint32_t tuple_bytes, uint32_t ring_lin
 }
 
 hipError_t launch_partition(const PartitionLaunch& a, hipStream_t stream) {
+  if (a.hashed != nullptr) {
+    PartitionLaunch none = a;
+    none.n = none.chunks = 0;
+    none.chunk_len = 1;
+    return launch_partition_pair(a, none, stream);
+  }
   if (a.type == KeyType::I32) return launch_partition_t<int32_t>(a, stream);
   return launch_partition_t<int64_t>(a, stream);
 }
 
 hipError_t launch_partition_pair(const PartitionLaunch& a, const PartitionLaunch& b, hipStream_t stream) {
-  hipError_t e = a.type == KeyType::I32 ? launch_partition_pair_t<int32_t>(a, b, stream)
-                                        : launch_partition_pair_t<int64_t>(a, b, stream);
+  if (a.hashed != nullptr)
+    return a.type == KeyType::I32 ? launch_partition_pair_t<int32_t, true>(a, b, stream)
+                                  : launch_partition_pair_t<int64_t, true>(a, b, stream);
+  hipError_t e = a.type == KeyType::I32 ? launch_partition_pair_t<int32_t, false>(a, b, stream)
+                                        : launch_partition_pair_t<int64_t, false>(a, b, stream);
   if (e != hipErrorNotSupported) return e;
   if ((e = launch_partition(a, stream)) != hipSuccess) return e;
   return launch_partition(b, stream);
@@ -642,16 +652,17 @@ hipError_t launch_partition_pair(const PartitionLaunch& a, const PartitionLaunch
 namespace {
 
 template <typename K>
-const void* batched_scatter_kernel(uint32_t block) {
-  return block == 512 ? reinterpret_cast<const void*>(scatter_swwc_batched_kernel<K, 512>)
-                      : reinterpret_cast<const void*>(scatter_swwc_batched_kernel<K, 1024>);
+auto batched_scatter_kernel(uint32_t block, bool adaptive) {
+  if (block == 512) return adaptive ? scatter_swwc_batched_kernel<K, 512, true> : scatter_swwc_batched_kernel<K, 512, false>;
+  return adaptive ? scatter_swwc_batched_kernel<K, 1024, true> : scatter_swwc_batched_kernel<K, 1024, false>;
 }
 
 // Ring of the batched scatter for this fanout and block: the deepest that
 // fits LDS, at most ring_cap lines when ring_cap is set (0: none fits).
 template <typename K>
 uint32_t batched_ring(uint32_t fanout, uint32_t lds_total, uint32_t block, uint32_t ring_cap) {
-  const uint32_t budget = dynamic_lds_budget(batched_scatter_kernel<K>(block), lds_total);
+  const uint32_t budget =
+      dynamic_lds_budget(reinterpret_cast<const void*>(batched_scatter_kernel<K>(block, false)), lds_total);
   const uint32_t top = ring_cap ? (ring_cap < 256 ? ring_cap : 256) : 256;
   for (uint32_t r = top; r >= 1; r /= 2)
     if (swwc_bytes(fanout, r, swwc_queue_len<K>(fanout, r, block)) <= budget) return r;
@@ -683,19 +694,16 @@ hipError_t scatter_params_batched_t(const void* keys, const void* pays, uint64_t
 
 template <typename K>
 hipError_t launch_partition_batched_t(const ScatterParams* jobs, const uint32_t* prefix, uint32_t njobs,
-                                      uint32_t blocks, uint32_t radix_bits, uint32_t lds_total, uint32_t block,
-                                      uint32_t ring_cap, hipStream_t stream) {
+                                      uint32_t blocks, uint32_t radix_bits, bool adaptive, uint32_t lds_total,
+                                      uint32_t block, uint32_t ring_cap, hipStream_t stream) {
   const uint32_t F = 1u << radix_bits;
   const uint32_t ring = batched_ring<K>(F, lds_total, block, ring_cap);
   if (ring == 0) return hipErrorNotSupported;
   const uint32_t lds = swwc_bytes(F, ring, swwc_queue_len<K>(F, ring, block));
-  (void)hipFuncSetAttribute(batched_scatter_kernel<K>(block), hipFuncAttributeMaxDynamicSharedMemorySize,
+  const auto kern = batched_scatter_kernel<K>(block, adaptive);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                             static_cast<int>(lds));
-  if (block == 512)
-    hipLaunchKernelGGL((scatter_swwc_batched_kernel<K, 512>), dim3(blocks), dim3(512), lds, stream, jobs, prefix, njobs);
-  else
-    hipLaunchKernelGGL((scatter_swwc_batched_kernel<K, 1024>), dim3(blocks), dim3(1024), lds, stream, jobs, prefix,
-                       njobs);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(block), lds, stream, jobs, prefix, njobs);
   return hipGetLastError();
 }
 
@@ -713,14 +721,14 @@ hipError_t scatter_params_batched(KeyType t, const void* keys, const void* pays,
 }
 
 hipError_t launch_partition_batched(KeyType t, const ScatterParams* jobs, const uint32_t* prefix, uint32_t njobs,
-                                    uint32_t blocks, uint32_t radix_bits, uint32_t lds_total, uint32_t block,
+                                    uint32_t blocks, uint32_t radix_bits, bool adaptive, uint32_t lds_total, uint32_t block,
                                     uint32_t ring_cap, hipStream_t stream) {
   if (blocks == 0) return hipSuccess;
   if (block != 512 && block != 1024) return hipErrorInvalidValue;
   if (t == KeyType::I32)
-    return launch_partition_batched_t<int32_t>(jobs, prefix, njobs, blocks, radix_bits, lds_total, block, ring_cap,
-                                               stream);
-  return launch_partition_batched_t<int64_t>(jobs, prefix, njobs, blocks, radix_bits, lds_total, block, ring_cap,
+    return launch_partition_batched_t<int32_t>(jobs, prefix, njobs, blocks, radix_bits, adaptive, lds_total, block,
+                                               ring_cap, stream);
+  return launch_partition_batched_t<int64_t>(jobs, prefix, njobs, blocks, radix_bits, adaptive, lds_total, block, ring_cap,
                                              stream);
 }
 

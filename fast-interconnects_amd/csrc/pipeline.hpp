@@ -120,6 +120,7 @@ struct PipelineDevice {
   uint32_t hbm_unit_cap;
   // single pass: 128 KiB block tables (one block per CU) instead of 64 KiB ones
   uint32_t big_block_tables;
+  uint32_t* hashed;           // adaptive digits (single pass): the decision of each join, or nullptr: radix digits
 };
 
 // One join side of a batched plan: its pass-1 region and where its

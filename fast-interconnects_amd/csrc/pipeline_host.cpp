@@ -88,6 +88,7 @@ PartitionLaunch scatter_of(const PipelineDevice& d, const PipelineSide& s, KeyTy
   a.block = block;
   a.lds_bytes = lds_total;
   a.buffered = true;
+  a.hashed = d.hashed;
   return a;
 }
 
@@ -100,11 +101,16 @@ hipError_t enqueue_pass1_prefix_sum(const PipelineDevice& d, KeyType t, uint32_t
   HistParams ha = hist_params(t, a->keys, a->n, a->g1, d.bits1, block, a->counts1, a->scan1);
   ha.stamp = d.stamps;
   HistParams hb = b ? hist_params(t, b->keys, b->n, b->g1, d.bits1, block, b->counts1, b->scan1) : ha;
+  if (d.hashed) {
+    const uint64_t n = d.sides & 1 ? d.build.n : 0;  // a server has looked at its build sides before
+    sample_build_keys(ha, d.build.keys, n, d.hashed);
+    sample_build_keys(hb, d.build.keys, n, d.hashed);
+  }
   if (key_copies) {
     ha.dst_keys = key_copies[a == &d.build ? 0 : 1];
     hb.dst_keys = key_copies[1];
   }
-  const hipError_t e = launch_hist_pair(t, ha, hb, a->g1, b ? b->g1 : 0, block, stream);
+  const hipError_t e = launch_hist_pair(t, ha, hb, a->g1, b ? b->g1 : 0, d.hashed != nullptr, block, stream);
   if (e != hipSuccess) return e;
   const OffsetsScan sa = scan_of(d, *a), sb = b ? scan_of(d, *b) : sa;
   return launch_offsets_scan(sa, b ? &sb : nullptr, stream);

@@ -38,6 +38,7 @@ struct fij_join_plan {
   uint32_t cus;
   uint32_t clock_khz;  // rate of the device clock the phases are stamped with
   uint32_t* done;      // [kDoneWords] finished blocks, zero between joins
+  uint32_t* hashed;    // single-pass joins: whether the last one's digits were hashed
   // what the last enqueued join wrote or did not launch
   struct Host {
     JoinAggregate result;
@@ -213,6 +214,7 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
         static_cast<uint32_t>(2ull * p->d.big_cap + (cfg->build_len + cfg->probe_len) / 65536 + 2);
     // (the block counters are cleared with the arena)
     if (st == FIJ_OK) st = alloc(p, &p->done, kDoneWords);
+    if (st == FIJ_OK) st = alloc(p, &p->hashed, 1);
     if (st == FIJ_OK && hipMemset(p->done, 0, kDoneWords * sizeof(uint32_t)) != hipSuccess)
       st = plan_fail(FIJ_DEVICE_ERROR, "clearing the block counters failed");
     void* arena = nullptr;
@@ -241,6 +243,9 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
   p->one.bits2 = 0;
   p->one.F1 = 1u << kOnePassBits;
   p->one.F2 = 1;
+  // (wider fanouts have no line rings)
+  p->one.hashed = p->hashed;
+  p->d.hashed = p->d.bits2 || p->d.bits1 > kOnePassBits ? nullptr : p->hashed;
   *out = p;
   return FIJ_OK;
 }

@@ -90,6 +90,7 @@ struct ResidentBuild {
   // of 2^table_lg entries instead of partitions (null: partitioned)
   void* table = nullptr;
   uint32_t table_lg = 0;
+  uint32_t* hashed = nullptr;  // one-pass builds: whether their digits are hashed
   std::vector<void*> allocs;
   uint64_t bytes = 0;
 };
@@ -161,6 +162,7 @@ PipelineDevice base_device(const fij_join_server* s, const ResidentBuild& b) {
   d.pad = pad_tuples(s->kt);
   d.tile2 = pipeline_tile2(s->kt);
   d.agg_len = s->agg_len;
+  d.hashed = b.hashed;
   return d;
 }
 
@@ -411,6 +413,7 @@ fij_status add_one_pass_build(fij_join_server* s, std::unique_ptr<ResidentBuild>
   b->n = len;
   const uint32_t F1 = 1u << b1;
   hipError_t e = alloc_pipeline_side(b->side, s->kt, len, F1, 1, s->cus, false, 0, b->allocs);
+  if (e == hipSuccess && (e = hipMalloc(&b->hashed, sizeof(uint32_t))) == hipSuccess) b->allocs.push_back(b->hashed);
   if (e != hipSuccess) {
     free_all(b->allocs);
     return hip_status(e, "hipMalloc");
