@@ -340,9 +340,9 @@ fij_status enqueue_class(fij_join_batch* b, ClassArena& a, const ClassKey& ck, c
   d.build.n = rel2[0];
   d.probe.n = rel2[1];
   d.hashed = a.hashed;
-  if (b2 == 0) {  // the class's largest build side chooses the block tables
+  if (b2 == 0) {  // the class's longest build side chooses the block tables
     d.build.n = static_cast<uint64_t>(J) * ck.build;
-    d.big_block_tables = big_block_tables_for(kt, ck.build, F1);
+    d.big_block_tables = one_pass_class(kt, ck.build).big_tables;
   }
   a.sub_joins = J;
   a.sub_blocks = blocks;
@@ -469,23 +469,14 @@ fij_join_tuning tuned_class(KeyType kt, uint64_t build_len, uint64_t probe_len, 
   return rule;
 }
 
-// The class that a batch runs a partitioned join of these lengths in.  Build
-// sides of up to two table fills per partition (one_pass_join) take a single
-// pass, in classes of a factor of four from 2^14 (int64: 2^13) tuples on: 5, 7
-// and 9 bits leave 512 to 2,048 (256 to 1,024) tuples in a partition, for 32
-// KiB tables; beyond, 9 bits with 64 KiB and then 128 KiB tables.
+// The class that a batch runs a partitioned join of these lengths in: a single
+// pass (one_pass_class) wherever one_pass_join takes it.
 ClassKey batch_class(KeyType kt, uint64_t build_len, uint64_t probe_len) {
   bool user = false;
   const fij_join_tuning tc = tuned_class(kt, build_len, probe_len, &user);
   if (user || !one_pass_join(kt, build_len, probe_len)) return {tc.radix_bits_1, tc.radix_bits_2, tc.ring_lines, tc.block, 0};
-  uint32_t b1 = 5;
-  uint64_t most = kt == KeyType::I32 ? 1u << 16 : 1u << 15;
-  for (; build_len > most && b1 < kOnePassBits; b1 += 2) most <<= 2;
-  if (build_len > most) {
-    most = static_cast<uint64_t>(pipeline_block_table_tuples(kt, false)) << kOnePassBits;
-    if (!block_tables_hold(kt, build_len, 1ull << kOnePassBits, false)) most = 2 * one_pass_fill(kt) << kOnePassBits;
-  }
-  return {b1, 0, 0, 1024, static_cast<uint32_t>(most)};
+  const OnePassClass c = one_pass_class(kt, build_len);
+  return {c.bits, 0, 0, 1024, c.build};
 }
 
 }  // namespace

@@ -114,6 +114,27 @@ inline uint32_t probe_heavy_bits2(KeyType t, uint64_t build_len) {
   while (b2 < 12 && (1ull << b2) < items) ++b2;
   return b2;
 }
+// The class of a batch's single-pass join: its bits, the longest build side of
+// the class and whether its tables are the 128 KiB ones.  A factor of four each
+// from 2^14 (int64: 2^13) tuples on: 5, 7 and 9 bits leave 512 to 2,048 (256 to
+// 1,024) tuples in a partition, for 32 KiB tables; beyond, 9 bits and 128 KiB
+// tables (64 KiB ones up to twice that: 3 joins of 550,000 x 2.2 M int64 tuples
+// 145 -> 160 us, of 2 M x 8 M int32 tuples 269 -> 273 us), in two classes that
+// overlap (in one, 6 joins of 1.2 to 3.4 M x 12 times as many int32 tuples
+// 1,108 -> 1,224 us).
+struct OnePassClass {
+  uint32_t bits, build;
+  bool big_tables;
+};
+inline OnePassClass one_pass_class(KeyType t, uint64_t build_len) {
+  uint32_t bits = 5;
+  uint64_t most = t == KeyType::I32 ? 1u << 16 : 1u << 15;
+  for (; build_len > most && bits < kOnePassBits; bits += 2) most <<= 2;
+  const bool big = build_len > most;
+  if (big) most <<= 1;
+  if (build_len > most) most = 2 * one_pass_fill(t) << kOnePassBits;
+  return {bits, static_cast<uint32_t>(most), big};
+}
 // big_block_tables of a single-pass plan of `partitions` partitions.
 inline uint32_t big_block_tables_for(KeyType t, uint64_t build_len, uint64_t partitions) {
   return block_tables_hold(t, build_len, partitions, false) ? 0u : 1u;
