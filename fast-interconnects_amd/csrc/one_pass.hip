@@ -4,9 +4,9 @@
 //
 //   one_pass_plan_kernel  partition lengths, and work units {build range, probe
 //                         range} of every partition pair; a build partition
-//                         beyond the LDS table fills it several times, beyond
-//                         kMaxFills fills it gets a hash table in the HBM arena
-//                         when the arena has room
+//                         beyond the LDS table fills it several times, a much
+//                         longer one (one_pass_lds_tuples) gets a hash table in
+//                         the HBM arena when the arena has room
 //   part_join_kernel      one block per unit: the build range goes into a
 //                         block-shared table, the probe range is streamed
 //                         against it; then the HBM tables, and the sum
@@ -31,24 +31,16 @@ __device__ __forceinline__ U uniform_load(const U* ptr) {
   return *(const __attribute__((address_space(4))) U*)(ptr);
 }
 
-// Slots of the block-shared table: 64 KiB of keys and values, half of that
-// for small partitions, or 128 KiB (big_block_tables).  A fill takes at most
-// 9/16 (int32) or 5/8 (int64) of them.
 template <typename K>
-constexpr uint32_t kSlots = 65536 / (2 * sizeof(K));
+constexpr KeyType kKeyType = sizeof(K) == 4 ? KeyType::I32 : KeyType::I64;
 
 constexpr uint32_t kTableUnitTuples = 65536;  // tuples of an HBM-table work unit
-
-// Table fills a build partition may take where the arena has room for a table:
-// every fill streams the probe tuples again (about 3 TB/s), an HBM table costs
-// a random access per probe tuple (about 45 G/s).
-constexpr uint32_t kMaxFills = 4;
 
 // One block per join.  `sides` == nullptr: one join, whose sides end at their
 // padded_len1; that block sets the counters.  In batches (which have no HBM
 // arena) the counters were reset by an earlier launch.
 __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, const BatchSide* sides, uint32_t F1j,
-                                                             uint32_t rcap) {
+                                                             uint32_t lds_tuples) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t wave_tmp[1024 / kWave + 1];
   __shared__ uint32_t s_base, s_slots, s_big, s_build_units, s_probe_units;
@@ -72,7 +64,7 @@ __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, c
     const uint32_t nb = range(d.build, end_b, p, at), np = range(d.probe, end_p, p, at);
     PartUnits cut = part_units_of(nb, np);
     if (cut.units) {
-      if (nb > kMaxFills * rcap && d.hbm_cap && nb <= (d.hbm_cap >> 1)) {
+      if (nb > lds_tuples && d.hbm_cap && nb <= (d.hbm_cap >> 1)) {
         // an HBM table of at least twice the build tuples, if the arena (at
         // most 2^26 slots) has room.  A partition that finds none takes no
         // slots; the sum of the others' stays below 2^32.
@@ -247,7 +239,7 @@ template <typename K, uint32_t CAP, uint32_t BLOCK>
 __global__ __launch_bounds__(BLOCK, CAP * 2 * sizeof(K) <= 32768 ? 6 : 4) void part_join_kernel(PipelineDevice d) {
   using V = TupleVec<K>;
   using VT = typename V::type;
-  constexpr uint32_t FILL = CAP / 16 * (sizeof(K) == 4 ? 9 : 10);  // build tuples per table fill (one_pass_fill)
+  constexpr uint32_t FILL = block_table_fill(kKeyType<K>, CAP);
   constexpr uint32_t NV = 2;                  // vectors in flight per buffer
   constexpr uint32_t NT = NV * V::N;          // their tuples
   constexpr uint32_t PROBES = 2;              // probed together
@@ -386,15 +378,15 @@ hipError_t launch_part_join(const PipelineDevice& d, uint32_t grid, hipStream_t 
 
 template <typename K>
 hipError_t launch_one_pass_join_t(const PipelineDevice& d, uint32_t grid, hipStream_t stream) {
-  // One block of 1,024 threads per CU with a 128 KiB table, two of 512 with
-  // 64 KiB, three with 32 KiB: those take partitions that fill them half on
-  // average (20 batched joins of 2^18..2^20 int32 build tuples: 283 us with 64
-  // KiB tables, 240 us).
+  // one block of 1,024 threads per CU with a 128 KiB table, two of 512 with 64
+  // KiB, three with 32 KiB
+  constexpr uint32_t SLOTS = block_table_slots(kKeyType<K>);
   auto blocks = [&](uint32_t n) { return d.job_results ? n : std::min(n, d.agg_len); };
-  if (d.big_block_tables) return launch_part_join<K, 2 * kSlots<K>, 1024>(d, blocks((grid + 1) / 2), stream);
-  if (d.build.n <= static_cast<uint64_t>(d.F1) * (kSlots<K> / 4))
-    return launch_part_join<K, kSlots<K> / 2, 512>(d, blocks(grid + grid / 2), stream);
-  return launch_part_join<K, kSlots<K>, 512>(d, blocks(grid), stream);
+  switch (one_pass_slots(kKeyType<K>, d.build.n, d.F1, d.big_block_tables != 0)) {
+    case 2 * SLOTS: return launch_part_join<K, 2 * SLOTS, 1024>(d, blocks((grid + 1) / 2), stream);
+    case SLOTS: return launch_part_join<K, SLOTS, 512>(d, blocks(grid), stream);
+    default: return launch_part_join<K, SLOTS / 2, 512>(d, blocks(grid + grid / 2), stream);
+  }
 }
 
 }  // namespace
@@ -409,7 +401,7 @@ hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchS
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(one_pass_plan_kernel, dim3(joins), dim3(1024), 3 * F1j * 4, stream, d, sides, F1j,
-                     pipeline_block_table_tuples(t, d.big_block_tables != 0));
+                     one_pass_lds_tuples(t, d.big_block_tables != 0));
   return hipGetLastError();
 }
 

@@ -45,6 +45,29 @@ constexpr uint32_t pipeline_block_table_tuples(KeyType t, bool big = false) {
   return (big ? 131072u : 65536u) / (t == KeyType::I32 ? 8u : 16u) * 3 / 4;
 }
 
+// Slots of the block-shared table of the single-pass joins: 64 KiB of keys and
+// values, 128 KiB (big_block_tables), or 32 KiB for partitions that fill those
+// half on average (20 batched joins of 2^18..2^20 int32 build tuples: 283 us
+// with 64 KiB tables, 240 us).
+constexpr uint32_t block_table_slots(KeyType t) { return t == KeyType::I32 ? 8192 : 4096; }
+inline uint32_t one_pass_slots(KeyType t, uint64_t build_len, uint64_t partitions, bool big) {
+  const uint32_t slots = block_table_slots(t);
+  return big ? 2 * slots : build_len <= partitions * (slots / 4) ? slots / 2 : slots;
+}
+// Build tuples of one fill of a table: 5/8 of the slots at int64, 9/16 at int32.
+// Fuller buckets overflow, and probes that leave theirs (in a table with
+// duplicate keys every one whose bucket is full) made fills of 70 % 0.7 to 0.9
+// times as fast as two passes, at int32 fills of 60 % 0.94 to 1.5 times.
+constexpr uint32_t block_table_fill(KeyType t, uint32_t slots) { return slots / 16 * (t == KeyType::I32 ? 9 : 10); }
+// Build tuples up to which a partition fills the table several times although
+// the arena would have room for an HBM table: three times the slots of the 64 or
+// 128 KiB table, up to 6 fills (5 at int64), of 32 KiB tables up to 11 (10).
+// Each fill streams the probe tuples again, an HBM table costs a random access
+// per probe tuple and a chain per repeated key.  Among 64 partitions one of
+// 10,000 int32 tuples, in 32 KiB tables: 490 to 540 us in LDS, 510 to 575 us in
+// HBM, of 20,000 910 to 980 and 340 to 400 us; of 14,000 with 500 copies of
+// every key 0.3 and 55 ms.
+constexpr uint32_t one_pass_lds_tuples(KeyType t, bool big) { return 3 * block_table_slots(t) * (big ? 2 : 1); }
 
 // Single-pass plans (fij_join_plan_bits, single-pass batched classes): 9
 // bits, the widest pass-1 fanout whose line rings fit LDS.
@@ -60,14 +83,8 @@ inline bool block_tables_hold(KeyType t, uint64_t build_len, uint64_t partitions
 inline bool one_pass_fits(KeyType t, uint64_t build_len) {
   return block_tables_hold(t, build_len, 1ull << kOnePassBits, true);
 }
-// Build tuples of one fill of a 128 KiB table in each of 2^kOnePassBits
-// partitions.  A fill takes 5/8 of the slots at int64, 9/16 at int32: fuller
-// buckets overflow, and probes that leave theirs (in a table with duplicate
-// keys every one whose bucket is full) made fills of 70 % 0.7 to 0.9 times as
-// fast as two passes, at int32 fills of 60 % 0.94 to 1.5 times.
-inline uint64_t one_pass_fill(KeyType t) {
-  return static_cast<uint64_t>(pipeline_block_table_tuples(t, true)) * (t == KeyType::I32 ? 9 : 10) / 12;
-}
+// Build tuples of one fill of a 128 KiB table.
+inline uint64_t one_pass_fill(KeyType t) { return block_table_fill(t, 2 * block_table_slots(t)); }
 // Whether the scatter's 32-bit offsets reach the end of a relation of `len`
 // tuples in this many partitions, each behind its padding.
 inline bool pass1_offsets_fit(KeyType t, uint64_t len, uint64_t partitions) {

@@ -13,6 +13,13 @@ PROGRAM = """
 #include "one_pass_rules.hpp"
 using namespace fij;
 int main(int argc, char** argv) {
+  if (argc == 5) {  // type, build tuples, partitions, big tables: slots, a fill, build tuples joined in LDS
+    const KeyType t = argv[1][0] == '0' ? KeyType::I32 : KeyType::I64;
+    const bool big = argv[4][0] == '1';
+    const uint32_t slots = one_pass_slots(t, strtoull(argv[2], nullptr, 10), strtoull(argv[3], nullptr, 10), big);
+    printf("%u %u %u\\n", slots, block_table_fill(t, slots), one_pass_lds_tuples(t, big));
+    return 0;
+  }
   if (argc == 4) {  // type, build and probe tuples: one pass, always one pass
     const KeyType t = argv[1][0] == '0' ? KeyType::I32 : KeyType::I64;
     const uint64_t b = strtoull(argv[2], nullptr, 10), p = strtoull(argv[3], nullptr, 10);
@@ -68,3 +75,14 @@ def test_single_pass_offsets_stay_below_2_32(rules, type, pad):
         assert rules([(type, build, last + 1)]) == [(0, 0)]
         assert rules([(type, build, (1 << 32) - 600)]) == [(0, 0)]
     assert rules([(type, 4_571_137, 5_000_000)]) == [(1, 0)]  # by its lengths, not always
+
+
+@pytest.mark.parametrize("type,fills", [(0, (2304, 4608, 9216)), (1, (1280, 2560, 5120))])
+def test_tables_and_their_fills(rules, type, fills):
+    """32 KiB tables up to half their slots on average, then 64 KiB ones; and how
+    often a partition may fill them before it takes an HBM table."""
+    half = 2048 >> type
+    for build, big, at, most in ((half << 9, 0, 0, (11, 10)), ((half << 9) + 1, 0, 1, (6, 5)), (1, 1, 2, (6, 5))):
+        [(slots, fill, lds)] = rules([(type, build, 512, big)])
+        assert slots == half << at + 1 and fill == fills[at]
+        assert -(-lds // fill) == most[type]
