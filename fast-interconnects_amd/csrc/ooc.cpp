@@ -262,8 +262,8 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
     for (int s = 0; s < NS; ++s) OOC_HIP(hipStreamSynchronize(st[s]));
     for (void* q : stream_allocs) OOC_HIP(hipFree(q));
     stream_allocs.clear();
-    cap = want;
-    const uint32_t max_tiles = static_cast<uint32_t>(cap / tile2 + F1 + 1);
+    cap = 0;
+    const uint32_t max_tiles = static_cast<uint32_t>(want / tile2 + F1 + 1);
     const uint64_t items = static_cast<uint64_t>(F1) * F2;
     OOC_HIP(place_on_device(stream_allocs, [&](Placer& a) {
       for (PipelineDevice& d : sd) {
@@ -275,8 +275,8 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
         d.tile2 = tile2;
         d.sides = 3;
         d.agg_len = join_grid;
-        d.unit_cap = static_cast<uint32_t>(items + 2 * cap / 65536 + 2);
-        for (PipelineSide* ps : {&d.build, &d.probe}) place_pipeline_side(*ps, kt, cap, F1, F2, 1, true, max_tiles, a);
+        d.unit_cap = static_cast<uint32_t>(items + 2 * want / 65536 + 2);
+        for (PipelineSide* ps : {&d.build, &d.probe}) place_pipeline_side(*ps, kt, want, F1, F2, 1, true, max_tiles, a);
         a.take(&d.work_counter, kJoinCounterWords);
         a.take(&d.overflow, items);
         a.take(&d.units, d.unit_cap);
@@ -286,6 +286,7 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
     // the deferred-item flags start at zero; every join leaves them at zero
     for (int s = 0; s < NS; ++s) OOC_HIP(hipMemsetAsync(sd[s].overflow, 0, items, st[s]));
     for (int s = 0; s < NS; ++s) OOC_HIP(hipStreamSynchronize(st[s]));
+    cap = want;
     return FIJ_OK;
   };
   // Enqueues pass 2 and the join of every group, alternating the streams;
@@ -463,9 +464,18 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
     // Keys in host memory cross the link once where a staging buffer's worth of
     // device memory holds each relation's: the histograms leave a copy for the
     // scatter (1,000,003 x 4,000,037 int64 tuples, 80 MB of columns: 4.32 ms with
-    // the keys read twice, 3.97 ms).
+    // the keys read twice, 3.97 ms).  The copies give way where there is no room
+    // for the cache or the join's buffers beside them.
     const size_t kb = key_bytes(kt);
     uint8_t* key_copy[2] = {nullptr, nullptr};
+    auto drop_copies = [&] {
+      (void)hipGetLastError();
+      if (!key_copy[0]) return false;
+      A.dev.erase(std::find(A.dev.begin(), A.dev.end(), static_cast<void*>(key_copy[0])));
+      (void)hipFree(key_copy[0]);  // one allocation
+      key_copy[0] = key_copy[1] = nullptr;
+      return true;
+    };
     if (std::max(build_len, probe_len) <= 2 * staging && !on_device(build_keys) && !on_device(probe_keys)) {
       const hipError_t e = place_on_device(A.dev, [&](Placer& a) {
         for (int r = 0; r < 2; ++r) a.take(&key_copy[r], lens[r] * kb);
@@ -502,11 +512,15 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
       s.cut_part = P;
       s.cut = P < F1 ? s.start(P) : s.padded_len;
     }
-    if (rel[0].cut || rel[1].cut)
-      OOC_HIP(place_on_device(A.dev, [&](Placer& a) {
+    if (rel[0].cut || rel[1].cut) {
+      auto place_cache = [&](Placer& a) {
         for (Pass1& s : rel)
           if (s.cut) a.take(&s.cache, (s.cut + 1) * tb);  // + the spare tuple of pass 2
-      }));
+      };
+      hipError_t e = place_on_device(A.dev, place_cache);
+      if (e == hipErrorOutOfMemory && drop_copies()) e = place_on_device(A.dev, place_cache);
+      OOC_HIP(e);
+    }
     // the spill regions keep the relations' alignment modulo 128 bytes, so the
     // scatter's full lines stay aligned there too
     auto place_spill = [&](Placer& a) {
@@ -551,7 +565,9 @@ extern "C" fij_status fij_ooc_join(const fij_ooc_config* cfg, const void* build_
     OOC_HIP(hipEventElapsedTime(&f, ev[1], ev[2]));
     partition_ms = f;
     const uint64_t whole = std::max(rel[0].padded_len, rel[1].padded_len);
-    fij_status fs = size_streams(std::max({std::min(staging, whole), longest(rel[0]), longest(rel[1])}));
+    const uint64_t want = std::max({std::min(staging, whole), longest(rel[0]), longest(rel[1])});
+    fij_status fs = size_streams(want);
+    if (fs == FIJ_OUT_OF_MEMORY && drop_copies()) fs = size_streams(want);
     if (fs != FIJ_OK) return fs;
     std::vector<Group> groups;
     make_groups(rel[0], rel[1], cap, groups);
