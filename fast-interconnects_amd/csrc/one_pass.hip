@@ -34,8 +34,6 @@ __device__ __forceinline__ U uniform_load(const U* ptr) {
 template <typename K>
 constexpr KeyType kKeyType = sizeof(K) == 4 ? KeyType::I32 : KeyType::I64;
 
-constexpr uint32_t kTableUnitTuples = 65536;  // tuples of an HBM-table work unit
-
 // One block per join.  `sides` == nullptr: one join, whose sides end at their
 // padded_len1; that block sets the counters.  In batches (which have no HBM
 // arena) the counters were reset by an earlier launch.
@@ -79,13 +77,12 @@ __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, c
         if (big < d.big_cap) {
           cut.units = 0;
           d.big[big] = make_uint4(j * F1j + p, slot, lg, 0u);
-          const uint32_t bu = range_count(nb, kTableUnitTuples), pu = range_count(np, kTableUnitTuples);
+          const uint32_t b_per = table_unit_tuples(nb), p_per = table_unit_tuples(np);
+          const uint32_t bu = range_count(nb, b_per), pu = range_count(np, p_per);
           const uint32_t b0 = atomicAdd(&s_build_units, bu), p0 = atomicAdd(&s_probe_units, pu);
-          for (uint32_t u = 0; u < bu; ++u)
-            d.hbm_units[b0 + u] = make_uint4(big, u * kTableUnitTuples, range_end(nb, kTableUnitTuples, u), 0u);
+          for (uint32_t u = 0; u < bu; ++u) d.hbm_units[b0 + u] = make_uint4(big, u * b_per, range_end(nb, b_per, u), 0u);
           for (uint32_t u = 0; u < pu; ++u)
-            d.hbm_units[d.hbm_unit_cap - 1 - (p0 + u)] =
-                make_uint4(big, u * kTableUnitTuples, range_end(np, kTableUnitTuples, u), 0u);
+            d.hbm_units[d.hbm_unit_cap - 1 - (p0 + u)] = make_uint4(big, u * p_per, range_end(np, p_per, u), 0u);
         }
       }
     }

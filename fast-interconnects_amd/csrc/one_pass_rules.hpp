@@ -59,6 +59,17 @@ inline uint32_t one_pass_slots(KeyType t, uint64_t build_len, uint64_t partition
 // duplicate keys every one whose bucket is full) made fills of 70 % 0.7 to 0.9
 // times as fast as two passes, at int32 fills of 60 % 0.94 to 1.5 times.
 constexpr uint32_t block_table_fill(KeyType t, uint32_t slots) { return slots / 16 * (t == KeyType::I32 ? 9 : 10); }
+// Tuples of a work unit of a partition with an HBM table.  A thread has one
+// random access in flight, so a unit takes as long as a thread has tuples, and
+// with blocks to wait for: a 128th of the range, but kTableUnitMin at least and
+// kTableUnitMax at most.  One of 64 partitions of 12,000 int64 tuples, in 32 KiB
+// tables, and 4 M probe tuples, 6 and 60 % of them in that partition: 743 and
+// 617 us with units of 65,536, 238 and 428 with a 64th, 182 and 305 so, 200 and
+// 468 with a 512th.
+constexpr uint32_t kTableUnitMin = 4096, kTableUnitMax = 65536;
+__host__ __device__ constexpr uint32_t table_unit_tuples(uint32_t n) {
+  return n / 128 < kTableUnitMin ? kTableUnitMin : n / 128 < kTableUnitMax ? n / 128 : kTableUnitMax;
+}
 // Build tuples up to which a partition fills the table several times although
 // the arena would have room for an HBM table: three times the slots of the 64 or
 // 128 KiB table, up to 6 fills (5 at int64), of 32 KiB tables up to 11 (10).

@@ -211,7 +211,7 @@ fij_status fij_join_plan_create(const fij_join_plan_config* cfg, fij_join_plan**
     p->d.hbm_cap = static_cast<uint32_t>(slots);
     p->d.big_cap = static_cast<uint32_t>(std::min<uint64_t>(items, slots / 256));
     p->d.hbm_unit_cap =
-        static_cast<uint32_t>(2ull * p->d.big_cap + (cfg->build_len + cfg->probe_len) / 65536 + 2);
+        static_cast<uint32_t>(2ull * p->d.big_cap + (cfg->build_len + cfg->probe_len) / kTableUnitMin + 2);
     // (the block counters are cleared with the arena)
     if (st == FIJ_OK) st = alloc(p, &p->done, kDoneWords);
     if (st == FIJ_OK) st = alloc(p, &p->hashed, 1);

@@ -13,6 +13,11 @@ PROGRAM = """
 #include "one_pass_rules.hpp"
 using namespace fij;
 int main(int argc, char** argv) {
+  if (argc == 2) {  // tuples of a partition with an HBM table: units, tuples of a unit, end of the last
+    const uint32_t n = strtoul(argv[1], nullptr, 10), per = table_unit_tuples(n), r = range_count(n, per);
+    printf("%u %u %u\\n", r, per, r ? range_end(n, per, r - 1) : 0u);
+    return 0;
+  }
   if (argc == 5) {  // type, build tuples, partitions, big tables: slots, a fill, build tuples joined in LDS
     const KeyType t = argv[1][0] == '0' ? KeyType::I32 : KeyType::I64;
     const bool big = argv[4][0] == '1';
@@ -86,3 +91,14 @@ def test_tables_and_their_fills(rules, type, fills):
         [(slots, fill, lds)] = rules([(type, build, 512, big)])
         assert slots == half << at + 1 and fill == fills[at]
         assert -(-lds // fill) == most[type]
+
+
+def test_units_of_partitions_with_hbm_tables(rules):
+    """At most as many as a plan has room for (one per 4,096 tuples and one), and
+    at least 32 of a long range: one block probed 65,536 tuples in 0.3 ms."""
+    for n in (1, 4095, 4096, 4097, 128 * 4096 - 1, 128 * 4096 + 127, 240_000, 128 * 65_536, 128 * 65_536 + 1, (1 << 32) - 20_000,
+              (1 << 32) - 1):
+        [(units, per, end)] = rules([(n,)])
+        assert end == n and (units - 1) * per < n <= units * per
+        assert units <= n // 4096 + 1
+        assert units >= min(32, n // 4096)
