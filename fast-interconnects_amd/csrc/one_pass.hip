@@ -38,7 +38,7 @@ constexpr KeyType kKeyType = sizeof(K) == 4 ? KeyType::I32 : KeyType::I64;
 // padded_len1; that block sets the counters.  In batches (which have no HBM
 // arena) the counters were reset by an earlier launch.
 __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, const BatchSide* sides, uint32_t F1j,
-                                                             uint32_t lds_tuples) {
+                                                             uint32_t fill, uint32_t lds_tuples) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t wave_tmp[1024 / kWave + 1];
   __shared__ uint32_t s_base, s_slots, s_big, s_build_units, s_probe_units;
@@ -57,10 +57,11 @@ __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, c
     at = s.off1[vp];
     return static_cast<uint32_t>((p + 1 < F1j ? s.off1[vp + 1] - d.pad : end) - at);
   };
+  const uint64_t mean = d.build.n / d.F1;
   for (uint32_t p = tid; p < F1j; p += blockDim.x) {
     uint64_t at;
     const uint32_t nb = range(d.build, end_b, p, at), np = range(d.probe, end_p, p, at);
-    PartUnits cut = part_units_of(nb, np);
+    PartUnits cut = part_units_of(nb, np, nb / 2 > mean ? fill : ~0u);
     if (cut.units) {
       if (nb > lds_tuples && d.hbm_cap && nb <= (d.hbm_cap >> 1)) {
         // an HBM table of at least twice the build tuples, if the arena (at
@@ -398,6 +399,7 @@ hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchS
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(one_pass_plan_kernel, dim3(joins), dim3(1024), 3 * F1j * 4, stream, d, sides, F1j,
+                     block_table_fill(t, one_pass_slots(t, d.build.n, d.F1, d.big_block_tables != 0)),
                      one_pass_lds_tuples(t, d.big_block_tables != 0));
   return hipGetLastError();
 }

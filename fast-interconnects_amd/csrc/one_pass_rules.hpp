@@ -27,13 +27,18 @@ constexpr uint64_t part_unit_cap(uint64_t partitions, uint64_t probe_len) {
 // Units of a partition pair, each of `per` probe tuples but for the last:
 // about 16 times the build tuples (a unit's build work is paid once per unit:
 // 20 batched joins of 2^18..2^20 int32 build tuples took 349 us with 8 times,
-// 283 us with 16), evenly.
+// 283 us with 16), evenly.  A unit streams them once per fill of the table, of
+// `fill` build tuples: those of a partition that stands out by more than two
+// fills are shorter, as the others will be done before them (one of 64
+// partitions of 10,000 int32 tuples, in 32 KiB tables: 490 -> 260 us; where all
+// partitions are of four fills more units only build more, 282 -> 328 us).
 struct PartUnits {
   uint32_t units, per;
 };
-__host__ __device__ constexpr PartUnits part_units_of(uint32_t build_n, uint32_t probe_n) {
+__host__ __device__ constexpr PartUnits part_units_of(uint32_t build_n, uint32_t probe_n, uint32_t fill = ~0u) {
   if (build_n == 0 || probe_n == 0) return {0, kPartUnitMin};
-  const uint32_t want = build_n < kPartUnitMax / 16 ? 16 * build_n : kPartUnitMax;
+  const uint32_t fills = range_count(build_n, fill), most = fills > 2 ? 2 * kPartUnitMax / fills : kPartUnitMax;
+  const uint32_t want = build_n < most / 16 ? 16 * build_n : most;
   const uint32_t units = range_count(probe_n, want < kPartUnitMin ? kPartUnitMin : want);
   return {units, range_count(probe_n, units)};
 }
@@ -75,9 +80,9 @@ __host__ __device__ constexpr uint32_t table_unit_tuples(uint32_t n) {
 // 128 KiB table, up to 6 fills (5 at int64), of 32 KiB tables up to 11 (10).
 // Each fill streams the probe tuples again, an HBM table costs a random access
 // per probe tuple and a chain per repeated key.  Among 64 partitions one of
-// 10,000 int32 tuples, in 32 KiB tables: 490 to 540 us in LDS, 510 to 575 us in
-// HBM, of 20,000 910 to 980 and 340 to 400 us; of 14,000 with 500 copies of
-// every key 0.3 and 55 ms.
+// 10,000 int32 tuples, in 32 KiB tables: 260 us in LDS, 145 to 255 us in HBM, of
+// 20,000 306 and 130 to 205 us; of 14,000 with 500 copies of every key 0.2 and 7
+// ms.  In larger tables LDS wins up to there.
 constexpr uint32_t one_pass_lds_tuples(KeyType t, bool big) { return 3 * block_table_slots(t) * (big ? 2 : 1); }
 
 // Single-pass plans (fij_join_plan_bits, single-pass batched classes): 9

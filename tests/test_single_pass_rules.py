@@ -18,6 +18,12 @@ int main(int argc, char** argv) {
     printf("%u %u %u\\n", r, per, r ? range_end(n, per, r - 1) : 0u);
     return 0;
   }
+  if (argc == 6) {  // tuples of a fill, build and probe tuples: units, tuples of a unit
+    const uint32_t fill = strtoul(argv[1], nullptr, 10);
+    const PartUnits u = part_units_of(strtoul(argv[2], nullptr, 10), strtoul(argv[3], nullptr, 10), fill);
+    printf("%u %u\\n", u.units, u.per);
+    return 0;
+  }
   if (argc == 5) {  // type, build tuples, partitions, big tables: slots, a fill, build tuples joined in LDS
     const KeyType t = argv[1][0] == '0' ? KeyType::I32 : KeyType::I64;
     const bool big = argv[4][0] == '1';
@@ -102,3 +108,15 @@ def test_units_of_partitions_with_hbm_tables(rules):
         assert end == n and (units - 1) * per < n <= units * per
         assert units <= n // 4096 + 1
         assert units >= min(32, n // 4096)
+
+
+def test_units_of_partitions_of_many_fills_are_shorter(rules):
+    """... down to 8,192 probe tuples; those of one or two fills are not."""
+    for fill in (1280, 9216):
+        for fills in (1, 2, 3, 5, 11, 400):
+            nb = fill * fills
+            for np_ in (1, 8193, 240_000, 1 << 24, (1 << 32) - 20_000):
+                [(units, per)] = rules([(fill, nb, np_, "", "")])
+                longest = max(8192, min(16 * nb, 65_536 if fills <= 2 else 131_072 // fills))
+                assert longest // 2 < per <= longest or np_ <= longest
+                assert (units - 1) * per < np_ <= units * per and units <= np_ // 8192 + 1
