@@ -32,9 +32,9 @@ __device__ __forceinline__ void hbm_insert(Tuple<K>* tab, uint32_t lg, K key, K 
 }
 
 // Every build tuple with this key matches; probing ends at the first free
-// slot.  (The i64 payload of a slot whose key was just installed may still
-// be in flight only while the build kernel runs; probes run in a later
-// launch.)
+// slot.  (The i64 payload of a slot whose key was just installed may still be
+// in flight while tables are built: probes run in a later launch, or behind the
+// wait for all build units.)
 template <typename K>
 __device__ __forceinline__ void hbm_probe(const Tuple<K>* tab, uint32_t lg, K key, K pay, uint64_t& cnt, uint64_t& sb,
                                           uint64_t& sp) {

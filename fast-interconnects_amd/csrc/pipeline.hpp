@@ -185,8 +185,9 @@ uint32_t pass1_chunks(KeyType t, uint64_t n, uint32_t most);
 // that every block has the same work and no launch waits for the tail of
 // another.  With one block per compute unit for each side in turn, the
 // histogram, scan and scatter of 2^20 + 2^24 int32 tuples at 9 bits took 26 +
-// 22 + 77 us, in one launch each 21 + 6 + 65 us; 2^27 + 2^27 int64 tuples 343 +
-// 22 + 1760 us and 330 + 6 + 1390 us (half as many pieces per partition).
+// 22 + 77 us, in one launch each 20 + 6 + 74 us; 2^27 + 2^27 int64 tuples 343 +
+// 22 + 1,760 us and 331 + 5 + 1,735 us (the scatter's time differs by more than
+// that from process to process).
 void split_chunks(KeyType t, uint64_t n_b, uint64_t n_p, uint32_t total, uint32_t* g_b, uint32_t* g_p);
 
 uint32_t pipeline_tile2(KeyType t);

@@ -336,7 +336,10 @@ fij_status fij_np_probe_sum(fij_type type, fij_hashing_scheme scheme, const void
  * passes: none where one block's LDS table holds it (12,288 int32 or 6,144
  * int64 tuples), one of 9 bits instead of two where its partitions then make at
  * most two table fills (up to 4.57 M tuples; 7.08 M int32 or 5.08 M int64 for
- * probe sides of at most 32 or 16 times the build side). */
+ * probe sides of at most 32 or 16 times the build side, of at most 2^32 less
+ * 16,386 (int64: 8,194) tuples).  Partitions of such joins are the library's
+ * own: if the build keys leave most radix digits of the pass unused (multiples
+ * of a power of two), it partitions by a hash of the key instead. */
 
 typedef struct fij_join_plan fij_join_plan;
 
@@ -408,11 +411,11 @@ fij_status fij_join_plan_execute(fij_join_plan *plan, const void *build_keys, co
  * whose build side fits one block's LDS table are joined together by one
  * persistent launch without partitioning.  Every other join is partitioned, in
  * one pass of 5, 7 or 9 bits by its build side up to two table fills per
- * partition (as a plan's join), else in two passes with the radix bits of its
- * size class (fij_join_autotune; also where fij_join_tuning_set has given the
- * class an entry),
- * all joins of a class together: one launch per pass (histograms, offsets,
- * scatter, pass 2, join) covers every join of the class.  The submission is
+ * partition (as a plan's join, by radix or hash), else in two passes with the
+ * radix bits of its size class (fij_join_autotune; also where
+ * fij_join_tuning_set has given the class an entry), all joins of a class
+ * together: one launch per pass (histograms, offsets, scatter, pass 2, join)
+ * covers every join of the class.  The submission is
  * recorded into one HIP graph when use_graph is set.  The size classes are
  * independent and are spread over `lanes` streams (forked from the
  * submission stream and joined back into it), so classes that do not fill
