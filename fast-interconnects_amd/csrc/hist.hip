@@ -57,42 +57,48 @@ __device__ void finish_histogram(uint32_t* hist, uint64_t* wave_tmp, uint32_t F,
 enum class HistCopy { None, Keys, Columns };
 
 // Whether a single-pass join's digits are hashed: if its build keys leave many
-// radix partitions empty.  Every block takes the same kSampleKeys keys, one from
-// each of as many equal parts of the column, and counts the digits among them:
-// of random keys F * (1 - e^(-kSampleKeys / F)), with a deviation of 5 at 512;
-// below nine tenths of that the digits are hashed.  Chunk 0 leaves the decision
-// for the launches behind.  (sample_n = 0: it has been made.)
+// radix partitions empty.  The first wave of every block takes the same
+// kSampleKeys keys, one from each of as many equal parts of the column, and
+// counts the digits among them: of random keys F * (1 - e^(-kSampleKeys / F)),
+// with a deviation of 3.3 at 512 and of 3.5 at 128; below 87 % of that the digits
+// are hashed.  Chunk 0 leaves the decision for the launches behind.  (sample_n =
+// 0: it has been made.)
 //
-// The keys are loaded with the block's first keys and counted behind the barrier
-// that its counters need anyway: 12.8 us instead of 12.4 for 65,539 x 1,000,003
-// int64 tuples (with 512 keys 13.0, with a look of its own before them 14.0).
+// The keys are loaded with the block's first keys and counted before the barrier
+// that its counters need anyway: 12.2 us instead of 11.9 for 65,539 x 1,000,003
+// int64 tuples (256 keys counted behind the barrier 12.3, 512 keys 12.6, a look of
+// its own before the first loads 13.6).
 template <typename K>
 struct SampledDigits {
   const HistParams& p;
-  uint32_t* seen;  // [16] LDS, 16-byte aligned
-  K key;           // sample threadIdx.x
-  __device__ __forceinline__ SampledDigits(const HistParams& params, uint32_t* lds) : p(params), seen(lds), key(0) {
-    if (threadIdx.x < p.sample_n) key = load(threadIdx.x);
-    if (threadIdx.x < 16) seen[threadIdx.x] = 0;
-  }
-  __device__ __forceinline__ K load(uint32_t i) const {
-    const uint32_t jitter = __umulhi(i * 2654435769u, p.sample_part);
-    return as_global(static_cast<const K*>(p.sample))[static_cast<uint64_t>(i) * p.sample_part + jitter];
-  }
-  // Behind a barrier; ends with one.
-  __device__ __forceinline__ bool hashed(uint32_t c) {
-    if (p.sample_n == 0) return scalar_load(p.hashed) != 0;
-    for (uint32_t i = threadIdx.x; i < p.sample_n; i += blockDim.x) {
-      const uint32_t d = static_cast<uint32_t>(i == threadIdx.x ? key : load(i)) & ((1u << p.radix_bits) - 1u);
-      atomicOr(&seen[d / 32], 1u << (d % 32));
+  uint32_t* lds;  // [16 + 1]: the digits seen, the decision
+  K key[2];       // samples threadIdx.x and threadIdx.x + kWave
+  __device__ __forceinline__ SampledDigits(const HistParams& params, uint32_t* seen) : p(params), lds(seen), key{} {
+    if (threadIdx.x >= kWave) return;
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+      const uint32_t i = k * kWave + threadIdx.x, jitter = __umulhi(i * 2654435769u, p.sample_part);
+      if (i < p.sample_n) key[k] = as_global(static_cast<const K*>(p.sample))[static_cast<uint64_t>(i) * p.sample_part + jitter];
     }
-    __syncthreads();
-    uint32_t digits = 0;
-    for (uint32_t i = 0; i < 16; ++i) digits += __popc(seen[i]);
-    const bool few = __builtin_amdgcn_readfirstlane(digits) < p.sample_digits;
-    if (c == 0 && threadIdx.x == 0) *p.hashed = few ? 1u : 0u;
-    return few;
+    if (threadIdx.x < 16) lds[threadIdx.x] = 0;
   }
+  // In the first wave; the others read the decision behind a barrier.
+  __device__ __forceinline__ void decide(uint32_t c) {
+    if (threadIdx.x >= kWave) return;
+    uint32_t digits = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+      const uint32_t d = static_cast<uint32_t>(key[k]) & ((1u << p.radix_bits) - 1u), bit = 1u << (d % 32);
+      const bool fresh = k * kWave + threadIdx.x < p.sample_n && (atomicOr(&lds[d / 32], bit) & bit) == 0;
+      digits += static_cast<uint32_t>(__popcll(__ballot(fresh)));
+    }
+    const uint32_t few = p.sample_n == 0 ? scalar_load(p.hashed) : digits < p.sample_digits ? 1u : 0u;
+    if (threadIdx.x == 0) {
+      lds[16] = few;
+      if (c == 0 && p.sample_n) *p.hashed = few;
+    }
+  }
+  __device__ __forceinline__ bool hashed() const { return __builtin_amdgcn_readfirstlane(lds[16]) != 0; }
 };
 
 // Histogram of chunk c of G (one block).
@@ -138,11 +144,12 @@ __device__ __forceinline__ void hist_body(const HistParams& p, uint32_t c, uint3
   VT xa[U], xb[U];
   bool hashed = false;
   if constexpr (ADAPTIVE) {
-    __shared__ __attribute__((aligned(16))) uint32_t seen[16];
+    __shared__ uint32_t seen[17];
     SampledDigits<K> sample(p, seen);
     if (nv) load(xa, 0);
+    sample.decide(c);
     __syncthreads();
-    hashed = sample.hashed(c);
+    hashed = sample.hashed();
   } else {
     if (nv) load(xa, 0);
     __syncthreads();
@@ -565,7 +572,7 @@ void sample_build_keys(HistParams& p, const void* keys, uint64_t n, uint32_t* ha
   p.sample = keys;
   p.sample_n = static_cast<uint32_t>(s);
   p.sample_part = static_cast<uint32_t>(n / std::max<uint64_t>(1, p.sample_n));
-  p.sample_digits = static_cast<uint32_t>(0.9 * F * (1.0 - std::exp(-s / F)) + 0.999);
+  p.sample_digits = static_cast<uint32_t>(0.87 * F * (1.0 - std::exp(-s / F)) + 0.999);
   p.hashed = hashed;
 }
 

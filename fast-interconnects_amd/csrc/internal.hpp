@@ -110,7 +110,7 @@ struct HistParams {
   uint32_t sample_n, sample_part, sample_digits, reserved;
   uint32_t* hashed;
 };
-constexpr uint32_t kSampleKeys = 256;
+constexpr uint32_t kSampleKeys = 128;
 
 // Contiguous histogram parameters of one relation of a paired or batched
 // launch, in chunks of balanced_chunk_len; scan_state (scan_state_words(2^radix_bits) words) is cleared by it.

@@ -38,7 +38,8 @@ constexpr KeyType kKeyType = sizeof(K) == 4 ? KeyType::I32 : KeyType::I64;
 // padded_len1; that block sets the counters.  In batches (which have no HBM
 // arena) the counters were reset by an earlier launch.
 __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, const BatchSide* sides, uint32_t F1j,
-                                                             uint32_t fill, uint32_t lds_tuples) {
+                                                             uint32_t fill, uint32_t long_tuples,
+                                                             uint32_t lds_tuples) {
   extern __shared__ uint32_t lds[];
   __shared__ uint32_t wave_tmp[1024 / kWave + 1];
   __shared__ uint32_t s_base, s_slots, s_big, s_build_units, s_probe_units;
@@ -57,11 +58,10 @@ __global__ __launch_bounds__(1024) void one_pass_plan_kernel(PipelineDevice d, c
     at = s.off1[vp];
     return static_cast<uint32_t>((p + 1 < F1j ? s.off1[vp + 1] - d.pad : end) - at);
   };
-  const uint64_t mean = d.build.n / d.F1;
   for (uint32_t p = tid; p < F1j; p += blockDim.x) {
     uint64_t at;
     const uint32_t nb = range(d.build, end_b, p, at), np = range(d.probe, end_p, p, at);
-    PartUnits cut = part_units_of(nb, np, nb / 2 > mean ? fill : ~0u);
+    PartUnits cut = part_units_of(nb, np, nb > long_tuples ? fill : ~0u);
     if (cut.units) {
       if (nb > lds_tuples && d.hbm_cap && nb <= (d.hbm_cap >> 1)) {
         // an HBM table of at least twice the build tuples, if the arena (at
@@ -249,6 +249,7 @@ __global__ __launch_bounds__(BLOCK, CAP * 2 * sizeof(K) <= 32768 ? 6 : 4) void p
   stamp_phase(d.stamps, 3);
   const uint32_t n_units = uniform_load(d.work_counter + kUnitCount);
   uint32_t job = 0;
+  bool hashed = d.hashed && uniform_load(d.hashed) != 0;  // the digits of the job's partitions
   for (uint32_t u = blockIdx.x; u < n_units;) {
     uint32_t ticket = 0;
     if (tid == 0) ticket = atomicAdd(d.work_counter + kBlockTicket, 1u);
@@ -256,6 +257,7 @@ __global__ __launch_bounds__(BLOCK, CAP * 2 * sizeof(K) <= 32768 ? 6 : 4) void p
     if (d.job_results && (unit.part >> d.job_shift) != job) {
       add_result<BLOCK>(d, red, job, cnt, sb, sp);
       job = unit.part >> d.job_shift;
+      hashed = uniform_load(d.hashed + job) != 0;
     }
     const uint32_t nb = unit.build_n;
     // a range as aligned 16-byte vectors: the first one may begin a tuple
@@ -271,7 +273,6 @@ __global__ __launch_bounds__(BLOCK, CAP * 2 * sizeof(K) <= 32768 ? 6 : 4) void p
       for (uint32_t k = 0; k < NV; ++k) x[k] = __builtin_nontemporal_load(vp + min(v0 + k * BLOCK + tid, nvp - 1));
     };
     const uint32_t digit = unit.part & ((1u << d.bits1) - 1u);
-    const bool hashed = d.hashed && uniform_load(d.hashed + (d.job_results ? unit.part >> d.job_shift : 0u)) != 0;
     const uint32_t other = hashed ? (digit ^ 1u) << (32u - d.bits1) : digit ^ 1u;
     const K free_key = static_cast<K>(hashed ? other * kDigitMulInverse : other);
     const K no_key = static_cast<K>(hashed ? (other + 1u) * kDigitMulInverse : other | (1u << d.bits1));
@@ -400,6 +401,7 @@ hipError_t launch_one_pass_plan(const PipelineDevice& d, KeyType t, const BatchS
   }
   hipLaunchKernelGGL(one_pass_plan_kernel, dim3(joins), dim3(1024), 3 * F1j * 4, stream, d, sides, F1j,
                      block_table_fill(t, one_pass_slots(t, d.build.n, d.F1, d.big_block_tables != 0)),
+                     static_cast<uint32_t>(std::min<uint64_t>(~0u, 2 * (d.build.n / d.F1))),
                      one_pass_lds_tuples(t, d.big_block_tables != 0));
   return hipGetLastError();
 }
